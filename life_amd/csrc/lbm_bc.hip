@@ -6,116 +6,59 @@
 // Compiled with -ffp-contract=off.
 #include <hip/hip_runtime.h>
 
-#include "d2q9_f64.h"
+#include "bc_site.h"
 #include "launch.h"
 
 namespace life {
 
-// GridClass::regularisedBC (Grid.cpp:387-465, Latt et al. 2008) on one
-// site's nine post-stream populations fs, with rho_n/u_n as set by applyBCs.
-// rhoNb1/rhoNb2 are the current densities at site + n and site + 2n, used
-// by the corner extrapolation (Utils.h:150-162).
-template <bool CM>
-__device__ void regularised64(const GridScalars& g, int type, int nx, int ny, int nd, double fs[kNV], double& rn,
-                              double& uxn, double& uyn, double rhoNb1, double rhoNb2) {
-    const bool velocity_like = (type == 1 || type == 2 || type == 3);  // wall, velocity, free-slip
-    const bool corner = (nx != 0 && ny != 0);
-    if (corner) {
-        if (velocity_like) rn = 2.0 * rhoNb1 - rhoNb2;
-    } else {
-        const int nn = nd == 0 ? nx : ny;
-        double fplus = 0.0, fzero = 0.0;
-#pragma unroll
-        for (int v = 0; v < kNV; v++) {
-            const int cn = nd == 0 ? kCX[v] : kCY[v];
-            if (cn == -nn) fplus += fs[v];
-            else if (cn == 0) fzero += fs[v];
-        }
-        if (velocity_like) rn = (2.0 * fplus + fzero) / (1.0 - nn * (nd == 0 ? uxn : uyn));
-        else if (type == 4) {
-            const double un = nn * (1.0 - (2.0 * fplus + fzero) / rn);
-            if (nd == 0) uxn = un;
-            else uyn = un;
-        }
-    }
-    const double rho = rn, ux = uxn, uy = uyn;
-    double Sxx = 0.0, Syy = 0.0, Sxy = 0.0;
-#pragma unroll
-    for (int v = 0; v < kNV; v++) {
-        const double feq = feq64<CM>(rho, ux, uy, v);
-        bool unknown;
-        if (corner) unknown = (kCX[v] == nx || kCY[v] == ny);
-        else unknown = ((nd == 0 ? kCX[v] : kCY[v]) == (nd == 0 ? nx : ny));
-        if (unknown) {
-            if (corner && nx * kCX[v] + ny * kCY[v] == 0) fs[v] = feq;
-            else fs[v] = feq + (fs[kOpp[v]] - feq64<CM>(rho, ux, uy, kOpp[v]));
-        }
-        const double fneq = fs[v] - feq;
-        Sxx += kCX[v] * kCX[v] * fneq;
-        Syy += kCY[v] * kCY[v] * fneq;
-        Sxy += kCX[v] * kCY[v] * fneq;
-    }
-#pragma unroll
-    for (int v = 0; v < kNV; v++)
-        fs[v] = feq64<CM>(rho, ux, uy, v) +
-                (w64(v) / (2.0 * g.cs4)) * (((kCX[v] * kCX[v] - g.cs2) * Sxx) + ((kCY[v] * kCY[v] - g.cs2) * Syy) +
-                                            (2.0 * kCX[v] * kCY[v] * Sxy));
-}
+// GridClass::applyBCs + regularisedBC / convectiveBC (Grid.cpp:302-474) on
+// the populations just streamed into dst, nine lanes per boundary site
+// (bc_site.h).  rho_n/u_n start as the site's end-of-previous-step moments
+// (the reference swaps its rho/u arrays at the start of the step,
+// Grid.cpp:43-45).
+//
+// The launch is bound by one chain of memory latency (site table,
+// populations) and arithmetic: one wavefront per workgroup and seven sites
+// per wavefront put the sites of even a small lattice on many CUs.
+// Measured against one lane per site in 256-lane workgroups: 256 x 256 FP32
+// BGK 10.5 -> 4.3 us, 1024 x 256 FP32 central moments 11.5 -> 5.2 us.
+constexpr int kBCBlock = 64;
 
-// One thread per boundary site: GridClass::applyBCs + regularisedBC /
-// convectiveBC (Grid.cpp:302-474) on the populations just streamed into
-// dst.  rho_n/u_n start as the site's end-of-previous-step moments (the
-// reference swaps its rho/u arrays at the start of the step, Grid.cpp:43-45).
 template <typename T, bool CM>
-__device__ inline void bc_site(const T* __restrict__ src, T* __restrict__ dst, const GridScalars& g, const BCArgs& a,
-                               const double* __restrict__ fibm, const double* __restrict__ rho0,
-                               const double* __restrict__ u0, int explicit_state, int k) {
-    if (k >= a.nbc) return;
+__device__ __forceinline__ void bc_wave(const T* __restrict__ src, T* __restrict__ dst, const GridScalars& g,
+                                        const BCArgs& a, const double* __restrict__ fibm,
+                                        const double* __restrict__ rho0, const double* __restrict__ u0,
+                                        int explicit_state, int block, double* share) {
+    const int slot = (int)threadIdx.x / kBCLanes, v = (int)threadIdx.x - slot * kBCLanes;
+    const int k = block * kBCPerWave + slot;
+    if (slot >= kBCPerWave || k >= a.nbc) return;
     const BCSite b = a.sites[k];
     const long long S = g.S, id = b.id;
     const int Ny = g.Ny, j = b.j;
     if (b.type == 5) {  // convective: f[2,6,8] = f_n + 3 w (delU . c)
-        const double dux = a.delU[2 * j], duy = a.delU[2 * j + 1];
-        const int vs[3] = {2, 6, 8};
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-            const int v = vs[q];
-            Pops<T>::put(dst, S, v, id, Pops<T>::get(src, S, v, id) + 3.0 * w64(v) * (dux * kCX[v] + duy * kCY[v]));
-        }
+        if (v == 2 || v == 6 || v == 8)
+            Pops<T>::put(dst, S, v, id, bc_convective(v, Pops<T>::get(src, S, v, id), a.delU[2 * j], a.delU[2 * j + 1]));
         return;
     }
     if (b.type == 0) return;
-    // the populations regularisedBC rebuilds from the others (the ones that
-    // entered from outside the domain) are never read, so only the known
-    // ones are loaded: six of nine on an edge
     const bool corner = b.nx != 0 && b.ny != 0;
-    // Every load the site needs is issued before the arithmetic (one round
-    // trip to memory, not up to three): its known populations, the two
-    // inward neighbours' populations (the zero gradient of free-slip and
-    // pressure sites, the density extrapolation of corners) and, at a
-    // pressure corner, its previous populations.
-    const bool nbr = b.type == 3 || b.type == 4 || corner;
+    // Every load the site needs is issued before the arithmetic: its
+    // populations, the two inward neighbours' and, at a pressure corner, its
+    // previous populations.
+    const bool nbr = bc_reads_neighbours(b.type, b.nx, b.ny);
     const bool prev = b.type == 4 && corner && !explicit_state;
     const long long id1 = (long long)(b.i + b.nx) * Ny + (j + b.ny);
     const long long id2 = (long long)(b.i + 2 * b.nx) * Ny + (j + 2 * b.ny);
     double fs[kNV], f1[kNV], f2[kNV], fp[kNV];
-#pragma unroll
-    for (int v = 0; v < kNV; v++) {
-        const bool unknown = corner ? (kCX[v] == b.nx || kCY[v] == b.ny)
-                                    : ((b.nd == 0 ? kCX[v] : kCY[v]) == (b.nd == 0 ? b.nx : b.ny));
-        fs[v] = unknown ? 0.0 : Pops<T>::get(dst, S, v, id);
-    }
+    load_site(dst, S, id, fs);
     if (nbr) {
         load_site(dst, S, id1, f1);
         load_site(dst, S, id2, f2);
     }
     if (prev) load_site(src, S, id, fp);
+    const double uwx = a.u_in[2 * j] * a.ramp, uwy = a.u_in[2 * j + 1] * a.ramp, rin = a.rho_in[j];
     // rho_n/u_n of the previous step outlive applyBCs + regularisedBC only
-    // at a pressure corner: everywhere else all three are overwritten below
-    // (wall/velocity set u, free-slip and pressure take u from the normal
-    // condition and the zero gradient, rho comes from the post-stream
-    // populations, the corner extrapolation or rho_in).  The previous
-    // populations, nine scattered loads per site, are read only there.
+    // at a pressure corner
     double rn = 0.0, uxn = 0.0, uyn = 0.0;
     if (b.type == 4 && corner) {
         if (explicit_state) {
@@ -127,66 +70,41 @@ __device__ inline void bc_site(const T* __restrict__ src, T* __restrict__ dst, c
                       rn, uxn, uyn);
         }
     }
-    double rho1 = 0.0, rho2 = 0.0;
-    switch (b.type) {
-        case 1:  // wall
-            uxn = 0.0;
-            uyn = 0.0;
-            break;
-        case 2:  // velocity
-            uxn = a.u_in[2 * j] * a.ramp;
-            uyn = a.u_in[2 * j + 1] * a.ramp;
-            break;
-        case 3:    // free slip
-        case 4: {  // pressure
-            if (b.type == 3) {
-                if (b.nd == 0) uxn = 0.0;
-                else uyn = 0.0;
-            } else {
-                rn = a.rho_in[j];
-            }
-            // Utils::zeroGradient order 2 on the current velocity (Utils.h:200-210)
-            double r1, r2, u1x, u1y, u2x, u2y;
-            moments64(f1, g.fcur ? g.fcur[id1] : g.Fx, g.fcur ? g.fcur[S + id1] : g.Fy, r1, u1x, u1y);
-            moments64(f2, g.fcur ? g.fcur[id2] : g.Fx, g.fcur ? g.fcur[S + id2] : g.Fy, r2, u2x, u2y);
-            if (b.nd != 0) uxn = (4.0 / 3.0) * u1x - (1.0 / 3.0) * u2x;
-            if (b.nd != 1) uyn = (4.0 / 3.0) * u1y - (1.0 / 3.0) * u2y;
-            break;
-        }
-        default:
-            break;
+    double F1 = b.nd != 0 ? g.Fx : g.Fy, F2 = F1;
+    if (g.fcur && nbr) {
+        F1 = g.fcur[(b.nd != 0 ? 0 : S) + id1];
+        F2 = g.fcur[(b.nd != 0 ? 0 : S) + id2];
     }
-    if (corner) {
-        rho1 = density64(f1);
-        rho2 = density64(f2);
-    }
-    regularised64<CM>(g, b.type, b.nx, b.ny, b.nd, fs, rn, uxn, uyn, rho1, rho2);
-#pragma unroll
-    for (int v = 0; v < kNV; v++) Pops<T>::put(dst, S, v, id, fs[v]);
+    Pops<T>::put(dst, S, v, id,
+                 bc_value<CM>(g, v, b.type, b.nx, b.ny, b.nd, fs, f1, f2, uwx, uwy, rin, rn, uxn, uyn, F1, F2,
+                              share + slot * kNV));
 }
 
 template <typename T, bool CM>
-__global__ __launch_bounds__(256) void k_bc(const T* __restrict__ src, T* __restrict__ dst, GridScalars g,
-                                            BCArgs a, const double* __restrict__ fibm,
-                                            const double* __restrict__ rho0, const double* __restrict__ u0,
-                                            int explicit_state) {
-    bc_site<T, CM>(src, dst, g, a, fibm, rho0, u0, explicit_state, blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(kBCBlock) void k_bc(const T* __restrict__ src, T* __restrict__ dst, GridScalars g,
+                                                 BCArgs a, const double* __restrict__ fibm,
+                                                 const double* __restrict__ rho0, const double* __restrict__ u0,
+                                                 int explicit_state) {
+    __shared__ double share[kBCPerWave * kNV];
+    bc_wave<T, CM>(src, dst, g, a, fibm, rho0, u0, explicit_state, blockIdx.x, share);
 }
 
 template <typename T, bool CM>
-__global__ __launch_bounds__(256) void k_bc_batch(const CaseDev* __restrict__ cases, const int* __restrict__ list) {
+__global__ __launch_bounds__(kBCBlock) void k_bc_batch(const CaseDev* __restrict__ cases,
+                                                       const int* __restrict__ list) {
+    __shared__ double share[kBCPerWave * kNV];
     const CaseDev& c = cases[list[blockIdx.y]];
-    bc_site<T, CM>(static_cast<const T*>(c.src), static_cast<T*>(c.dst), c.g, c.bc, c.fibm, c.rho0, c.u0,
-                   c.explicit_state, blockIdx.x * blockDim.x + threadIdx.x);
+    bc_wave<T, CM>(static_cast<const T*>(c.src), static_cast<T*>(c.dst), c.g, c.bc, c.fibm, c.rho0, c.u0,
+                   c.explicit_state, blockIdx.x, share);
 }
 
 template <typename T>
 void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, const double* fibm, const double* rho0,
                const double* u0, bool explicit_state, hipStream_t s) {
     if (a.nbc <= 0) return;
-    const unsigned nb = (unsigned)((a.nbc + 255) / 256);
-    if (g.cm) k_bc<T, true><<<nb, 256, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
-    else k_bc<T, false><<<nb, 256, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
+    const unsigned nb = (unsigned)((a.nbc + kBCPerWave - 1) / kBCPerWave);
+    if (g.cm) k_bc<T, true><<<nb, kBCBlock, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
+    else k_bc<T, false><<<nb, kBCBlock, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
 }
 
 // GridClass::convectiveSpeed (Grid.cpp:477-495) on the end-of-previous-step
@@ -299,9 +217,9 @@ void launch_convective_speed(const T* src, const GridScalars& g, const double* f
 template <typename T>
 void launch_bc_batch(bool cm, const CaseDev* cases, const int* list, int n, int max_nbc, hipStream_t s) {
     if (n <= 0 || max_nbc <= 0) return;
-    const dim3 grid((unsigned)((max_nbc + 255) / 256), (unsigned)n);
-    if (cm) k_bc_batch<T, true><<<grid, 256, 0, s>>>(cases, list);
-    else k_bc_batch<T, false><<<grid, 256, 0, s>>>(cases, list);
+    const dim3 grid((unsigned)((max_nbc + kBCPerWave - 1) / kBCPerWave), (unsigned)n);
+    if (cm) k_bc_batch<T, true><<<grid, kBCBlock, 0, s>>>(cases, list);
+    else k_bc_batch<T, false><<<grid, kBCBlock, 0, s>>>(cases, list);
 }
 
 template <typename T>
