@@ -7,6 +7,7 @@
 // on the host; everything on the lattice runs on the device.
 //
 // Compiled with -ffp-contract=off.
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -664,8 +665,21 @@ int life_case_destroy(life_case* c) {
 int life_case_step(life_case* c, int nsteps) {
     return guarded([&] {
         LIFE_HIP(hipSetDevice(c->g->device));
-        for (int s = 0; s < nsteps; s++) {
-            case_step(c, nullptr, nullptr, s + 1 < nsteps, nullptr, nullptr);
+        for (int s = 0; s < nsteps;) {
+            // without bodies, several steps go in one launch, up to the next
+            // step that the blow-up scan reads
+            int k = 0;
+            if (!c->hasIBM && !c->timing->on) {
+                const int every = c->g->check_every;
+                const int to_check = every > 0 ? every - c->t % every : nsteps;
+                k = lbm_multi_step(c->g, c->t + 1, std::min(nsteps - s, to_check));
+                c->t += k;
+            }
+            if (k == 0) {
+                k = 1;
+                case_step(c, nullptr, nullptr, s + 1 < nsteps, nullptr, nullptr);
+            }
+            s += k;
             case_blowup_cadence(c);
         }
         lbm_join(c->g);

@@ -1,7 +1,8 @@
 // FP32-shifted D2Q9 site arithmetic shared by the single-case and batched
 // stream-collide kernels.  Stored value g_v = f_v - w_v (rho0 = 1) in FP32.
-// Include only from translation units compiled with -ffp-contract=fast (the
-// fused multiply-adds are part of the method's rounding).
+// Include only from translation units compiled with
+// -ffp-contract=fast-honor-pragmas (the fused multiply-adds are part of the
+// method's rounding; d2q9_f32_rn.h has the forms that state them).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -165,25 +166,6 @@ LIFE_DF void push32_explicit_site(const float* __restrict__ src, float* __restri
     const float drho = (float)(rho0[id] - 1.0);
     const float ux = (float)u0[2 * id], uy = (float)u0[2 * id + 1];
     const float Fx = (float)(g.Fx + fibm[id]), Fy = (float)(g.Fy + fibm[S + id]);
-    collide32<CM>(g, gs, drho, ux, uy, Fx, Fy, go);
-    push_site32(dst, g, id, go);
-}
-
-// Support site of the last spread: moments and forcing with force_xy +
-// force_ibm (IBMNode.cpp:97-136).
-template <bool CM>
-LIFE_DF void support_push32_site(const float* __restrict__ src, float* __restrict__ dst, const GridScalars& g,
-                                 const double* __restrict__ fibm, long long id) {
-    const long long S = g.S;
-    float gs[kNV], go[kNV];
-#pragma unroll
-    for (int v = 0; v < kNV; v++) gs[v] = src[v * S + id];
-    // moments as stored at the end of the previous step (its force_xy),
-    // forcing of this step
-    const float Fxm = (float)(g.Fxm + fibm[id]), Fym = (float)(g.Fym + fibm[S + id]);
-    const float Fx = (float)(g.Fx + fibm[id]), Fy = (float)(g.Fy + fibm[S + id]);
-    float drho, ux, uy;
-    moments32(gs, Fxm, Fym, drho, ux, uy);
     collide32<CM>(g, gs, drho, ux, uy, Fx, Fy, go);
     push_site32(dst, g, id, go);
 }

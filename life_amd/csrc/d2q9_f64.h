@@ -6,12 +6,17 @@
 // compiled with -ffp-contract=off (no fused multiply-add) and without any
 // fast-math flag.  Integer lattice velocities are kept as int and promoted
 // exactly where the reference promotes them; the compiler only folds
-// value-preserving identities (x*1.0, x*-1.0).
+// value-preserving identities (x*1.0, x*-1.0).  A translation unit that also
+// holds contracted FP32 arithmetic (-ffp-contract=fast-honor-pragmas)
+// includes this header after it: the pragma keeps everything from here to
+// the end of the file uncontracted.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include "life_dev.h"
+
+#pragma clang fp contract(off)
 
 namespace life {
 
@@ -72,17 +77,24 @@ LIFE_DI double density64(const double fs[kNV]) {
     return r;
 }
 
-// BGK collision + Guo forcing (Grid.cpp:236-244).
+// BGK collision + Guo forcing (Grid.cpp:236-244).  FORCE false: the site's
+// force is zero, whose terms (a zero each) are left out.
+template <bool FORCE = true>
 LIFE_DI void collide_bgk64(double omega, const double fs[kNV], double rho, double ux, double uy, double Fx,
                            double Fy, double fo[kNV]) {
     const double c2 = 1.0 - 0.5 * omega;
 #pragma unroll
-    for (int v = 0; v < kNV; v++)
-        fo[v] = fs[v] + omega * (feq64<false>(rho, ux, uy, v) - fs[v]) + c2 * guo64(ux, uy, Fx, Fy, v);
+    for (int v = 0; v < kNV; v++) {
+        fo[v] = fs[v] + omega * (feq64<false>(rho, ux, uy, v) - fs[v]);
+        if (FORCE) fo[v] = fo[v] + c2 * guo64(ux, uy, Fx, Fy, v);
+    }
 }
 
 // Central-moments collision (Grid.cpp:106-223, De Rosis 2019).  The nine
 // back-transformation rows keep the reference's term order and grouping.
+// FORCE false: the site's force is zero, whose terms (k1, k2, k6, k7, a zero
+// each) are left out.
+template <bool FORCE = true>
 LIFE_DI void collide_cm64(double omega, double cs2, double cs4, const double fs[kNV], double rho, double ux,
                           double uy, double Fx, double Fy, double fo[kNV]) {
     double k4p = 0.0, k5p = 0.0;
@@ -98,52 +110,58 @@ LIFE_DI void collide_cm64(double omega, double cs2, double cs4, const double fs[
     const double X = ux, Y = uy, XX = ux * ux, YY = uy * uy;
     const double XXYY = XX * YY, XYY = X * YY, XXY = XX * Y, XY = X * Y;
 
-    fo[0] = (XX * YY - XX - YY + 1.0) * k0 + (2.0 * X * YY - 2.0 * X) * k1 + (2.0 * Y * XX - 2.0 * Y) * k2 +
-            (0.5 * XX + 0.5 * YY - 1.0) * k3 + (0.5 * YY - 0.5 * XX) * k4 + 4.0 * X * Y * k5 + 2.0 * Y * k6 +
-            2.0 * X * k7 + k8;
-    fo[1] = (0.5 * XX - 0.5 * XXYY - 0.5 * XYY + 0.5 * X) * k0 + (X - X * YY - 0.5 * YY + 0.5) * k1 +
-            (-Y * XX - Y * X) * k2 + (-0.25 * XX - 0.25 * X - 0.25 * YY + 0.25) * k3 +
-            (0.25 * XX + 0.25 * X - 0.25 * YY + 0.25) * k4 + (-Y - 2.0 * X * Y) * k5 + (-Y) * k6 +
-            (-X - 0.5) * k7 - 0.5 * k8;
-    fo[2] = (-0.5 * XXYY + 0.5 * XX + 0.5 * XYY - 0.5 * X) * k0 + (X - X * YY + 0.5 * YY - 0.5) * k1 +
-            (-Y * XX + Y * X) * k2 + (-0.25 * XX + 0.25 * X - 0.25 * YY + 0.25) * k3 +
-            (0.25 * XX - 0.25 * X - 0.25 * YY + 0.25) * k4 + (Y - 2.0 * X * Y) * k5 + (-Y) * k6 +
-            (0.5 - X) * k7 - 0.5 * k8;
-    fo[3] = (0.5 * YY - 0.5 * XXY - 0.5 * XXYY + 0.5 * Y) * k0 + (-X * YY - X * Y) * k1 +
-            (Y - XX * Y - 0.5 * XX + 0.5) * k2 + (-0.25 * XX - 0.25 * YY - 0.25 * Y + 0.25) * k3 +
-            (0.25 * XX - 0.25 * YY - 0.25 * Y - 0.25) * k4 + (-X - 2.0 * X * Y) * k5 + (-Y - 0.5) * k6 +
-            (-X) * k7 - 0.5 * k8;
-    fo[4] = (-0.5 * XXYY + 0.5 * XXY + 0.5 * YY - 0.5 * Y) * k0 + (-X * YY + X * Y) * k1 +
-            (Y - XX * Y + 0.5 * XX - 0.5) * k2 + (-0.25 * XX - 0.25 * YY + 0.25 * Y + 0.25) * k3 +
-            (0.25 * XX - 0.25 * YY + 0.25 * Y - 0.25) * k4 + (X - 2.0 * X * Y) * k5 + (0.5 - Y) * k6 +
-            (-X) * k7 - 0.5 * k8;
-    fo[5] = (0.25 * XXYY + 0.25 * XXY + 0.25 * XYY + 0.25 * XY) * k0 +
-            (0.25 * Y + 0.5 * XY + 0.5 * XYY + 0.25 * YY) * k1 + (0.25 * X + 0.5 * XY + 0.5 * XXY + 0.25 * XX) * k2 +
-            (0.125 * XX + 0.125 * X + 0.125 * YY + 0.125 * Y) * k3 +
-            (-0.125 * XX - 0.125 * X + 0.125 * YY + 0.125 * Y) * k4 + (0.5 * X + 0.5 * Y + X * Y + 0.25) * k5 +
-            (0.5 * Y + 0.25) * k6 + (0.5 * X + 0.25) * k7 + 0.25 * k8;
-    fo[6] = (0.25 * XXYY - 0.25 * XXY - 0.25 * XYY + 0.25 * XY) * k0 +
-            (0.25 * Y - 0.5 * XY + 0.5 * XYY - 0.25 * YY) * k1 + (0.25 * X - 0.5 * XY + 0.5 * XXY - 0.25 * XX) * k2 +
-            (0.125 * XX - 0.125 * X + 0.125 * YY - 0.125 * Y) * k3 +
-            (-0.125 * XX + 0.125 * X + 0.125 * YY - 0.125 * Y) * k4 + (X * Y - 0.5 * Y - 0.5 * X + 0.25) * k5 +
-            (0.5 * Y - 0.25) * k6 + (0.5 * X - 0.25) * k7 + 0.25 * k8;
-    fo[7] = (0.25 * XXYY - 0.25 * XXY + 0.25 * XYY - 0.25 * XY) * k0 +
-            (0.5 * XYY - 0.5 * XY - 0.25 * Y + 0.25 * YY) * k1 + (0.5 * XY - 0.25 * X + 0.5 * XXY - 0.25 * XX) * k2 +
-            (0.125 * XX + 0.125 * X + 0.125 * YY - 0.125 * Y) * k3 +
-            (-0.125 * XX - 0.125 * X + 0.125 * YY - 0.125 * Y) * k4 + (0.5 * Y - 0.5 * X + X * Y - 0.25) * k5 +
-            (0.5 * Y - 0.25) * k6 + (0.5 * X + 0.25) * k7 + 0.25 * k8;
-    fo[8] = (0.25 * XXYY + 0.25 * XXY - 0.25 * XYY - 0.25 * XY) * k0 +
-            (0.5 * XY - 0.25 * Y + 0.5 * XYY - 0.25 * YY) * k1 + (0.5 * XXY - 0.5 * XY - 0.25 * X + 0.25 * XX) * k2 +
-            (0.125 * XX - 0.125 * X + 0.125 * YY + 0.125 * Y) * k3 +
-            (-0.125 * XX + 0.125 * X + 0.125 * YY + 0.125 * Y) * k4 + (0.5 * X - 0.5 * Y + X * Y - 0.25) * k5 +
-            (0.5 * Y + 0.25) * k6 + (0.5 * X - 0.25) * k7 + 0.25 * k8;
+    fo[0] = (XX * YY - XX - YY + 1.0) * k0;
+    if (FORCE) fo[0] = fo[0] + (2.0 * X * YY - 2.0 * X) * k1 + (2.0 * Y * XX - 2.0 * Y) * k2;
+    fo[0] = fo[0] + (0.5 * XX + 0.5 * YY - 1.0) * k3 + (0.5 * YY - 0.5 * XX) * k4 + 4.0 * X * Y * k5;
+    if (FORCE) fo[0] = fo[0] + 2.0 * Y * k6 + 2.0 * X * k7;
+    fo[0] = fo[0] + k8;
+    fo[1] = (0.5 * XX - 0.5 * XXYY - 0.5 * XYY + 0.5 * X) * k0;
+    if (FORCE) fo[1] = fo[1] + (X - X * YY - 0.5 * YY + 0.5) * k1 + (-Y * XX - Y * X) * k2;
+    fo[1] = fo[1] + (-0.25 * XX - 0.25 * X - 0.25 * YY + 0.25) * k3 + (0.25 * XX + 0.25 * X - 0.25 * YY + 0.25) * k4 + (-Y - 2.0 * X * Y) * k5;
+    if (FORCE) fo[1] = fo[1] + (-Y) * k6 + (-X - 0.5) * k7;
+    fo[1] = fo[1] - 0.5 * k8;
+    fo[2] = (-0.5 * XXYY + 0.5 * XX + 0.5 * XYY - 0.5 * X) * k0;
+    if (FORCE) fo[2] = fo[2] + (X - X * YY + 0.5 * YY - 0.5) * k1 + (-Y * XX + Y * X) * k2;
+    fo[2] = fo[2] + (-0.25 * XX + 0.25 * X - 0.25 * YY + 0.25) * k3 + (0.25 * XX - 0.25 * X - 0.25 * YY + 0.25) * k4 + (Y - 2.0 * X * Y) * k5;
+    if (FORCE) fo[2] = fo[2] + (-Y) * k6 + (0.5 - X) * k7;
+    fo[2] = fo[2] - 0.5 * k8;
+    fo[3] = (0.5 * YY - 0.5 * XXY - 0.5 * XXYY + 0.5 * Y) * k0;
+    if (FORCE) fo[3] = fo[3] + (-X * YY - X * Y) * k1 + (Y - XX * Y - 0.5 * XX + 0.5) * k2;
+    fo[3] = fo[3] + (-0.25 * XX - 0.25 * YY - 0.25 * Y + 0.25) * k3 + (0.25 * XX - 0.25 * YY - 0.25 * Y - 0.25) * k4 + (-X - 2.0 * X * Y) * k5;
+    if (FORCE) fo[3] = fo[3] + (-Y - 0.5) * k6 + (-X) * k7;
+    fo[3] = fo[3] - 0.5 * k8;
+    fo[4] = (-0.5 * XXYY + 0.5 * XXY + 0.5 * YY - 0.5 * Y) * k0;
+    if (FORCE) fo[4] = fo[4] + (-X * YY + X * Y) * k1 + (Y - XX * Y + 0.5 * XX - 0.5) * k2;
+    fo[4] = fo[4] + (-0.25 * XX - 0.25 * YY + 0.25 * Y + 0.25) * k3 + (0.25 * XX - 0.25 * YY + 0.25 * Y - 0.25) * k4 + (X - 2.0 * X * Y) * k5;
+    if (FORCE) fo[4] = fo[4] + (0.5 - Y) * k6 + (-X) * k7;
+    fo[4] = fo[4] - 0.5 * k8;
+    fo[5] = (0.25 * XXYY + 0.25 * XXY + 0.25 * XYY + 0.25 * XY) * k0;
+    if (FORCE) fo[5] = fo[5] + (0.25 * Y + 0.5 * XY + 0.5 * XYY + 0.25 * YY) * k1 + (0.25 * X + 0.5 * XY + 0.5 * XXY + 0.25 * XX) * k2;
+    fo[5] = fo[5] + (0.125 * XX + 0.125 * X + 0.125 * YY + 0.125 * Y) * k3 + (-0.125 * XX - 0.125 * X + 0.125 * YY + 0.125 * Y) * k4 + (0.5 * X + 0.5 * Y + X * Y + 0.25) * k5;
+    if (FORCE) fo[5] = fo[5] + (0.5 * Y + 0.25) * k6 + (0.5 * X + 0.25) * k7;
+    fo[5] = fo[5] + 0.25 * k8;
+    fo[6] = (0.25 * XXYY - 0.25 * XXY - 0.25 * XYY + 0.25 * XY) * k0;
+    if (FORCE) fo[6] = fo[6] + (0.25 * Y - 0.5 * XY + 0.5 * XYY - 0.25 * YY) * k1 + (0.25 * X - 0.5 * XY + 0.5 * XXY - 0.25 * XX) * k2;
+    fo[6] = fo[6] + (0.125 * XX - 0.125 * X + 0.125 * YY - 0.125 * Y) * k3 + (-0.125 * XX + 0.125 * X + 0.125 * YY - 0.125 * Y) * k4 + (X * Y - 0.5 * Y - 0.5 * X + 0.25) * k5;
+    if (FORCE) fo[6] = fo[6] + (0.5 * Y - 0.25) * k6 + (0.5 * X - 0.25) * k7;
+    fo[6] = fo[6] + 0.25 * k8;
+    fo[7] = (0.25 * XXYY - 0.25 * XXY + 0.25 * XYY - 0.25 * XY) * k0;
+    if (FORCE) fo[7] = fo[7] + (0.5 * XYY - 0.5 * XY - 0.25 * Y + 0.25 * YY) * k1 + (0.5 * XY - 0.25 * X + 0.5 * XXY - 0.25 * XX) * k2;
+    fo[7] = fo[7] + (0.125 * XX + 0.125 * X + 0.125 * YY - 0.125 * Y) * k3 + (-0.125 * XX - 0.125 * X + 0.125 * YY - 0.125 * Y) * k4 + (0.5 * Y - 0.5 * X + X * Y - 0.25) * k5;
+    if (FORCE) fo[7] = fo[7] + (0.5 * Y - 0.25) * k6 + (0.5 * X + 0.25) * k7;
+    fo[7] = fo[7] + 0.25 * k8;
+    fo[8] = (0.25 * XXYY + 0.25 * XXY - 0.25 * XYY - 0.25 * XY) * k0;
+    if (FORCE) fo[8] = fo[8] + (0.5 * XY - 0.25 * Y + 0.5 * XYY - 0.25 * YY) * k1 + (0.5 * XXY - 0.5 * XY - 0.25 * X + 0.25 * XX) * k2;
+    fo[8] = fo[8] + (0.125 * XX - 0.125 * X + 0.125 * YY + 0.125 * Y) * k3 + (-0.125 * XX + 0.125 * X + 0.125 * YY + 0.125 * Y) * k4 + (0.5 * X - 0.5 * Y + X * Y - 0.25) * k5;
+    if (FORCE) fo[8] = fo[8] + (0.5 * Y + 0.25) * k6 + (0.5 * X - 0.25) * k7;
+    fo[8] = fo[8] + 0.25 * k8;
 }
 
-template <bool CM>
+template <bool CM, bool FORCE = true>
 LIFE_DI void collide64(const GridScalars& g, const double fs[kNV], double rho, double ux, double uy, double Fx,
                        double Fy, double fo[kNV]) {
-    if (CM) collide_cm64(g.omega, g.cs2, g.cs4, fs, rho, ux, uy, Fx, Fy, fo);
-    else collide_bgk64(g.omega, fs, rho, ux, uy, Fx, Fy, fo);
+    if (CM) collide_cm64<FORCE>(g.omega, g.cs2, g.cs4, fs, rho, ux, uy, Fx, Fy, fo);
+    else collide_bgk64<FORCE>(g.omega, fs, rho, ux, uy, Fx, Fy, fo);
 }
 
 // 3-point regularised delta (Utils::diracDelta, Utils.h:220-232).
@@ -162,6 +180,7 @@ struct Pops;
 template <>
 struct Pops<double> {
     static LIFE_DI double get(const double* f, long long S, int v, long long id) { return f[v * S + id]; }
+    static LIFE_DI double from(double x, double) { return x; }  // stored value of weight w
     static LIFE_DI void put(double* f, long long S, int v, long long id, double x) { f[v * S + id] = x; }
 };
 
@@ -170,6 +189,7 @@ struct Pops<float> {
     static LIFE_DI double get(const float* f, long long S, int v, long long id) {
         return (double)f[v * S + id] + w64(v);
     }
+    static LIFE_DI double from(float x, double w) { return (double)x + w; }
     static LIFE_DI void put(float* f, long long S, int v, long long id, double x) {
         f[v * S + id] = (float)(x - w64(v));
     }

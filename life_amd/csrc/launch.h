@@ -34,6 +34,33 @@ struct BCArgs {
 template <typename T>
 void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, const double* fibm, const double* rho0,
                const double* u0, bool explicit_state, hipStream_t s);
+// Tiled step (lbm_tile.hip): stream-collide and boundaries of a.steps steps
+// in one launch.  The lattice has no immersed bodies, no convective outlet
+// and no pressure corner, has in each direction boundary conditions on both
+// sides or on neither, and is periodic in i if it is in j; tiles are at
+// least 3 sites wide (CI, CJ >= 5).
+constexpr int kTileMaxSteps = 8;
+constexpr int kTileMaxSites = 1024;  // lanes of a workgroup: tile and rim
+struct TileShape {
+    int CI, CJ;  // largest tile, without its rim
+    int steps;   // steps per launch
+};
+struct TileArgs {
+    int steps;
+    int per_i, per_j;            // periodic in i / j
+    int wall[4];                 // left, right, bottom, top (eLatType)
+    double F[kTileMaxSteps + 1][2];  // force_xy of the step before and of each step
+    double ramp[kTileMaxSteps];  // inlet ramp of each step
+    const double* u_in;
+    const double* rho_in;
+    // set by the launcher
+    int ni, nj;          // tiles; the first ri (rj) of them have qi + 1 (qj + 1) sites, the others qi (qj)
+    int qi, ri, qj, rj;
+    int EJ, PS;      // row and plane strides in LDS
+    unsigned bc_off, share_off;  // byte offsets of the boundary sites and their scratch in LDS
+};
+template <typename T>
+void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, const TileShape& shape, hipStream_t s);
 template <typename T>
 void launch_convective_speed(const T* src, const GridScalars& g, const double* fibm, const double* u0,
                              bool explicit_state, double* ucol, double* delU, bool ordered, hipStream_t s);

@@ -41,43 +41,44 @@ __device__ __forceinline__ void bc_wave(const T* __restrict__ src, T* __restrict
         return;
     }
     if (b.type == 0) return;
-    const bool corner = b.nx != 0 && b.ny != 0;
+    const BCLane l = bc_lane(g, v, b.type, b.nx, b.ny, b.nd);
     // Every load the site needs is issued before the arithmetic: its
     // populations, the two inward neighbours' and, at a pressure corner, its
     // previous populations.
-    const bool nbr = bc_reads_neighbours(b.type, b.nx, b.ny);
-    const bool prev = b.type == 4 && corner && !explicit_state;
     const long long id1 = (long long)(b.i + b.nx) * Ny + (j + b.ny);
     const long long id2 = (long long)(b.i + 2 * b.nx) * Ny + (j + 2 * b.ny);
-    double fs[kNV], f1[kNV], f2[kNV], fp[kNV];
-    load_site(dst, S, id, fs);
-    if (nbr) {
+    const BCPops q = bc_read(l, [&](int u, double w) { return Pops<T>::from(dst[u * S + id], w); });
+    double f1[kNV], f2[kNV], fp[kNV];
+    if (l.nbr) {
         load_site(dst, S, id1, f1);
         load_site(dst, S, id2, f2);
     }
-    if (prev) load_site(src, S, id, fp);
+    const bool pcorner = b.type == 4 && l.corner;
+    if (pcorner && !explicit_state) load_site(src, S, id, fp);
     const double uwx = a.u_in[2 * j] * a.ramp, uwy = a.u_in[2 * j + 1] * a.ramp, rin = a.rho_in[j];
-    // rho_n/u_n of the previous step outlive applyBCs + regularisedBC only
-    // at a pressure corner
-    double rn = 0.0, uxn = 0.0, uyn = 0.0;
-    if (b.type == 4 && corner) {
+    // u_n of the previous step outlives applyBCs + regularisedBC only at a
+    // pressure corner, across its side (nd = 1 there)
+    double pun = 0.0;
+    if (pcorner) {
         if (explicit_state) {
-            rn = rho0[id];
-            uxn = u0[2 * id];
-            uyn = u0[2 * id + 1];
+            pun = u0[2 * id + 1];
         } else {
+            double rn, uxn;
             moments64(fp, (g.fprev ? g.fprev[id] : g.Fxm) + fibm[id], (g.fprev ? g.fprev[S + id] : g.Fym) + fibm[S + id],
-                      rn, uxn, uyn);
+                      rn, uxn, pun);
         }
     }
-    double F1 = b.nd != 0 ? g.Fx : g.Fy, F2 = F1;
-    if (g.fcur && nbr) {
-        F1 = g.fcur[(b.nd != 0 ? 0 : S) + id1];
-        F2 = g.fcur[(b.nd != 0 ? 0 : S) + id2];
+    double r1 = 0.0, u1 = 0.0, r2 = 0.0, u2 = 0.0;
+    if (l.nbr) {
+        double F1 = b.nd != 0 ? g.Fx : g.Fy, F2 = F1;
+        if (g.fcur) {
+            F1 = g.fcur[(b.nd != 0 ? 0 : S) + id1];
+            F2 = g.fcur[(b.nd != 0 ? 0 : S) + id2];
+        }
+        bc_neighbour(f1, b.nd, F1, r1, u1);
+        bc_neighbour(f2, b.nd, F2, r2, u2);
     }
-    Pops<T>::put(dst, S, v, id,
-                 bc_value<CM>(g, v, b.type, b.nx, b.ny, b.nd, fs, f1, f2, uwx, uwy, rin, rn, uxn, uyn, F1, F2,
-                              share + slot * kNV));
+    Pops<T>::put(dst, S, v, id, bc_value<CM>(l, g, q, r1, u1, r2, u2, uwx, uwy, rin, pun, share + slot * kNV));
 }
 
 template <typename T, bool CM>

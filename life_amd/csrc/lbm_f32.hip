@@ -15,7 +15,8 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "d2q9_f32.h"
+#include "d2q9_f32_rn.h"
+#pragma clang fp contract(fast)
 #include "dev_util.h"
 #include "launch.h"
 
@@ -85,14 +86,11 @@ __device__ __forceinline__ void push32_lds_block(SP __restrict__ src, DP __restr
     const long long S = g.S;
     const int Ny = g.Ny;
     const int i = (int)(idc / Ny), j = (int)(idc - (long long)i * Ny);
-    float gs[kNV], go[kNV];
+    float gs[kNV];
 #pragma unroll
     for (int v = 0; v < kNV; v++) gs[v] = valid ? __builtin_nontemporal_load(&src[v * S + idc]) : 0.0f;
-    float drho, ux, uy;
-    const float Fx = (float)g.Fx, Fy = (float)g.Fy;
-    moments32(gs, (float)g.Fxm, (float)g.Fym, drho, ux, uy);
-    collide32<CM>(g, gs, drho, ux, uy, Fx, Fy, go);
-    push_store_realigned<float, NTS, BS>(dst, S, g.Nx, Ny, g.N, base, t, idc, i, j, go, valid, st);
+    step_site32<CM, false>(g, gs, (float)g.Fxm, (float)g.Fym, (float)g.Fx, (float)g.Fy);
+    push_store_realigned<float, NTS, BS>(dst, S, g.Nx, Ny, g.N, base, t, idc, i, j, gs, valid, st);
 }
 
 // Bulk stream-collide with LDS-realigned stores (see push_store_realigned).

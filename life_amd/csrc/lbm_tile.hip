@@ -1,23 +1,24 @@
-// Tiled lattice step: stream-collide, support sites and boundaries of one
-// or several time steps in one launch.
+// Tiled lattice step: stream-collide and boundaries of several time steps in
+// one launch, for a lattice without immersed bodies.
 //
-// The plain step is a bulk push kernel followed by small launches (support
-// sites, boundaries) that wait for each other.  On a lattice of up to about
-// a million sites those small launches, each a few microseconds of launch
-// and dependent memory latency, are most of the step.  Here a workgroup owns
-// a tile of the lattice plus a rim of `steps` sites around it, keeps all
-// nine populations of those sites on the CU, and runs the whole step on
-// them: collide in registers, push through LDS, boundary sites from LDS.
-// The rim is recomputed by every tile that needs it and shrinks by one site
-// per step, so after `steps` steps exactly the tile is valid and is stored;
-// the lattice crosses memory once per launch instead of once per step, and
-// boundaries cost no launch of their own.
+// The plain step is a bulk push kernel and a boundary kernel that wait for
+// each other: two launches of 4-5 us on a small lattice, and one trip of the
+// whole lattice through memory per step on a large one.  Here a workgroup
+// owns a tile plus a rim of `steps` sites around it, keeps the nine
+// populations of each site on the CU and runs whole steps on them: collide
+// in registers, push through LDS, boundary sites from LDS.  The rim is
+// recomputed by every tile that needs it and shrinks by one site per step,
+// so after `steps` steps exactly the tile is valid and is stored: one launch
+// and one trip through memory for `steps` steps.
 //
-// Every site update is the arithmetic of the plain kernels (collide64 /
-// collide32, bc_values), operand for operand, so the values are the same.
+// Every site update is the plain kernels' arithmetic (collide64,
+// step_site32, bc_value), so the values are the same bit for bit.  Bound by
+// the arithmetic of tile and rim and by one step's chain (collide, two
+// barriers, the boundary sites); the tile sizes and their measured times
+// stand at the rule that picks them (tile_shape in runtime.cpp).
 #include <hip/hip_runtime.h>
 
-#include "d2q9_f32.h"
+#include "d2q9_f32_rn.h"
 // (uncontracted from here on, see d2q9_f64.h)
 #include "bc_site.h"
 #include "dev_util.h"
@@ -30,46 +31,37 @@ namespace {
 // Site arithmetic by storage type: moments and collision of one site.
 // Fm: force_xy of the previous step (moments), F: of this step, both with
 // force_ibm where the lattice has immersed bodies.
-template <typename T, bool CM>
+template <typename T, bool CM, bool FORCE>
 struct TileOps;
 
-template <bool CM>
-struct TileOps<double, CM> {
+template <bool CM, bool FORCE>
+struct TileOps<double, CM, FORCE> {
     static __device__ __forceinline__ void step(const GridScalars& g, double f[kNV], double Fxm, double Fym, double Fx,
                                                 double Fy) {
         double rho, ux, uy, fo[kNV];
         moments64(f, Fxm, Fym, rho, ux, uy);
-        collide64<CM>(g, f, rho, ux, uy, Fx, Fy, fo);
+        collide64<CM, FORCE>(g, f, rho, ux, uy, Fx, Fy, fo);
 #pragma unroll
         for (int v = 0; v < kNV; v++) f[v] = fo[v];
     }
 };
 
-template <bool CM>
-struct TileOps<float, CM> {
+template <bool CM, bool FORCE>
+struct TileOps<float, CM, FORCE> {
     static __device__ __forceinline__ void step(const GridScalars& g, float f[kNV], double Fxm, double Fym, double Fx,
                                                 double Fy) {
-        // Scalars opaque to the optimiser: hoisted out of the step loop, they
-        // would leave the compiler other multiply-add pairs to fuse than in
-        // the plain kernels, and the results would differ in the last bit.
-        float om = (float)g.omega, c2 = (float)g.cs2, c4 = (float)g.cs4;
-        float xm = (float)Fxm, ym = (float)Fym, x = (float)Fx, y = (float)Fy;
-        asm volatile("" : "+v"(om), "+v"(c2), "+v"(c4), "+v"(xm), "+v"(ym), "+v"(x), "+v"(y));
-        float drho, ux, uy, fo[kNV];
-        moments32(f, xm, ym, drho, ux, uy);
-        if (CM) collide_cm32(om, c2, c4, f, drho, ux, uy, x, y, fo);
-        else collide_bgk32(om, f, drho, ux, uy, x, y, fo);
-#pragma unroll
-        for (int v = 0; v < kNV; v++) f[v] = fo[v];
+        step_site32<CM, false, FORCE>(g, f, (float)Fxm, (float)Fym, (float)Fx, (float)Fy);
     }
 };
 
-// A boundary site of the tile: where it lies in the tile, and its type and
-// normal (BCSite's, resolved from the walls alone).
+// A boundary site of the tile: where it lies in the tile, its type and
+// normal (BCSite's, resolved from the walls alone) and what its condition
+// reads from memory.
 struct TileBC {
-    int t;       // tile-local index a * EJ + b
-    int i, j;    // lattice coordinates
+    int t;              // tile-local index a * EJ + b
     signed char type, nx, ny, nd;
+    double ux, uy;      // inlet velocity without the ramp
+    double rho_in;
 };
 
 // Site type and normal of (i, j), as site_type and normal_vector of the
@@ -98,8 +90,6 @@ __device__ __forceinline__ bool tile_bc(const TileArgs& a, int Nx, int Ny, int i
             nx = 0;
         }
     }
-    b.i = i;
-    b.j = j;
     b.type = (signed char)type;
     b.nx = (signed char)nx;
     b.ny = (signed char)ny;
@@ -107,19 +97,9 @@ __device__ __forceinline__ bool tile_bc(const TileArgs& a, int Nx, int Ny, int i
     return true;
 }
 
-// Value of population v at tile-local index t, in FP64 (Pops<T>::get on the
-// tile's LDS planes).
-template <typename T>
-__device__ __forceinline__ void lds_site(const T* P, int PS, int t, double f[kNV]) {
-#pragma unroll
-    for (int v = 0; v < kNV; v++) f[v] = Pops<T>::get(P, PS, v, t);
-}
-
-// One tile of CI x CJ sites (at most) and its rim, one site per lane.  SUP:
-// the lattice has immersed bodies, so force_ibm is added to every site's
-// force (it is zero away from the supports of the last spread, which gives
-// the plain kernels' values there); one step per launch then.
-template <typename T, bool CM, bool SUP>
+// One tile of CI x CJ sites (at most) and its rim, one site per lane.  FORCE
+// false: no force in these steps.
+template <typename T, bool CM, bool FORCE>
 __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict__ src, T* __restrict__ dst,
                                                              GridScalars g, TileArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
@@ -130,8 +110,8 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
     // the tile: rows [i0, i1) and columns [j0, j1), dealt out evenly
     const unsigned tile = xcd_block(blockIdx.x, gridDim.x);
     const int ti = (int)(tile / (unsigned)a.nj), tj = (int)(tile - (unsigned)ti * (unsigned)a.nj);
-    const int i0 = (int)((long long)ti * Nx / a.ni), i1 = (int)((long long)(ti + 1) * Nx / a.ni);
-    const int j0 = (int)((long long)tj * Ny / a.nj), j1 = (int)((long long)(tj + 1) * Ny / a.nj);
+    const int i0 = ti * a.qi + min(ti, a.ri), i1 = i0 + a.qi + (ti < a.ri ? 1 : 0);
+    const int j0 = tj * a.qj + min(tj, a.rj), j1 = j0 + a.qj + (tj < a.rj ? 1 : 0);
     // with its rim; a side of the lattice with boundary conditions ends it
     const int li = a.per_i ? i0 - n : (i0 - n > 0 ? i0 - n : 0), hi = a.per_i ? i1 + n : (i1 + n < Nx ? i1 + n : Nx);
     const int lj = a.per_j ? j0 - n : (j0 - n > 0 ? j0 - n : 0), hj = a.per_j ? j1 + n : (j1 + n < Ny ? j1 + n : Ny);
@@ -147,61 +127,46 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
     if (a.per_i) i = ((i % Nx) + Nx) % Nx;
     if (a.per_j) j = ((j % Ny) + Ny) % Ny;
     const long long id = act ? (long long)i * Ny + j : 0;
+    const int tl = act ? t : 0;
     T f[kNV];
 #pragma unroll
     for (int v = 0; v < kNV; v++) f[v] = src[v * S + id];
-    double Bx = 0.0, By = 0.0;
-    if (SUP) {
-        Bx = a.fibm[id];
-        By = a.fibm[S + id];
-    }
     if (t == 0) s_nbc = 0;
     __syncthreads();
     {
+        // The boundary sites are gathered: in place, each wavefront of a
+        // tile along a wall would run the boundary arithmetic for its few
+        // sites.
         TileBC b;
         if (act && tile_bc(a, Nx, Ny, i, j, b)) {
             b.t = t;
+            b.ux = a.u_in[2 * j];
+            b.uy = a.u_in[2 * j + 1];
+            b.rho_in = a.rho_in[j];
             bcs[atomicAdd(&s_nbc, 1)] = b;
         }
     }
     __syncthreads();
-    // The boundary sites are gathered so that the first lanes take one each
-    // (their FP64 arithmetic is several times a site's collision: in place,
-    // every wavefront of a tile along a wall would pay for it).
+    // nine lanes per boundary site, seven sites per wavefront (bc_site.h);
+    // the launch has wavefronts enough for all of them
     const int nbc = s_nbc;
-    TileBC b{};
-    double uwx = 0.0, uwy = 0.0, rin = 1.0;
-    const bool bcl = t < nbc;
+    const int wave = t / 64, slot = t % 64 / kBCLanes, bv = t % 64 - slot * kBCLanes;
+    const int bk = wave * kBCPerWave + slot;
+    const bool bcl = slot < kBCPerWave && bk < nbc;
+    double* share = reinterpret_cast<double*>(tile_lds + a.share_off) + bk * kNV;
+    // site and lane in one word: what the boundary arithmetic derives from it
+    // is formed again in each step, since held over the collision it would
+    // cost the registers that let two workgroups share a CU
+    unsigned bword = 0;
     if (bcl) {
-        b = bcs[t];
-        uwx = a.u_in[2 * b.j];
-        uwy = a.u_in[2 * b.j + 1];
-        rin = a.rho_in[b.j];
-    }
-    double dux = 0.0, duy = 0.0, fo2 = 0.0, fo6 = 0.0, fo8 = 0.0;
-    double rn = 0.0, uxn = 0.0, uyn = 0.0;
-    if (bcl && b.type == 5) {
-        // convective outlet (one step per launch): its old populations and
-        // the extrapolated velocity change
-        const long long bid = (long long)b.i * Ny + b.j;
-        dux = a.delU[2 * b.j];
-        duy = a.delU[2 * b.j + 1];
-        fo2 = Pops<T>::get(src, S, 2, bid);
-        fo6 = Pops<T>::get(src, S, 6, bid);
-        fo8 = Pops<T>::get(src, S, 8, bid);
-    }
-    if (bcl && b.type == 4 && b.nx != 0 && b.ny != 0) {
-        // pressure corner (one step per launch): its previous moments
-        const long long bid = (long long)b.i * Ny + b.j;
-        double fp[kNV];
-        load_site(src, S, bid, fp);
-        moments64(fp, a.F[0][0] + a.fibm[bid], a.F[0][1] + a.fibm[S + bid], rn, uxn, uyn);
+        const TileBC& b = bcs[bk];
+        bword = (unsigned)b.t | (unsigned)bv << 12 | (unsigned)b.type << 16 | (unsigned)(b.nx + 1) << 20 |
+                (unsigned)(b.ny + 1) << 22 | (unsigned)b.nd << 24;
     }
     for (int s = 0; s < n; s++) {
         const double Fxm = a.F[s][0], Fym = a.F[s][1], Fx = a.F[s + 1][0], Fy = a.F[s + 1][1];
         if (act) {
-            if (SUP) TileOps<T, CM>::step(g, f, Fxm + Bx, Fym + By, Fx + Bx, Fy + By);
-            else TileOps<T, CM>::step(g, f, Fxm, Fym, Fx + 0.0, Fy + 0.0);
+            TileOps<T, CM, FORCE>::step(g, f, Fxm, Fym, Fx + 0.0, Fy + 0.0);
             // push; a value that leaves the tile's last column lands on the
             // next row's first entry, which no other source writes and whose
             // population is either rebuilt by its boundary condition or
@@ -211,34 +176,32 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
         }
         __syncthreads();
         if (nbc) {
+            asm volatile("" : "+v"(bword));
+            const int bt = bword & 0xfff, v = bword >> 12 & 0xf, type = bword >> 16 & 0xf;
+            const TileBC& b = bcs[bk];
             if (bcl) {
-                if (b.type == 5) {
-                    Pops<T>::put(P, PS, 2, b.t, fo2 + 3.0 * w64(2) * (dux * kCX[2] + duy * kCY[2]));
-                    Pops<T>::put(P, PS, 6, b.t, fo6 + 3.0 * w64(6) * (dux * kCX[6] + duy * kCY[6]));
-                    Pops<T>::put(P, PS, 8, b.t, fo8 + 3.0 * w64(8) * (dux * kCX[8] + duy * kCY[8]));
-                } else {
-                    double fs[kNV], f1[kNV], f2[kNV];
-                    const bool nbr = bc_reads_neighbours(b.type, b.nx, b.ny);
-#pragma unroll
-                    for (int v = 0; v < kNV; v++)
-                        fs[v] = bc_unknown(b.nx, b.ny, b.nd, v) ? 0.0 : Pops<T>::get(P, PS, v, b.t);
-                    if (nbr) {
-                        lds_site(P, PS, b.t + b.nx * EJ + b.ny, f1);
-                        lds_site(P, PS, b.t + 2 * (b.nx * EJ + b.ny), f2);
+                const int nx = (int)(bword >> 20 & 3) - 1, ny = (int)(bword >> 22 & 3) - 1, nd = bword >> 24 & 1;
+                const BCLane l = bc_lane(g, v, type, nx, ny, nd);
+                double r1 = 0.0, u1 = 0.0, r2 = 0.0, u2 = 0.0;
+                if (l.nbr) {
+                    // one neighbour at a time, for the registers
+#pragma unroll 1
+                    for (int q = 1; q <= 2; q++) {
+                        double fn[kNV];
+                        r1 = r2;
+                        u1 = u2;
+                        load_site(P, PS, bt + q * (nx * EJ + ny), fn);
+                        bc_neighbour(fn, nd, nd != 0 ? Fx : Fy, r2, u2);
                     }
-                    const double F12[2] = {Fx, Fy};
-                    bc_values<CM>(g, b.type, b.nx, b.ny, b.nd, fs, f1, f2, uwx * a.ramp[s], uwy * a.ramp[s], rin, rn,
-                                  uxn, uyn, F12, F12);
-#pragma unroll
-                    for (int v = 0; v < kNV; v++) Pops<T>::put(P, PS, v, b.t, fs[v]);
                 }
+                const BCPops q = bc_read(l, [&](int u, double w) { return Pops<T>::from(P[u * PS + bt], w); });
+                Pops<T>::put(P, PS, v, bt, bc_value<CM>(l, g, q, r1, u1, r2, u2, b.ux * a.ramp[s], b.uy * a.ramp[s],
+                                                        b.rho_in, 0.0, share));
             }
             __syncthreads();
         }
-        if (act) {
 #pragma unroll
-            for (int v = 0; v < kNV; v++) f[v] = P[v * PS + t];
-        }
+        for (int v = 0; v < kNV; v++) f[v] = P[v * PS + tl];
         if (s + 1 < n) __syncthreads();  // the next push overwrites what others still read
     }
     if (act && li + ra >= i0 && li + ra < i1 && lj + rb >= j0 && lj + rb < j1) {
@@ -247,30 +210,46 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
     }
 }
 
-template <typename T, bool CM, bool SUP>
+template <typename T, bool CM, bool FORCE>
 void launch_tile_t(const T* src, T* dst, const GridScalars& g, const TileArgs& a, unsigned threads, size_t lds,
                    hipStream_t s) {
-    k_tile_step<T, CM, SUP><<<(unsigned)(a.ni * a.nj), threads, lds, s>>>(src, dst, g, a);
+    // tiles of four steps with their rim exceed the default limit in FP64
+    static const bool once = (hipFuncSetAttribute((const void*)k_tile_step<T, CM, FORCE>,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) == hipSuccess);
+    (void)once;
+    k_tile_step<T, CM, FORCE><<<(unsigned)(a.ni * a.nj), threads, lds, s>>>(src, dst, g, a);
 }
 
 }  // namespace
 
 template <typename T>
-void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, const TileShape& shape, bool sup,
-                      hipStream_t s) {
+void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, const TileShape& shape, hipStream_t s) {
     const int n = a.steps;
     a.ni = (g.Nx + shape.CI - 1) / shape.CI;
     a.nj = (g.Ny + shape.CJ - 1) / shape.CJ;
-    const int ci = (g.Nx + a.ni - 1) / a.ni, cj = (g.Ny + a.nj - 1) / a.nj;  // largest tile
+    a.qi = g.Nx / a.ni;
+    a.ri = g.Nx % a.ni;
+    a.qj = g.Ny / a.nj;
+    a.rj = g.Ny % a.nj;
+    const int ci = a.qi + (a.ri ? 1 : 0), cj = a.qj + (a.rj ? 1 : 0);  // largest tile
     const int EI = ci + 2 * n;
     a.EJ = cj + 2 * n;
     a.PS = EI * a.EJ + 2 * (a.EJ + 1);
     const size_t planes = ((size_t)kNV * a.PS * sizeof(T) + 15) / 16 * 16;
     a.bc_off = (unsigned)planes;
-    // boundary sites of a tile lie on at most two rows and two columns of it
-    const size_t lds = planes + sizeof(TileBC) * (size_t)(2 * (EI + a.EJ));
-    const unsigned threads = (unsigned)((EI * a.EJ + 63) / 64 * 64);
-    if (sup) {
+    // boundary sites of a tile and its rim: on the sides of the lattice it
+    // reaches, both of them where the tile spans the lattice
+    const int reach_i = a.per_i ? 0 : (a.ni == 1 || a.qi <= n ? 2 : 1);
+    const int reach_j = a.per_j ? 0 : (a.nj == 1 || a.qj <= n ? 2 : 1);
+    const int max_bc = reach_i * (a.EJ < g.Ny || a.per_j ? a.EJ : g.Ny) + reach_j * (EI < g.Nx || a.per_i ? EI : g.Nx);
+    unsigned threads = (unsigned)((EI * a.EJ + 63) / 64 * 64);
+    const unsigned bc_threads = (unsigned)((max_bc + kBCPerWave - 1) / kBCPerWave * 64);
+    if (threads < bc_threads) threads = bc_threads;
+    a.share_off = (unsigned)(planes + sizeof(TileBC) * (size_t)max_bc);
+    const size_t lds = a.share_off + sizeof(double) * (size_t)(threads / 64 * kBCPerWave * kNV);
+    bool force = false;
+    for (int k = 0; k <= n; k++) force = force || a.F[k][0] != 0.0 || a.F[k][1] != 0.0;
+    if (force) {
         if (g.cm) launch_tile_t<T, true, true>(src, dst, g, a, threads, lds, s);
         else launch_tile_t<T, false, true>(src, dst, g, a, threads, lds, s);
     } else {
@@ -279,9 +258,9 @@ void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, co
     }
 }
 
-template void launch_tile_step<double>(const double*, double*, const GridScalars&, TileArgs, const TileShape&, bool,
+template void launch_tile_step<double>(const double*, double*, const GridScalars&, TileArgs, const TileShape&,
                                        hipStream_t);
-template void launch_tile_step<float>(const float*, float*, const GridScalars&, TileArgs, const TileShape&, bool,
+template void launch_tile_step<float>(const float*, float*, const GridScalars&, TileArgs, const TileShape&,
                                       hipStream_t);
 
 }  // namespace life

@@ -46,6 +46,7 @@ struct GridScalars {
     int cm;                 // central moments (else BGK)
     double omega;
     double cs2, cs4;        // c_s*c_s and c_s*c_s*c_s*c_s with the reference's rounding
+    double wq[3];           // w_v / (2 c_s^4) of the rest, axis and diagonal populations (Grid.cpp:460)
     double Fx, Fy;          // force_xy (uniform)
     double Fx0, Fy0;        // force_xy + 0.0 (force_xy + force_ibm at non-support sites)
     double Fxm, Fym;        // force_xy of the previous step: the moments of the incoming populations

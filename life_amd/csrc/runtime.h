@@ -83,6 +83,7 @@ struct life_grid {
     double* delU = nullptr;
     double* ucol = nullptr;
     std::vector<int> type_host;
+    bool tile_multi = false;  // the sides allow the tiled step (lbm_tile.hip), several steps per launch
     // markers
     life::MarkerDev md{};
     int nbodies = 0;
@@ -136,6 +137,9 @@ namespace life {
 // Enqueue one lbmKernel on the grid stream; if ev_begin/ev_end are given,
 // they are recorded around the fused stream-collide launch.
 void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end);
+// Steps t .. t + k - 1 of a lattice without bodies in one launch, 1 <= k <=
+// left; returns k, or 0 (nothing launched) where lbm_step is to be used.
+int lbm_multi_step(life_grid* g, int t, int left);
 // The same step in two parts.  lbm_bulk_early launches the bulk
 // stream-collide of the next step on the second stream as soon as the
 // populations of the current step are final (it reads only f and the
