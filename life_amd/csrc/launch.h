@@ -40,6 +40,10 @@ void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, cons
 // sides or on neither, and is periodic in i if it is in j; tiles are at
 // least 3 sites wide (CI, CJ >= 5).
 constexpr int kTileMaxSteps = 8;
+constexpr int kTileMaxOutlet = 2048;  // rows of a lattice whose convective outlet a tile takes
+// Threads of the outlet-mean kernel, whose tree of sums the FP32-shifted
+// storage keeps everywhere.
+constexpr int kConvThreads = 1024;
 constexpr int kTileMaxSites = 1024;  // lanes of a workgroup: tile and rim
 struct TileShape {
     int CI, CJ;  // largest tile, without its rim
@@ -53,11 +57,16 @@ struct TileArgs {
     double ramp[kTileMaxSteps];  // inlet ramp of each step
     const double* u_in;
     const double* rho_in;
+    // one step per launch, on the state of the step before (steps = 1):
+    // force_ibm of the last spread, or null without immersed bodies
+    int one;
+    const double* fibm;
+    const int *site_uid, *uniq, *uniq_n;  // its support sites (SpreadScratch)
     // set by the launcher
     int ni, nj;          // tiles; the first ri (rj) of them have qi + 1 (qj + 1) sites, the others qi (qj)
     int qi, ri, qj, rj;
     int EJ, PS;      // row and plane strides in LDS
-    unsigned bc_off, share_off;  // byte offsets of the boundary sites and their scratch in LDS
+    unsigned bc_off, share_off, out_off;  // byte offsets in LDS: boundary sites, their scratch, the outlet's
 };
 template <typename T>
 void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, const TileShape& shape, hipStream_t s);

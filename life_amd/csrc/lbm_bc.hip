@@ -112,7 +112,6 @@ void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, cons
 // velocity of the last three columns.  One workgroup.  ordered = true keeps
 // the reference's serial left-to-right mean (plain method); otherwise an
 // FP64 tree reduction is used.
-constexpr int kConvThreads = 1024;
 
 // Outlet velocity of column c = 0..2 from the right wall, row j: stored in
 // ucol (one thread per (c, j), many workgroups).

@@ -31,6 +31,8 @@ namespace {
 // Site arithmetic by storage type: moments and collision of one site.
 // Fm: force_xy of the previous step (moments), F: of this step, both with
 // force_ibm where the lattice has immersed bodies.
+// FORCE false: no uniform force.  site: the same with the force of a support
+// site, rounded as the support-site kernels round.
 template <typename T, bool CM, bool FORCE>
 struct TileOps;
 
@@ -44,6 +46,10 @@ struct TileOps<double, CM, FORCE> {
 #pragma unroll
         for (int v = 0; v < kNV; v++) f[v] = fo[v];
     }
+    static __device__ __forceinline__ void site(const GridScalars& g, double f[kNV], double Fxm, double Fym, double Fx,
+                                                double Fy) {
+        TileOps<double, CM, true>::step(g, f, Fxm, Fym, Fx, Fy);
+    }
 };
 
 template <bool CM, bool FORCE>
@@ -51,6 +57,10 @@ struct TileOps<float, CM, FORCE> {
     static __device__ __forceinline__ void step(const GridScalars& g, float f[kNV], double Fxm, double Fym, double Fx,
                                                 double Fy) {
         step_site32<CM, false, FORCE>(g, f, (float)Fxm, (float)Fym, (float)Fx, (float)Fy);
+    }
+    static __device__ __forceinline__ void site(const GridScalars& g, float f[kNV], double Fxm, double Fym, double Fx,
+                                                double Fy) {
+        step_site32<CM, true>(g, f, (float)Fxm, (float)Fym, (float)Fx, (float)Fy);
     }
 };
 
@@ -62,6 +72,8 @@ struct TileBC {
     signed char type, nx, ny, nd;
     double ux, uy;      // inlet velocity without the ramp
     double rho_in;
+    // one step per launch only:
+    double old[3];      // convective: populations 2, 6, 8 before the step; [0] at a pressure corner: its previous u_y
 };
 
 // Site type and normal of (i, j), as site_type and normal_vector of the
@@ -97,9 +109,52 @@ __device__ __forceinline__ bool tile_bc(const TileArgs& a, int Nx, int Ny, int i
     return true;
 }
 
+// Population v as the FP64 value (Pops<T>::get of a register).
+__device__ __forceinline__ double to64(double f, int) { return f; }
+__device__ __forceinline__ double to64(float f, int v) { return (double)f + w64(v); }
+
+// GridClass::convectiveSpeed's mean (Grid.cpp:477-487) over the outlet
+// velocities col[0..Ny) in LDS, by the whole workgroup: serial in row order
+// for FP64 populations, else the tree of convective_finish (its threads'
+// sums of rows tid, tid + kConvThreads, ..., combined in halves), which
+// leaves the sum in red[0].  The caller synchronises before reading it.
+template <typename T>
+__device__ __forceinline__ void tile_outlet_sum(const double* col, int Ny, double* red) {
+    const int t = threadIdx.x, nt = blockDim.x;
+    if (sizeof(T) == 8) {
+        if (t == 0) {
+            double s = 0.0;
+            int j = 0;
+            for (; j + 8 <= Ny; j += 8) {
+                double c[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) c[q] = col[j + q];
+#pragma unroll
+                for (int q = 0; q < 8; q++) s += c[q];
+            }
+            for (; j < Ny; j++) s += col[j];
+            red[0] = s;
+        }
+        return;
+    }
+    for (int q = t; q < kConvThreads; q += nt) {
+        double part = 0.0;
+        for (int j = q; j < Ny; j += kConvThreads) part += col[j];
+        red[q] = part;
+    }
+    __syncthreads();
+    for (int w = kConvThreads / 2; w > 0; w >>= 1) {
+        for (int q = t; q < w; q += nt) red[q] += red[q + w];
+        __syncthreads();
+    }
+}
+
 // One tile of CI x CJ sites (at most) and its rim, one site per lane.  FORCE
-// false: no force in these steps.
-template <typename T, bool CM, bool FORCE>
+// false: no uniform force in these steps.  ONE: one step per launch, with
+// what depends on the step before: force_ibm at the support sites of the last
+// spread (a.fibm; it is zero elsewhere), a convective outlet, a pressure
+// corner.
+template <typename T, bool CM, bool FORCE, bool ONE>
 __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict__ src, T* __restrict__ dst,
                                                              GridScalars g, TileArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
@@ -131,6 +186,43 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
     T f[kNV];
 #pragma unroll
     for (int v = 0; v < kNV; v++) f[v] = src[v * S + id];
+    double Bx = 0.0, By = 0.0;
+    bool site = false;  // a support site of the last spread
+    if (ONE && a.fibm) {
+        Bx = a.fibm[id];
+        By = a.fibm[S + id];
+        site = Bx != 0.0 || By != 0.0;
+        if (sizeof(T) == 4 && !site) {
+            // FP32 rounds a support site its own way also where the force is
+            // exactly zero: look it up in the spread's site list
+            const int u = a.site_uid[id];
+            site = (unsigned)u < (unsigned)*a.uniq_n && a.uniq[u] == id;
+        }
+    }
+    // outlet: every tile on that side forms the mean velocity of the last
+    // column itself (launches of their own, with their own waits, cost more)
+    const bool outlet = ONE && a.wall[1] == 5 && hi == Nx;
+    double* u3 = reinterpret_cast<double*>(tile_lds + a.out_off);  // 3 columns x EJ rows x 2
+    double* red = u3 + 6 * EJ;
+    double* col = red + (sizeof(T) == 8 ? 1 : kConvThreads);
+    if (outlet) {
+        for (int q = t; q < Ny; q += (int)blockDim.x) {
+            const long long cid = (long long)(Nx - 1) * Ny + q;
+            double fc[kNV], r, ux, uy;
+            load_site(src, S, cid, fc);
+            moments64(fc, a.F[0][0] + (a.fibm ? a.fibm[cid] : 0.0), a.F[0][1] + (a.fibm ? a.fibm[S + cid] : 0.0), r, ux,
+                      uy);
+            col[q] = ux;
+        }
+        if (act && i >= Nx - 3) {
+            double fc[kNV], r, ux, uy;
+#pragma unroll
+            for (int v = 0; v < kNV; v++) fc[v] = to64(f[v], v);
+            moments64(fc, a.F[0][0] + Bx, a.F[0][1] + By, r, ux, uy);
+            u3[((Nx - 1 - i) * EJ + rb) * 2] = ux;
+            u3[((Nx - 1 - i) * EJ + rb) * 2 + 1] = uy;
+        }
+    }
     if (t == 0) s_nbc = 0;
     __syncthreads();
     {
@@ -143,9 +235,20 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
             b.ux = a.u_in[2 * j];
             b.uy = a.u_in[2 * j + 1];
             b.rho_in = a.rho_in[j];
+            if (ONE && b.type == 5) {
+                b.old[0] = to64(f[2], 2);
+                b.old[1] = to64(f[6], 6);
+                b.old[2] = to64(f[8], 8);
+            } else if (ONE && b.type == 4 && b.nx != 0 && b.ny != 0) {
+                double fp[kNV], rn, uxn;
+#pragma unroll
+                for (int v = 0; v < kNV; v++) fp[v] = to64(f[v], v);
+                moments64(fp, a.F[0][0] + Bx, a.F[0][1] + By, rn, uxn, b.old[0]);
+            }
             bcs[atomicAdd(&s_nbc, 1)] = b;
         }
     }
+    if (outlet) tile_outlet_sum<T>(col, Ny, red);
     __syncthreads();
     // nine lanes per boundary site, seven sites per wavefront (bc_site.h);
     // the launch has wavefronts enough for all of them
@@ -166,7 +269,8 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
     for (int s = 0; s < n; s++) {
         const double Fxm = a.F[s][0], Fym = a.F[s][1], Fx = a.F[s + 1][0], Fy = a.F[s + 1][1];
         if (act) {
-            TileOps<T, CM, FORCE>::step(g, f, Fxm, Fym, Fx + 0.0, Fy + 0.0);
+            if (ONE && site) TileOps<T, CM, FORCE>::site(g, f, Fxm + Bx, Fym + By, Fx + Bx, Fy + By);
+            else TileOps<T, CM, FORCE>::step(g, f, Fxm, Fym, Fx + 0.0, Fy + 0.0);
             // push; a value that leaves the tile's last column lands on the
             // next row's first entry, which no other source writes and whose
             // population is either rebuilt by its boundary condition or
@@ -179,7 +283,16 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
             asm volatile("" : "+v"(bword));
             const int bt = bword & 0xfff, v = bword >> 12 & 0xf, type = bword >> 16 & 0xf;
             const TileBC& b = bcs[bk];
-            if (bcl) {
+            if (ONE && bcl && type == 5) {
+                if (v == 2 || v == 6 || v == 8) {
+                    // delU of GridClass::convectiveSpeed (Grid.cpp:488-494)
+                    const double uOut = red[0] / (double)Ny;
+                    const double* u = u3 + 2 * (bt % EJ);
+                    const double dux = (-uOut / 2.0) * (3.0 * u[0] - 4.0 * u[2 * EJ] + u[4 * EJ]);
+                    const double duy = (-uOut / 2.0) * (3.0 * u[1] - 4.0 * u[2 * EJ + 1] + u[4 * EJ + 1]);
+                    Pops<T>::put(P, PS, v, bt, bc_convective(v, b.old[v == 2 ? 0 : (v == 6 ? 1 : 2)], dux, duy));
+                }
+            } else if (bcl) {
                 const int nx = (int)(bword >> 20 & 3) - 1, ny = (int)(bword >> 22 & 3) - 1, nd = bword >> 24 & 1;
                 const BCLane l = bc_lane(g, v, type, nx, ny, nd);
                 double r1 = 0.0, u1 = 0.0, r2 = 0.0, u2 = 0.0;
@@ -196,7 +309,7 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
                 }
                 const BCPops q = bc_read(l, [&](int u, double w) { return Pops<T>::from(P[u * PS + bt], w); });
                 Pops<T>::put(P, PS, v, bt, bc_value<CM>(l, g, q, r1, u1, r2, u2, b.ux * a.ramp[s], b.uy * a.ramp[s],
-                                                        b.rho_in, 0.0, share));
+                                                        b.rho_in, ONE ? b.old[0] : 0.0, share));
             }
             __syncthreads();
         }
@@ -210,14 +323,26 @@ __global__ __launch_bounds__(kTileMaxSites) void k_tile_step(const T* __restrict
     }
 }
 
-template <typename T, bool CM, bool FORCE>
+template <typename T, bool CM, bool FORCE, bool ONE>
 void launch_tile_t(const T* src, T* dst, const GridScalars& g, const TileArgs& a, unsigned threads, size_t lds,
                    hipStream_t s) {
     // tiles of four steps with their rim exceed the default limit in FP64
-    static const bool once = (hipFuncSetAttribute((const void*)k_tile_step<T, CM, FORCE>,
+    static const bool once = (hipFuncSetAttribute((const void*)k_tile_step<T, CM, FORCE, ONE>,
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) == hipSuccess);
     (void)once;
-    k_tile_step<T, CM, FORCE><<<(unsigned)(a.ni * a.nj), threads, lds, s>>>(src, dst, g, a);
+    k_tile_step<T, CM, FORCE, ONE><<<(unsigned)(a.ni * a.nj), threads, lds, s>>>(src, dst, g, a);
+}
+
+template <typename T, bool ONE>
+void launch_tile_cf(const T* src, T* dst, const GridScalars& g, const TileArgs& a, bool force, unsigned threads,
+                    size_t lds, hipStream_t s) {
+    if (g.cm) {
+        if (force) launch_tile_t<T, true, true, ONE>(src, dst, g, a, threads, lds, s);
+        else launch_tile_t<T, true, false, ONE>(src, dst, g, a, threads, lds, s);
+    } else {
+        if (force) launch_tile_t<T, false, true, ONE>(src, dst, g, a, threads, lds, s);
+        else launch_tile_t<T, false, false, ONE>(src, dst, g, a, threads, lds, s);
+    }
 }
 
 }  // namespace
@@ -246,16 +371,14 @@ void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, co
     const unsigned bc_threads = (unsigned)((max_bc + kBCPerWave - 1) / kBCPerWave * 64);
     if (threads < bc_threads) threads = bc_threads;
     a.share_off = (unsigned)(planes + sizeof(TileBC) * (size_t)max_bc);
-    const size_t lds = a.share_off + sizeof(double) * (size_t)(threads / 64 * kBCPerWave * kNV);
+    a.out_off = a.share_off + (unsigned)(sizeof(double) * (threads / 64 * kBCPerWave * kNV));
+    const bool one = a.one != 0;
+    const size_t outlet = one && a.wall[1] == 5 ? 6 * (size_t)a.EJ + kConvThreads + (size_t)g.Ny : 0;
+    const size_t lds = a.out_off + sizeof(double) * outlet;
     bool force = false;
     for (int k = 0; k <= n; k++) force = force || a.F[k][0] != 0.0 || a.F[k][1] != 0.0;
-    if (force) {
-        if (g.cm) launch_tile_t<T, true, true>(src, dst, g, a, threads, lds, s);
-        else launch_tile_t<T, false, true>(src, dst, g, a, threads, lds, s);
-    } else {
-        if (g.cm) launch_tile_t<T, true, false>(src, dst, g, a, threads, lds, s);
-        else launch_tile_t<T, false, false>(src, dst, g, a, threads, lds, s);
-    }
+    if (one) launch_tile_cf<T, true>(src, dst, g, a, force, threads, lds, s);
+    else launch_tile_cf<T, false>(src, dst, g, a, force, threads, lds, s);
 }
 
 template void launch_tile_step<double>(const double*, double*, const GridScalars&, TileArgs, const TileShape&,

@@ -394,10 +394,50 @@ TileShape tile_shape(const life_grid* g) {
     return cm ? TileShape{12, 28, 2} : TileShape{10, 26, 3};
 }
 
+// As tile_shape, for a launch of one step of any lattice, bodies and
+// convective outlet included: one launch instead of two to six (outlet
+// speed, bulk, support sites, boundaries).  Whole step of a cylinder case,
+// plain | tiled: 441 x 83 FP64, pressure outlet 21.1 | 15.7 us, convective
+// 28.2 | 16.6; 1024 x 256 FP32, 31.1 | 28.4 and 36.5 | 29.4; 1024 x 1024
+// FP64 90 | 83 and 130 | 92, FP32 79.0 | 79.6 and 86 | 81; a cavity of 256 x
+// 256 without bodies FP64 8.5 | 6.8, of 512 x 512 11.5 | 12.6.  Tiles of
+// 14 x 14 sites with their rim while they are few, of 16 x 32 (three
+// workgroups to a CU, longer rows) above; past the sizes below the rim's
+// second reading costs more than the launches.  LIFE_TILE = 0 selects the
+// plain kernels here too, LIFE_TILE1 = "CI,CJ" a tile, for sweeps.
+TileShape tile_shape_one(const life_grid* g) {
+    const TileShape plain{0, 0, 0};
+    if (!g->tile_ok || std::getenv("LIFE_PUSH32") || std::getenv("LIFE_PUSH64")) return plain;
+    if (g->convective && g->p.Ny > kTileMaxOutlet) return plain;
+    if (const char* e = std::getenv("LIFE_TILE"))
+        if (std::atoi(e) == 0) return plain;
+    const long long N = (long long)g->p.Nx * g->p.Ny;
+    if (const char* e = std::getenv("LIFE_TILE1")) {
+        TileShape s{0, 0, 1};
+        if (std::sscanf(e, "%d,%d", &s.CI, &s.CJ) != 2 || s.CI < 5 || s.CJ < 5 ||
+            (long long)(s.CI + 2) * (s.CJ + 2) > 512 || s.CI + s.CJ > 52)
+            return plain;
+        return s;
+    }
+    const bool f32 = g->prec == LIFE_FP32_SHIFTED;
+    const long long most = g->convective ? 1100000 : (g->md.n > 0 ? (f32 ? 300000 : 1100000) : 150000);
+    if (N > most) return plain;
+    return N <= 150000 ? TileShape{12, 12, 1} : TileShape{14, 30, 1};
+}
+
 // Launch steps t .. t + shape.steps - 1 on stream s.
-void tile_launch(life_grid* g, int t, const TileShape& shape, hipStream_t s) {
+// one: a single step on the state of the step before (bodies, convective
+// outlet, pressure corner).
+void tile_launch(life_grid* g, int t, const TileShape& shape, bool one, hipStream_t s) {
     TileArgs a{};
     a.steps = shape.steps;
+    a.one = one ? 1 : 0;
+    if (g->md.n > 0) {
+        a.fibm = g->fibm;
+        a.site_uid = g->sc.site_uid;
+        a.uniq = g->sc.uniq;
+        a.uniq_n = g->sc.uniq_n;
+    }
     a.per_i = g->p.wall_left == LIFE_FLUID;
     a.per_j = g->p.wall_bottom == LIFE_FLUID;
     a.wall[0] = g->p.wall_left;
@@ -433,7 +473,7 @@ int lbm_multi_step(life_grid* g, int t, int left) {
     if (shape.steps > left) shape.steps = left;
     lbm_join(g);
     g->g = step_scalars(*g, t);
-    tile_launch(g, t, shape, g->stream);
+    tile_launch(g, t, shape, false, g->stream);
     LIFE_HIP(hipGetLastError());
     const int k = shape.steps;
     g->g = step_scalars(*g, t + k - 1);
@@ -470,7 +510,13 @@ void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end) {
             off = true;
         }
     }
-    if (g->prec == kFP64) {
+    TileShape shape{0, 0, 0};
+    if (!early && !ex) shape = tile_shape_one(g);
+    if (shape.CI > 0) {
+        if (ev_begin) LIFE_HIP(hipEventRecord(ev_begin, s));
+        tile_launch(g, t, shape, true, s);
+        if (ev_end) LIFE_HIP(hipEventRecord(ev_end, s));
+    } else if (g->prec == kFP64) {
         const double* fs = static_cast<const double*>(g->f[src]);
         double* fd = static_cast<double*>(g->f[dst]);
         if (g->convective) launch_convective_speed<double>(fs, g->g, g->fibm, g->u0, ex, g->ucol, g->delU, true, s);
@@ -947,8 +993,8 @@ int life_grid_create(const life_params* p, int precision, int device, life_grid*
             // j would leave corner sites that stream from the far side.  A
             // convective outlet reads the mean of its column and a pressure
             // corner its previous moments before every step.
-            g->tile_multi = wl == wr && wb == wt && !(wl && !wb) && !site_force &&
-                            p->wall_right != LIFE_CONVECTIVE &&
+            g->tile_ok = wl == wr && wb == wt && !(wl && !wb) && !site_force;
+            g->tile_multi = g->tile_ok && p->wall_right != LIFE_CONVECTIVE &&
                             p->wall_bottom != LIFE_PRESSURE && p->wall_top != LIFE_PRESSURE;
         }
 

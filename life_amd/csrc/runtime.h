@@ -83,7 +83,9 @@ struct life_grid {
     double* delU = nullptr;
     double* ucol = nullptr;
     std::vector<int> type_host;
-    bool tile_multi = false;  // the sides allow the tiled step (lbm_tile.hip), several steps per launch
+    // the sides allow the tiled step (lbm_tile.hip), and several steps per
+    // launch of it without bodies
+    bool tile_ok = false, tile_multi = false;
     // markers
     life::MarkerDev md{};
     int nbodies = 0;

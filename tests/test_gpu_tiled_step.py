@@ -90,3 +90,46 @@ def test_blow_up_is_reported_at_its_scan(gpu_lib, monkeypatch):
         msg.append(str(e.value))
         c.close()
     assert msg[0] == msg[1] and "t = 10)" in msg[0]
+
+
+def one_step_cases(cm):
+    cyl, g = cfg.cylinder_channel(Nx=241, Ny=61, D=10.0, u_max=0.05, Re=60.0, ramp_steps=0.0, centre=(60.2, 29.7))
+    yield "cylinder, convective", cyl.replace(central_moments=cm), g
+    yield "cylinder, pressure", cyl.replace(central_moments=cm, wall_right=cfg.PRESSURE), g
+    # larger tiles; body two columns from the outlet, so that its supports carry force in the outlet's three columns
+    p, g = cfg.cylinder_channel(Nx=410, Ny=391, D=40.0, u_max=0.05, Re=60.0, ramp_steps=0.0, centre=(387.3, 190.2))
+    yield "cylinder at the outlet", p.replace(central_moments=cm), g
+    # more outlet rows than threads of the outlet mean
+    yield "tall channel", bc_mix_params("channel_convective", Nx=60, Ny=1100, cm=cm)[0], ""
+    yield "thin channel", bc_mix_params("channel_convective", Nx=6, Ny=5, cm=cm)[0], ""
+    yield "pressure corners", cfg.lattice_case(50, 33, 0.7, wall_left=cfg.VELOCITY, wall_right=cfg.PRESSURE,
+                                               wall_bottom=cfg.PRESSURE, wall_top=cfg.FREESLIP, profile=cfg.UNIFORM,
+                                               uxInlet_p=0.03, central_moments=cm), ""
+    p, g = cfg.womersley_cylinder(central_moments=cm)
+    yield "oscillating force with a body", p, g
+    # markers half-way between rows: supports whose force is exactly zero
+    p, g = cfg.inverted_flag(200, 100, 0.25, 12, Re=100.0, kb=0.6, central_moments=cm)
+    yield "flag", p, g
+
+
+@pytest.mark.parametrize("cm", [0, 1])
+def test_single_tiled_step_equals_plain_kernels(gpu_lib, monkeypatch, cm):
+    """One step per launch, with support sites, convective outlet and pressure corners."""
+    for name, p, g in one_step_cases(cm):
+        for prec in (L.LIFE_FP64, L.LIFE_FP32_SHIFTED):
+            out = []
+            for tile in (None, "0"):
+                monkeypatch.delenv("LIFE_TILE", raising=False)
+                if tile:
+                    monkeypatch.setenv("LIFE_TILE", tile)
+                c = Case(p, g, precision=prec)
+                c.step(25)
+                o = list(c.fields())
+                if c.n_markers:
+                    m = c.markers()
+                    o += [m["pos"], m["force"]]
+                c.close()
+                out.append(o)
+            assert np.isfinite(out[0][0]).all()
+            for a, b in zip(*out):
+                assert np.array_equal(a, b), (name, cm, prec, float(np.abs(a - b).max()))
