@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "launch.h"
+
 namespace life {
 
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X, each
@@ -92,6 +94,41 @@ __device__ __forceinline__ void push_store_realigned(DP __restrict__ dst, long l
                 put<T, NT>(&dst[kv[q] * S + (long long)id_row * Ny + j], st.slot[q][t + 1]);
             }
         }
+    }
+}
+
+// s plus x[0..n) (in LDS) added one after the other, in order, by one lane.
+// The next sixteen operands are on their way while sixteen are added, so the
+// chain waits for the additions alone.
+__device__ inline double serial_sum(double s, const double* x, int n) {
+    constexpr int U = 16;
+    double c[U];
+    int j = 0;
+    if (n >= U) {
+#pragma unroll
+        for (int q = 0; q < U; q++) c[q] = x[q];
+        for (j = U; j + U <= n; j += U) {
+            double d[U];
+#pragma unroll
+            for (int q = 0; q < U; q++) d[q] = x[j + q];
+#pragma unroll
+            for (int q = 0; q < U; q++) s += c[q];
+#pragma unroll
+            for (int q = 0; q < U; q++) c[q] = d[q];
+        }
+#pragma unroll
+        for (int q = 0; q < U; q++) s += c[q];
+    }
+    for (; j < n; j++) s += x[j];
+    return s;
+}
+
+// red[0] = the kConvThreads values of red (in LDS) combined in halves, by the
+// whole workgroup; the caller synchronises before and after.
+__device__ inline void tree_sum(double* red) {
+    for (int w = kConvThreads / 2; w > 0; w >>= 1) {
+        for (int q = threadIdx.x; q < w; q += (int)blockDim.x) red[q] += red[q + w];
+        __syncthreads();
     }
 }
 

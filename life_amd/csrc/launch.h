@@ -27,7 +27,7 @@ struct BCArgs {
     int nbc;
     const double* u_in;   // Ny*2
     const double* rho_in; // Ny
-    const double* delU;   // Ny*2
+    const double* ucol;   // outlet velocities [column][d][row] and their mean (launch_convective_speed)
     double ramp;
 };
 
@@ -72,7 +72,7 @@ template <typename T>
 void launch_tile_step(const T* src, T* dst, const GridScalars& g, TileArgs a, const TileShape& shape, hipStream_t s);
 template <typename T>
 void launch_convective_speed(const T* src, const GridScalars& g, const double* fibm, const double* u0,
-                             bool explicit_state, double* ucol, double* delU, bool ordered, hipStream_t s);
+                             bool explicit_state, double* ucol, bool ordered, hipStream_t s);
 template <typename T>
 void launch_init_equilibrium(T* f, const GridScalars& g, const double* rho0, const double* u0, hipStream_t s);
 template <typename T>

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bc_site.h"
+#include "dev_util.h"
 #include "launch.h"
 
 namespace life {
@@ -36,8 +37,14 @@ __device__ __forceinline__ void bc_wave(const T* __restrict__ src, T* __restrict
     const long long S = g.S, id = b.id;
     const int Ny = g.Ny, j = b.j;
     if (b.type == 5) {  // convective: f[2,6,8] = f_n + 3 w (delU . c)
-        if (v == 2 || v == 6 || v == 8)
-            Pops<T>::put(dst, S, v, id, bc_convective(v, Pops<T>::get(src, S, v, id), a.delU[2 * j], a.delU[2 * j + 1]));
+        if (v == 2 || v == 6 || v == 8) {
+            // delU of GridClass::convectiveSpeed (Grid.cpp:488-494)
+            const double uOut = a.ucol[6 * (long long)Ny];
+            const double* u = a.ucol + j;
+            const double dux = (-uOut / 2.0) * (3.0 * u[0] - 4.0 * u[2LL * Ny] + u[4LL * Ny]);
+            const double duy = (-uOut / 2.0) * (3.0 * u[Ny] - 4.0 * u[3LL * Ny] + u[5LL * Ny]);
+            Pops<T>::put(dst, S, v, id, bc_convective(v, Pops<T>::get(src, S, v, id), dux, duy));
+        }
         return;
     }
     if (b.type == 0) return;
@@ -109,12 +116,20 @@ void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, cons
 }
 
 // GridClass::convectiveSpeed (Grid.cpp:477-495) on the end-of-previous-step
-// velocity of the last three columns.  One workgroup.  ordered = true keeps
-// the reference's serial left-to-right mean (plain method); otherwise an
-// FP64 tree reduction is used.
+// velocity of the last three columns: many workgroups form the velocities
+// (ucol), one the mean outlet speed, and the outlet sites delU from both.
+// ordered = true keeps the reference's serial left-to-right mean (plain
+// method); otherwise an FP64 tree reduction is used.  The serial mean is one
+// chain of Ny additions: its operands come from LDS, sixteen ahead (read one
+// by one from memory, the chain waited for each).  Both launches on a lattice
+// of 451 | 4096 rows: FP64 8.3 | 34 us (20.3 | 143 so), FP32 6.7 | 7.7 (5.9 | 10.6
+// with delU formed by the one workgroup).  One launch, whose last workgroup
+// takes the mean, is slower (FP32 7.4 | 12.1): the device-wide fences cost
+// more than the second launch.
+constexpr int kOutletChunk = 2048;
 
 // Outlet velocity of column c = 0..2 from the right wall, row j: stored in
-// ucol (one thread per (c, j), many workgroups).
+// ucol (one thread per (c, j)).
 template <typename T>
 __device__ inline void convective_column(const T* __restrict__ src, const GridScalars& g,
                                          const double* __restrict__ fibm, const double* __restrict__ u0,
@@ -138,40 +153,43 @@ __device__ inline void convective_column(const T* __restrict__ src, const GridSc
     ucol[(c * 2 + 1) * (long long)Ny + j] = uy;
 }
 
-// uOut and delU from ucol, one workgroup of kConvThreads.  ordered: the
-// reference's serial left-to-right mean; otherwise each thread sums its
-// rows j = tid, tid + kConvThreads, ... in increasing j and a fixed tree
-// combines the threads.
-__device__ inline void convective_finish(const GridScalars& g, const double* __restrict__ ucol,
-                                         double* __restrict__ delU, int ordered, double* red, double& uOutS) {
-    const int Ny = g.Ny;
-    double part = 0.0;
-    for (int j = threadIdx.x; j < Ny; j += blockDim.x) part += ucol[j];
-    red[threadIdx.x] = part;
-    __syncthreads();
+// red[0] = the sum of the outlet velocities u, by one workgroup of
+// kConvThreads.  ordered: the
+// reference's serial left-to-right mean; otherwise kConvThreads partial sums
+// (q sums the rows q, q + kConvThreads, ... in increasing order) combined by
+// a fixed tree.  The rows are brought to LDS in chunks, whose loads are all in
+// flight together.
+__device__ inline void convective_sum(const double* __restrict__ u, int Ny, int ordered, double* __restrict__ red) {
+    __shared__ double col[kOutletChunk];
+    const int t = threadIdx.x;
+    constexpr int R = kOutletChunk / kConvThreads;
+    double s = 0.0;
+    if (!ordered) red[t] = 0.0;
+    for (int c0 = 0; c0 < Ny; c0 += kOutletChunk) {
+        double x[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int j = c0 + r * kConvThreads + t;
+            x[r] = j < Ny ? u[j] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; r++) col[r * kConvThreads + t] = x[r];
+        __syncthreads();
+        const int n = min(Ny - c0, kOutletChunk);
+        if (ordered) {
+            if (t == 0) s = serial_sum(s, col, n);
+        } else {
+            static_assert(kOutletChunk % kConvThreads == 0, "rows of a partial sum in order");
+            for (int j = t; j < n; j += kConvThreads) red[t] += col[j];
+        }
+    }
     if (ordered) {
-        if (threadIdx.x == 0) {
-            double uOut = 0.0;
-            for (int j = 0; j < Ny; j++) uOut += ucol[j];
-            uOutS = uOut / (double)Ny;
-        }
-    } else {
-        for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) uOutS = red[0] / (double)Ny;
+        if (t == 0) red[0] = s;
+        return;
     }
     __syncthreads();
-    const double uOut = uOutS;
-    for (int j = threadIdx.x; j < Ny; j += blockDim.x) {
-        for (int d = 0; d < 2; d++) {
-            const double u1 = ucol[(0 * 2 + d) * (long long)Ny + j];
-            const double u2 = ucol[(1 * 2 + d) * (long long)Ny + j];
-            const double u3 = ucol[(2 * 2 + d) * (long long)Ny + j];
-            delU[2 * j + d] = (-uOut / 2.0) * (3.0 * u1 - 4.0 * u2 + u3);
-        }
-    }
+    tree_sum(red);
 }
 
 template <typename T>
@@ -182,11 +200,11 @@ __global__ __launch_bounds__(256) void k_convective_cols(const T* __restrict__ s
     convective_column(src, g, fibm, u0, explicit_state, ucol, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-__global__ __launch_bounds__(kConvThreads) void k_convective_finish(GridScalars g, const double* __restrict__ ucol,
-                                                                    double* __restrict__ delU, int ordered) {
+// uOut lies behind the velocities in ucol.
+__global__ __launch_bounds__(kConvThreads) void k_convective_mean(int Ny, double* __restrict__ ucol, int ordered) {
     __shared__ double red[kConvThreads];
-    __shared__ double uOutS;
-    convective_finish(g, ucol, delU, ordered, red, uOutS);
+    convective_sum(ucol, Ny, ordered, red);
+    if (threadIdx.x == 0) ucol[6 * (long long)Ny] = red[0] / (double)Ny;
 }
 
 // Serving: grid.y = listed case (cases with a convective outlet).
@@ -198,20 +216,20 @@ __global__ __launch_bounds__(256) void k_convective_cols_batch(const CaseDev* __
                       blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-__global__ __launch_bounds__(kConvThreads) void k_convective_finish_batch(const CaseDev* __restrict__ cases,
-                                                                          const int* __restrict__ list, int ordered) {
+__global__ __launch_bounds__(kConvThreads) void k_convective_mean_batch(const CaseDev* __restrict__ cases,
+                                                                        const int* __restrict__ list, int ordered) {
     __shared__ double red[kConvThreads];
-    __shared__ double uOutS;
     const CaseDev& c = cases[list[blockIdx.x]];
-    convective_finish(c.g, c.ucol, const_cast<double*>(c.bc.delU), ordered, red, uOutS);
+    convective_sum(c.ucol, c.g.Ny, ordered, red);
+    if (threadIdx.x == 0) c.ucol[6 * (long long)c.g.Ny] = red[0] / (double)c.g.Ny;
 }
 
 template <typename T>
 void launch_convective_speed(const T* src, const GridScalars& g, const double* fibm, const double* u0,
-                             bool explicit_state, double* ucol, double* delU, bool ordered, hipStream_t s) {
+                             bool explicit_state, double* ucol, bool ordered, hipStream_t s) {
     k_convective_cols<T><<<(unsigned)((3 * g.Ny + 255) / 256), 256, 0, s>>>(src, g, fibm, u0, explicit_state ? 1 : 0,
                                                                            ucol);
-    k_convective_finish<<<1, kConvThreads, 0, s>>>(g, ucol, delU, ordered ? 1 : 0);
+    k_convective_mean<<<1, kConvThreads, 0, s>>>(g.Ny, ucol, ordered ? 1 : 0);
 }
 
 template <typename T>
@@ -226,7 +244,7 @@ template <typename T>
 void launch_convective_batch(const CaseDev* cases, const int* list, int n, int max_ny, bool ordered, hipStream_t s) {
     if (n <= 0 || max_ny <= 0) return;
     k_convective_cols_batch<T><<<dim3((unsigned)((3 * max_ny + 255) / 256), (unsigned)n), 256, 0, s>>>(cases, list);
-    k_convective_finish_batch<<<(unsigned)n, kConvThreads, 0, s>>>(cases, list, ordered ? 1 : 0);
+    k_convective_mean_batch<<<(unsigned)n, kConvThreads, 0, s>>>(cases, list, ordered ? 1 : 0);
 }
 
 // f = f_eq(rho, u) at every site (Grid.cpp:1048-1061).
@@ -412,7 +430,7 @@ void launch_blowup_scan(const T* f, const GridScalars& g, unsigned long long* fl
     template void launch_bc<T>(const T*, T*, const GridScalars&, const BCArgs&, const double*, const double*,        \
                                const double*, bool, hipStream_t);                                                    \
     template void launch_convective_speed<T>(const T*, const GridScalars&, const double*, const double*, bool,       \
-                                             double*, double*, bool, hipStream_t);                                   \
+                                             double*, bool, hipStream_t);                                            \
     template void launch_init_equilibrium<T>(T*, const GridScalars&, const double*, const double*, hipStream_t);     \
     template void launch_materialise<T>(const T*, const GridScalars&, const double*, const double*, const double*,   \
                                         bool, double*, double*, double*, double*, hipStream_t);                      \

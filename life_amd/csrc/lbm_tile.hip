@@ -122,19 +122,7 @@ template <typename T>
 __device__ __forceinline__ void tile_outlet_sum(const double* col, int Ny, double* red) {
     const int t = threadIdx.x, nt = blockDim.x;
     if (sizeof(T) == 8) {
-        if (t == 0) {
-            double s = 0.0;
-            int j = 0;
-            for (; j + 8 <= Ny; j += 8) {
-                double c[8];
-#pragma unroll
-                for (int q = 0; q < 8; q++) c[q] = col[j + q];
-#pragma unroll
-                for (int q = 0; q < 8; q++) s += c[q];
-            }
-            for (; j < Ny; j++) s += col[j];
-            red[0] = s;
-        }
+        if (t == 0) red[0] = serial_sum(0.0, col, Ny);
         return;
     }
     for (int q = t; q < kConvThreads; q += nt) {
@@ -143,10 +131,7 @@ __device__ __forceinline__ void tile_outlet_sum(const double* col, int Ny, doubl
         red[q] = part;
     }
     __syncthreads();
-    for (int w = kConvThreads / 2; w > 0; w >>= 1) {
-        for (int q = t; q < w; q += nt) red[q] += red[q + w];
-        __syncthreads();
-    }
+    tree_sum(red);
 }
 
 // One tile of CI x CJ sites (at most) and its rim, one site per lane.  FORCE

@@ -487,7 +487,7 @@ void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end) {
     g->t_step = t;
     const double ramp = ramp_coefficient(g->p, g->cs.Dt, t);
     const int src = g->cur, dst = 1 - g->cur;
-    BCArgs a{g->bc, g->nbc, g->u_in, g->rho_in, g->delU, ramp};
+    BCArgs a{g->bc, g->nbc, g->u_in, g->rho_in, g->ucol, ramp};
     const bool ex = g->explicit_state;
     hipStream_t s = g->stream;
     const bool early = g->bulk_pending;
@@ -519,7 +519,7 @@ void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end) {
     } else if (g->prec == kFP64) {
         const double* fs = static_cast<const double*>(g->f[src]);
         double* fd = static_cast<double*>(g->f[dst]);
-        if (g->convective) launch_convective_speed<double>(fs, g->g, g->fibm, g->u0, ex, g->ucol, g->delU, true, s);
+        if (g->convective) launch_convective_speed<double>(fs, g->g, g->fibm, g->u0, ex, g->ucol, true, s);
         if (!early) {
             if (ev_begin) LIFE_HIP(hipEventRecord(ev_begin, s));
             launch_push64(fs, fd, g->g, g->rho0, g->u0, g->fibm, ex, s);
@@ -530,7 +530,7 @@ void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end) {
     } else {
         const float* fs = static_cast<const float*>(g->f[src]);
         float* fd = static_cast<float*>(g->f[dst]);
-        if (g->convective) launch_convective_speed<float>(fs, g->g, g->fibm, g->u0, ex, g->ucol, g->delU, false, s);
+        if (g->convective) launch_convective_speed<float>(fs, g->g, g->fibm, g->u0, ex, g->ucol, false, s);
         if (!early) {
             if (ev_begin) LIFE_HIP(hipEventRecord(ev_begin, s));
             launch_push32(fs, fd, g->g, g->rho0, g->u0, g->fibm, ex, s);
@@ -1056,14 +1056,12 @@ int life_grid_create(const life_params* p, int precision, int device, life_grid*
         g->bc = dalloc<BCSite>(g->nbc);
         g->u_in = dalloc<double>(2 * Ny);
         g->rho_in = dalloc<double>(Ny);
-        g->delU = dalloc<double>(2 * Ny);
-        g->ucol = dalloc<double>(6 * Ny);
+        g->ucol = dalloc<double>(6 * Ny + 1);  // and the mean behind them
         hipStream_t st = g->stream;
         if (g->nbc)
             LIFE_HIP(hipMemcpyAsync(g->bc, g->bc_host.data(), sizeof(BCSite) * g->nbc, hipMemcpyHostToDevice, st));
         LIFE_HIP(hipMemcpyAsync(g->u_in, g->u_in_host.data(), sizeof(double) * 2 * Ny, hipMemcpyHostToDevice, st));
         LIFE_HIP(hipMemcpyAsync(g->rho_in, g->rho_in_host.data(), sizeof(double) * Ny, hipMemcpyHostToDevice, st));
-        launch_fill_f64(g->delU, 0.0, 2 * Ny, st);
         launch_fill_f64(g->fibm, 0.0, 2 * (long long)S, st);
         // initial moments (Grid.cpp:1004-1033) and f = f_eq (Grid.cpp:1048-1061)
         int mode = 0;
@@ -1103,7 +1101,7 @@ int life_grid_destroy(life_grid* g) {
         free_markers(g);
         // the grid's work is done (synchronised above): its lattice blocks can be handed out again
         for (void* p : {g->f[0], g->f[1], (void*)g->rho0, (void*)g->u0, (void*)g->fibm}) dfree_cached(p);
-        for (void* p : {(void*)g->bc, (void*)g->u_in, (void*)g->rho_in, (void*)g->delU, (void*)g->ucol, (void*)g->epsA,
+        for (void* p : {(void*)g->bc, (void*)g->u_in, (void*)g->rho_in, (void*)g->ucol, (void*)g->epsA,
                         (void*)g->eps_first, (void*)g->eps_n, (void*)g->eps_off, (void*)g->eps_outside,
                         (void*)g->eps_band, (void*)g->eps_y, (void*)g->fsite[0], (void*)g->fsite[1]})
             dfree(p);

@@ -80,7 +80,6 @@ struct life_grid {
     std::vector<double> u_in_host, rho_in_host;
     double* u_in = nullptr;
     double* rho_in = nullptr;
-    double* delU = nullptr;
     double* ucol = nullptr;
     std::vector<int> type_host;
     // the sides allow the tiled step (lbm_tile.hip), and several steps per

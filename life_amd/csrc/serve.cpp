@@ -384,7 +384,7 @@ void fill_table(life_server* s) {
         d.fibm = g->fibm;
         d.explicit_state = g->explicit_state ? 1 : 0;
         d.convective = g->convective ? 1 : 0;
-        d.bc = BCArgs{g->bc, g->nbc, g->u_in, g->rho_in, g->delU, ramp_coefficient(g->p, g->cs.Dt, sl.c->t + 1)};
+        d.bc = BCArgs{g->bc, g->nbc, g->u_in, g->rho_in, g->ucol, ramp_coefficient(g->p, g->cs.Dt, sl.c->t + 1)};
         d.ucol = g->ucol;
         d.m = g->md;
         d.sc = g->sc;
