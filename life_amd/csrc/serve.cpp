@@ -479,6 +479,8 @@ void lattice_phase(life_server* s) {
         LIFE_HIP(hipEventRecord(s->ev_bulk_up, s->stream));
         s->bulk_up_pending = true;
         run_phase(s, s->graph_bulk, s->exec_bulk, s->stream, [&](hipStream_t st) { launch_bulk(s, st); });
+        // the last reader of the table so far (launch_bulk_early rewrites it)
+        LIFE_HIP(hipEventRecord(s->ev_bulk, s->stream));
     }
     run_phase(s, s->graph, s->exec, s->stream, [&](hipStream_t st) { launch_tail(s, st); });
 }
@@ -504,12 +506,15 @@ void launch_bulk_early(life_server* s) {
         d.dst = g->f[1 - g->cur];
         d.explicit_state = 0;
     }
-    // The table goes up on stream2 behind the previous bulk kernel (the
-    // last reader of the old table) and ahead of the wait for this step's
-    // lattice phase: it is in place by the time that phase ends, and the
-    // bulk kernel starts on the event alone.  (A profiled run showed about
+    // The table goes up on stream2 behind the previous bulk kernel, the last
+    // reader of the old table (which ran on the engine's stream if this step
+    // had no early launch: waited for, or its last workgroups could read the
+    // next step's entries), and ahead of the wait for this step's lattice
+    // phase: it is in place by the time that phase ends, and the bulk kernel
+    // starts on the event alone.  (A profiled run showed about
     // 40 us between the boundaries and the bulk kernel with the copy after
     // the wait; unprofiled capacity is the same within the spread.)
+    LIFE_HIP(hipStreamWaitEvent(s->stream2, s->ev_bulk, 0));
     s->cases_bulk.upload(s->slots.size(), s->stream2);
     LIFE_HIP(hipEventRecord(s->ev_bulk_up, s->stream2));
     s->bulk_up_pending = true;
