@@ -26,9 +26,6 @@ namespace life {
 // few marker counts; freed blocks are therefore kept, by size, for the next
 // array of that size (pinned_take / pinned_give, runtime.cpp), up to a cap,
 // and stay allocated until the process ends.
-void* pinned_take(size_t bytes);
-void pinned_give(void* p, size_t bytes);
-
 template <typename T>
 struct PinnedAllocator {
     using value_type = T;

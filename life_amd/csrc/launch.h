@@ -75,19 +75,30 @@ void launch_convective_speed(const T* src, const GridScalars& g, const double* f
                              bool explicit_state, double* ucol, bool ordered, hipStream_t s);
 template <typename T>
 void launch_init_equilibrium(T* f, const GridScalars& g, const double* rho0, const double* u0, hipStream_t s);
+// State in the reference layout, sites [first, first + n) at a time, to and
+// from page-locked host memory whose first entries are site `first`.
 template <typename T>
 void launch_materialise(const T* f, const GridScalars& g, const double* fibm, const double* rho0, const double* u0,
-                        bool explicit_state, double* f_aos, double* rho, double* u, double* fibm_aos,
-                        hipStream_t s);
+                        bool explicit_state, long long first, long long n, double* f_aos, double* rho, double* u,
+                        double* fibm_aos, hipStream_t s);
 template <typename T>
-void launch_upload(T* f, const GridScalars& g, const double* f_aos, hipStream_t s);
+void launch_upload(T* f, const GridScalars& g, long long first, long long n, const double* f_aos, const double* rho,
+                   const double* u, const double* fibm_in, double* rho0, double* u0, double* fibm, hipStream_t s);
 void launch_init_moments(double* rho0, double* u0, const GridScalars& g, int mode, double ux, double uy,
                          const double* u_in, const BCSite* bc, int nbc, hipStream_t s);
-void launch_fibm_from_aos(double* fibm, const GridScalars& g, const double* fibm_aos, hipStream_t s);
 // NaN velocity scan (GridClass::writeInfo): *flag = smallest lattice id
 // whose |u| is NaN, or ~0 when there is none.
 template <typename T>
 void launch_blowup_scan(const T* f, const GridScalars& g, unsigned long long* flag, hipStream_t s);
+// Copies of 4-byte words, several arrays in one launch (device or
+// page-locked host memory on either side).
+struct WordCopies {
+    const unsigned* src[8];
+    unsigned* dst[8];
+    int words[8];
+    int n;
+};
+void launch_copy_words(const WordCopies& w, hipStream_t s);
 void launch_fill_f64(double* p, double v, long long n, hipStream_t s);
 void launch_fill_i32(int* p, int v, long long n, hipStream_t s);
 

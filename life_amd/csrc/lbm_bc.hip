@@ -265,21 +265,37 @@ void launch_init_equilibrium(T* f, const GridScalars& g, const double* rho0, con
     else k_init_eq<T, false><<<nb, 256, 0, s>>>(f, g, rho0, u0);
 }
 
-// Reference-layout state: f AoS, rho, u (macroscopic with force_xy +
-// force_ibm, as left by IBMNodeClass::updateMacroscopic), force_ibm AoS.
+// Reference-layout state of sites [first, first + n): f AoS, rho, u
+// (macroscopic with force_xy + force_ibm, as left by
+// IBMNodeClass::updateMacroscopic), force_ibm AoS; any output may be null,
+// and site `first` is each output's first.  The outputs are page-locked host
+// memory: bound by the link to the host, so every wavefront stores whole
+// runs of consecutive doubles (the AoS populations through LDS).
+constexpr int kStateBlock = 256;
+
 template <typename T>
-__global__ __launch_bounds__(256) void k_materialise(const T* __restrict__ f, GridScalars g,
-                                                     const double* __restrict__ fibm, const double* __restrict__ rho0,
-                                                     const double* __restrict__ u0, int explicit_state,
-                                                     double* __restrict__ f_aos, double* __restrict__ rho,
-                                                     double* __restrict__ u, double* __restrict__ fibm_aos) {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= g.N) return;
+__global__ __launch_bounds__(kStateBlock) void k_materialise(const T* __restrict__ f, GridScalars g,
+                                                             const double* __restrict__ fibm,
+                                                             const double* __restrict__ rho0,
+                                                             const double* __restrict__ u0, int explicit_state,
+                                                             long long first, long long n,
+                                                             double* __restrict__ f_aos, double* __restrict__ rho,
+                                                             double2* __restrict__ u, double2* __restrict__ fibm_aos) {
+    __shared__ double sh[kStateBlock * kNV];
+    const int t = threadIdx.x;
+    const long long k0 = (long long)blockIdx.x * kStateBlock, k = k0 + t;
+    const bool in = k < n;
+    const long long id = first + (in ? k : 0);
     double fs[kNV];
     load_site(f, g.S, id, fs);
-    if (f_aos)
+    if (f_aos) {
 #pragma unroll
-        for (int v = 0; v < kNV; v++) f_aos[id * kNV + v] = fs[v];
+        for (int v = 0; v < kNV; v++) sh[t * kNV + v] = fs[v];
+        __syncthreads();
+        const int m = (int)(n - k0 < kStateBlock ? n - k0 : kStateBlock) * kNV;
+        for (int q = t; q < m; q += kStateBlock) f_aos[k0 * kNV + q] = sh[q];
+    }
+    if (!in) return;
     if (rho || u) {
         double r, ux, uy;
         if (explicit_state) {
@@ -290,50 +306,80 @@ __global__ __launch_bounds__(256) void k_materialise(const T* __restrict__ f, Gr
             moments64(fs, (g.fcur ? g.fcur[id] : g.Fx) + fibm[id], (g.fcur ? g.fcur[g.S + id] : g.Fy) + fibm[g.S + id],
                       r, ux, uy);
         }
-        if (rho) rho[id] = r;
-        if (u) {
-            u[2 * id] = ux;
-            u[2 * id + 1] = uy;
-        }
+        if (rho) rho[k] = r;
+        if (u) u[k] = make_double2(ux, uy);
     }
-    if (fibm_aos) {
-        fibm_aos[2 * id] = fibm[id];
-        fibm_aos[2 * id + 1] = fibm[g.S + id];
-    }
+    if (fibm_aos) fibm_aos[k] = make_double2(fibm[id], fibm[g.S + id]);
 }
 
 template <typename T>
 void launch_materialise(const T* f, const GridScalars& g, const double* fibm, const double* rho0, const double* u0,
-                        bool explicit_state, double* f_aos, double* rho, double* u, double* fibm_aos,
-                        hipStream_t s) {
-    const unsigned nb = (unsigned)((g.N + 255) / 256);
-    k_materialise<T><<<nb, 256, 0, s>>>(f, g, fibm, rho0, u0, explicit_state ? 1 : 0, f_aos, rho, u, fibm_aos);
+                        bool explicit_state, long long first, long long n, double* f_aos, double* rho, double* u,
+                        double* fibm_aos, hipStream_t s) {
+    if (n <= 0) return;
+    const unsigned nb = (unsigned)((n + kStateBlock - 1) / kStateBlock);
+    k_materialise<T><<<nb, kStateBlock, 0, s>>>(f, g, fibm, rho0, u0, explicit_state ? 1 : 0, first, n, f_aos, rho,
+                                                reinterpret_cast<double2*>(u), reinterpret_cast<double2*>(fibm_aos));
 }
 
+// The reverse: sites [first, first + n) from page-locked host memory (fibm_in
+// may be null).
 template <typename T>
-__global__ __launch_bounds__(256) void k_upload(T* __restrict__ f, GridScalars g, const double* __restrict__ f_aos) {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= g.N) return;
+__global__ __launch_bounds__(kStateBlock) void k_upload(T* __restrict__ f, GridScalars g, long long first, long long n,
+                                                        const double* __restrict__ f_aos,
+                                                        const double* __restrict__ rho, const double2* __restrict__ u,
+                                                        const double2* __restrict__ fibm_in, double* __restrict__ rho0,
+                                                        double* __restrict__ u0, double* __restrict__ fibm) {
+    __shared__ double sh[kStateBlock * kNV];
+    const int t = threadIdx.x;
+    const long long k0 = (long long)blockIdx.x * kStateBlock, k = k0 + t;
+    const int m = (int)(n - k0 < kStateBlock ? n - k0 : kStateBlock) * kNV;
+    double x[kNV];
 #pragma unroll
-    for (int v = 0; v < kNV; v++) Pops<T>::put(f, g.S, v, id, f_aos[id * kNV + v]);
+    for (int v = 0; v < kNV; v++) {
+        const int q = v * kStateBlock + t;
+        x[v] = q < m ? f_aos[k0 * kNV + q] : 0.0;
+    }
+#pragma unroll
+    for (int v = 0; v < kNV; v++) sh[v * kStateBlock + t] = x[v];
+    __syncthreads();
+    if (k >= n) return;
+    const long long id = first + k;
+    const double r = rho[k];
+    const double2 w = u[k];
+#pragma unroll
+    for (int v = 0; v < kNV; v++) Pops<T>::put(f, g.S, v, id, sh[t * kNV + v]);
+    rho0[id] = r;
+    u0[2 * id] = w.x;
+    u0[2 * id + 1] = w.y;
+    if (fibm_in) {
+        const double2 b = fibm_in[k];
+        fibm[id] = b.x;
+        fibm[g.S + id] = b.y;
+    }
 }
 
 template <typename T>
-void launch_upload(T* f, const GridScalars& g, const double* f_aos, hipStream_t s) {
-    const unsigned nb = (unsigned)((g.N + 255) / 256);
-    k_upload<T><<<nb, 256, 0, s>>>(f, g, f_aos);
+void launch_upload(T* f, const GridScalars& g, long long first, long long n, const double* f_aos, const double* rho,
+                   const double* u, const double* fibm_in, double* rho0, double* u0, double* fibm, hipStream_t s) {
+    if (n <= 0) return;
+    const unsigned nb = (unsigned)((n + kStateBlock - 1) / kStateBlock);
+    k_upload<T><<<nb, kStateBlock, 0, s>>>(f, g, first, n, f_aos, rho, reinterpret_cast<const double2*>(u),
+                                           reinterpret_cast<const double2*>(fibm_in), rho0, u0, fibm);
 }
 
-__global__ void k_fibm_from_aos(double* __restrict__ fibm, GridScalars g, const double* __restrict__ a) {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= g.N) return;
-    fibm[id] = a[2 * id];
-    fibm[g.S + id] = a[2 * id + 1];
+__global__ __launch_bounds__(256) void k_copy_words(WordCopies w) {
+    const unsigned* __restrict__ src = w.src[blockIdx.y];
+    unsigned* __restrict__ dst = w.dst[blockIdx.y];
+    for (int k = blockIdx.x * 256 + threadIdx.x; k < w.words[blockIdx.y]; k += (int)gridDim.x * 256) dst[k] = src[k];
 }
 
-void launch_fibm_from_aos(double* fibm, const GridScalars& g, const double* fibm_aos, hipStream_t s) {
-    const unsigned nb = (unsigned)((g.N + 255) / 256);
-    k_fibm_from_aos<<<nb, 256, 0, s>>>(fibm, g, fibm_aos);
+void launch_copy_words(const WordCopies& w, hipStream_t s) {
+    int most = 0;
+    for (int q = 0; q < w.n; q++) most = most > w.words[q] ? most : w.words[q];
+    if (most <= 0) return;
+    const int nb = (most + 255) / 256;
+    k_copy_words<<<dim3((unsigned)(nb < 256 ? nb : 256), (unsigned)w.n), 256, 0, s>>>(w);
 }
 
 __global__ void k_fill_f64(double* p, double v, long long n) {
@@ -433,8 +479,10 @@ void launch_blowup_scan(const T* f, const GridScalars& g, unsigned long long* fl
                                              double*, bool, hipStream_t);                                            \
     template void launch_init_equilibrium<T>(T*, const GridScalars&, const double*, const double*, hipStream_t);     \
     template void launch_materialise<T>(const T*, const GridScalars&, const double*, const double*, const double*,   \
-                                        bool, double*, double*, double*, double*, hipStream_t);                      \
-    template void launch_upload<T>(T*, const GridScalars&, const double*, hipStream_t);                             \
+                                        bool, long long, long long, double*, double*, double*, double*,              \
+                                        hipStream_t);                                                                \
+    template void launch_upload<T>(T*, const GridScalars&, long long, long long, const double*, const double*,       \
+                                   const double*, const double*, double*, double*, double*, hipStream_t);            \
     template void launch_bc_batch<T>(bool, const CaseDev*, const int*, int, int, hipStream_t);                       \
     template void launch_convective_batch<T>(const CaseDev*, const int*, int, int, bool, hipStream_t);
 LIFE_INST(double)

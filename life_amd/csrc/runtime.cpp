@@ -5,11 +5,13 @@
 
 #include "lu.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <new>
@@ -74,6 +76,46 @@ void pinned_give(void* p, size_t bytes) {
     }
     (void)hipHostFree(p);
 }
+
+namespace {
+// Small page-locked slots (a grid's overflow flags), cut from shared pages:
+// page-locking memory for each grid would cost more than building a small
+// one.  Pages are freed with the pools.
+struct PinnedSlots {
+    static constexpr size_t kSlot = 64, kPage = 4096;
+    std::mutex mu;
+    std::vector<char*> pages, free;
+    char* take() {
+        std::lock_guard<std::mutex> lock(mu);
+        if (free.empty()) {
+            void* p = nullptr;
+            if (hipHostMalloc(&p, kPage, hipHostMallocDefault) != hipSuccess) throw std::bad_alloc();
+            pages.push_back(static_cast<char*>(p));
+            for (size_t o = 0; o < kPage; o += kSlot) free.push_back(pages.back() + o);
+        }
+        char* s = free.back();
+        free.pop_back();
+        return s;
+    }
+    void give(void* s) {
+        if (!s) return;
+        std::lock_guard<std::mutex> lock(mu);
+        free.push_back(static_cast<char*>(s));
+    }
+    // With every slot given back.
+    void release() {
+        std::lock_guard<std::mutex> lock(mu);
+        if (free.size() != pages.size() * (kPage / kSlot)) return;
+        for (char* p : pages) (void)hipHostFree(p);
+        pages.clear();
+        free.clear();
+    }
+};
+PinnedSlots& pinned_slots() {
+    static PinnedSlots* s = new PinnedSlots();  // never destroyed, like the blocks above
+    return *s;
+}
+}  // namespace
 
 static thread_local std::string g_error;
 
@@ -319,6 +361,111 @@ GridScalars step_scalars(const life_grid& g, int t) {
     }
     return s;
 }
+
+namespace {
+
+// One transfer of a grid's state in the reference layout, in chunks of sites
+// through page-locked buffers: the device reads or writes a buffer over the
+// link (launch_materialise, launch_upload) while the host's threads copy
+// others from or to the caller's arrays.  A copy straight to pageable memory
+// runs at 18 GB/s, this at the link's rate (57 GB/s) as far as the host's
+// threads keep up, and needs no device memory: 4096 x 2048, rho and u
+// (201 MB) 12.0 -> 4.2 ms, 8192 x 4096 47 -> 15.  The buffers come from the pool of page-locked blocks and go
+// back to it.
+class StateChunks {
+  public:
+    struct Part {
+        long long first, n;
+        double *f, *rho, *u, *fibm;
+    };
+    StateChunks(life_grid* g, double* f, double* rho, double* u, double* fibm) : g_(g), user_{f, rho, u, fibm} {
+        size_t per = 0;  // doubles per site
+        for (int a = 0; a < 4; a++)
+            if (user_[a]) per += kWidth[a];
+        const size_t N = (size_t)g->g.N;
+        if (per == 0) return;
+        // buffers of a power of two, so that lattices of many sizes share them
+        bytes_ = kMinBytes;
+        while (bytes_ < kMaxBytes && bytes_ < N * per * sizeof(double)) bytes_ *= 2;
+        sites_ = bytes_ / (per * sizeof(double));
+        if (sites_ > 64) sites_ = sites_ / 64 * 64;
+        count_ = (N + sites_ - 1) / sites_;
+        depth_ = count_ < kDepth ? count_ : kDepth;
+        for (size_t b = 0; b < depth_; b++) {
+            buf_[b] = static_cast<double*>(pinned_take(bytes_));
+            if (!g->ev_state[b]) LIFE_HIP(hipEventCreateWithFlags(&g->ev_state[b], hipEventDisableTiming));
+        }
+    }
+    StateChunks(const StateChunks&) = delete;
+    StateChunks& operator=(const StateChunks&) = delete;
+    ~StateChunks() {
+        // the device is done with the buffers (an error may have come between)
+        if (open_) (void)hipStreamSynchronize(g_->stream);
+        for (size_t b = 0; b < depth_; b++)
+            if (buf_[b]) pinned_give(buf_[b], bytes_);
+    }
+    size_t count() const { return count_; }
+    size_t depth() const { return depth_; }
+    Part part(size_t k) const {
+        Part p{(long long)(k * sites_), 0, nullptr, nullptr, nullptr, nullptr};
+        p.n = (long long)std::min(sites_, (size_t)g_->g.N - k * sites_);
+        double* at = buf_[k % depth_];
+        double** out[4] = {&p.f, &p.rho, &p.u, &p.fibm};
+        for (int a = 0; a < 4; a++) {
+            if (!user_[a]) continue;
+            *out[a] = at;
+            at += kWidth[a] * sites_;
+        }
+        return p;
+    }
+    // Chunk k's launch is queued.
+    void record(size_t k) {
+        open_ = true;
+        LIFE_HIP(hipGetLastError());
+        LIFE_HIP(hipEventRecord(g_->ev_state[k % depth_], g_->stream));
+    }
+    void wait(size_t k) {
+        LIFE_HIP(hipEventSynchronize(g_->ev_state[k % depth_]));
+        if (k + 1 == count_) open_ = false;
+    }
+    // Chunk k between its buffer and the caller's arrays.
+    void copy(size_t k, bool to_user) const {
+        const Part p = part(k);
+        double* buf[4] = {p.f, p.rho, p.u, p.fibm};
+        struct Piece {
+            double *dst, *src;
+            size_t n;
+        };
+        std::vector<Piece> pieces;
+        constexpr size_t kPiece = 1 << 15;  // doubles a thread takes at a time
+        for (int a = 0; a < 4; a++) {
+            if (!user_[a]) continue;
+            const size_t n = kWidth[a] * (size_t)p.n;
+            double* user = user_[a] + kWidth[a] * (size_t)p.first;
+            for (size_t o = 0; o < n; o += kPiece) {
+                const size_t m = std::min(kPiece, n - o);
+                if (to_user) pieces.push_back({user + o, buf[a] + o, m});
+                else pieces.push_back({buf[a] + o, user + o, m});
+            }
+        }
+        const int np = (int)pieces.size();
+#pragma omp parallel for schedule(dynamic, 1) if (np > 4)
+        for (int q = 0; q < np; q++) std::memcpy(pieces[q].dst, pieces[q].src, pieces[q].n * sizeof(double));
+    }
+
+  private:
+    static constexpr size_t kWidth[4] = {9, 1, 2, 2};  // doubles per site of f, rho, u, force_ibm
+    static constexpr size_t kMinBytes = size_t(64) << 10, kMaxBytes = size_t(16) << 20;
+    static constexpr size_t kDepth = life_grid::kStateDepth;
+    life_grid* g_;
+    double* user_[4];
+    double* buf_[kDepth] = {};
+    size_t bytes_ = 0, sites_ = 1, count_ = 0, depth_ = 0;
+    bool open_ = false;
+};
+constexpr size_t StateChunks::kWidth[4];
+
+}  // namespace
 
 void lbm_join(life_grid* g) {
     if (!g->tail_pending) return;
@@ -624,8 +771,83 @@ void ibm_find_support(life_grid* g, int flexible_only) {
     LIFE_HIP(hipGetLastError());
 }
 
+namespace {
+constexpr size_t kStageMatrix = size_t(512) << 10;
+
+// The grid's page-locked block for marker arrays, at least `bytes`.  Its
+// last reader on the device is done when this returns.
+char* stage(life_grid* g, size_t bytes) {
+    if (g->stage_busy) {
+        LIFE_HIP(hipEventSynchronize(g->ev_stage));
+        g->stage_busy = false;
+    }
+    if (bytes > g->stage_bytes) {
+        LIFE_HIP(hipStreamSynchronize(g->stream));
+        size_t b = 4096;
+        while (b < bytes) b *= 2;
+        pinned_give(g->stage, g->stage_bytes);
+        g->stage = nullptr;
+        g->stage_bytes = 0;
+        g->stage = static_cast<char*>(pinned_take(b));
+        g->stage_bytes = b;
+    }
+    return g->stage;
+}
+
+struct MarkerCopy {
+    void* host;
+    void* dev;
+    size_t bytes;
+};
+
+// Marker arrays to the host (which waits) or to the device (which does
+// not), all of them in one launch through the page-locked block: a copy of
+// its own for each array to or from pageable memory costs 10-20 us.
+void move_markers(life_grid* g, std::initializer_list<MarkerCopy> copies, bool to_host) {
+    WordCopies w{};
+    size_t bytes = 0;
+    for (const MarkerCopy& c : copies)
+        if (c.host) bytes += (c.bytes + 15) / 16 * 16;
+    if (bytes == 0) return;
+    char* const base = stage(g, bytes);
+    size_t at = 0;
+    for (const MarkerCopy& c : copies) {
+        if (!c.host || c.bytes == 0) continue;
+        if (!to_host) std::memcpy(base + at, c.host, c.bytes);
+        w.src[w.n] = reinterpret_cast<const unsigned*>(to_host ? c.dev : base + at);
+        w.dst[w.n] = reinterpret_cast<unsigned*>(to_host ? base + at : c.dev);
+        w.words[w.n++] = (int)(c.bytes / sizeof(unsigned));
+        at += (c.bytes + 15) / 16 * 16;
+    }
+    launch_copy_words(w, g->stream);
+    LIFE_HIP(hipGetLastError());
+    if (!to_host) {
+        if (!g->ev_stage) LIFE_HIP(hipEventCreateWithFlags(&g->ev_stage, hipEventDisableTiming));
+        LIFE_HIP(hipEventRecord(g->ev_stage, g->stream));
+        g->stage_busy = true;
+        return;
+    }
+    LIFE_HIP(hipStreamSynchronize(g->stream));
+    at = 0;
+    for (const MarkerCopy& c : copies) {
+        if (!c.host || c.bytes == 0) continue;
+        std::memcpy(c.host, base + at, c.bytes);
+        at += (c.bytes + 15) / 16 * 16;
+    }
+}
+}  // namespace
+
 void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host) {
     const size_t need = (size_t)n * n;
+    if (need * sizeof(double) <= kStageMatrix) {
+        // small systems: assembled straight into page-locked memory
+        double* A = reinterpret_cast<double*>(stage(g, need * sizeof(double)));
+        launch_epsilon_matrix(g->md, g->g, first, n, A, g->stream);
+        LIFE_HIP(hipGetLastError());
+        LIFE_HIP(hipStreamSynchronize(g->stream));
+        std::memcpy(A_host, A, need * sizeof(double));
+        return;
+    }
     if (need > g->epsA_cap) {
         dfree(g->epsA);
         g->epsA = dalloc<double>(need);
@@ -694,9 +916,8 @@ std::vector<int> ibm_epsilon_band_dense(const life_grid* g) {
 
 void check_flags(life_grid* g) {
     if (!g->flags) return;
-    int h[2] = {0, 0};
-    LIFE_HIP(hipMemcpyAsync(h, g->flags, sizeof h, hipMemcpyDeviceToHost, g->stream));
     LIFE_HIP(hipStreamSynchronize(g->stream));
+    const volatile int* h = g->flags;
     if (h[0]) throw std::runtime_error("Support buffer size is not big enough for number of support points");
     if (h[1]) throw std::runtime_error("more than 64 markers share one support site");
 }
@@ -707,8 +928,9 @@ static void free_markers(life_grid* g) {
                     (void*)m.supp_cnt, (void*)m.supp_site, (void*)m.supp_ij, (void*)m.supp_delta,
                     (void*)g->body_first, (void*)g->body_n, (void*)g->body_flex, (void*)g->sc.site_count,
                     (void*)g->sc.site_uid, (void*)g->sc.uniq, (void*)g->sc.uniq_n, (void*)g->sc.pair_slot,
-                    (void*)g->sc.list, (void*)g->flags})
+                    (void*)g->sc.list})
         dfree(p);
+    pinned_slots().give(g->flags);
     m = MarkerDev{};
     g->sc = SpreadScratch{};
     g->body_first = g->body_n = g->body_flex = nullptr;
@@ -787,6 +1009,7 @@ static void release_pools(bool streams) {
         dc.bytes = 0;
     }
     pinned_release_all();
+    pinned_slots().release();
     if (!streams) return;
     {
         std::lock_guard<std::mutex> lock(g_stream_mu);
@@ -1109,6 +1332,10 @@ int life_grid_destroy(life_grid* g) {
         if (g->blow_h) (void)hipHostFree(g->blow_h);
         dfree(g->blow_d);
         if (g->ev_blow) (void)hipEventDestroy(g->ev_blow);
+        for (hipEvent_t e : g->ev_state)
+            if (e) (void)hipEventDestroy(e);
+        if (g->ev_stage) (void)hipEventDestroy(g->ev_stage);
+        pinned_give(g->stage, g->stage_bytes);
         for (hipEvent_t e : {g->ev_a, g->ev_b, g->ev_k0, g->ev_k1, g->ev_ready, g->ev_bulk, g->ev_tail})
             if (e) (void)hipEventDestroy(e);
         // the coupling stream of a split grid is the device's, not the grid's
@@ -1164,30 +1391,24 @@ int life_grid_download(life_grid* g, double* f_aos, double* rho, double* u, doub
     return guarded([&] {
         LIFE_HIP(hipSetDevice(g->device));
         lbm_join(g);
-        const size_t N = (size_t)g->g.N;
-        double *df = nullptr, *dr = nullptr, *du = nullptr, *db = nullptr;
-        try {
-            if (f_aos) df = dalloc<double>(9 * N);
-            if (rho) dr = dalloc<double>(N);
-            if (u) du = dalloc<double>(2 * N);
-            if (force_ibm) db = dalloc<double>(2 * N);
+        StateChunks ch(g, f_aos, rho, u, force_ibm);
+        const size_t n = ch.count(), depth = ch.depth();
+        // a buffer is filled by the device while the host empties the others
+        for (size_t k = 0; k < n + depth; k++) {
+            if (k >= depth) {
+                ch.wait(k - depth);
+                ch.copy(k - depth, true);
+            }
+            if (k >= n) continue;
+            const StateChunks::Part p = ch.part(k);
             if (g->prec == kFP64)
                 launch_materialise<double>(static_cast<const double*>(g->f[g->cur]), g->g, g->fibm, g->rho0, g->u0,
-                                           g->explicit_state, df, dr, du, db, g->stream);
+                                           g->explicit_state, p.first, p.n, p.f, p.rho, p.u, p.fibm, g->stream);
             else
                 launch_materialise<float>(static_cast<const float*>(g->f[g->cur]), g->g, g->fibm, g->rho0, g->u0,
-                                          g->explicit_state, df, dr, du, db, g->stream);
-            LIFE_HIP(hipGetLastError());
-            if (df) LIFE_HIP(hipMemcpyAsync(f_aos, df, 9 * N * sizeof(double), hipMemcpyDeviceToHost, g->stream));
-            if (dr) LIFE_HIP(hipMemcpyAsync(rho, dr, N * sizeof(double), hipMemcpyDeviceToHost, g->stream));
-            if (du) LIFE_HIP(hipMemcpyAsync(u, du, 2 * N * sizeof(double), hipMemcpyDeviceToHost, g->stream));
-            if (db) LIFE_HIP(hipMemcpyAsync(force_ibm, db, 2 * N * sizeof(double), hipMemcpyDeviceToHost, g->stream));
-            LIFE_HIP(hipStreamSynchronize(g->stream));
-        } catch (...) {
-            dfree(df), dfree(dr), dfree(du), dfree(db);
-            throw;
+                                          g->explicit_state, p.first, p.n, p.f, p.rho, p.u, p.fibm, g->stream);
+            ch.record(k);
         }
-        dfree(df), dfree(dr), dfree(du), dfree(db);
     });
 }
 
@@ -1196,29 +1417,22 @@ int life_grid_upload(life_grid* g, const double* f_aos, const double* rho, const
         if (!f_aos || !rho || !u) throw std::runtime_error("life_grid_upload needs f, rho and u");
         LIFE_HIP(hipSetDevice(g->device));
         lbm_join(g);
-        const size_t N = (size_t)g->g.N;
-        double* df = dalloc<double>(9 * N);
-        double* db = nullptr;
-        try {
-            LIFE_HIP(hipMemcpyAsync(df, f_aos, 9 * N * sizeof(double), hipMemcpyHostToDevice, g->stream));
-            LIFE_HIP(hipMemcpyAsync(g->rho0, rho, N * sizeof(double), hipMemcpyHostToDevice, g->stream));
-            LIFE_HIP(hipMemcpyAsync(g->u0, u, 2 * N * sizeof(double), hipMemcpyHostToDevice, g->stream));
-            if (g->prec == kFP64) launch_upload<double>(static_cast<double*>(g->f[g->cur]), g->g, df, g->stream);
-            else launch_upload<float>(static_cast<float*>(g->f[g->cur]), g->g, df, g->stream);
-            if (force_ibm) {
-                db = dalloc<double>(2 * N);
-                LIFE_HIP(hipMemcpyAsync(db, force_ibm, 2 * N * sizeof(double), hipMemcpyHostToDevice, g->stream));
-                launch_fibm_from_aos(g->fibm, g->g, db, g->stream);
-            } else {
-                launch_fill_f64(g->fibm, 0.0, 2 * g->g.S, g->stream);
-            }
-            LIFE_HIP(hipGetLastError());
-            LIFE_HIP(hipStreamSynchronize(g->stream));
-        } catch (...) {
-            dfree(df), dfree(db);
-            throw;
+        StateChunks ch(g, const_cast<double*>(f_aos), const_cast<double*>(rho), const_cast<double*>(u),
+                       const_cast<double*>(force_ibm));
+        if (!force_ibm) launch_fill_f64(g->fibm, 0.0, 2 * g->g.S, g->stream);
+        for (size_t k = 0; k < ch.count(); k++) {
+            if (k >= ch.depth()) ch.wait(k - ch.depth());
+            ch.copy(k, false);
+            const StateChunks::Part p = ch.part(k);
+            if (g->prec == kFP64)
+                launch_upload<double>(static_cast<double*>(g->f[g->cur]), g->g, p.first, p.n, p.f, p.rho, p.u, p.fibm,
+                                      g->rho0, g->u0, g->fibm, g->stream);
+            else
+                launch_upload<float>(static_cast<float*>(g->f[g->cur]), g->g, p.first, p.n, p.f, p.rho, p.u, p.fibm,
+                                     g->rho0, g->u0, g->fibm, g->stream);
+            ch.record(k);
         }
-        dfree(df), dfree(db);
+        LIFE_HIP(hipStreamSynchronize(g->stream));
         g->explicit_state = true;
         g->dense_clear_next = true;
     });
@@ -1270,7 +1484,10 @@ int life_ibm_set_markers(life_grid* g, int n, const double* pos, const double* v
         g->body_first = dalloc<int>(nbodies);
         g->body_n = dalloc<int>(nbodies);
         g->body_flex = dalloc<int>(nbodies);
-        g->flags = dalloc<int>(2);
+        // in page-locked host memory: a kernel writes one only on an overflow,
+        // and the host reads them without a copy
+        g->flags = reinterpret_cast<int*>(pinned_slots().take());
+        g->flags[0] = g->flags[1] = 0;
         m.body_first = g->body_first;
         m.body_n = g->body_n;
         m.body_flex = g->body_flex;
@@ -1300,7 +1517,6 @@ int life_ibm_set_markers(life_grid* g, int n, const double* pos, const double* v
         launch_fill_f64(m.eps, 0.0, n, s);
         launch_fill_f64(m.ds, 0.0, n, s);
         launch_fill_i32(m.supp_cnt, 0, n, s);
-        launch_fill_i32(g->flags, 0, 2, s);
         launch_fill_i32(sc.site_count, 0, g->g.N, s);
         launch_fill_i32(sc.uniq_n, 0, 1, s);
         LIFE_HIP(hipGetLastError());
@@ -1313,8 +1529,8 @@ int life_ibm_update_markers(life_grid* g, const double* pos, const double* vel) 
     return guarded([&] {
         LIFE_HIP(hipSetDevice(g->device));
         const size_t n = (size_t)g->md.n;
-        if (pos) LIFE_HIP(hipMemcpyAsync(g->md.pos, pos, sizeof(double) * 2 * n, hipMemcpyHostToDevice, g->stream));
-        if (vel) LIFE_HIP(hipMemcpyAsync(g->md.vel, vel, sizeof(double) * 2 * n, hipMemcpyHostToDevice, g->stream));
+        move_markers(g, {{const_cast<double*>(pos), g->md.pos, 16 * n}, {const_cast<double*>(vel), g->md.vel, 16 * n}},
+                     false);
     });
 }
 
@@ -1337,8 +1553,7 @@ int life_ibm_epsilon_matrix(life_grid* g, int first, int n, double* A) {
 int life_ibm_set_epsilon(life_grid* g, const double* eps) {
     return guarded([&] {
         LIFE_HIP(hipSetDevice(g->device));
-        LIFE_HIP(hipMemcpyAsync(g->md.eps, eps, sizeof(double) * g->md.n, hipMemcpyHostToDevice, g->stream));
-        LIFE_HIP(hipStreamSynchronize(g->stream));
+        move_markers(g, {{const_cast<double*>(eps), g->md.eps, sizeof(double) * g->md.n}}, false);
     });
 }
 
@@ -1346,11 +1561,7 @@ int life_ibm_interpolate(life_grid* g, double* force) {
     return guarded([&] {
         LIFE_HIP(hipSetDevice(g->device));
         ibm_interpolate(g);
-        if (force) {
-            LIFE_HIP(hipMemcpyAsync(force, g->md.force, sizeof(double) * 2 * g->md.n, hipMemcpyDeviceToHost,
-                                    g->stream));
-            LIFE_HIP(hipStreamSynchronize(g->stream));
-        }
+        if (force) move_markers(g, {{force, g->md.force, 16 * (size_t)g->md.n}}, true);
     });
 }
 
@@ -1366,19 +1577,17 @@ int life_ibm_download(life_grid* g, double* pos, double* vel, double* force, dou
     return guarded([&] {
         LIFE_HIP(hipSetDevice(g->device));
         const size_t n = (size_t)g->md.n;
-        hipStream_t s = g->stream;
-        auto cp = [&](void* dst, const void* src, size_t bytes) {
-            if (dst && bytes) LIFE_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-        };
-        cp(pos, g->md.pos, 16 * n);
-        cp(vel, g->md.vel, 16 * n);
-        cp(force, g->md.force, 16 * n);
-        cp(eps, g->md.eps, 8 * n);
-        cp(ds, g->md.ds, 8 * n);
-        cp(supp_count, g->md.supp_cnt, 4 * n);
-        cp(supp_ij, g->md.supp_ij, 4 * n * kSupp * 2);
-        cp(supp_delta, g->md.supp_delta, 8 * n * kSupp);
-        LIFE_HIP(hipStreamSynchronize(s));
+        const MarkerDev& m = g->md;
+        move_markers(g,
+                     {{pos, m.pos, 16 * n},
+                      {vel, m.vel, 16 * n},
+                      {force, m.force, 16 * n},
+                      {eps, m.eps, 8 * n},
+                      {ds, m.ds, 8 * n},
+                      {supp_count, m.supp_cnt, 4 * n},
+                      {supp_ij, m.supp_ij, 4 * n * kSupp * 2},
+                      {supp_delta, m.supp_delta, 8 * n * kSupp}},
+                     true);
         check_flags(g);
     });
 }

@@ -35,6 +35,10 @@ CaseScalars derive_scalars(const life_params& p);
 // GridClass::getRampCoefficient, Grid.cpp:548-556.
 double ramp_coefficient(const life_params& p, double Dt, int t);
 
+// Page-locked host memory from a pool of freed blocks (runtime.cpp).
+void* pinned_take(size_t bytes);
+void pinned_give(void* p, size_t bytes);
+
 template <typename T>
 T* dalloc(size_t n) {
     void* p = nullptr;
@@ -93,7 +97,7 @@ struct life_grid {
     int* body_flex = nullptr;
     std::vector<int> body_first_h, body_n_h, body_flex_h;
     life::SpreadScratch sc{};
-    int* flags = nullptr;  // [0] support overflow, [1] spread overflow
+    int* flags = nullptr;  // page-locked: [0] support overflow, [1] spread overflow
     double* epsA = nullptr;  // epsilon matrix scratch
     size_t epsA_cap = 0;
     // banded epsilon systems (flexible bodies)
@@ -129,6 +133,15 @@ struct life_grid {
     unsigned long long* blow_d = nullptr;
     unsigned long long* blow_h = nullptr;  // page-locked
     hipEvent_t ev_blow = nullptr;
+    // buffers of a state transfer in flight at once, an event each
+    static constexpr size_t kStateDepth = 4;
+    hipEvent_t ev_state[kStateDepth] = {};
+    // page-locked block for marker arrays on their way to or from the device;
+    // busy: the device may still read it (ev_stage recorded)
+    char* stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t ev_stage = nullptr;
+    bool stage_busy = false;
     int blow_t = -1;  // step of the scan in flight, -1 none
 
     void* f_cur() { return f[cur]; }
