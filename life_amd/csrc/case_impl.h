@@ -12,6 +12,7 @@
 
 #include "fem.h"
 #include "fem_dev.h"
+#include "lu.h"
 #include "runtime.h"
 
 namespace life {
@@ -103,8 +104,7 @@ struct life_case {
     int subIt = 0, simDOFs = 0;
     double subRes = 0.0, subNum = 0.0, subDen = 0.0, relax = 1.0;
     std::vector<double> A;
-    std::vector<double> luw;
-    std::vector<int> luiw;
+    life::LuWork luw;
     std::vector<double> rhs, sol;
     bool forces_on_host = false;
     std::unique_ptr<life::PhaseTimes> timing{new life::PhaseTimes()};

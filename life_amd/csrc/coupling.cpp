@@ -291,13 +291,21 @@ void life::case_fem(life_case* c) {
     c->subIt++;
 }
 
-// computeEpsilon's solve of one system by the dense path.
+// computeEpsilon's solve of one system on the host: its non-zeros from the
+// device, or the whole matrix where a row has too many of them.
 void life::case_solve_eps_dense(life_case* c, int first, int n) {
-    c->A.resize((size_t)n * n);
-    ibm_epsilon_matrix(c->g, first, n, c->A.data());
+    if (n <= 0) return;
     c->rhs.assign(n, 1.0);
     c->sol.assign(n, 0.0);
-    lu_solve_sparse(n, 0, c->A.data(), c->rhs.data(), c->sol.data(), c->luw, c->luiw);
+    const int *count, *col;
+    const double* val;
+    if (ibm_epsilon_rows(c->g, first, n, count, col, val)) {
+        lu_solve_rows(n, kEpsRowCap, count, col, val, c->rhs.data(), c->sol.data(), c->luw);
+    } else {
+        c->A.resize((size_t)n * n);
+        ibm_epsilon_matrix(c->g, first, n, c->A.data());
+        lu_solve_sparse(n, 0, c->A.data(), c->rhs.data(), c->sol.data(), c->luw);
+    }
     std::memcpy(&c->eps[first], c->sol.data(), sizeof(double) * n);
     LIFE_HIP(hipMemcpyAsync(c->g->md.eps + first, &c->eps[first], sizeof(double) * n, hipMemcpyHostToDevice,
                             c->g->stream));

@@ -137,6 +137,11 @@ void launch_find_support(const MarkerDev& m, const GridScalars& g, int flexible_
 void launch_support_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s);
 void launch_compute_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s);
 void launch_epsilon_matrix(const MarkerDev& m, const GridScalars& g, int first, int n, double* A, hipStream_t s);
+// Its non-zeros row by row: count[r] of them (counted past kEpsRowCap, but not
+// stored), columns ascending in col[r * kEpsRowCap ..], values in val.
+constexpr int kEpsRowCap = 32;
+void launch_epsilon_rows(const MarkerDev& m, const GridScalars& g, int first, int n, int* count, int* col, double* val,
+                         hipStream_t s);
 // Banded epsilon systems (one per entry of sys_first/sys_n), assembled and
 // solved on the device into m.eps; outside[k] is written: 1 for a system whose
 // matrix is not confined to the band (left for the dense host path).  cr:

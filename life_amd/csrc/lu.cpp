@@ -1,56 +1,91 @@
 #include "lu.h"
 
+#include <emmintrin.h>
+
 #include <cmath>
 #include <cstring>
 
 namespace life {
 
-int lu_solve_sparse(int n, int bc, const double* A, const double* b, double* x, std::vector<double>& work,
-                    std::vector<int>& iwork) {
-    const int m = n - bc;
-    work.resize((size_t)m * m + m);
-    iwork.resize(m);
-    double* B = work.data();
-    double* y = B + (size_t)m * m;
-    for (int i = 0; i < m; i++) {
-        std::memcpy(B + (size_t)i * m, A + (size_t)(i + bc) * n + bc, sizeof(double) * m);
-        y[i] = b[i + bc];
+namespace {
+
+// The elimination on the m rows in w (rows B, their non-zero patterns bits,
+// right-hand sides y), into x[0..m).  Rows stay where they are: row[p] is the
+// row at position p of the canonical algorithm, pos its inverse.
+//
+// A row takes part from the column of its first non-zero on (before that its
+// entries in the pivot column are zero), so a step looks at the active rows
+// only, and at the pattern of the pivot row instead of all columns.
+int eliminate(LuWork& w, int m, double* x) {
+    const int words = (m + 63) / 64;
+    double* const B = w.B.data();
+    double* const y = w.y.data();
+    uint64_t* const bits = w.bits.data();
+    auto row = [&](int r) { return B + (size_t)r * m; };
+    auto pat = [&](int r) { return bits + (size_t)r * words; };
+    w.row.resize(m);
+    w.pos.resize(m);
+    w.head.assign(m + 1, -1);
+    w.next.resize(m);
+    w.cols.resize(m);
+    w.act.clear();
+    for (int r = 0; r < m; r++) {
+        w.row[r] = w.pos[r] = r;
+        int f = m;  // first non-zero column
+        for (int q = 0; q < words && f == m; q++)
+            if (pat(r)[q]) f = q * 64 + __builtin_ctzll(pat(r)[q]);
+        w.next[r] = w.head[f];
+        w.head[f] = r;
     }
     int info = 0;
-    int* cols = iwork.data();
+    int* const cols = w.cols.data();
     for (int k = 0; k < m; k++) {
+        for (int r = w.head[k]; r >= 0; r = w.next[r])
+            if (w.pos[r] >= k) w.act.push_back(r);  // (else U's row of a column without a pivot)
+        // first row of maximum magnitude, by position
         int p = k;
-        double best = std::fabs(B[(size_t)k * m + k]);
-        for (int i = k + 1; i < m; i++) {
-            const double a = std::fabs(B[(size_t)i * m + k]);
-            if (a > best) {
+        double best = std::fabs(row(w.row[k])[k]);
+        for (int r : w.act) {
+            const double a = std::fabs(row(r)[k]);
+            if (a > best || (a == best && w.pos[r] < p)) {
                 best = a;
-                p = i;
+                p = w.pos[r];
             }
         }
         if (best == 0.0) {
             if (!info) info = k + 1;
+            // the row at position k keeps its place, as U's row k
+            for (size_t q = 0; q < w.act.size(); q++)
+                if (w.pos[w.act[q]] == k) {
+                    w.act[q] = w.act.back();
+                    w.act.pop_back();
+                    break;
+                }
             continue;
         }
-        if (p != k) {
-            double* rk = B + (size_t)k * m;
-            double* rp = B + (size_t)p * m;
-            for (int j = 0; j < m; j++) {
-                const double t = rk[j];
-                rk[j] = rp[j];
-                rp[j] = t;
-            }
-            const double t = y[k];
-            y[k] = y[p];
-            y[p] = t;
-        }
-        const double* rk = B + (size_t)k * m;
+        const int rp = w.row[p], rq = w.row[k];
+        w.row[p] = rq;
+        w.pos[rq] = p;
+        w.row[k] = rp;
+        w.pos[rp] = k;
+        const double* const rk = row(rp);
+        const uint64_t* const pk = pat(rp);
         const double piv = rk[k];
         int nc = 0;
-        for (int j = k + 1; j < m; j++)
-            if (rk[j] != 0.0) cols[nc++] = j;
-        for (int i = k + 1; i < m; i++) {
-            double* ri = B + (size_t)i * m;
+        const int w0 = (k + 1) / 64;
+        for (int q = w0; q < words; q++) {
+            uint64_t b = pk[q];
+            if (q == w0) b &= ~uint64_t(0) << ((k + 1) % 64);
+            for (; b; b &= b - 1) {
+                const int j = q * 64 + __builtin_ctzll(b);
+                if (rk[j] != 0.0) cols[nc++] = j;
+            }
+        }
+        size_t keep = 0;
+        for (int r : w.act) {
+            if (r == rp) continue;
+            w.act[keep++] = r;
+            double* const ri = row(r);
             if (ri[k] == 0.0) continue;
             const double l = ri[k] / piv;
             ri[k] = l;
@@ -58,17 +93,83 @@ int lu_solve_sparse(int n, int bc, const double* A, const double* b, double* x, 
                 const int j = cols[q];
                 ri[j] = ri[j] - l * rk[j];
             }
-            y[i] = y[i] - l * y[k];
+            uint64_t* const pi = pat(r);
+            for (int q = w0; q < words; q++) pi[q] |= pk[q];
+            y[r] = y[r] - l * y[rp];
         }
+        w.act.resize(keep);
     }
     for (int i = m - 1; i >= 0; i--) {
-        const double* ri = B + (size_t)i * m;
-        double s = y[i];
-        for (int j = i + 1; j < m; j++)
-            if (ri[j] != 0.0) s = s - ri[j] * x[j + bc];
-        x[i + bc] = s / ri[i];
+        const int r = w.row[i];
+        const double* const ri = row(r);
+        const uint64_t* const pi = pat(r);
+        double s = y[r];
+        const int w0 = (i + 1) / 64;
+        for (int q = w0; q < words; q++) {
+            uint64_t b = pi[q];
+            if (q == w0) b &= ~uint64_t(0) << ((i + 1) % 64);
+            for (; b; b &= b - 1) {
+                const int j = q * 64 + __builtin_ctzll(b);
+                if (ri[j] != 0.0) s = s - ri[j] * x[j];
+            }
+        }
+        x[i] = s / ri[i];
     }
+    return info;
+}
+
+}  // namespace
+
+int lu_solve_sparse(int n, int bc, const double* A, const double* b, double* x, LuWork& w) {
+    const int m = n - bc, words = (m + 63) / 64;
+    w.rows_m = 0;  // B is overwritten as a whole
+    w.B.resize((size_t)m * m);
+    w.y.resize(m);
+    w.bits.assign((size_t)m * words, 0);
+    for (int i = 0; i < m; i++) {
+        const double* a = A + (size_t)(i + bc) * n + bc;
+        std::memcpy(&w.B[(size_t)i * m], a, sizeof(double) * m);
+        uint64_t* p = &w.bits[(size_t)i * words];
+        int j = 0;
+        for (; j + 2 <= m; j += 2)
+            p[j / 64] |= (uint64_t)_mm_movemask_pd(_mm_cmpneq_pd(_mm_loadu_pd(a + j), _mm_setzero_pd())) << (j % 64);
+        for (; j < m; j++) p[j / 64] |= (uint64_t)(a[j] != 0.0) << (j % 64);
+        w.y[i] = b[i + bc];
+    }
+    const int info = eliminate(w, m, x + bc);
     for (int i = 0; i < bc; i++) x[i] = 0.0;
+    return info;
+}
+
+int lu_solve_rows(int n, int cap, const int* count, const int* col, const double* val, const double* b, double* x,
+                  LuWork& w) {
+    const int words = (n + 63) / 64;
+    if (w.rows_m != n) {
+        w.B.assign((size_t)n * n, 0.0);
+        w.bits.assign((size_t)n * words, 0);
+        w.y.resize(n);
+        w.rows_m = n;
+    }
+    for (int r = 0; r < n; r++) {
+        double* const ri = &w.B[(size_t)r * n];
+        uint64_t* const p = &w.bits[(size_t)r * words];
+        for (int q = 0; q < count[r]; q++) {
+            const int j = col[(size_t)r * cap + q];
+            ri[j] = val[(size_t)r * cap + q];
+            p[j / 64] |= uint64_t(1) << (j % 64);
+        }
+        w.y[r] = b[r];
+    }
+    const int info = eliminate(w, n, x);
+    // zero again for the next system: only what the patterns name was written
+    for (int r = 0; r < n; r++) {
+        double* const ri = &w.B[(size_t)r * n];
+        uint64_t* const p = &w.bits[(size_t)r * words];
+        for (int q = 0; q < words; q++) {
+            for (uint64_t v = p[q]; v; v &= v - 1) ri[q * 64 + __builtin_ctzll(v)] = 0.0;
+            p[q] = 0;
+        }
+    }
     return info;
 }
 

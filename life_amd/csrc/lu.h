@@ -12,16 +12,29 @@
 #pragma once
 
 #include <cstddef>
+#include <cstdint>
 #include <vector>
 
 namespace life {
+
+// Work space of the two sparse solvers, kept between calls.
+struct LuWork {
+    std::vector<double> B, y;
+    std::vector<uint64_t> bits;
+    std::vector<int> row, pos, head, next, act, cols;
+    int rows_m = 0;  // B is all zero and of this size (lu_solve_rows), else 0
+};
 
 // Solve B x = b for the trailing block B = A[bc:, bc:] of the row-major
 // n x n matrix A; x[0..bc) = 0.  Skips rows with a zero multiplier and
 // columns that are zero in the pivot row.  Returns 0, or k+1 if column k
 // had no non-zero pivot.
-int lu_solve_sparse(int n, int bc, const double* A, const double* b, double* x, std::vector<double>& work,
-                    std::vector<int>& iwork);
+int lu_solve_sparse(int n, int bc, const double* A, const double* b, double* x, LuWork& work);
+
+// The same (bc = 0) for a matrix given by its non-zeros: row r has count[r]
+// of them, columns col[r * cap + q] ascending, values val[r * cap + q].
+int lu_solve_rows(int n, int cap, const int* count, const int* col, const double* val, const double* b, double* x,
+                  LuWork& work);
 
 // Banded storage: row r holds columns [r-kl, r+kl+ku] at
 // data[r*(2*kl+ku+1) + (c - r + kl)] (room for the fill-in of partial

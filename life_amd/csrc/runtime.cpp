@@ -859,6 +859,24 @@ void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host) {
     LIFE_HIP(hipStreamSynchronize(g->stream));
 }
 
+bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const int*& col, const double*& val) {
+    // values, then counts, then columns, in the page-locked block
+    const size_t nv = (size_t)n * kEpsRowCap;
+    char* p = stage(g, nv * sizeof(double) + (size_t)n * sizeof(int) + nv * sizeof(int));
+    double* v = reinterpret_cast<double*>(p);
+    int* c = reinterpret_cast<int*>(v + nv);
+    int* j = c + n;
+    launch_epsilon_rows(g->md, g->g, first, n, c, j, v, g->stream);
+    LIFE_HIP(hipGetLastError());
+    LIFE_HIP(hipStreamSynchronize(g->stream));
+    count = c;
+    col = j;
+    val = v;
+    for (int r = 0; r < n; r++)
+        if (c[r] > kEpsRowCap) return false;
+    return true;
+}
+
 void ibm_epsilon_band_setup(life_grid* g, const std::vector<int>& first, const std::vector<int>& n, int KB) {
     for (void* p : {(void*)g->eps_first, (void*)g->eps_n, (void*)g->eps_off, (void*)g->eps_outside,
                     (void*)g->eps_band, (void*)g->eps_y})
@@ -1441,9 +1459,13 @@ int life_grid_upload(life_grid* g, const double* f_aos, const double* rho, const
 int life_solve_lapack(int n, int bc, const double* A, const double* b, double* x) {
     return guarded([&] {
         if (n < 0 || bc < 0 || bc > n) throw std::runtime_error("bad system size");
-        std::vector<double> w;
-        std::vector<int> iw;
-        const int info = lu_solve_sparse(n, bc, A, b, x, w, iw);
+        // Kept per thread for systems of up to 512 unknowns: allocated and freed
+        // in each call, the work space was new pages each time (110 us of
+        // page faults for 82 unknowns, whose solve takes 10).
+        static thread_local LuWork kept;
+        LuWork own;
+        LuWork& w = n - bc <= 512 ? kept : own;
+        const int info = lu_solve_sparse(n, bc, A, b, x, w);
         if (info) throw std::runtime_error("singular matrix (zero pivot column " + std::to_string(info - 1) + ")");
     });
 }

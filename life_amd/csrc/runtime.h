@@ -211,6 +211,10 @@ void ibm_spread(life_grid* g);
 void ibm_interp_spread(life_grid* g);
 void ibm_find_support(life_grid* g, int flexible_only);
 void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host);
+// The same matrix by its non-zeros, kEpsRowCap a row, in page-locked memory
+// that stays valid until the grid's next marker transfer; false where a row
+// has more.  Waits for the stream.
+bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const int*& col, const double*& val);
 // Declare the banded epsilon systems [first[k], first[k]+n[k]) once.
 void ibm_epsilon_band_setup(life_grid* g, const std::vector<int>& first, const std::vector<int>& n, int KB);
 // Assemble and solve them on the device (epsilon lands in md.eps) and, with
