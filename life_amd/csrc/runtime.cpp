@@ -1459,12 +1459,7 @@ int life_grid_upload(life_grid* g, const double* f_aos, const double* rho, const
 int life_solve_lapack(int n, int bc, const double* A, const double* b, double* x) {
     return guarded([&] {
         if (n < 0 || bc < 0 || bc > n) throw std::runtime_error("bad system size");
-        // Kept per thread for systems of up to 512 unknowns: allocated and freed
-        // in each call, the work space was new pages each time (110 us of
-        // page faults for 82 unknowns, whose solve takes 10).
-        static thread_local LuWork kept;
-        LuWork own;
-        LuWork& w = n - bc <= 512 ? kept : own;
+        LuWork w;
         const int info = lu_solve_sparse(n, bc, A, b, x, w);
         if (info) throw std::runtime_error("singular matrix (zero pivot column " + std::to_string(info - 1) + ")");
     });
