@@ -389,7 +389,7 @@ void object_kernel_dev(life_case* c, EarlyBulk& eb, int mode) {
         // the out-of-band flags reach the host with the FEM's sums
         compute_epsilon(c, false, false);
         T.lap(g, 1);
-        ibm_interpolate(g);
+        ibm_interpolate(g, true);
         if (mode == 2) launch_pending(c, eb);
         T.lap(g, 2);
         // femKernel; again with epsilon from the dense path if a system was
@@ -459,7 +459,7 @@ void object_kernel(life_case* c, EarlyBulk& eb, int mode) {
     do {
         if (c->hasFlex) recompute_object_vals(c);
         T.lap(c->g, 1);
-        ibm_interpolate(c->g);
+        ibm_interpolate(c->g, true);
         // mode 2: the next step's stream-collide starts once the first
         // pass of the coupling kernels is queued, beside the host FEM
         if (mode == 2) launch_pending(c, eb);

@@ -6,6 +6,7 @@
 // Compiled with -ffp-contract=off.
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdlib>
 
 #include <stdexcept>
@@ -32,13 +33,21 @@ hipError_t set_coupling_priority(int level) {
     return hipMemcpyToSymbol(HIP_SYMBOL(g_coupling_prio), &level, sizeof(int));
 }
 
+// Orders LDS writes of some lanes before later reads by other lanes of the
+// same wavefront (LDS operations of a wavefront complete in order; the
+// fence stops the compiler from reordering them across lanes).
+__device__ __forceinline__ void lane_exchange_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // IBMNodeClass::findSupport (IBMNode.cpp:139-179): lattice sites within 1.5
 // spacings of the marker in both directions, scanned i-major over the 5x5
 // block around the nearest site, kept in scan order (at most 9).
 __device__ inline void find_support_xy(const MarkerDev& m, const GridScalars& g, int k, double x, double y) {
     const double Dx = g.Dx;
     const int inear = (int)round(x / Dx), jnear = (int)round(y / Dx);
-    int n = 0;
+    int n = 0, i0 = 0, j0 = 0, nj = 0;
     for (int i = inear - 2; i <= inear + 2; i++) {
         const double dx = fabs(x / Dx - i);
         for (int j = jnear - 2; j <= jnear + 2; j++) {
@@ -52,6 +61,11 @@ __device__ inline void find_support_xy(const MarkerDev& m, const GridScalars& g,
                 m.supp_ij[(k * kSupp + n) * 2] = i;
                 m.supp_ij[(k * kSupp + n) * 2 + 1] = j;
                 m.supp_delta[k * kSupp + n] = dirac64(dx) * dirac64(dy);
+                if (n == 0) {
+                    i0 = i;
+                    j0 = j;
+                }
+                if (i == i0) nj++;
                 n++;
             }
         }
@@ -63,17 +77,16 @@ __device__ inline void find_support_xy(const MarkerDev& m, const GridScalars& g,
         m.supp_delta[k * kSupp + s] = 0.0;
     }
     m.supp_cnt[k] = n;
+    int* box = m.supp_box + 4 * k;
+    box[0] = i0;
+    box[1] = j0;
+    box[2] = n > 0 ? n / nj : 0;
+    box[3] = nj;
 }
 
 __device__ inline void find_support_one(const MarkerDev& m, const GridScalars& g, int flexible_only, int k) {
     if (flexible_only && m.body_flex[m.body[k]] != 0) return;
     find_support_xy(m, g, k, m.pos[2 * k], m.pos[2 * k + 1]);
-}
-
-__global__ void k_find_support(MarkerDev m, GridScalars g, int flexible_only) {
-    coupling_priority();
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < m.n) find_support_one(m, g, flexible_only, k);
 }
 
 __global__ void k_find_support_batch(const CaseDev* __restrict__ cases, const int* __restrict__ list,
@@ -143,12 +156,6 @@ __device__ inline void compute_ds_body(const MarkerDev& m, const GridScalars& g,
     if (flexible_only && m.body_flex[b] != 0) return;
     const int first = m.body_first[b], cnt = m.body_n[b];
     ds_from_positions(m, g, first, cnt, stage_body_positions(m, first, cnt, spos));
-}
-
-__global__ void k_compute_ds(MarkerDev m, GridScalars g, int flexible_only) {
-    coupling_priority();
-    extern __shared__ double spos[];
-    compute_ds_body(m, g, flexible_only, blockIdx.x, spos);
 }
 
 // Supports and spacing of one body per workgroup in one launch: the two
@@ -394,14 +401,6 @@ __global__ void k_eps_far_check_batch(const CaseDev* __restrict__ cases, const C
 // The skipped dense operations all involve an exact zero, so the values
 // equal the dense elimination's.  A single wavefront is latency-bound
 // here: every step is one dependent chain (search, division, update).
-
-// Orders LDS writes of some lanes before later reads by other lanes of the
-// same wavefront (LDS operations of a wavefront complete in order; the
-// fence stops the compiler from reordering them across lanes).
-__device__ __forceinline__ void lane_exchange_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 // Lane `lane`'s value as a wavefront-uniform (SGPR) value.
 __device__ inline double uniform64(double v, int lane) {
@@ -1076,6 +1075,17 @@ constexpr int kInterpMarkers = 28;
 constexpr int kInterpThreads = kInterpMarkers * kSupp;  // 252
 
 template <typename T>
+__device__ __forceinline__ void interpolate_terms(const T* __restrict__ f, const GridScalars& g, long long id, double d,
+                                                  double& a, double& bx, double& by) {
+    double fs[kNV], rho, ux, uy;
+    load_site(f, g.S, id, fs);
+    moments64(fs, g.fcur ? g.fcur[id] : g.Fx, g.fcur ? g.fcur[g.S + id] : g.Fy, rho, ux, uy);
+    a = rho * d * 1.0 * 1.0;
+    bx = rho * ux * d * 1.0 * 1.0;
+    by = rho * uy * d * 1.0 * 1.0;
+}
+
+template <typename T>
 __device__ inline void interpolate_slots(const T* __restrict__ f, const MarkerDev& m, const GridScalars& g,
                                          int k0, double* __restrict__ sh, int t) {
     const int km = t / kSupp, s = t - km * kSupp;
@@ -1084,14 +1094,7 @@ __device__ inline void interpolate_slots(const T* __restrict__ f, const MarkerDe
     double* bx = sh + kInterpThreads;
     double* by = sh + 2 * kInterpThreads;
     if (t < kInterpThreads && k < m.n && s < m.supp_cnt[k]) {
-        const long long id = m.supp_site[k * kSupp + s];
-        double fs[kNV], rho, ux, uy;
-        load_site(f, g.S, id, fs);
-        moments64(fs, g.fcur ? g.fcur[id] : g.Fx, g.fcur ? g.fcur[g.S + id] : g.Fy, rho, ux, uy);
-        const double d = m.supp_delta[k * kSupp + s];
-        a[t] = rho * d * 1.0 * 1.0;
-        bx[t] = rho * ux * d * 1.0 * 1.0;
-        by[t] = rho * uy * d * 1.0 * 1.0;
+        interpolate_terms(f, g, m.supp_site[k * kSupp + s], m.supp_delta[k * kSupp + s], a[t], bx[t], by[t]);
     }
     __syncthreads();
     if (t < kInterpThreads && s == 0 && k < m.n) {
@@ -1108,10 +1111,21 @@ __device__ inline void interpolate_slots(const T* __restrict__ f, const MarkerDe
     }
 }
 
+__device__ inline void spread_clear_one(double* __restrict__ fibm, long long S, const int* __restrict__ uniq,
+                                        const int* __restrict__ uniq_n, int k);
+
+// Workgroups past the first ib zero the force at the sites of the last spread,
+// for a launch that a spread with new supports follows: the interpolation does
+// not read that force, so the clear costs the chain no launch of its own.
 template <typename T>
-__global__ __launch_bounds__(256) void k_interpolate(const T* __restrict__ f, MarkerDev m, GridScalars g) {
+__global__ __launch_bounds__(256) void k_interpolate(const T* __restrict__ f, MarkerDev m, GridScalars g, int ib,
+                                                     SpreadScratch sc, double* __restrict__ fibm) {
     __shared__ double sh[3 * kInterpThreads];
     coupling_priority();
+    if ((int)blockIdx.x >= ib) {
+        spread_clear_one(fibm, g.S, sc.uniq, sc.uniq_n, ((int)blockIdx.x - ib) * kInterpThreads + (int)threadIdx.x);
+        return;
+    }
     interpolate_slots(f, m, g, blockIdx.x * kInterpMarkers, sh, (int)threadIdx.x);
 }
 
@@ -1135,6 +1149,7 @@ __device__ inline void spread_clear_one(double* __restrict__ fibm, long long S, 
                                         const int* __restrict__ uniq_n, int k) {
     if (k >= *uniq_n) return;
     const long long id = uniq[k];
+    if (id < 0) return;
     fibm[id] = 0.0;
     fibm[S + id] = 0.0;
 }
@@ -1218,55 +1233,197 @@ __global__ void k_spread_reduce(MarkerDev m, SpreadScratch sc, double* __restric
     spread_reduce_one(m, sc, fibm, S, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-// The whole spread of a case with few marker-support pairs in one
-// workgroup: the clear, reset, count, scatter and reduce passes of the
-// separate launches in turn, each the same per-pair or per-site code,
-// separated by workgroup barriers (which make one pass's writes to the
-// scratch in device memory visible to the next).  Same pairs, same order at
-// each site, same sums; one launch instead of five, which is most of the
-// spread's time for a case of a few hundred markers.
-constexpr int kSpreadOneBlock = 1024;
-constexpr int kSpreadOneMaxPairs = 8192;
+// Spread of a case with few markers without lists: one wavefront per marker k
+// finds the markers whose support blocks overlap k's (all blocks compared, 64
+// a round, in ascending order; the four wavefronts of a workgroup share the
+// reading, a quarter each), forms their contributions, seven markers of
+// nine support lanes at a time, in a table by k's own sites, and lane o < 9
+// adds up site o in marker order.  The first marker at a site owns it and
+// writes its sum; the same additions in the same order as the passes above,
+// with no atomics and no sorting.  The site list of the last spread has one
+// entry per marker-support pair here, -1 where another marker owns the site.
+// Every support site is overwritten, so only sites outside the present
+// supports have to be cleared before.
+//
+// INTERP: the forces are not read but interpolated from the populations f on
+// the way, by every wavefront that needs them (those of about seven markers
+// each; the marker's own wavefront stores its force): interpolation and
+// spread of rigid bodies in one launch without a wait between them.
+//
+// Bound by the launch and a chain of four dependent reads (blocks, supports,
+// populations, sums in LDS).  The passes in one workgroup, with their atomics
+// and lists in device memory, took 26 us for 530 markers against 6 us here; with
+// the interpolation 17 us for 126 markers against 6 us.
+// Up to kScanMaxMarkers markers: the comparisons grow with the square of their
+// number, the five passes do not.  Spread with the clear at 1000, 2000, 4000
+// and 8000 markers: 10, 12, 15 and 24 us here, 19, 21, 25 and 33 us by the
+// passes.
+constexpr int kScanMaxMarkers = 8192;
+constexpr int kScanWaves = 4;    // markers per workgroup
+constexpr int kScanGroup = 7;    // neighbours at a time, of kSupp lanes each
+// More overlapping markers than this put more than kMaxPerSite pairs on one
+// of the nine sites.
+constexpr int kScanNear = kSupp * kMaxPerSite;
 
-__device__ inline void spread_passes_wg(const MarkerDev& m, const SpreadScratch& sc, double* __restrict__ fibm,
-                                        long long S, int clear) {
-    const int t = threadIdx.x, nt = blockDim.x;
-    const int np = m.n * kSupp;
-    if (clear)
-        for (int k = t; k < sc.cap; k += nt) spread_clear_one(fibm, S, sc.uniq, sc.uniq_n, k);
-    __syncthreads();
-    if (t == 0) *sc.uniq_n = 0;
-    __syncthreads();
-    for (int p = t; p < np; p += nt) spread_count_one(m, sc, p);
-    __syncthreads();
-    for (int p = t; p < np; p += nt) spread_scatter_one(m, sc, p);
-    __syncthreads();
-    for (int u = t; u < sc.cap; u += nt) spread_reduce_one(m, sc, fibm, S, u);
-}
-
-__global__ __launch_bounds__(kSpreadOneBlock) void k_spread_one(MarkerDev m, SpreadScratch sc,
-                                                                double* __restrict__ fibm, long long S, int clear) {
+template <typename T, bool INTERP>
+__global__ __launch_bounds__(64 * kScanWaves) void k_spread_scan(const T* __restrict__ f, MarkerDev m, GridScalars g,
+                                                                 SpreadScratch sc, double* __restrict__ fibm) {
+    __shared__ unsigned short near_s[kScanWaves][kScanWaves][kScanNear];  // marker, quarter
+    __shared__ int near_n[kScanWaves][kScanWaves];
+    __shared__ double tx_s[kScanWaves][64], ty_s[kScanWaves][64];
+    __shared__ int has_s[kScanWaves][64];
+    __shared__ double terms_s[kScanWaves][INTERP ? 3 * 64 : 1];
     coupling_priority();
-    spread_passes_wg(m, sc, fibm, S, clear);
-}
-
-// Rigid bodies of a small case, where the spread follows the interpolation
-// with nothing between them: both in one workgroup.  Four groups of 256
-// lanes take kInterpMarkers markers each per round with the interpolation's
-// own per-marker code (kInterpThreads of each group's lanes); a barrier;
-// then the spread passes as in k_spread_one.
-template <typename T>
-__global__ __launch_bounds__(kSpreadOneBlock) void k_interp_spread_one(const T* __restrict__ f, MarkerDev m,
-                                                                       GridScalars g, SpreadScratch sc,
-                                                                       double* __restrict__ fibm, int clear) {
-    __shared__ double sh[kSpreadOneBlock / 256][3 * kInterpThreads];
-    coupling_priority();
-    constexpr int kGroups = kSpreadOneBlock / 256;
-    const int grp = (int)threadIdx.x / 256, tl = (int)threadIdx.x % 256;
-    for (int k0 = 0; k0 < m.n; k0 += kGroups * kInterpMarkers)
-        interpolate_slots(f, m, g, k0 + grp * kInterpMarkers, sh[grp], tl);
+    const int wv = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
+    const int k = (int)blockIdx.x * kScanWaves + wv;
+    const int4* box = reinterpret_cast<const int4*>(m.supp_box);
+    const int k0 = (int)blockIdx.x * kScanWaves;
+    const int4 bk = box[min(k, m.n - 1)];
+    // each wavefront compares a quarter of the markers with all four of the
+    // workgroup
+    int4 bs[kScanWaves];
+    int have[kScanWaves], lx = INT_MAX, ly = INT_MAX, hx = INT_MIN, hy = INT_MIN;
+#pragma unroll
+    for (int w = 0; w < kScanWaves; w++) {
+        bs[w] = box[min(k0 + w, m.n - 1)];
+        have[w] = 0;
+        lx = min(lx, bs[w].x);
+        ly = min(ly, bs[w].y);
+        hx = max(hx, bs[w].x + bs[w].z);
+        hy = max(hy, bs[w].y + bs[w].w);
+    }
+    const int part = (m.n + kScanWaves - 1) / kScanWaves, cb = wv * part, ce = min(cb + part, m.n);
+    constexpr int U = 4;
+    for (int c0 = cb; c0 < ce; c0 += 64 * U) {
+        int4 bc[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) bc[u] = box[min(c0 + 64 * u + lane, m.n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int c = c0 + 64 * u + lane;
+            const int4 b = bc[u];
+            // mostly none of the 64 is near any of the four
+            const bool any = (b.x < hx && lx < b.x + b.z && b.y < hy && ly < b.y + b.w) || c / kScanWaves == (int)blockIdx.x;
+            if (!__ballot(any)) continue;
+#pragma unroll
+            for (int w = 0; w < kScanWaves; w++) {
+                const bool overlap = b.z > 0 && bs[w].z > 0 && b.x < bs[w].x + bs[w].z && bs[w].x < b.x + b.z &&
+                                     b.y < bs[w].y + bs[w].w && bs[w].y < b.y + b.w;
+                const bool in = c < ce && (overlap || c == k0 + w);
+                const unsigned long long mask = __ballot(in);
+                const int at = have[w] + __popcll(mask & ((1ull << lane) - 1));
+                if (in && at < kScanNear) near_s[w][wv][at] = (unsigned short)c;
+                have[w] += __popcll(mask);
+            }
+        }
+    }
+    if (lane == 0)
+#pragma unroll
+        for (int w = 0; w < kScanWaves; w++) near_n[w][wv] = have[w];
     __syncthreads();
-    spread_passes_wg(m, sc, fibm, g.S, clear);
+    if (k >= m.n) return;  // the whole wavefront; no workgroup barriers below
+    double *tx = tx_s[wv], *ty = ty_s[wv];
+    int* has = has_s[wv];
+    const int own_site = lane < kSupp ? m.supp_site[k * kSupp + lane] : -1;
+    // the quarters one after the other: neighbour e is entry e - end[h - 1] of
+    // quarter h
+    int end[kScanWaves], total = 0;
+    bool full = false;
+#pragma unroll
+    for (int h = 0; h < kScanWaves; h++) {
+        const int c = near_n[wv][h];
+        full = full || c > kScanNear;
+        end[h] = total += min(c, kScanNear);
+    }
+    if (full && lane == 0) *sc.overflow = 1;
+    auto near = [&](int e) -> int {
+        int h = 0, at = e;
+#pragma unroll
+        for (int r = 0; r + 1 < kScanWaves; r++)
+            if (e >= end[r]) {
+                h = r + 1;
+                at = e - end[r];
+            }
+        return near_s[wv][h][at];
+    };
+    const int q = lane / kSupp, s = lane - q * kSupp;
+    double fx = 0.0, fy = 0.0;
+    int pairs = 0;
+    bool owner = false;
+    for (int g0 = 0; g0 < total; g0 += kScanGroup) {
+        const int qn = min(kScanGroup, total - g0);
+        const bool on = q < qn;
+        const int j = near(on ? g0 + q : 0), p = j * kSupp + s;
+        const int4 bj = box[j];
+        const bool act = on && s < bj.z * bj.w;
+        const int site = m.supp_site[p];
+        const double d = m.supp_delta[p], e = m.eps[j], ds = m.ds[j];
+        double Fx, Fy;
+        if constexpr (INTERP) {
+            double *ta = terms_s[wv], *tbx = ta + 64, *tby = ta + 128;
+            const double vx = m.vel[2 * j], vy = m.vel[2 * j + 1];
+            if (act) interpolate_terms(f, g, site, d, ta[lane], tbx[lane], tby[lane]);
+            lane_exchange_fence();
+            // every lane of the marker adds the terms up in support order
+            double iR = 0.0, mx = 0.0, my = 0.0;
+            const int first = q * kSupp, cnt = on ? bj.z * bj.w : 0;
+#pragma unroll
+            for (int r = 0; r < kSupp; r++) {
+                const double va = ta[min(first + r, 63)], vbx = tbx[min(first + r, 63)], vby = tby[min(first + r, 63)];
+                if (r < cnt) {
+                    iR += va;
+                    mx += vbx;
+                    my += vby;
+                }
+            }
+            Fx = 2.0 * (g.velScale * iR * vx - mx);
+            Fy = 2.0 * (g.velScale * iR * vy - my);
+            if (on && s == 0 && j == k) {
+                m.force[2 * k] = Fx;
+                m.force[2 * k + 1] = Fy;
+            }
+        } else {
+            Fx = m.force[2 * j];
+            Fy = m.force[2 * j + 1];
+        }
+        has[lane] = 0;
+        lane_exchange_fence();
+        const int w = max(bj.w, 1), i = bj.x + s / w - bk.x, jj = bj.y + s % w - bk.y;
+        if (act && i >= 0 && i < bk.z && jj >= 0 && jj < bk.w) {
+            const int o = q * kSupp + i * bk.w + jj;
+            has[o] = 1;
+            tx[o] = Fx * e * ds * 1.0 * d;
+            ty[o] = Fy * e * ds * 1.0 * d;
+        }
+        lane_exchange_fence();
+        if (lane < kSupp) {
+#pragma unroll
+            for (int r = 0; r < kScanGroup; r++) {
+                const int o = r * kSupp + lane;
+                const bool hit = r < qn && has[o] != 0;
+                const double cx = tx[o], cy = ty[o];
+                if (hit) {
+                    if (pairs == 0) owner = near(g0 + r) == k;
+                    pairs++;
+                    fx += cx;
+                    fy += cy;
+                }
+            }
+        }
+        lane_exchange_fence();
+    }
+    if (lane < kSupp) {
+        const int p = k * kSupp + lane;
+        const bool mine = owner && own_site >= 0;
+        sc.uniq[p] = mine ? own_site : -1;
+        if (mine) {
+            sc.site_uid[own_site] = p;
+            fibm[own_site] = fx;
+            fibm[g.S + own_site] = fy;
+            if (pairs > kMaxPerSite) *sc.overflow = 1;
+        }
+        if (p == 0) *sc.uniq_n = m.n * kSupp;
+    }
 }
 
 // Batched spread, grid.y = case (the reset: one thread per case).
@@ -1364,19 +1521,9 @@ void launch_eps_band(const MarkerDev& m, const GridScalars& g, const int* sys_fi
         sys_first, sys_n, outside, band, band_off, ywork, m.eps, rows, cr ? kCrMaxRows : 0);
 }
 
-void launch_find_support(const MarkerDev& m, const GridScalars& g, int flexible_only, hipStream_t s) {
-    if (m.n <= 0) return;
-    k_find_support<<<(m.n + 127) / 128, 128, 0, s>>>(m, g, flexible_only);
-}
-
 void launch_support_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s) {
     if (m.n <= 0 || nbodies <= 0) return;
     k_support_ds<<<nbodies, 256, sizeof(double) * 2 * kDsLdsMarkers, s>>>(m, g, flexible_only);
-}
-
-void launch_compute_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s) {
-    if (m.n <= 0 || nbodies <= 0) return;
-    k_compute_ds<<<nbodies, 256, sizeof(double) * 2 * kDsLdsMarkers, s>>>(m, g, flexible_only);
 }
 
 void launch_epsilon_matrix(const MarkerDev& m, const GridScalars& g, int first, int n, double* A, hipStream_t s) {
@@ -1392,26 +1539,35 @@ void launch_epsilon_rows(const MarkerDev& m, const GridScalars& g, int first, in
 }
 
 template <typename T>
-void launch_interpolate(const T* f, const MarkerDev& m, const GridScalars& g, hipStream_t s) {
+void launch_interpolate(const T* f, const MarkerDev& m, const GridScalars& g, bool clear, double* fibm,
+                        const SpreadScratch& sc, hipStream_t s) {
     if (m.n <= 0) return;
-    k_interpolate<T><<<(m.n + kInterpMarkers - 1) / kInterpMarkers, kInterpThreads, 0, s>>>(f, m, g);
+    const int ib = (m.n + kInterpMarkers - 1) / kInterpMarkers;
+    const int cb = clear ? (sc.cap + kInterpThreads - 1) / kInterpThreads : 0;
+    k_interpolate<T><<<ib + cb, kInterpThreads, 0, s>>>(f, m, g, ib, sc, fibm);
 }
-template void launch_interpolate<double>(const double*, const MarkerDev&, const GridScalars&, hipStream_t);
-template void launch_interpolate<float>(const float*, const MarkerDev&, const GridScalars&, hipStream_t);
+template void launch_interpolate<double>(const double*, const MarkerDev&, const GridScalars&, bool, double*,
+                                         const SpreadScratch&, hipStream_t);
+template void launch_interpolate<float>(const float*, const MarkerDev&, const GridScalars&, bool, double*,
+                                        const SpreadScratch&, hipStream_t);
 
-void launch_spread(const MarkerDev& m, const GridScalars& g, double* fibm, SpreadScratch& sc, bool dense_clear,
+bool spread_scans(const MarkerDev& m) { return m.n <= kScanMaxMarkers; }
+
+static unsigned scan_blocks(const MarkerDev& m) { return (unsigned)((m.n + kScanWaves - 1) / kScanWaves); }
+
+void launch_spread(const MarkerDev& m, const GridScalars& g, double* fibm, SpreadScratch& sc, SpreadClear clear,
                    hipStream_t s) {
     const int np = m.n * kSupp;
     const int cap = sc.cap;
-    if (np > 0 && np <= kSpreadOneMaxPairs && cap >= np) {
-        if (dense_clear) launch_fill_f64(fibm, 0.0, g.S * 2, s);
-        k_spread_one<<<1, kSpreadOneBlock, 0, s>>>(m, sc, fibm, g.S, dense_clear ? 0 : 1);
-        return;
-    }
-    if (dense_clear) {
+    const bool scan = np > 0 && spread_scans(m);
+    if (clear == SpreadClear::kAll) {
         launch_fill_f64(fibm, 0.0, g.S * 2, s);
-    } else if (cap > 0) {
+    } else if (cap > 0 && (clear == SpreadClear::kList || !scan)) {
         k_spread_clear<<<(cap + 255) / 256, 256, 0, s>>>(fibm, g.S, sc.uniq, sc.uniq_n);
+    }
+    if (scan) {
+        k_spread_scan<double, false><<<scan_blocks(m), 64 * kScanWaves, 0, s>>>(nullptr, m, g, sc, fibm);
+        return;
     }
     k_spread_reset<<<1, 1, 0, s>>>(sc.uniq_n);
     if (np <= 0) return;
@@ -1420,19 +1576,15 @@ void launch_spread(const MarkerDev& m, const GridScalars& g, double* fibm, Sprea
     k_spread_reduce<<<(cap + 127) / 128, 128, 0, s>>>(m, sc, fibm, g.S);
 }
 
-bool launch_interp_spread_small(const void* f, bool f64, const MarkerDev& m, const GridScalars& g, double* fibm,
-                                SpreadScratch& sc, bool dense_clear, hipStream_t s) {
-    const int np = m.n * kSupp;
-    if (np <= 0 || np > kSpreadOneMaxPairs || sc.cap < np) return false;
-    if (dense_clear) launch_fill_f64(fibm, 0.0, g.S * 2, s);
-    if (f64)
-        k_interp_spread_one<double><<<1, kSpreadOneBlock, 0, s>>>(static_cast<const double*>(f), m, g, sc, fibm,
-                                                                  dense_clear ? 0 : 1);
-    else
-        k_interp_spread_one<float><<<1, kSpreadOneBlock, 0, s>>>(static_cast<const float*>(f), m, g, sc, fibm,
-                                                                 dense_clear ? 0 : 1);
-    return true;
+template <typename T>
+void launch_interp_spread(const T* f, const MarkerDev& m, const GridScalars& g, double* fibm, SpreadScratch& sc,
+                          hipStream_t s) {
+    k_spread_scan<T, true><<<scan_blocks(m), 64 * kScanWaves, 0, s>>>(f, m, g, sc, fibm);
 }
+template void launch_interp_spread<double>(const double*, const MarkerDev&, const GridScalars&, double*, SpreadScratch&,
+                                           hipStream_t);
+template void launch_interp_spread<float>(const float*, const MarkerDev&, const GridScalars&, double*, SpreadScratch&,
+                                          hipStream_t);
 
 // ---------------------------------------------------------------- batched launchers
 void launch_find_support_batch(const CaseDev* cases, const int* list, int n, int max_markers, int flexible_only,

@@ -118,13 +118,14 @@ struct MarkerDev {
     int* supp_site;    // n*9, lattice id or -1
     int* supp_ij;      // n*9*2
     double* supp_delta;// n*9
+    int* supp_box;     // n*4: first column and row of the support block, its columns and rows
     int* overflow;     // 1: set when a marker finds more than 9 supports
 };
 
 struct SpreadScratch {
     int* site_count;   // N, zero between spreads
     int* site_uid;     // N
-    int* uniq;         // cap, lattice ids of support sites of the last spread
+    int* uniq;         // cap, lattice ids of support sites of the last spread, -1: no entry
     int* uniq_n;       // 1
     int* pair_slot;    // n*9
     int* list;         // cap*kMaxPerSite
@@ -132,10 +133,8 @@ struct SpreadScratch {
     int cap;
 };
 
-void launch_find_support(const MarkerDev& m, const GridScalars& g, int flexible_only, hipStream_t s);
-// launch_find_support + launch_compute_ds in one launch (one workgroup per body).
+// Support sites and spacing of the markers of all (or all flexible) bodies.
 void launch_support_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s);
-void launch_compute_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s);
 void launch_epsilon_matrix(const MarkerDev& m, const GridScalars& g, int first, int n, double* A, hipStream_t s);
 // Its non-zeros row by row: count[r] of them (counted past kEpsRowCap, but not
 // stored), columns ascending in col[r * kEpsRowCap ..], values in val.
@@ -150,15 +149,23 @@ void launch_epsilon_rows(const MarkerDev& m, const GridScalars& g, int first, in
 void launch_eps_band(const MarkerDev& m, const GridScalars& g, const int* sys_first, const int* sys_n,
                      const int* host_n, int nsys, int KB, double* band, const long long* band_off, int* outside,
                      double* ywork, bool cr, hipStream_t s);
+// clear: zero the force at the sites of the last spread in the same launch.
 template <typename T>
-void launch_interpolate(const T* f, const MarkerDev& m, const GridScalars& g, hipStream_t s);
-void launch_spread(const MarkerDev& m, const GridScalars& g, double* fibm, SpreadScratch& sc, bool dense_clear,
+void launch_interpolate(const T* f, const MarkerDev& m, const GridScalars& g, bool clear, double* fibm,
+                        const SpreadScratch& sc, hipStream_t s);
+// What a spread has to zero before it: the whole force field, the sites of the
+// last spread, or nothing (no site outside the present supports holds a force;
+// a spread of more markers than spread_scans takes clears its list all the same).
+enum class SpreadClear { kAll, kList, kNone };
+void launch_spread(const MarkerDev& m, const GridScalars& g, double* fibm, SpreadScratch& sc, SpreadClear clear,
                    hipStream_t s);
-// Interpolation (populations f, FP64 or FP32-shifted) and then the spread in
-// one launch, for a case of at most 8192 marker-support pairs; false (and
-// nothing launched) otherwise.
-bool launch_interp_spread_small(const void* f, bool f64, const MarkerDev& m, const GridScalars& g, double* fibm,
-                                SpreadScratch& sc, bool dense_clear, hipStream_t s);
+// Few enough markers for the spread without lists.
+bool spread_scans(const MarkerDev& m);
+// Interpolation and spread in one launch, where spread_scans holds and nothing
+// is to be cleared.
+template <typename T>
+void launch_interp_spread(const T* f, const MarkerDev& m, const GridScalars& g, double* fibm, SpreadScratch& sc,
+                          hipStream_t s);
 
 // ---------------------------------------------------------------- serving
 // Batched forms of the kernels above for the serving engine.  Every

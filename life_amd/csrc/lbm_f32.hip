@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_support_push32_batch(const CaseDev* __r
                                                               const int* __restrict__ list) {
     const CaseDev& c = cases[list[blockIdx.y]];
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c.explicit_state || c.m.n <= 0 || k >= *c.sc.uniq_n) return;
+    if (c.explicit_state || c.m.n <= 0 || k >= *c.sc.uniq_n || c.sc.uniq[k] < 0) return;
     support_push32_site<CM>(static_cast<const float*>(c.src), static_cast<float*>(c.dst), c.g, c.fibm, c.sc.uniq[k]);
 }
 
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(256) void k_support_push32(const float* __restrict_
                                                         const int* __restrict__ sites,
                                                         const int* __restrict__ count) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= *count) return;
+    if (k >= *count || sites[k] < 0) return;
     support_push32_site<CM>(src, dst, g, fibm, sites[k]);
 }
 

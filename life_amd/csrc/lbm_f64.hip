@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void k_support_push64(const double* __restrict
                                                         const int* __restrict__ sites,
                                                         const int* __restrict__ count) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < *count) support_push64_site<CM>(src, dst, g, fibm, sites[k]);
+    if (k < *count && sites[k] >= 0) support_push64_site<CM>(src, dst, g, fibm, sites[k]);
 }
 
 template <bool CM>
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256) void k_support_push64_batch(const CaseDev* __r
                                                               const int* __restrict__ list) {
     const CaseDev& c = cases[list[blockIdx.y]];
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c.explicit_state || c.m.n <= 0 || k >= *c.sc.uniq_n) return;
+    if (c.explicit_state || c.m.n <= 0 || k >= *c.sc.uniq_n || c.sc.uniq[k] < 0) return;
     support_push64_site<CM>(static_cast<const double*>(c.src), static_cast<double*>(c.dst), c.g, c.fibm,
                             c.sc.uniq[k]);
 }

@@ -738,35 +738,50 @@ void blowup_cadence(life_grid* g, int t, hipStream_t s) {
     blowup_scan(g, t, s);
 }
 
-void ibm_interpolate(life_grid* g) {
+void ibm_interpolate(life_grid* g, bool spread_follows) {
     if (g->md.n <= 0) return;
     lbm_join(g);
-    if (g->prec == kFP64) launch_interpolate<double>(static_cast<const double*>(g->f[g->cur]), g->md, g->g, g->stream);
-    else launch_interpolate<float>(static_cast<const float*>(g->f[g->cur]), g->md, g->g, g->stream);
+    const bool clear = spread_follows && !g->spread_current && !g->dense_clear_next && spread_scans(g->md);
+    if (g->prec == kFP64)
+        launch_interpolate<double>(static_cast<const double*>(g->f[g->cur]), g->md, g->g, clear, g->fibm, g->sc,
+                                   g->stream);
+    else
+        launch_interpolate<float>(static_cast<const float*>(g->f[g->cur]), g->md, g->g, clear, g->fibm, g->sc,
+                                  g->stream);
+    if (clear) g->spread_current = true;
     LIFE_HIP(hipGetLastError());
 }
 
 void ibm_spread(life_grid* g) {
-    launch_spread(g->md, g->g, g->fibm, g->sc, g->dense_clear_next, g->stream);
+    launch_spread(g->md, g->g, g->fibm, g->sc,
+                  g->dense_clear_next ? SpreadClear::kAll
+                                      : (g->spread_current ? SpreadClear::kNone : SpreadClear::kList),
+                  g->stream);
     g->dense_clear_next = false;
+    g->spread_current = true;
     LIFE_HIP(hipGetLastError());
 }
 
 void ibm_interp_spread(life_grid* g) {
     if (g->md.n <= 0) return;
-    lbm_join(g);
-    if (launch_interp_spread_small(g->f[g->cur], g->prec == kFP64, g->md, g->g, g->fibm, g->sc, g->dense_clear_next,
-                                   g->stream)) {
-        g->dense_clear_next = false;
-        LIFE_HIP(hipGetLastError());
+    if (!g->spread_current || g->dense_clear_next || !spread_scans(g->md)) {
+        ibm_interpolate(g, true);
+        ibm_spread(g);
         return;
     }
-    ibm_interpolate(g);
-    ibm_spread(g);
+    // the supports are those of the last spread (rigid bodies after their
+    // first step): nothing to clear, one launch
+    lbm_join(g);
+    if (g->prec == kFP64)
+        launch_interp_spread<double>(static_cast<const double*>(g->f[g->cur]), g->md, g->g, g->fibm, g->sc, g->stream);
+    else
+        launch_interp_spread<float>(static_cast<const float*>(g->f[g->cur]), g->md, g->g, g->fibm, g->sc, g->stream);
+    LIFE_HIP(hipGetLastError());
 }
 
 void ibm_find_support(life_grid* g, int flexible_only) {
     if (g->md.n <= 0) return;
+    g->spread_current = false;
     launch_support_ds(g->md, g->g, g->nbodies, flexible_only, g->stream);
     LIFE_HIP(hipGetLastError());
 }
@@ -943,7 +958,7 @@ void check_flags(life_grid* g) {
 static void free_markers(life_grid* g) {
     MarkerDev& m = g->md;
     for (void* p : {(void*)m.pos, (void*)m.vel, (void*)m.force, (void*)m.eps, (void*)m.ds, (void*)m.body,
-                    (void*)m.supp_cnt, (void*)m.supp_site, (void*)m.supp_ij, (void*)m.supp_delta,
+                    (void*)m.supp_cnt, (void*)m.supp_site, (void*)m.supp_ij, (void*)m.supp_delta, (void*)m.supp_box,
                     (void*)g->body_first, (void*)g->body_n, (void*)g->body_flex, (void*)g->sc.site_count,
                     (void*)g->sc.site_uid, (void*)g->sc.uniq, (void*)g->sc.uniq_n, (void*)g->sc.pair_slot,
                     (void*)g->sc.list})
@@ -1498,6 +1513,7 @@ int life_ibm_set_markers(life_grid* g, int n, const double* pos, const double* v
         m.supp_site = dalloc<int>((size_t)n * kSupp);
         m.supp_ij = dalloc<int>((size_t)n * kSupp * 2);
         m.supp_delta = dalloc<double>((size_t)n * kSupp);
+        m.supp_box = dalloc<int>((size_t)n * 4);
         g->body_first = dalloc<int>(nbodies);
         g->body_n = dalloc<int>(nbodies);
         g->body_flex = dalloc<int>(nbodies);
@@ -1534,11 +1550,13 @@ int life_ibm_set_markers(life_grid* g, int n, const double* pos, const double* v
         launch_fill_f64(m.eps, 0.0, n, s);
         launch_fill_f64(m.ds, 0.0, n, s);
         launch_fill_i32(m.supp_cnt, 0, n, s);
+        launch_fill_i32(m.supp_box, 0, 4 * (long long)n, s);
         launch_fill_i32(sc.site_count, 0, g->g.N, s);
         launch_fill_i32(sc.uniq_n, 0, 1, s);
         LIFE_HIP(hipGetLastError());
         LIFE_HIP(hipStreamSynchronize(s));
         g->dense_clear_next = true;
+        g->spread_current = false;
     });
 }
 

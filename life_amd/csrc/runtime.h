@@ -76,6 +76,9 @@ struct life_grid {
     double* fibm = nullptr;
     double* fsite[2] = {nullptr, nullptr};  // per-site force_xy planes (WOMERSLEY with gravity)
     bool dense_clear_next = false;
+    // no site outside the present supports holds a force_ibm: set by a spread
+    // (or the clear before it), reset where supports are found again
+    bool spread_current = false;
     // boundaries
     std::vector<life::BCSite> bc_host;
     life::BCSite* bc = nullptr;
@@ -205,9 +208,12 @@ void blowup_check(life_grid* g, bool wait);
 // Scan after step t when the cadence says so (reading the previous scan
 // first if it is done).
 void blowup_cadence(life_grid* g, int t, hipStream_t s);
-void ibm_interpolate(life_grid* g);
+// spread_follows: the launch may zero the force of the last spread, since a
+// spread is next and nothing reads force_ibm in between.
+void ibm_interpolate(life_grid* g, bool spread_follows = false);
 void ibm_spread(life_grid* g);
-// ibm_interpolate then ibm_spread, in one launch for a small case.
+// ibm_interpolate then ibm_spread, in one launch where the supports are those
+// of the last spread and the markers few.
 void ibm_interp_spread(life_grid* g);
 void ibm_find_support(life_grid* g, int flexible_only);
 void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host);
