@@ -41,144 +41,108 @@ __device__ __forceinline__ void lane_exchange_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// Supports and spacing take half a wavefront (kHalf lanes) per marker: one lane
+// per site of the 5x5 block, and every 32nd marker of the body per lane.  With
+// one lane per marker the 25 sites and the body's markers came one after the
+// other in each lane, and one workgroup per body left all but a few CUs idle:
+// 27 us for two bodies of 530 markers and 10 us for one filament, 5.5 us for both now.
+constexpr int kHalf = 32;
+
 // IBMNodeClass::findSupport (IBMNode.cpp:139-179): lattice sites within 1.5
 // spacings of the marker in both directions, scanned i-major over the 5x5
-// block around the nearest site, kept in scan order (at most 9).
-__device__ inline void find_support_xy(const MarkerDev& m, const GridScalars& g, int k, double x, double y) {
+// block around the nearest site, kept in scan order (at most 9).  l: lane of
+// the half wavefront.
+__device__ __forceinline__ void find_support_half(const MarkerDev& m, const GridScalars& g, int k, double x, double y,
+                                                  int l) {
     const double Dx = g.Dx;
     const int inear = (int)round(x / Dx), jnear = (int)round(y / Dx);
-    int n = 0, i0 = 0, j0 = 0, nj = 0;
-    for (int i = inear - 2; i <= inear + 2; i++) {
-        const double dx = fabs(x / Dx - i);
-        for (int j = jnear - 2; j <= jnear + 2; j++) {
-            const double dy = fabs(y / Dx - j);
-            if (dx < 1.5 && dy < 1.5 && i >= 0 && i <= g.Nx - 1 && j >= 0 && j <= g.Ny - 1) {
-                if (n == kSupp) {
-                    *m.overflow = 1;
-                    continue;
-                }
-                m.supp_site[k * kSupp + n] = i * g.Ny + j;
-                m.supp_ij[(k * kSupp + n) * 2] = i;
-                m.supp_ij[(k * kSupp + n) * 2 + 1] = j;
-                m.supp_delta[k * kSupp + n] = dirac64(dx) * dirac64(dy);
-                if (n == 0) {
-                    i0 = i;
-                    j0 = j;
-                }
-                if (i == i0) nj++;
-                n++;
-            }
-        }
+    const int i = inear - 2 + l / 5, j = jnear - 2 + l % 5;
+    const double dx = fabs(x / Dx - i), dy = fabs(y / Dx - j);
+    const bool in = l < 25 && dx < 1.5 && dy < 1.5 && i >= 0 && i <= g.Nx - 1 && j >= 0 && j <= g.Ny - 1;
+    const unsigned mask = (unsigned)(__ballot(in) >> (threadIdx.x & 32));  // this half's lanes
+    const int at = __popc(mask & ((1u << l) - 1)), found = __popc(mask), n = min(found, kSupp);
+    if (in && at < kSupp) {
+        m.supp_site[k * kSupp + at] = i * g.Ny + j;
+        m.supp_ij[(k * kSupp + at) * 2] = i;
+        m.supp_ij[(k * kSupp + at) * 2 + 1] = j;
+        m.supp_delta[k * kSupp + at] = dirac64(dx) * dirac64(dy);
     }
-    for (int s = n; s < kSupp; s++) {
-        m.supp_site[k * kSupp + s] = -1;
-        m.supp_ij[(k * kSupp + s) * 2] = 0;
-        m.supp_ij[(k * kSupp + s) * 2 + 1] = 0;
-        m.supp_delta[k * kSupp + s] = 0.0;
+    if (l >= n && l < kSupp) {
+        m.supp_site[k * kSupp + l] = -1;
+        m.supp_ij[(k * kSupp + l) * 2] = 0;
+        m.supp_ij[(k * kSupp + l) * 2 + 1] = 0;
+        m.supp_delta[k * kSupp + l] = 0.0;
     }
-    m.supp_cnt[k] = n;
-    int* box = m.supp_box + 4 * k;
-    box[0] = i0;
-    box[1] = j0;
-    box[2] = n > 0 ? n / nj : 0;
-    box[3] = nj;
+    if (l == 0) {
+        if (found > kSupp) *m.overflow = 1;
+        const int first = n > 0 ? __ffs(mask) - 1 : 0, rows = __popc(mask & (31u << (first / 5 * 5)));
+        m.supp_cnt[k] = n;
+        int* box = m.supp_box + 4 * k;
+        box[0] = n > 0 ? inear - 2 + first / 5 : 0;
+        box[1] = n > 0 ? jnear - 2 + first % 5 : 0;
+        box[2] = n > 0 ? n / rows : 0;
+        box[3] = rows;
+    }
 }
 
-__device__ inline void find_support_one(const MarkerDev& m, const GridScalars& g, int flexible_only, int k) {
-    if (flexible_only && m.body_flex[m.body[k]] != 0) return;
-    find_support_xy(m, g, k, m.pos[2 * k], m.pos[2 * k + 1]);
-}
-
-__global__ void k_find_support_batch(const CaseDev* __restrict__ cases, const int* __restrict__ list,
-                                     int flexible_only) {
-    const CaseDev& c = cases[list[blockIdx.y]];
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < c.m.n) find_support_one(c.m, c.g, flexible_only, k);
-}
-
-// IBMNodeClass::computeDs (IBMNode.cpp:182-204): distance (lattice units)
-// to the nearest other marker of the same body, starting from 10.  One
-// workgroup per body; the body's positions are staged in LDS when they fit.
-constexpr int kDsLdsMarkers = 2048;
-
-// The positions of body markers [first, first + cnt) staged in LDS (spos)
-// when they fit, else read from device memory; all lanes of the workgroup.
-__device__ inline const double* stage_body_positions(const MarkerDev& m, int first, int cnt, double* spos) {
-    const bool lds = cnt <= kDsLdsMarkers;
-    if (lds)
-        for (int t = threadIdx.x; t < 2 * cnt; t += blockDim.x) spos[t] = m.pos[2 * first + t];
-    __syncthreads();
-    return lds ? spos : m.pos + 2 * first;
-}
-
-__device__ inline void ds_from_positions(const MarkerDev& m, const GridScalars& g, int first, int cnt,
-                                         const double* P) {
+// IBMNodeClass::computeDs (IBMNode.cpp:182-204): distance (lattice units) of
+// marker q0 of a body, at (x, y), to the nearest of the body's other markers
+// (positions P, cnt of them), starting from 10.  sqrt(.)/Dx is monotone, so
+// the minimum of sqrt(d.d)/Dx over the other markers is sqrt(min d.d)/Dx; the
+// minimum does not depend on the order of the comparisons.  The result is in
+// every lane of the half wavefront.
+__device__ __forceinline__ double spacing_half(const double* P, int cnt, int q0, double x, double y, double Dx, int l) {
     const double2* P2 = reinterpret_cast<const double2*>(P);
-    // sqrt(.)/Dx is monotone, so the minimum of sqrt(d.d)/Dx over the other
-    // markers is sqrt(min d.d)/Dx: one square root per marker, same value.
-    // The minimum of a set does not depend on the order of the comparisons,
-    // so eight running minima take eight markers per round, their positions
-    // loaded (16 bytes each) before the comparisons.
-    constexpr int U = 8;
-    for (int k = threadIdx.x; k < cnt; k += blockDim.x) {
-        const double x = P[2 * k], y = P[2 * k + 1];
-        double mn[U];
+    constexpr int U = 4;  // positions loaded before the first is used
+    double mn = INFINITY;
+    for (int b = 0; b < cnt; b += U * kHalf) {
+        double2 pq[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) mn[u] = INFINITY;
-        int q0 = 0;
-        for (; q0 + U <= cnt; q0 += U) {
-            double2 pq[U];
+        for (int u = 0; u < U; u++) pq[u] = P2[min(b + u * kHalf + l, cnt - 1)];
 #pragma unroll
-            for (int u = 0; u < U; u++) pq[u] = P2[q0 + u];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const double dx = x - pq[u].x, dy = y - pq[u].y;
-                const double d2 = 0.0 + dx * dx + dy * dy;
-                if (q0 + u != k && d2 < mn[u]) mn[u] = d2;
-            }
-        }
-        for (int q = q0; q < cnt; q++) {
-            const double dx = x - P[2 * q], dy = y - P[2 * q + 1];
+        for (int u = 0; u < U; u++) {
+            const int q = b + u * kHalf + l;
+            const double dx = x - pq[u].x, dy = y - pq[u].y;
             const double d2 = 0.0 + dx * dx + dy * dy;
-            if (q != k && d2 < mn[0]) mn[0] = d2;
+            if (q < cnt && q != q0 && d2 < mn) mn = d2;
         }
-        double d2min = mn[0];
-#pragma unroll
-        for (int u = 1; u < U; u++)
-            if (mn[u] < d2min) d2min = mn[u];
-        const double mag = sqrt(d2min) / g.Dx;
-        m.ds[first + k] = mag < 10.0 ? mag : 10.0;
     }
+#pragma unroll
+    for (int o = kHalf / 2; o > 0; o /= 2) {
+        const double other = __shfl_xor(mn, o, kHalf);
+        if (other < mn) mn = other;
+    }
+    const double mag = sqrt(mn) / Dx;
+    return mag < 10.0 ? mag : 10.0;
 }
 
-__device__ inline void compute_ds_body(const MarkerDev& m, const GridScalars& g, int flexible_only, int b,
-                                       double* spos) {
+// Both for the markers of this workgroup: the two are independent (the
+// spacing reads only positions), so the coupling chain has one kernel fewer
+// to wait for.
+constexpr int kSupportThreads = 256;
+
+__device__ __forceinline__ void support_ds_body(const MarkerDev& m, const GridScalars& g, int flexible_only) {
+    const int k = (int)(blockIdx.x * (kSupportThreads / kHalf) + threadIdx.x / kHalf), l = (int)threadIdx.x % kHalf;
+    if (k >= m.n) return;
+    const int b = m.body[k];
+    const double x = m.pos[2 * k], y = m.pos[2 * k + 1];
+    const int first = m.body_first[b], cnt = m.body_n[b];
     if (flexible_only && m.body_flex[b] != 0) return;
-    const int first = m.body_first[b], cnt = m.body_n[b];
-    ds_from_positions(m, g, first, cnt, stage_body_positions(m, first, cnt, spos));
+    find_support_half(m, g, k, x, y, l);
+    const double ds = spacing_half(m.pos + 2 * first, cnt, k - first, x, y, g.Dx, l);
+    if (l == 0) m.ds[k] = ds;
 }
 
-// Supports and spacing of one body per workgroup in one launch: the two
-// are independent (spacing reads only positions), so the coupling chain
-// has one kernel fewer to wait for.
-// The body's positions are read once (into LDS), and its kind once per
-// workgroup, so beside a bandwidth-bound kernel the chain of dependent
-// device-memory reads is two long (body table, positions).
-__global__ void k_support_ds(MarkerDev m, GridScalars g, int flexible_only) {
+__global__ __launch_bounds__(kSupportThreads) void k_support_ds(MarkerDev m, GridScalars g, int flexible_only) {
     coupling_priority();
-    extern __shared__ double spos[];
-    const int b = blockIdx.x;
-    const int first = m.body_first[b], cnt = m.body_n[b];
-    if (flexible_only && m.body_flex[b] != 0) return;  // the whole workgroup
-    const double* P = stage_body_positions(m, first, cnt, spos);
-    for (int k = threadIdx.x; k < cnt; k += blockDim.x) find_support_xy(m, g, first + k, P[2 * k], P[2 * k + 1]);
-    ds_from_positions(m, g, first, cnt, P);
+    support_ds_body(m, g, flexible_only);
 }
 
-__global__ void k_compute_ds_batch(const CaseDev* __restrict__ cases, const int* __restrict__ list, int flexible_only) {
-    extern __shared__ double spos[];
+__global__ __launch_bounds__(kSupportThreads) void k_support_ds_batch(const CaseDev* __restrict__ cases,
+                                                                      const int* __restrict__ list,
+                                                                      int flexible_only) {
     const CaseDev& c = cases[list[blockIdx.y]];
-    if ((int)blockIdx.x < c.nbodies) compute_ds_body(c.m, c.g, flexible_only, blockIdx.x, spos);
+    support_ds_body(c.m, c.g, flexible_only);
 }
 
 // A_ij of ObjectsClass::computeEpsilon (Objects.cpp:271-300) for the system
@@ -954,8 +918,8 @@ __global__ __launch_bounds__(256) void k_eps_band_cr_batch(const CaseDev* __rest
 // The device half of recomputeObjectVals (Objects.cpp:217-227 and the
 // computeEpsilon of flexible bodies, Objects.cpp:235-321) for one flexible
 // body per workgroup, without global round trips between the stages:
-// supports of its markers (to global memory, as k_find_support), spacing
-// from positions staged in LDS (as k_compute_ds), the band of its epsilon
+// supports of its markers (to global memory) and spacing, from positions
+// staged in LDS (as k_support_ds), the band of its epsilon
 // system built in LDS (as eps_band_entry), the out-of-band check (as
 // eps_far_pair) and, if the system is banded, the solve by wavefront 0
 // (as k_eps_band_solve).  Same operations in the same order as those
@@ -983,28 +947,23 @@ __device__ __forceinline__ void recompute_body(const MarkerDev& m, const GridSca
         *flag = 0;
         *bw_sh = 0;
     }
-    for (int k = tid; k < n; k += nt) {
+    const int half = tid / kHalf, nhalf = nt / kHalf, l = tid % kHalf;
+    for (int k = half; k < n; k += nhalf) {
         // the position and the body kind are read side by side
         const double x = m.pos[2 * (first + k)], y = m.pos[2 * (first + k) + 1];
-        if (m.body_flex[m.body[first + k]] == 0) find_support_xy(m, g, first + k, x, y);
-        P[2 * k] = x;
-        P[2 * k + 1] = y;
+        if (m.body_flex[m.body[first + k]] == 0) find_support_half(m, g, first + k, x, y, l);
+        if (l == 0) {
+            P[2 * k] = x;
+            P[2 * k + 1] = y;
+        }
     }
     __syncthreads();
-    // computeDs (IBMNode.cpp:182-204), as compute_ds_body
-    for (int k = tid; k < n; k += nt) {
-        const double x = P[2 * k], y = P[2 * k + 1];
-        double d2min = INFINITY;
-        for (int q = 0; q < n; q++) {
-            if (q == k) continue;
-            const double dx = x - P[2 * q], dy = y - P[2 * q + 1];
-            const double d2 = 0.0 + dx * dx + dy * dy;
-            if (d2 < d2min) d2min = d2;
+    for (int k = half; k < n; k += nhalf) {
+        const double ds = spacing_half(P, n, k, P[2 * k], P[2 * k + 1], g.Dx, l);
+        if (l == 0) {
+            m.ds[first + k] = ds;
+            dsl[k] = ds;
         }
-        const double mag = sqrt(d2min) / g.Dx;
-        const double ds = mag < 10.0 ? mag : 10.0;
-        m.ds[first + k] = ds;
-        dsl[k] = ds;
     }
     __syncthreads();
     // band entries (as eps_band_entry, reading the staged positions and ds)
@@ -1521,9 +1480,14 @@ void launch_eps_band(const MarkerDev& m, const GridScalars& g, const int* sys_fi
         sys_first, sys_n, outside, band, band_off, ywork, m.eps, rows, cr ? kCrMaxRows : 0);
 }
 
-void launch_support_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s) {
-    if (m.n <= 0 || nbodies <= 0) return;
-    k_support_ds<<<nbodies, 256, sizeof(double) * 2 * kDsLdsMarkers, s>>>(m, g, flexible_only);
+static unsigned support_blocks(int markers) {
+    constexpr int per = kSupportThreads / kHalf;
+    return (unsigned)((markers + per - 1) / per);
+}
+
+void launch_support_ds(const MarkerDev& m, const GridScalars& g, int flexible_only, hipStream_t s) {
+    if (m.n <= 0) return;
+    k_support_ds<<<support_blocks(m.n), kSupportThreads, 0, s>>>(m, g, flexible_only);
 }
 
 void launch_epsilon_matrix(const MarkerDev& m, const GridScalars& g, int first, int n, double* A, hipStream_t s) {
@@ -1587,18 +1551,11 @@ template void launch_interp_spread<float>(const float*, const MarkerDev&, const 
                                           hipStream_t);
 
 // ---------------------------------------------------------------- batched launchers
-void launch_find_support_batch(const CaseDev* cases, const int* list, int n, int max_markers, int flexible_only,
-                               hipStream_t s) {
-    if (n <= 0 || max_markers <= 0) return;
-    k_find_support_batch<<<dim3((unsigned)((max_markers + 127) / 128), (unsigned)n), 128, 0, s>>>(cases, list,
-                                                                                                 flexible_only);
-}
-
-void launch_compute_ds_batch(const CaseDev* cases, const int* list, int n, int max_bodies, int flexible_only,
+void launch_support_ds_batch(const CaseDev* cases, const int* list, int n, int max_markers, int flexible_only,
                              hipStream_t s) {
-    if (n <= 0 || max_bodies <= 0) return;
-    k_compute_ds_batch<<<dim3((unsigned)max_bodies, (unsigned)n), 256, sizeof(double) * 2 * kDsLdsMarkers, s>>>(
-        cases, list, flexible_only);
+    if (n <= 0 || max_markers <= 0) return;
+    k_support_ds_batch<<<dim3(support_blocks(max_markers), (unsigned)n), kSupportThreads, 0, s>>>(cases, list,
+                                                                                                flexible_only);
 }
 
 void launch_eps_band_batch(const CaseDev* cases, const CaseSys* sys, int nsys, int max_n, int* outside_out,

@@ -134,7 +134,7 @@ struct SpreadScratch {
 };
 
 // Support sites and spacing of the markers of all (or all flexible) bodies.
-void launch_support_ds(const MarkerDev& m, const GridScalars& g, int nbodies, int flexible_only, hipStream_t s);
+void launch_support_ds(const MarkerDev& m, const GridScalars& g, int flexible_only, hipStream_t s);
 void launch_epsilon_matrix(const MarkerDev& m, const GridScalars& g, int first, int n, double* A, hipStream_t s);
 // Its non-zeros row by row: count[r] of them (counted past kEpsRowCap, but not
 // stored), columns ascending in col[r * kEpsRowCap ..], values in val.
@@ -236,9 +236,7 @@ void launch_markers_in_batch(const CaseDev* cases, const int* list, int n, int m
                              hipStream_t s);
 void launch_markers_out_batch(const CaseDev* cases, const int* list, int n, int max_markers, double* stage,
                               hipStream_t s);
-void launch_find_support_batch(const CaseDev* cases, const int* list, int n, int max_markers, int flexible_only,
-                               hipStream_t s);
-void launch_compute_ds_batch(const CaseDev* cases, const int* list, int n, int max_bodies, int flexible_only,
+void launch_support_ds_batch(const CaseDev* cases, const int* list, int n, int max_markers, int flexible_only,
                              hipStream_t s);
 // outside_out[q] = 1 for a listed system that is not banded (no solve done;
 // outside_out may be page-locked host memory, readable after the stream is

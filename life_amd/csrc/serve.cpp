@@ -181,7 +181,7 @@ struct life_server {
     Mirror<double> stage_in, stage_out;
     LatticePlan plan;
     int off_conv = 0, off_ibm[2] = {0, 0}, off_bc[2] = {0, 0}, off_ibm_all = 0, n_ibm_all = 0;
-    int total_markers = 0, max_markers = 0, max_bodies = 0;
+    int total_markers = 0, max_markers = 0;
     hipGraph_t graph = nullptr;  // lattice tail
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph_bulk = nullptr;  // bulk stream-collide
@@ -285,7 +285,7 @@ void admit(life_server* s) {
 void rebuild(life_server* s) {
     LatticePlan& P = s->plan;
     P = LatticePlan{};
-    s->total_markers = s->max_markers = s->max_bodies = 0;
+    s->total_markers = s->max_markers = 0;
     std::vector<int> ibm_all;
     for (int q = 0; q < (int)s->slots.size(); q++) {
         Slot& sl = s->slots[q];
@@ -310,7 +310,6 @@ void rebuild(life_server* s) {
         sl.moff = s->total_markers;
         s->total_markers += sl.c->nm;
         s->max_markers = std::max(s->max_markers, sl.c->nm);
-        s->max_bodies = std::max(s->max_bodies, g->nbodies);
     }
     for (int k = 0; k < 2; k++) {
         s->blocks[k].reserve(P.blocks[k].size());
@@ -724,8 +723,7 @@ void coupling_phase(life_server* s) {
                                launch_recompute_fused_batch(s->cases.d, s->sys.d, (int)sysl.size(), max_n,
                                                             s->outside.h, cr, st);
             if (!fused) {
-                launch_find_support_batch(s->cases.d, s->dyn.d, na, s->max_markers, 1, st);
-                launch_compute_ds_batch(s->cases.d, s->dyn.d, na, s->max_bodies, 1, st);
+                launch_support_ds_batch(s->cases.d, s->dyn.d, na, s->max_markers, 1, st);
                 if (!sysl.empty())
                     launch_eps_band_batch(s->cases.d, s->sys.d, (int)sysl.size(), max_n, s->outside.h, cr, st);
             }
