@@ -346,25 +346,31 @@ __global__ void k_eps_far_check_batch(const CaseDev* __restrict__ cases, const C
 //
 // With lower and upper bandwidth KB, every non-zero that step k of the
 // dense elimination reads or writes lies in rows k..k+KB and columns
-// k..k+2KB (row swaps widen the upper band by KB).  That window stays in
-// registers: register slot r holds row k+r, and lane L < C holds the
-// window column j with j = L (mod C), so columns never move between lanes.
-// Step k:
-//  - the lane holding column k finds the pivot (first row of maximum
-//    magnitude; rows past n hold zeros) in its own registers, and one
-//    v_readlane makes the row index uniform;
-//  - rows k and k+p are swapped in every column;
-//  - column k goes through LDS to lanes 1..KB, lane r forms the multiplier
-//    l_r = a(k+r, k) / a(k, k) (one division for the whole wavefront), and
-//    the multipliers come back through LDS;
-//  - every other column gets a_ij - l_i a_kj once, from the same operands
-//    as the dense algorithm (rows past n get l = 0: no change), and row k
-//    of U is emitted.
-// The slots then shift by one row (row k+R enters), and column k's lane
-// takes column k+C, whose entries in rows k+1..k+KB are structural zeros.
-// The skipped dense operations all involve an exact zero, so the values
-// equal the dense elimination's.  A single wavefront is latency-bound
-// here: every step is one dependent chain (search, division, update).
+// k..k+2KB (row swaps widen the upper band by KB).  Row r lives in the
+// registers of lane r % 64, column c of it in register c % C, C = 2KB + 1: rows
+// and columns stay where they are for the whole elimination, the steps are
+// unrolled C times so that every register index is a constant, and the lanes
+// of rows k+1..k+KB are selected by an execution mask that moves up by one a
+// step.  Step k:
+//  - the pivot's lane is read by every lane (v_readlane); if no entry of
+//    column k in the window reaches its magnitude, it is the pivot;
+//  - otherwise the first row of maximum magnitude is found, and the two lanes'
+//    registers change places;
+//  - every lane divides (l = a(i, k) / a(k, k)) and the window's lanes take
+//    l times row k from their own row: columns k+1..k+KB, and up to k+2KB
+//    within KB steps of a swap, past which those columns of row k are zero.
+// Rows of U stay in place; half the lanes at a time store theirs and take the
+// rows 64 further on.  The skipped dense operations all involve an exact
+// zero, so the values equal the dense elimination's.
+//
+// A single wavefront is bound by the chain of dependent FP64 operations here
+// (readlane, compare, a division of ten operations, product, difference), about
+// 330 cycles a step at KB = 3; the back substitution, with the diagonal's
+// reciprocals formed beforehand, 175.  Columns in lanes and rows in registers,
+// shifted every step, took 950 for both; with swaps at every step 1500 (1030
+// before), which the matrices of markers one spacing apart do not have.
+// 91 markers, KB = 3: 39 us before, 25 us with the staging by four
+// wavefronts.
 
 // Lane `lane`'s value as a wavefront-uniform (SGPR) value.
 __device__ inline double uniform64(double v, int lane) {
@@ -374,157 +380,264 @@ __device__ inline double uniform64(double v, int lane) {
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// Back substitution on one lane in increasing column order, two rows per
-// iteration (no register shuffling between them); rows of U stored with
-// half-bandwidth KBS, window half-bandwidth KB.  Terms past n are 0 * 0
-// (structural zeros of U times the zero-initialised x window), which
-// leave s unchanged, so rows need no bounds tests.
+// This lane's bit of a wavefront-uniform mask.
+__device__ __forceinline__ bool lane_in(unsigned long long mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// The band is stored with half-bandwidth KBS (W = 3KBS + 1 per row); the
+// elimination window has half-bandwidth KB <= KBS, which must bound every
+// non-zero of the matrix (|column - row| <= KB).
 template <int KB, int KBS>
-__device__ __forceinline__ void band_back_substitute(int first, int n, const double* __restrict__ B,
-                                                     const double* __restrict__ y, double* __restrict__ eps) {
-    constexpr int W = 3 * KBS + 1;
-    double xa[2 * KB + 1];  // xa[q] = x[i+1+q] for the row pair (i, i-1)
+struct BandRows {
+    static constexpr int C = 2 * KB + 1, W = 3 * KBS + 1;
+    double w[C], wr;       // this lane's row and its right-hand side
+    bool swapped = false;  // a pivot was not on the diagonal
+
+    // Row r of the band (zero past n): register j takes column
+    // (r - KB) + (j - (r - KB)) mod C.
+    __device__ __forceinline__ void load(int r, int n, const double* __restrict__ B) {
+        const bool in = r < n;
+        const double* src = B + (size_t)(in ? r : 0) * W + (KBS - KB);
+        int q = (KB - r) % C;
+        if (q < 0) q += C;
 #pragma unroll
-    for (int q = 0; q <= 2 * KB; q++) xa[q] = 0.0;
-    int i = n - 1;
-    for (; i >= 1; i -= 2) {
-        const double* U1 = B + i * W + KBS;
-        const double* U0 = B + (i - 1) * W + KBS;
-        double u1[2 * KB + 1], u0[2 * KB + 1];
-#pragma unroll
-        for (int q = 0; q <= 2 * KB; q++) {
-            u1[q] = U1[q];
-            u0[q] = U0[q];
+        for (int j = 0; j < C; j++) {
+            const double v = src[q];
+            w[j] = in ? v : 0.0;
+            q = q + 1 == C ? 0 : q + 1;
         }
+        wr = in ? 1.0 : 0.0;
+    }
+
+    // Row r of U (columns r .. r + 2KB) in place of row r of the band.
+    __device__ __forceinline__ void store(int r, int n, double* __restrict__ B, double* __restrict__ y) const {
+        if (r >= n) return;
+        double* dst = B + (size_t)r * W + KBS;
+        int q = (-r) % C;
+        if (q < 0) q += C;
+#pragma unroll
+        for (int j = 0; j < C; j++) {
+            dst[q] = w[j];
+            q = q + 1 == C ? 0 : q + 1;
+        }
+        y[r] = wr;
+    }
+
+    __device__ __forceinline__ void swap_lanes(int L, int a, int b) {
+        auto sw = [&](double& v) {
+            const double va = uniform64(v, a), vb = uniform64(v, b);
+            v = L == a ? vb : (L == b ? va : v);
+        };
+#pragma unroll
+        for (int j = 0; j < C; j++) sw(w[j]);
+        sw(wr);
+    }
+
+    // Step k, column k in register J; window: the lanes of rows k+1..k+KB;
+    // wide: steps left in which row k may reach past column k+KB.
+    template <int J>
+    __device__ __forceinline__ void step(int k, unsigned long long window, int& wide, int L) {
+        const int a = k & 63;
+        const double p0 = uniform64(w[J], a);
+        double piv = p0;
+        // also where the whole column is zero (rows past n are zero)
+        if (__builtin_expect((__ballot(fabs(w[J]) >= fabs(p0)) & window) != 0, 0)) {
+            double best = fabs(p0);
+            int b = a;
+            for (int r = 1; r <= KB; r++) {
+                const double v = fabs(uniform64(w[J], (k + r) & 63));
+                if (v > best) {
+                    best = v;
+                    b = (k + r) & 63;
+                }
+            }
+            if (b != a) {
+                swap_lanes(L, a, b);
+                piv = uniform64(w[J], a);
+                wide = KB + 1;
+                swapped = true;
+            }
+            if (piv == 0.0) piv = 1.0;  // zero column: all multipliers 0
+        }
+        double p[KB + 1];
+#pragma unroll
+        for (int d = 1; d <= KB; d++) p[d] = uniform64(w[(J + d) % C], a);
+        const double pr = uniform64(wr, a);
+        const double l = w[J] / piv;
+        if (lane_in(window)) {
+            w[J] = 0.0;  // column k + C from here on
+#pragma unroll
+            for (int d = 1; d <= KB; d++) w[(J + d) % C] = w[(J + d) % C] - l * p[d];
+            wr = wr - l * pr;
+        }
+        if (__builtin_expect(wide > 0, 0)) {
+            wide--;
+#pragma unroll
+            for (int d = KB + 1; d <= 2 * KB; d++) {
+                const double q = uniform64(w[(J + d) % C], a);
+                if (lane_in(window)) w[(J + d) % C] = w[(J + d) % C] - l * q;
+            }
+        }
+    }
+
+    // Steps k .. k+C-1 (FULL) or those of them below kend.
+    template <bool FULL, int J = 0>
+    __device__ __forceinline__ void steps(int k, int kend, unsigned long long& window, int& wide, int L) {
+        if constexpr (J < C) {
+            if (FULL || k < kend) {
+                step<J>(k, window, wide, L);
+                window = (window << 1) | (window >> 63);
+                steps<FULL, J + 1>(k + 1, kend, window, wide, L);
+            }
+        }
+    }
+};
+
+// One wavefront; true if a row swap was made.
+template <int KB, int KBS>
+__device__ __forceinline__ bool band_eliminate(int n, double* __restrict__ B, double* __restrict__ y) {
+    constexpr int C = 2 * KB + 1;
+    const int L = threadIdx.x;
+    BandRows<KB, KBS> s;
+    s.load(L, n, B);
+    unsigned long long window = ((1ull << KB) - 1) << 1;
+    int wide = 0, saved = 0;
+    for (int k = 0; k < n; k += C) {
+        // the half wavefront whose rows are done: a block of C steps and its
+        // window stay within the 64 rows from `saved`
+        if (k >= saved + 32) {
+            if (L / 32 == (saved / 32) % 2) {
+                const int r = saved + L % 32;
+                s.store(r, n, B, y);
+                s.load(r + 64, n, B);
+            }
+            saved += 32;
+        }
+        if (k + C <= n) s.template steps<true>(k, n, window, wide, L);
+        else s.template steps<false>(k, n, window, wide, L);
+    }
+    for (int end = saved + 64; saved < end; saved += 32)
+        if (L / 32 == (saved / 32) % 2) s.store(saved + L % 32, n, B, y);
+    return s.swapped;
+}
+
+// Between the solve's phases: writes of some lanes, reads by others of the
+// same wavefront, in LDS or in device memory.
+template <bool LDS_>
+__device__ __forceinline__ void band_fence() {
+    if (LDS_) lane_exchange_fence();
+    else __threadfence_block();
+}
+
+__device__ __forceinline__ bool mid_range(double v) {
+    const double a = fabs(v);
+    return a > 0x1p-300 && a < 0x1p300;
+}
+
+// a / b from y, the correctly rounded 1 / b (Markstein, IBM J. Res. Dev. 34,
+// 1990): the first correction leaves a quotient within one unit in the last
+// place, the second rounds it correctly.  For values clear of overflow and
+// underflow (mid_range).
+__device__ __forceinline__ double div_by(double a, double b, double y) {
+    double q = a * y;
+    q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
+// Back substitution by one wavefront (every lane the same), in increasing
+// column order: rows of U of half-bandwidth T = KB, no swap having widened
+// them.  Terms past n are 0 * 0, which leaves a sum unchanged.  The
+// reciprocals and the results go into the two sub-diagonal entries that the
+// elimination left unused.  False, with nothing of use written, if a diagonal
+// entry or a result is not mid_range (a singular matrix among them).
+template <int T, int KBS, bool LDS_>
+__device__ __forceinline__ bool band_back_fast(int first, int n, double* __restrict__ B, const double* __restrict__ y,
+                                               double* __restrict__ eps) {
+    constexpr int W = 3 * KBS + 1;
+    bool ok = true;
+    for (int r = threadIdx.x; r < n; r += 64) {
+        const double d = B[(size_t)r * W + KBS];
+        ok = ok && mid_range(d);
+        B[(size_t)r * W + KBS - 1] = 1.0 / d;
+    }
+    if (__ballot(!ok)) return false;
+    band_fence<LDS_>();
+    struct Row {
+        double u[T + 1], r, s;
+    };
+    auto load = [&](Row& v, int i) {
+        const double* U = B + (size_t)max(i, 0) * W + KBS;
+#pragma unroll
+        for (int q = 0; q <= T; q++) v.u[q] = U[q];
+        v.r = U[-1];
+        v.s = y[max(i, 0)];
+    };
+    double x[T];  // x[q] = solution at i + 1 + q
+#pragma unroll
+    for (int q = 0; q < T; q++) x[q] = 0.0;
+    auto solve = [&](const Row& v, int i) {
+        double t = v.s;
+#pragma unroll
+        for (int q = 0; q < T; q++) t = t - v.u[1 + q] * x[q];
+        const double xi = div_by(t, v.u[0], v.r);
+        if (i >= 0) B[(size_t)i * W + KBS - 2] = xi;
+#pragma unroll
+        for (int q = T - 1; q > 0; q--) x[q] = x[q - 1];
+        x[0] = xi;
+    };
+    // rows loaded two ahead
+    Row a, b, c;
+    load(a, n - 1);
+    load(b, n - 2);
+    for (int i = n - 1; i >= 0; i -= 3) {
+        load(c, i - 2);
+        solve(a, i);
+        load(a, i - 3);
+        solve(b, i - 1);
+        load(b, i - 4);
+        solve(c, i - 2);
+    }
+    band_fence<LDS_>();
+    for (int r = threadIdx.x; r < n; r += 64) {
+        const double v = B[(size_t)r * W + KBS - 2];
+        ok = ok && mid_range(v);
+        eps[first + r] = v;
+    }
+    return !__ballot(!ok);
+}
+
+// The same for any U of half-bandwidth T, with divisions.
+template <int T, int KBS>
+__device__ __forceinline__ void band_back_rows(int first, int n, const double* __restrict__ B,
+                                               const double* __restrict__ y, double* __restrict__ eps) {
+    constexpr int W = 3 * KBS + 1;
+    double x[T];
+#pragma unroll
+    for (int q = 0; q < T; q++) x[q] = 0.0;
+    for (int i = n - 1; i >= 0; i--) {
+        const double* U = B + (size_t)i * W + KBS;
         double s = y[i];
 #pragma unroll
-        for (int q = 0; q < 2 * KB; q++) s = s - u1[1 + q] * xa[q];
-        const double x1 = s / u1[0];
-        eps[first + i] = x1;
-        double t = y[i - 1];
-        t = t - u0[1] * x1;
+        for (int q = 0; q < T; q++) s = s - U[1 + q] * x[q];
+        const double xi = s / U[0];
+        if (threadIdx.x == 0) eps[first + i] = xi;
 #pragma unroll
-        for (int q = 1; q < 2 * KB; q++) t = t - u0[1 + q] * xa[q - 1];
-        const double x0 = t / u0[0];
-        eps[first + i - 1] = x0;
-#pragma unroll
-        for (int q = 2 * KB; q > 1; q--) xa[q] = xa[q - 2];
-        xa[1] = x1;
-        xa[0] = x0;
-    }
-    if (i == 0) {
-        const double* U = B + KBS;
-        double s = y[0];
-#pragma unroll
-        for (int q = 0; q < 2 * KB; q++) s = s - U[1 + q] * xa[q];
-        eps[first] = s / U[0];
+        for (int q = T - 1; q > 0; q--) x[q] = x[q - 1];
+        x[0] = xi;
     }
 }
 
 // B: the band (rows of U replace it), y: the right-hand side; both either
 // in LDS or in global memory (LDS_ selects the instantiation, so that every
-// access is compiled for its own address space).  xb: 2R doubles of LDS.
-// The band is stored with half-bandwidth KBS (W = 3KBS + 1 per row); the
-// elimination window has half-bandwidth KB <= KBS, which must bound every
-// non-zero of the matrix (|column - row| <= KB).
-template <int KB, int KBS, bool LDS_, bool ONE_WAVE = false>
+// access is compiled for its own address space).  Wavefront 0 of the workgroup.
+template <int KB, int KBS, bool LDS_>
 __device__ __forceinline__ void eps_band_solve_impl(int first, int n, double* __restrict__ B, double* __restrict__ y,
-                                                    double* __restrict__ eps, double* __restrict__ xb) {
-    static_assert(KB <= KBS, "window wider than the stored band");
-    constexpr int R = KB + 1, C = 2 * KB + 1, W = 3 * KBS + 1;
-    const int L = threadIdx.x;
-    // lanes 0..C-1 hold the window columns; lane C holds the right-hand
-    // side, which the row operations treat as one more column
-    const bool rhs_lane = L == C;
-    double w[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int q = L - r + KBS;
-        const bool in = L < C && r < n && L < n && q >= 0 && q < W;
-        const double a = B[in ? r * W + q : 0];
-        w[r] = in ? a : (rhs_lane && r < n ? 1.0 : 0.0);
-    }
-    int pl = 0;   // lane holding column k
-    int off = L;  // this lane holds column k + off
-    for (int k = 0; k < n; k++) {
-        // row k+R enters this lane's column after the step (band offset
-        // q = column - row + KBS, always inside the stored band here); the
-        // load is unconditional (clamped address) so that its latency
-        // overlaps the step
-        const int cn = L == pl ? C : off;
-        const bool in = L < C && k + R < n && k + cn < n;
-        const double a_in = B[in ? (k + R) * W + (cn - R + KBS) : 0];
-        double best = fabs(w[0]);
-        int pr = 0;
-#pragma unroll
-        for (int r = 1; r < R; r++) {
-            const double a = fabs(w[r]);
-            const bool gt = a > best;
-            best = gt ? a : best;
-            pr = gt ? r : pr;
-        }
-        const int p = __builtin_amdgcn_readlane(pr, pl);
-        if (__builtin_expect(p != 0, 0)) {
-            const double tw = w[0];
-#pragma unroll
-            for (int r = 1; r < R; r++)
-                if (r == p) {
-                    w[0] = w[r];
-                    w[r] = tw;
-                }
-        }
-        double l[R];
-        if constexpr (KB <= 4) {
-            // narrow window: column k and the multipliers as wavefront-
-            // uniform values (v_readlane), no LDS round trip
-            const double piv0 = uniform64(w[0], pl);
-            const double piv = piv0 != 0.0 ? piv0 : 1.0;  // zero column: all multipliers 0
-            double num = 0.0;
-#pragma unroll
-            for (int r = 1; r < R; r++) {
-                const double a = uniform64(w[r], pl);
-                num = L == r ? a : num;
-            }
-            const double lm = num / piv;
-#pragma unroll
-            for (int r = 1; r < R; r++) l[r] = uniform64(lm, r);
-        } else {
-            if (L == pl) {
-#pragma unroll
-                for (int r = 0; r < R; r++) xb[r] = w[r];
-            }
-            // other lanes read what lane pl wrote: a wavefront-scope fence
-            // keeps the compiler from moving their reads above the write
-            lane_exchange_fence();
-            const double piv0 = xb[0];
-            const double piv = piv0 != 0.0 ? piv0 : 1.0;  // zero column: all multipliers 0
-            const double num = (L >= 1 && L < R) ? xb[L] : 0.0;
-            if (L >= 1 && L < R) xb[R + L] = num / piv;
-            lane_exchange_fence();
-#pragma unroll
-            for (int r = 1; r < R; r++) l[r] = xb[R + r];
-        }
-#pragma unroll
-        for (int r = 1; r < R; r++) {
-            const double upd = w[r] - l[r] * w[0];
-            w[r] = L == pl ? 0.0 : upd;
-        }
-        // row k of U (in place of row k of the band) and the final y_k
-        if (L < C && k + off < n) B[k * W + (off + KBS)] = w[0];
-        if (rhs_lane) y[k] = w[0];
-        // drop row k, take in row k+R; column k's lane takes column k+C
-#pragma unroll
-        for (int r = 0; r < R - 1; r++) w[r] = w[r + 1];
-        w[R - 1] = in ? a_in : (rhs_lane && k + R < n ? 1.0 : 0.0);
-        off = L == pl ? C - 1 : off - 1;
-        pl = pl == C - 1 ? 0 : pl + 1;
-        if constexpr (KB > 4) lane_exchange_fence();  // xb is rewritten next step
-        else __builtin_amdgcn_wave_barrier();
-    }
-    // lane 0 reads the rows of U and y the other lanes wrote
-    if (ONE_WAVE) lane_exchange_fence();
-    else __syncthreads();
-    if (L == 0) band_back_substitute<KB, KBS>(first, n, B, y, eps);
+                                                    double* __restrict__ eps) {
+    static_assert(KB <= KBS && KB >= 2, "window wider than the stored band, or no sub-diagonal pair");
+    if (threadIdx.x >= 64) return;
+    const bool swapped = band_eliminate<KB, KBS>(n, B, y);
+    band_fence<LDS_>();
+    if (!swapped && band_back_fast<KB, KBS, LDS_>(first, n, B, y, eps)) return;
+    band_back_rows<2 * KB, KBS>(first, n, B, y, eps);
 }
 
 // Largest |column - row| over the non-zero entries of rows [r0, r1) of a
@@ -543,74 +656,81 @@ __device__ __forceinline__ int band_width_rows(const double* __restrict__ B, lon
 // Elimination with the narrowest window that holds the matrix's non-zeros
 // (bandwidth bw): the same operations on the non-zero entries, fewer on
 // structural zeros, so the same values.
-template <int KBS, bool LDS_, bool ONE_WAVE = false>
+template <int KBS, bool LDS_>
 __device__ __forceinline__ void eps_band_solve_bw(int bw, int first, int n, double* __restrict__ B,
-                                                  double* __restrict__ y, double* __restrict__ eps,
-                                                  double* __restrict__ xb) {
-    if (bw <= 2) eps_band_solve_impl<2, KBS, LDS_, ONE_WAVE>(first, n, B, y, eps, xb);
-    else if (bw == 3) eps_band_solve_impl<3, KBS, LDS_, ONE_WAVE>(first, n, B, y, eps, xb);
-    else if (bw == 4) eps_band_solve_impl<4, KBS, LDS_, ONE_WAVE>(first, n, B, y, eps, xb);
-    else eps_band_solve_impl<KBS, KBS, LDS_, ONE_WAVE>(first, n, B, y, eps, xb);
+                                                  double* __restrict__ y, double* __restrict__ eps) {
+    if (bw <= 2) eps_band_solve_impl<2, KBS, LDS_>(first, n, B, y, eps);
+    else if (bw == 3) eps_band_solve_impl<3, KBS, LDS_>(first, n, B, y, eps);
+    else if (bw == 4) eps_band_solve_impl<4, KBS, LDS_>(first, n, B, y, eps);
+    else eps_band_solve_impl<KBS, KBS, LDS_>(first, n, B, y, eps);
 }
 
-// One system per 64-lane workgroup: stage the band in LDS when it fits,
-// measure its bandwidth on the way, and solve with the matching window.
-// bw_sh: one int of LDS.
+// One system per workgroup of kBandThreads lanes: all of them stage the band in
+// LDS when it fits and measure its bandwidth on the way, the first wavefront
+// solves with the matching window.  bw_sh: one int of LDS.
+constexpr int kBandThreads = 256;
+
 template <int KB>
 __device__ __forceinline__ void eps_band_solve_body(int first, int n, double* __restrict__ G, double* __restrict__ ywork,
-                                                    double* __restrict__ eps, int lds_rows, double* sm,
-                                                    double* xb, int* bw_sh) {
+                                                    double* __restrict__ eps, int lds_rows, double* sm, int* bw_sh) {
     constexpr int W = 3 * KB + 1;
     const int nw = n * W;
     if (threadIdx.x == 0) *bw_sh = 0;
     __syncthreads();
     int bw = 0;
     if (n <= lds_rows) {
-#pragma unroll 8
-        for (int t = threadIdx.x; t < nw; t += 64) {
-            const double v = G[t];
-            sm[t] = v;
-            const int q = t % W;
-            if (q <= 2 * KB && v != 0.0) bw = max(bw, q < KB ? KB - q : q - KB);
+        constexpr int U = 8;  // loads in flight
+        for (int t0 = threadIdx.x; t0 < nw; t0 += U * kBandThreads) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = G[min(t0 + u * kBandThreads, nw - 1)];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int t = t0 + u * kBandThreads, q = t % W;
+                if (t < nw) {
+                    sm[t] = v[u];
+                    if (q <= 2 * KB && v[u] != 0.0) bw = max(bw, q < KB ? KB - q : q - KB);
+                }
+            }
         }
     } else {
-        bw = band_width_rows<KB>(G, threadIdx.x, nw, 64);
+        bw = band_width_rows<KB>(G, threadIdx.x, nw, kBandThreads);
     }
-    atomicMax(bw_sh, bw);
+    if (bw) atomicMax(bw_sh, bw);
     __syncthreads();
     bw = *bw_sh;
-    if (n <= lds_rows) eps_band_solve_bw<KB, true>(bw, first, n, sm, sm + (long long)nw, eps, xb);
-    else eps_band_solve_bw<KB, false>(bw, first, n, G, ywork + first, eps, xb);
+    if (n <= lds_rows) eps_band_solve_bw<KB, true>(bw, first, n, sm, sm + (long long)nw, eps);
+    else eps_band_solve_bw<KB, false>(bw, first, n, G, ywork + first, eps);
 }
 
 template <int KB>
-__global__ __launch_bounds__(64) void k_eps_band_solve(const int* __restrict__ sys_first, const int* __restrict__ sys_n,
-                                                       const int* __restrict__ outside, double* __restrict__ band,
-                                                       const long long* __restrict__ band_off,
-                                                       double* __restrict__ ywork, double* __restrict__ eps,
-                                                       int lds_rows, int skip_upto) {
+__global__ __launch_bounds__(kBandThreads) void k_eps_band_solve(const int* __restrict__ sys_first,
+                                                                 const int* __restrict__ sys_n,
+                                                                 const int* __restrict__ outside,
+                                                                 double* __restrict__ band,
+                                                                 const long long* __restrict__ band_off,
+                                                                 double* __restrict__ ywork, double* __restrict__ eps,
+                                                                 int lds_rows, int skip_upto) {
     extern __shared__ double sm[];
-    __shared__ double xb[2 * (KB + 1)];
     __shared__ int bw;
     const int sys = blockIdx.x;
     coupling_priority();
     // skip_upto: systems of up to that many rows are the reduction's
     if (outside[sys] || sys_n[sys] <= skip_upto) return;
-    eps_band_solve_body<KB>(sys_first[sys], sys_n[sys], band + band_off[sys], ywork, eps, lds_rows, sm, xb, &bw);
+    eps_band_solve_body<KB>(sys_first[sys], sys_n[sys], band + band_off[sys], ywork, eps, lds_rows, sm, &bw);
 }
 
 template <int KB>
-__global__ __launch_bounds__(64) void k_eps_band_solve_batch(const CaseDev* __restrict__ cases,
-                                                             const CaseSys* __restrict__ sys, int lds_rows,
-                                                             int skip_upto) {
+__global__ __launch_bounds__(kBandThreads) void k_eps_band_solve_batch(const CaseDev* __restrict__ cases,
+                                                                       const CaseSys* __restrict__ sys, int lds_rows,
+                                                                       int skip_upto) {
     extern __shared__ double sm[];
-    __shared__ double xb[2 * (KB + 1)];
     __shared__ int bw;
     const CaseSys q = sys[blockIdx.x];
     const CaseDev& c = cases[q.c];
     if (c.eps.outside[q.k] || c.eps.n[q.k] <= skip_upto) return;
     eps_band_solve_body<KB>(c.eps.first[q.k], c.eps.n[q.k], c.eps.band + c.eps.off[q.k], c.eps.y, c.m.eps, lds_rows,
-                            sm, xb, &bw);
+                            sm, &bw);
 }
 
 // ---------------------------------------------------------------- epsilon by cyclic reduction
@@ -874,15 +994,12 @@ static void allow_lds(const void* kernel, size_t bytes) {
 
 // One system per workgroup: the reduction, or for a band wider than
 // kCrMaxBw the pivoted elimination on the band in device memory (ywork: its
-// right-hand side).  That elimination's lanes are those of wavefront 0; the
-// other wavefronts run along without storing anything and meet it at the
-// workgroup barrier before the back substitution.
+// right-hand side) by wavefront 0.
 __device__ __forceinline__ void eps_cr_or_pivot(double* __restrict__ G, int first, int n, double* __restrict__ ywork,
-                                                double* __restrict__ eps, double* sm, double* xb, int* bw_sh,
-                                                int maxbw) {
+                                                double* __restrict__ eps, double* sm, int* bw_sh, int maxbw) {
     const int bw = band_width_wg(G, n, bw_sh);
     if (bw > maxbw) {
-        eps_band_solve_bw<8, false>(bw, first, n, G, ywork + first, eps, xb);
+        eps_band_solve_bw<8, false>(bw, first, n, G, ywork + first, eps);
         return;
     }
     const int nb = (n + kCrMaxBw - 1) / kCrMaxBw;
@@ -894,24 +1011,22 @@ __global__ __launch_bounds__(256) void k_eps_band_cr(const int* __restrict__ sys
                                                      const long long* __restrict__ band_off,
                                                      double* __restrict__ ywork, double* __restrict__ eps, int maxbw) {
     extern __shared__ double sm[];
-    __shared__ double xb[2 * (8 + 1)];
     __shared__ int bw_sh;
     const int sys = blockIdx.x, n = sys_n[sys];
     coupling_priority();
     if (outside[sys] || n > kCrMaxRows) return;
-    eps_cr_or_pivot(band + band_off[sys], sys_first[sys], n, ywork, eps, sm, xb, &bw_sh, maxbw);
+    eps_cr_or_pivot(band + band_off[sys], sys_first[sys], n, ywork, eps, sm, &bw_sh, maxbw);
 }
 
 __global__ __launch_bounds__(256) void k_eps_band_cr_batch(const CaseDev* __restrict__ cases,
                                                            const CaseSys* __restrict__ sys, int maxbw) {
     extern __shared__ double sm[];
-    __shared__ double xb[2 * (8 + 1)];
     __shared__ int bw_sh;
     const CaseSys q = sys[blockIdx.x];
     const CaseDev& c = cases[q.c];
     const int n = c.eps.n[q.k];
     if (c.eps.outside[q.k] || n > kCrMaxRows) return;
-    eps_cr_or_pivot(c.eps.band + c.eps.off[q.k], c.eps.first[q.k], n, c.eps.y, c.m.eps, sm, xb, &bw_sh, maxbw);
+    eps_cr_or_pivot(c.eps.band + c.eps.off[q.k], c.eps.first[q.k], n, c.eps.y, c.m.eps, sm, &bw_sh, maxbw);
 }
 
 // ---------------------------------------------------------------- fused recompute
@@ -935,8 +1050,7 @@ constexpr int kFusedMaxMarkers = 256;
 template <int KB>
 __device__ __forceinline__ void recompute_body(const MarkerDev& m, const GridScalars& g, int first, int n,
                                                int* __restrict__ outside, double* __restrict__ sm,
-                                               double* __restrict__ xb, int* __restrict__ flag,
-                                               int* __restrict__ bw_sh, int cr_bw) {
+                                               int* __restrict__ flag, int* __restrict__ bw_sh, int cr_bw) {
     constexpr int W = 3 * KB + 1;
     double* P = sm;                // 2n positions
     double* dsl = sm + 2 * n;      // n spacings
@@ -1001,8 +1115,7 @@ __device__ __forceinline__ void recompute_body(const MarkerDev& m, const GridSca
                         blk + (size_t)nb * (3 * kCrMaxBw * kCrMaxBw + kCrMaxBw));
         return;
     }
-    if (tid >= 64) return;
-    eps_band_solve_bw<KB, true, true>(*bw_sh, first, n, Bl, yl, m.eps, xb);
+    eps_band_solve_bw<KB, true>(*bw_sh, first, n, Bl, yl, m.eps);
 }
 
 // Lanes per body workgroup (at least one wavefront for the solve).  Beside
@@ -1015,11 +1128,10 @@ template <int KB>
 __global__ __launch_bounds__(512) void k_recompute_body_batch(const CaseDev* __restrict__ cases,
                                                               const CaseSys* __restrict__ sys, int cr_bw) {
     extern __shared__ double sm[];
-    __shared__ double xb[2 * (KB + 1)];
     __shared__ int flag, bw;
     const CaseSys q = sys[blockIdx.x];
     const CaseDev& c = cases[q.c];
-    recompute_body<KB>(c.m, c.g, c.eps.first[q.k], c.eps.n[q.k], c.eps.outside + q.k, sm, xb, &flag, &bw, cr_bw);
+    recompute_body<KB>(c.m, c.g, c.eps.first[q.k], c.eps.n[q.k], c.eps.outside + q.k, sm, &flag, &bw, cr_bw);
 }
 
 // ObjectsClass::ibmKernelInterp body (IBMNode.cpp:26-58): rho and rho*u at
@@ -1476,7 +1588,7 @@ void launch_eps_band(const MarkerDev& m, const GridScalars& g, const int* sys_fi
     }
     // band, then right-hand side, in LDS for systems of up to lds_rows rows
     const int rows = eps_lds_rows(KB, max_n);
-    k_eps_band_solve<8><<<nsys, 64, sizeof(double) * (size_t)rows * (W + 1), s>>>(
+    k_eps_band_solve<8><<<nsys, kBandThreads, sizeof(double) * (size_t)rows * (W + 1), s>>>(
         sys_first, sys_n, outside, band, band_off, ywork, m.eps, rows, cr ? kCrMaxRows : 0);
 }
 
@@ -1574,7 +1686,7 @@ void launch_eps_band_batch(const CaseDev* cases, const CaseSys* sys, int nsys, i
     }
     if (!cr || max_n > kCrMaxRows) {
         const int rows = eps_lds_rows(KB, max_n);
-        k_eps_band_solve_batch<KB><<<(unsigned)nsys, 64, sizeof(double) * (size_t)rows * (W + 1), s>>>(
+        k_eps_band_solve_batch<KB><<<(unsigned)nsys, kBandThreads, sizeof(double) * (size_t)rows * (W + 1), s>>>(
             cases, sys, rows, cr ? kCrMaxRows : 0);
     }
     k_eps_outside_gather_batch<<<nb, 256, 0, s>>>(cases, sys, nsys, outside_out);
