@@ -413,7 +413,7 @@ void object_kernel_dev(life_case* c, EarlyBulk& eb, int mode) {
         const bool spec = c->spec_spread && c->subIt + 1 >= c->prev_subits;
         for (;;) {
             so.seq = fd.seq += 1.0;
-            launch_fem_dynamic(fd.d_bodies, nullptr, fd.nb, fd.lds, redo, g->stream, so);
+            launch_fem_dynamic(fd.d_bodies, nullptr, fd.nb, fd.lds, fd.max_nel, redo, g->stream, so);
             LIFE_HIP(hipEventRecord(c->ev_forces, g->stream));
             if (spec) ibm_spread(g);
             spread_done = spec;

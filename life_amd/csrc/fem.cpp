@@ -188,6 +188,7 @@ void FemBody::layout(Layout& out) const {
             }
         for (const Map& m : e.map) {
             out.map_node.push_back(m.node);
+            out.map_el.push_back((int)out.map_start.size() - 1);
             out.map_z.push_back(m.z1);
             out.map_z.push_back(m.z2);
         }

@@ -81,7 +81,7 @@ class FemBody {
     // z1, z2) and the marker-to-element map (element, zeta).
     struct Layout {
         std::vector<double> node, el, Mloc, KLloc, map_z, pm_zeta;
-        std::vector<int> map_start, map_node, pm_el;
+        std::vector<int> map_start, map_node, map_el, pm_el;
     };
     void layout(Layout& out) const;
     // Back from the device: the vectors (U, Ud, Udd, Un, Unm1, Unm2, Udn,

@@ -38,6 +38,7 @@ struct FemDevBody {
     const double* mats;    // nel x 2 x kFemMatNZ: M's then KL's upper-triangle non-zeros (constant)
     const int* map_start;  // nel + 1
     const int* map_node;   // marker (body-local) of each load-map entry
+    const int* map_el;     // its element
     const double* map_z;   // 2 per entry
     const int* pm_el;      // nm: element of each marker
     const double* pm_zeta; // nm
@@ -54,6 +55,7 @@ struct FemDevBody {
 // Device FEM of one case's flexible bodies (in the case's body order).
 struct FemDevCase {
     int nb = 0;
+    int max_nel = 0;               // most elements of a body
     std::vector<FemDevBody> host;  // descriptors (device pointers)
     FemDevBody* d_bodies = nullptr;
     std::vector<void*> blocks;     // device allocations
@@ -122,7 +124,7 @@ void fem_wait_sums(const FemSumsOut& so, hipEvent_t ev, double spin_us);
 // so.done set (bodies 0 .. nb-1 only), the last workgroup also writes the
 // sums over the bodies and the flags to the host (synchronise the stream
 // before reading them).
-void launch_fem_dynamic(const FemDevBody* b, const int* list, int nb, size_t lds, bool redo, hipStream_t st,
+void launch_fem_dynamic(const FemDevBody* b, const int* list, int nb, size_t lds, int max_nel, bool redo, hipStream_t st,
                         const FemSumsOut& so = FemSumsOut());
 // out[0..2] of the listed bodies packed into outs (3 per body; outs may be
 // page-locked host memory, readable after the stream is synchronised).

@@ -10,18 +10,20 @@
 //  - the load vector: a node's three DOFs take the terms of the element on
 //    its left (its second node), then of the one on its right, each in
 //    load-map order, exactly the host's accumulation order;
-//  - the banded elimination: one wavefront, the row updates of a step in
-//    parallel (each entry is updated once per step), the pivot search and
-//    the back substitution in the host's order;
-//  - dot products: one lane, in index order.
+//  - the linear solve: block cyclic reduction (block_solve_d), which agrees
+//    with the host's elimination to rounding;
+//  - dot products: their terms side by side, added up by one lane in index
+//    order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
 
+#include "dev_util.h"
 #include "fem.h"
 #include "fem_dev.h"
 #include "runtime.h"
@@ -147,7 +149,9 @@ __host__ __device__ inline int mat_nz(int r, int c) {
 FDI const double* elp(const FemDevBody& B, int e) { return B.el + (size_t)e * kFemElStride; }
 
 // FemBody::update_fem (FEMBody.cpp:198-223)
-FDI void update_fem_d(const FemDevBody& B) {
+// beside: work without barriers for any lanes, done beside the elements'.
+template <typename Fn>
+FDI void update_fem_d(const FemDevBody& B, Fn beside) {
     const int tid = threadIdx.x, nt = blockDim.x;
     const double* U = vecp(B, kFU);
     for (int n = tid; n < B.nnode; n += nt) {
@@ -157,6 +161,7 @@ FDI void update_fem_d(const FemDevBody& B) {
         nd[5] = nd[4] + U[3 * n + 2];
     }
     __syncthreads();
+    beside();
     for (int e = tid; e < B.nel; e += nt) {
         const double* n0 = B.node + 6 * e;
         const double* n1 = B.node + 6 * (e + 1);
@@ -172,6 +177,9 @@ FDI void update_fem_d(const FemDevBody& B) {
         el[8] = sin(angle);
     }
     __syncthreads();
+}
+FDI void update_fem_d(const FemDevBody& B) {
+    update_fem_d(B, [] {});
 }
 
 // FemBody::finish_newmark (FEMBody.cpp:129-144)
@@ -309,38 +317,13 @@ FDI void load_entry_d(const FemDevBody& B, const double* mk, int q, int k, doubl
     mul_t6_d(T, R, RG);
 }
 
-// The load-map entries en0 .. en1-1 of element q, added in map order onto
-// acc (the node's terms of the element: its first node's RG[0..2] or its
-// second node's RG[3..5]).  The entries' map values are loaded eight at a
-// time, ahead of the arithmetic.
-FDI void add_entries_d(const FemDevBody& B, const double* mk, int q, int en0, int en1, int half, double acc[3]) {
-    constexpr int U = 8;
-    for (int base = en0; base < en1; base += U) {
-        int kk[U];
-        double za[U], zb[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int en = base + u;
-            kk[u] = en < en1 ? gload(B.map_node + en) : 0;
-            za[u] = en < en1 ? gload(B.map_z + 2 * en) : 0.0;
-            zb[u] = en < en1 ? gload(B.map_z + 2 * en + 1) : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (base + u < en1) {
-                double RG[6];
-                load_entry_d(B, mk, q, kk[u], za[u], zb[u], RG);
-                acc[0] += RG[3 * half];
-                acc[1] += RG[3 * half + 1];
-                acc[2] += RG[3 * half + 2];
-            }
-        }
-    }
-}
-
 // R (FEMBodyClass::constructRVector) into LDS: node n's DOFs take the terms
 // of element n-1 (its second node) then of element n (its first node),
-// each in load-map order, onto 0.0.
+// each in load-map order, onto 0.0.  The entries of the two elements follow
+// each other in the map.  Every entry's terms are formed first, one lane per
+// entry, into the K and M bands' space (in chunks where they do not fit), then
+// one lane per DOF adds its terms up: 280 markers on 41 nodes took 18 400
+// cycles with one lane per node doing both, 6 500 now.
 FDI void load_vector_d(const FemDevBody& B, const FemLds& S) {
     const int tid = threadIdx.x, nt = blockDim.x;
     for (int k = tid; k < B.nm; k += nt) {
@@ -348,19 +331,42 @@ FDI void load_vector_d(const FemDevBody& B, const FemLds& S) {
         S.mk[3 * k + 1] = gload(B.mforce + 2 * k + 1);
         S.mk[3 * k + 2] = gload(B.meps + k);
     }
+    for (int d = tid; d < B.ndof; d += nt) S.R[d] = 0.0;
     __syncthreads();
-    for (int n = tid; n < B.nnode; n += nt) {
-        double acc[3] = {0.0, 0.0, 0.0};
-        const int s0 = n >= 1 ? gload(B.map_start + n - 1) : 0;
-        const int s1 = gload(B.map_start + n);
-        const int s2 = n < B.nel ? gload(B.map_start + n + 1) : 0;
-        if (n >= 1) add_entries_d(B, S.mk, n - 1, s0, s1, 1, acc);
-        if (n < B.nel) add_entries_d(B, S.mk, n, s1, s2, 0, acc);
-        S.R[3 * n] = acc[0];
-        S.R[3 * n + 1] = acc[1];
-        S.R[3 * n + 2] = acc[2];
+    const int entries = gload(B.map_start + B.nel), chunk = B.ndof * (kFemBandW + kMBand) / 6;
+    double* rg = S.K;
+    for (int c0 = 0; c0 < entries; c0 += chunk) {
+        const int c1 = min(c0 + chunk, entries);
+        for (int en = c0 + tid; en < c1; en += nt) {
+            const int k = gload(B.map_node + en);
+            const double za = gload(B.map_z + 2 * en), zb = gload(B.map_z + 2 * en + 1);
+            double RG[6];
+            load_entry_d(B, S.mk, gload(B.map_el + en), k, za, zb, RG);
+#pragma unroll
+            for (int j = 0; j < 6; j++) rg[6 * (en - c0) + j] = RG[j];
+        }
+        __syncthreads();
+        for (int d = tid; d < B.ndof; d += nt) {
+            const int n = d / 3, j = d - 3 * n;
+            const int s0 = max(n >= 1 ? gload(B.map_start + n - 1) : gload(B.map_start), c0);
+            const int s1 = gload(B.map_start + n), s2 = min(n < B.nel ? gload(B.map_start + n + 1) : s1, c1);
+            double acc = S.R[d];
+            constexpr int U = 8;  // terms read ahead of the sums
+            for (int base = s0; base < s2; base += U) {
+                double v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int en = min(base + u, s2 - 1);
+                    v[u] = rg[6 * (en - c0) + (en < s1 ? 3 : 0) + j];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (base + u < s2) acc += v[u];
+            }
+            S.R[d] = acc;
+        }
+        __syncthreads();
     }
-    __syncthreads();
 }
 
 // Entry (r, c) of the element's rotation matrix make_T(ca, sa).
@@ -397,27 +403,46 @@ FDI void rotate_row_d(double ca, double sa, int i, const double a0[6], const dou
     }
 }
 
-// Row r of the element's geometric stiffness K_NL (FEMElement.cpp:119-131).
-FDI void knl_row(int r, double Fa, double V0, double L0, double out[6]) {
-#pragma unroll
-    for (int j = 0; j < 6; j++) out[j] = 0.0;
-    switch (r) {
-        case 0: out[1] = -V0 / L0; out[4] = V0 / L0; break;
-        case 1: out[0] = -V0 / L0; out[1] = Fa / L0; out[3] = V0 / L0; out[4] = -Fa / L0; break;
-        case 3: out[1] = V0 / L0; out[4] = -V0 / L0; break;
-        case 4: out[0] = V0 / L0; out[1] = -Fa / L0; out[3] = -V0 / L0; out[4] = Fa / L0; break;
-        default: break;
+// Row r of the element's geometric stiffness K_NL (FEMElement.cpp:119-131),
+// v = V0 / L0 and f = Fa / L0 (a quotient changes sign with its dividend).
+FDI void knl_row(int r, double v, double f, double out[6]) {
+    out[0] = r == 1 ? -v : (r == 4 ? v : 0.0);
+    out[1] = r == 0 ? -v : (r == 1 ? f : (r == 3 ? v : (r == 4 ? -f : 0.0)));
+    out[2] = 0.0;
+    out[3] = r == 1 ? v : (r == 4 ? -v : 0.0);
+    out[4] = r == 0 ? v : (r == 1 ? -f : (r == 3 ? -v : (r == 4 ? f : 0.0)));
+    out[5] = 0.0;
+}
+
+// What a lane that forms row i of an element needs to know of the pattern:
+// the rows of A that row i of Transpose(T) A reads (rb: -1, one row), and where
+// the entries of those rows lie among the matrices' non-zeros (mat_nz, four
+// bits each, 15: a zero).  The same for all elements and Newton iterations.
+struct RowPattern {
+    int i, ra, rb;
+    unsigned za, zb;
+};
+FDI RowPattern row_pattern(int i) {
+    RowPattern p{i, kNZdRow(i, 0), kNZdRow(i, 1), 0, 0};
+    for (int j = 0; j < 6; j++) {
+        p.za |= (unsigned)(mat_nz(p.ra, j) & 15) << (4 * j);
+        p.zb |= (unsigned)(mat_nz(p.rb >= 0 ? p.rb : p.ra, j) & 15) << (4 * j);
     }
+    return p;
 }
 
 // force_vector + mass_stiff of element q (FEMElement.cpp:72-138), row i of
-// the element's terms (one lane per row): added onto the global F, M and K
-// in LDS.  Each entry takes the same operations as the whole-element form.
-// Every value the row reads from device memory is loaded first, so the
-// loads share one round trip.
-FDI void element_row_d(const FemDevBody& B, const FemLds& S, int q, int i) {
-    const int ra = kNZdRow(i, 0), rb = kNZdRow(i, 1);
-    const int rb1 = rb >= 0 ? rb : ra;
+// the element's terms of the global F, M and K (one lane per row).  Each entry
+// takes the same operations as the whole-element form.
+struct ElementRow {
+    double F, M[6], K[6];
+};
+FDI ElementRow element_row_d(const FemDevBody& B, RowPattern p, int q) {
+    ElementRow o;
+    // keeps the comparisons with the row here: moved out of the loops, their
+    // masks fill the scalar registers and are spilled and fetched lane by lane
+    asm("" : "+v"(p.i), "+v"(p.ra), "+v"(p.rb), "+v"(p.za), "+v"(p.zb));
+    const int i = p.i, ra = p.ra, rb = p.rb, rb1 = rb >= 0 ? rb : ra;
     const double* e = B.el + (size_t)q * kFemElStride;
     const double* Mc = B.mats + 2 * kFemMatNZ * (size_t)q;
     const double* Kc = Mc + kFemMatNZ;
@@ -427,11 +452,13 @@ FDI void element_row_d(const FemDevBody& B, const FemLds& S, int q, int i) {
     const double nth0 = B.node[6 * q + 5], nth1 = B.node[6 * (q + 1) + 5];
 #pragma unroll
     for (int j = 0; j < 6; j++) {
-        const int za = mat_nz(ra, j), zb = mat_nz(rb1, j);
-        m0[j] = za >= 0 ? Mc[za] : 0.0;
-        m1[j] = zb >= 0 ? Mc[zb] : 0.0;
-        k0[j] = za >= 0 ? Kc[za] : 0.0;
-        k1[j] = zb >= 0 ? Kc[zb] : 0.0;
+        const unsigned za = p.za >> (4 * j) & 15, zb = p.zb >> (4 * j) & 15;
+        const double ma = Mc[min(za, kFemMatNZ - 1u)], mb = Mc[min(zb, kFemMatNZ - 1u)];
+        const double ka = Kc[min(za, kFemMatNZ - 1u)], kb = Kc[min(zb, kFemMatNZ - 1u)];
+        m0[j] = za != 15 ? ma : 0.0;
+        m1[j] = zb != 15 ? mb : 0.0;
+        k0[j] = za != 15 ? ka : 0.0;
+        k1[j] = zb != 15 ? kb : 0.0;
     }
     const double L0 = ev[0], L = ev[1], angle = ev[2], A = ev[3], I = ev[4], E = ev[5];
     const double ca = ev[7], sa = ev[8];
@@ -444,73 +471,81 @@ FDI void element_row_d(const FemDevBody& B, const FemLds& S, int q, int i) {
     // Fe (the element's local forces): the two entries row i reads
     const double Fsum = (1.0 / L0) * (M1 + M2);
     auto fe = [&](int r) {
-        switch (r) {
-            case 0: return -F0;
-            case 1: return Fsum;
-            case 2: return M1;
-            case 3: return F0;
-            case 4: return -((1.0 / L0) * (M1 + M2));
-            default: return M2;
-        }
+        return r == 0 ? -F0 : (r == 1 ? Fsum : (r == 2 ? M1 : (r == 3 ? F0 : (r == 4 ? -Fsum : M2))));
     };
     // row i of Transpose(T) Fe (mul_t6_d)
     double fg = 0.0;
     fg += t_entry(ca, sa, ra, i) * fe(ra);
     if (rb >= 0) fg += t_entry(ca, sa, rb, i) * fe(rb);
-    const int d0 = 3 * q, row = d0 + i;
     double G[6], N[6], n0[6], n1[6];
-    rotate_row_d(ca, sa, i, m0, m1, G);
-    S.F[row] += fg;
-#pragma unroll
-    for (int j = 0; j < 6; j++) mband(S.M, row, d0 + j) += G[j];
+    o.F = fg;
+    rotate_row_d(ca, sa, i, m0, m1, o.M);
     rotate_row_d(ca, sa, i, k0, k1, G);
-    const double Fa = F0, V0 = -((1.0 / L0) * (M1 + M2));
-    knl_row(ra, Fa, V0, L0, n0);
-    knl_row(rb1, Fa, V0, L0, n1);
+    const double V0 = -Fsum, kv = V0 / L0, kf = F0 / L0;
+    knl_row(ra, kv, kf, n0);
+    knl_row(rb1, kv, kf, n1);
     rotate_row_d(ca, sa, i, n0, n1, N);
 #pragma unroll
-    for (int j = 0; j < 6; j++) band(S.K, row, d0 + j) += G[j] + N[j];
+    for (int j = 0; j < 6; j++) o.K[j] = G[j] + N[j];
+    return o;
 }
 
 // FemBody::build_global (FEMBody.cpp:90-109) into LDS.  Elements q and q+1
-// share a node, so the even elements go first, then the odd ones; an entry
-// takes at most two terms, whose sum does not depend on their order.
-FDI void build_global_d(const FemDevBody& B, const FemLds& S) {
+// share a node, so the even elements are added first, then the odd ones; an
+// entry takes at most two terms, whose sum does not depend on their order.
+// The rows of both are formed together before (40 elements: 18 700 cycles with
+// the two parities one after the other, 12 000 now).
+FDI void build_global_d(const FemDevBody& B, const FemLds& S, const RowPattern& p) {
     const int tid = threadIdx.x, nt = blockDim.x;
     for (int k = tid; k < B.ndof * kFemBandW; k += nt) S.K[k] = 0.0;
     for (int k = tid; k < B.ndof * kMBand; k += nt) S.M[k] = 0.0;
     for (int k = tid; k < B.ndof; k += nt) S.F[k] = 0.0;
     __syncthreads();
-    const int nph = (B.nel + 1) / 2;  // elements of one parity, at most
-    for (int ph = 0; ph < 2; ph++) {
-        for (int t = tid; t < 6 * nph; t += nt) {
-            const int q = ph + 2 * (t / 6);
-            if (q < B.nel) element_row_d(B, S, q, t % 6);
+    const int per = nt / 6;  // elements a round
+    for (int q0 = 0; q0 < B.nel; q0 += per) {
+        const int q = q0 + tid / 6, i = p.i;
+        const bool on = tid < 6 * per && q < B.nel;
+        ElementRow e;
+        if (on) e = element_row_d(B, p, q);
+        for (int ph = 0; ph < 2; ph++) {
+            if (on && (q & 1) == ph) {
+                const int d0 = 3 * q, row = d0 + i;
+                S.F[row] += e.F;
+#pragma unroll
+                for (int j = 0; j < 6; j++) {
+                    mband(S.M, row, d0 + j) += e.M[j];
+                    band(S.K, row, d0 + j) += e.K[j];
+                }
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
 }
 
-// Inverse of a 3x3 block (row-major, in place) by its adjugate.
-FDI void inv3_d(double* D) {
+// Entry e of the inverse of a 3x3 block (row-major) by its adjugate.  sel: the
+// entry's cofactor, D[p] D[q] - D[u] D[v], as p | q << 4 | u << 8 | v << 12.
+FDI unsigned cofactor_sel(int e) {
+    constexpr unsigned t[9] = {0x7584, 0x8172, 0x4251, 0x8365, 0x6280, 0x5032, 0x6473, 0x7061, 0x3140};
+    unsigned s = t[0];
+#pragma unroll
+    for (int k = 1; k < 9; k++) s = e == k ? t[k] : s;
+    return s;
+}
+FDI double inv3_entry_d(const double* D, unsigned sel) {
     const double a = D[0], b = D[1], c = D[2], d = D[3], e = D[4], f = D[5], g = D[6], h = D[7], i = D[8];
+    const double p = D[sel & 15], q = D[sel >> 4 & 15], u = D[sel >> 8 & 15], v = D[sel >> 12];
     const double c00 = e * i - f * h, c01 = f * g - d * i, c02 = d * h - e * g;
     const double det = a * c00 + b * c01 + c * c02;
     const double r = 1.0 / det;
-    D[0] = c00 * r;
-    D[1] = (c * h - b * i) * r;
-    D[2] = (b * f - c * e) * r;
-    D[3] = c01 * r;
-    D[4] = (a * i - c * g) * r;
-    D[5] = (c * d - a * f) * r;
-    D[6] = c02 * r;
-    D[7] = (b * g - a * h) * r;
-    D[8] = (a * e - b * d) * r;
+    return (p * q - u * v) * r;
 }
 
 // Node blocks of the cyclic reduction: sub-diagonal A, diagonal D (its
 // inverse once the node is eliminated), super-diagonal C, right-hand side f.
 constexpr int kBlkA = 0, kBlkD = 9, kBlkC = 18, kBlkF = 27, kBlk = 30;
+constexpr int kSolveNodes = 3;   // nodes per wavefront of a forward level, 18 lanes each
+constexpr int kInvertNodes = 7;  // nodes per wavefront, nine lanes each
+constexpr int kBackNodes = 21;   // nodes per wavefront, three lanes each
 
 // K x = F (K + a0 M from newton_d, band in LDS) with x = 0 on the nbc
 // clamped DOFs.  An element couples two neighbouring nodes, so K is block
@@ -524,85 +559,110 @@ constexpr int kBlkA = 0, kBlkD = 9, kBlkC = 18, kBlkF = 27, kBlk = 30;
 // symmetric positive definite (the Newmark mass term dominates), so no
 // pivoting is needed.  The values agree with the host's scalar elimination
 // to rounding, not bit for bit.  Blocks: kBlk doubles per node in the M
-// band's space (free once K + a0 M is formed); a level's new blocks are
-// staged in the K band's space (free once the blocks are read out of it).
+// band's space (free once K + a0 M is formed).  Lanes of one wavefront share a
+// node: 18 (nine per neighbour, an entry each, the products' left factors
+// exchanged through the K band's space) in the forward levels, three in the
+// back substitution.  A node's new blocks replace the old ones in place (all
+// its lanes have read before one writes), and the inverse that the next level
+// takes out is formed, an entry per lane, without a barrier in between: one
+// barrier a level.  The bound is the instructions each lane issues, six levels
+// one after the other.  41 nodes: 25 000 cycles with nine lanes per node that
+// took both neighbours' whole products, the inverse by one lane and three
+// barriers a level, 19 000 now.
 FDI void block_solve_d(const FemDevBody& B, const FemLds& S) {
-    const int tid = threadIdx.x, nt = blockDim.x;
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid % 64, wave = tid / 64, waves = nt / 64;
     const int N = B.nnode, nbc = B.nbc;
-    // constrained DOFs: identity rows and columns, zero right-hand side
-    for (int t = tid; t < nbc * (2 * kFemKL + 1); t += nt) {
-        const int d = t / (2 * kFemKL + 1), o = t % (2 * kFemKL + 1) - kFemKL;  // o = column - row
-        const int c = d + o;
-        if (c >= 0 && c < B.ndof) {
-            band(S.K, d, c) = (o == 0) ? 1.0 : 0.0;  // row d
-            if (o != 0) band(S.K, c, d) = 0.0;        // column d
-        }
-    }
-    for (int d = tid; d < nbc; d += nt) S.F[d] = 0.0;
-    __syncthreads();
     double* blk = S.M;
-    for (int t = tid; t < N * kBlk; t += nt) {
-        const int n = t / kBlk, q = t % kBlk;
-        double v;
-        if (q < kBlkF) {
-            const int cn = n + q / 9 - 1, i = (q % 9) / 3, j = q % 3;  // column node n-1, n, n+1
-            v = (cn < 0 || cn >= N) ? 0.0 : band(S.K, 3 * n + i, 3 * cn + j);
-        } else {
-            v = S.F[3 * n + q - kBlkF];
+    {
+        // 32 lanes per node, entry q of its blocks each (nt is a multiple of 32)
+        const int q = tid % 32, i = (q % 9) / 3, j = q % 3, part = q / 9 - 1;
+        for (int n = tid / 32; n < N; n += nt / 32) {
+            double v;
+            if (q < kBlkF) {
+                const int cn = n + part, r = 3 * n + i, c = 3 * cn + j;  // column node n-1, n, n+1
+                // constrained DOFs: identity rows and columns, zero right-hand side
+                if (cn < 0 || cn >= N) v = 0.0;
+                else if (r < nbc || c < nbc) v = r == c ? 1.0 : 0.0;
+                else v = band(S.K, r, c);
+            } else {
+                const int r = 3 * n + q - kBlkF;
+                v = r < nbc || q >= kBlk ? 0.0 : S.F[r];
+            }
+            if (q < kBlk) blk[kBlk * n + q] = v;
         }
-        blk[t] = v;
     }
     __syncthreads();
-    double* stage = S.K;
+    const int en = lane % 9, r = en / 3, c = en % 3;
+    const unsigned sel = cofactor_sel(en);
+    // entry en of inv(D_j) in place of D_j: nine lanes of a wavefront together
+    auto invert = [&](bool act, int j) {
+        double* D = blk + kBlk * j + kBlkD;
+        wave_fence();
+        const double v = act ? inv3_entry_d(D, sel) : 0.0;
+        wave_fence();
+        if (act) D[en] = v;
+    };
+    // level 1 takes the odd nodes out (a single node is inverted as it is)
+    for (int k0 = 0; k0 == 0 || 2 * k0 + 1 < N; k0 += waves * kInvertNodes) {
+        const int k = k0 + wave * kInvertNodes + lane / 9, j = N == 1 ? k : 2 * k + 1;
+        invert(lane < 9 * kInvertNodes && j < N, j);
+    }
+    __syncthreads();
+    const int slots = waves * kSolveNodes, slot = wave * kSolveNodes + lane / 18, side = lane % 18 / 9;
+    const bool on = lane < 18 * kSolveNodes;
+    double* left = S.K + 18 * slot + 9 * side;  // this neighbour's left factor
     int s = 1;
     for (; s < N; s *= 2) {
-        // nodes j = s, 3s, 5s, ... leave: D_j becomes its inverse
-        for (int j = s + 2 * s * tid; j < N; j += 2 * s * nt) inv3_d(blk + kBlk * j + kBlkD);
-        __syncthreads();
-        // nodes i = 0, 2s, 4s, ... take them out, entry (r, c) per lane:
+        // nodes j = s, 3s, 5s, ... leave (D_j holds its inverse); nodes
+        // i = 0, 2s, 4s, ... take them out, entry (r, c) per lane and side:
         //   al = A_i inv(D_{i-s}), ga = C_i inv(D_{i+s})
         //   D_i - al C_{i-s} - ga A_{i+s},  -al A_{i-s},  -ga C_{i+s},
         //   f_i - al f_{i-s} - ga f_{i+s}
         const int nr = (N - 1) / (2 * s) + 1;
-        for (int t = tid; t < 9 * nr; t += nt) {
-            const int k = t / 9, r = (t % 9) / 3, c = t % 3, i = 2 * s * k;
-            const double* bi = blk + kBlk * i;
-            double Dn = bi[kBlkD + 3 * r + c], An = 0.0, Cn = 0.0, fn = bi[kBlkF + r];
-            if (i - s >= 0) {
-                const double* bj = blk + kBlk * (i - s);
-                double al[3];
-#pragma unroll
-                for (int q = 0; q < 3; q++)
-                    al[q] = bi[kBlkA + 3 * r] * bj[kBlkD + q] + bi[kBlkA + 3 * r + 1] * bj[kBlkD + 3 + q] +
-                            bi[kBlkA + 3 * r + 2] * bj[kBlkD + 6 + q];
-                Dn = Dn - (al[0] * bj[kBlkC + c] + al[1] * bj[kBlkC + 3 + c] + al[2] * bj[kBlkC + 6 + c]);
-                An = -(al[0] * bj[kBlkA + c] + al[1] * bj[kBlkA + 3 + c] + al[2] * bj[kBlkA + 6 + c]);
-                fn = fn - (al[0] * bj[kBlkF] + al[1] * bj[kBlkF + 1] + al[2] * bj[kBlkF + 2]);
+        for (int k0 = 0; k0 < nr; k0 += slots) {
+            const int k = k0 + slot, i = 2 * s * k, j = side ? i + s : i - s;
+            const bool act = on && k < nr, has = act && j >= 0 && j < N;
+            double* bi = blk + kBlk * i;
+            const double* bj = blk + kBlk * j;
+            const int oX = side ? kBlkC : kBlkA, oY = side ? kBlkA : kBlkC;
+            double dD = 0.0, dX = 0.0, df = 0.0, D = 0.0, f = 0.0;
+            if (has) {
+                const double* X = bi + oX + 3 * r;
+                left[en] = X[0] * bj[kBlkD + c] + X[1] * bj[kBlkD + 3 + c] + X[2] * bj[kBlkD + 6 + c];
             }
-            if (i + s < N) {
-                const double* bj = blk + kBlk * (i + s);
-                double ga[3];
-#pragma unroll
-                for (int q = 0; q < 3; q++)
-                    ga[q] = bi[kBlkC + 3 * r] * bj[kBlkD + q] + bi[kBlkC + 3 * r + 1] * bj[kBlkD + 3 + q] +
-                            bi[kBlkC + 3 * r + 2] * bj[kBlkD + 6 + q];
-                Dn = Dn - (ga[0] * bj[kBlkA + c] + ga[1] * bj[kBlkA + 3 + c] + ga[2] * bj[kBlkA + 6 + c]);
-                Cn = -(ga[0] * bj[kBlkC + c] + ga[1] * bj[kBlkC + 3 + c] + ga[2] * bj[kBlkC + 6 + c]);
-                fn = fn - (ga[0] * bj[kBlkF] + ga[1] * bj[kBlkF + 1] + ga[2] * bj[kBlkF + 2]);
+            wave_fence();
+            if (has) {
+                const double l0 = left[3 * r], l1 = left[3 * r + 1], l2 = left[3 * r + 2];
+                dD = l0 * bj[oY + c] + l1 * bj[oY + 3 + c] + l2 * bj[oY + 6 + c];
+                dX = -(l0 * bj[oX + c] + l1 * bj[oX + 3 + c] + l2 * bj[oX + 6 + c]);
+                df = l0 * bj[kBlkF] + l1 * bj[kBlkF + 1] + l2 * bj[kBlkF + 2];
             }
-            double* o = stage + kBlk * k;
-            o[kBlkA + 3 * r + c] = An;
-            o[kBlkD + 3 * r + c] = Dn;
-            o[kBlkC + 3 * r + c] = Cn;
-            if (c == 0) o[kBlkF + r] = fn;
+            if (act) {
+                D = bi[kBlkD + en];
+                f = bi[kBlkF + r];
+            }
+            // the first nine lanes take the second neighbour's terms after their own
+            const double dD2 = __shfl_down(dD, 9), df2 = __shfl_down(df, 9);
+            wave_fence();  // the lanes of the node have read the old blocks
+            if (act) bi[oX + en] = dX;
+            if (act && side == 0) {
+                if (has) {
+                    D = D - dD;
+                    f = f - df;
+                }
+                if (i + s < N) {
+                    D = D - dD2;
+                    f = f - df2;
+                }
+                bi[kBlkD + en] = D;
+                if (c == 0) bi[kBlkF + r] = f;
+            }
+            // the nodes of the next level, and after the last one node 0
+            invert(act && side == 0 && ((k & 1) || 2 * s >= N), i);
         }
-        __syncthreads();
-        for (int t = tid; t < kBlk * nr; t += nt) blk[kBlk * 2 * s * (t / kBlk) + t % kBlk] = stage[t];
         __syncthreads();
     }
     // node 0 alone: x_0 = inv(D_0) f_0
-    if (tid == 0) inv3_d(blk + kBlkD);
-    __syncthreads();
     if (tid < 3) {
         const double* b0 = blk;
         S.x[tid] = b0[kBlkD + 3 * tid] * b0[kBlkF] + b0[kBlkD + 3 * tid + 1] * b0[kBlkF + 1] +
@@ -610,25 +670,27 @@ FDI void block_solve_d(const FemDevBody& B, const FemLds& S) {
     }
     __syncthreads();
     // back substitution, levels in reverse: x_j = inv(D_j) (f_j - A_j x_{j-s} - C_j x_{j+s})
+    const int a = lane % 3;
     for (s /= 2; s >= 1; s /= 2) {
         const int ne = (N + s - 1) / (2 * s);
-        for (int t = tid; t < 3 * ne; t += nt) {
-            const int j = s + 2 * s * (t / 3), r = t % 3;
-            const double* bj = blk + kBlk * j;
-            const double* xl = S.x + 3 * (j - s);
-            double v[3];
-#pragma unroll
-            for (int a = 0; a < 3; a++)
-                v[a] = bj[kBlkF + a] - (bj[kBlkA + 3 * a] * xl[0] + bj[kBlkA + 3 * a + 1] * xl[1] +
-                                        bj[kBlkA + 3 * a + 2] * xl[2]);
-            if (j + s < N) {
-                const double* xr = S.x + 3 * (j + s);
-#pragma unroll
-                for (int a = 0; a < 3; a++)
-                    v[a] = v[a] - (bj[kBlkC + 3 * a] * xr[0] + bj[kBlkC + 3 * a + 1] * xr[1] +
-                                   bj[kBlkC + 3 * a + 2] * xr[2]);
+        for (int k0 = 0; k0 < ne; k0 += waves * kBackNodes) {
+            const int k = k0 + wave * kBackNodes + lane / 3, j = s + 2 * s * k;
+            const bool act = lane < 3 * kBackNodes && k < ne;
+            double* bj = blk + kBlk * j;
+            if (act) {
+                const double* xl = S.x + 3 * (j - s);
+                double v = bj[kBlkF + a] -
+                           (bj[kBlkA + 3 * a] * xl[0] + bj[kBlkA + 3 * a + 1] * xl[1] + bj[kBlkA + 3 * a + 2] * xl[2]);
+                if (j + s < N) {
+                    const double* xr = S.x + 3 * (j + s);
+                    v = v - (bj[kBlkC + 3 * a] * xr[0] + bj[kBlkC + 3 * a + 1] * xr[1] + bj[kBlkC + 3 * a + 2] * xr[2]);
+                }
+                bj[kBlkF + a] = v;
             }
-            S.x[3 * j + r] = bj[kBlkD + 3 * r] * v[0] + bj[kBlkD + 3 * r + 1] * v[1] + bj[kBlkD + 3 * r + 2] * v[2];
+            wave_fence();
+            if (act)
+                S.x[3 * j + a] = bj[kBlkD + 3 * a] * bj[kBlkF] + bj[kBlkD + 3 * a + 1] * bj[kBlkF + 1] +
+                                 bj[kBlkD + 3 * a + 2] * bj[kBlkF + 2];
         }
         __syncthreads();
     }
@@ -638,9 +700,9 @@ FDI void block_solve_d(const FemDevBody& B, const FemLds& S) {
 
 // FemBody::newton_dynamic (FEMBody.cpp:71-87, 112-126) and the residual
 // test of dynamic(): returns resNR (every lane).
-FDI double newton_d(const FemDevBody& B, const FemLds& S) {
+FDI double newton_d(const FemDevBody& B, const FemLds& S, const RowPattern& p) {
     const int tid = threadIdx.x, nt = blockDim.x;
-    build_global_d(B, S);
+    build_global_d(B, S, p);
     const double Dt = B.s.Dt, al = B.s.alpha;
     const double a0 = 1.0 / (al * (Dt * Dt));
     const double a2 = 1.0 / (al * Dt);
@@ -649,26 +711,40 @@ FDI double newton_d(const FemDevBody& B, const FemLds& S) {
     double *U = vecp(B, kFU), *Un = vecp(B, kFUn), *Ud = vecp(B, kFUd), *Udd = vecp(B, kFUdd);
     for (int k = tid; k < nd; k += nt) S.vec[k] = a0 * (Un[k] - U[k]) + a2 * Ud[k] + a3 * Udd[k];
     __syncthreads();
-    const int kb = kFemKL;
+    static_assert(kMBand == kFemBandW, "rows of M and K of one width");
     for (int i = tid; i < nd; i += nt) {
+        // the row's entries read before the first is used
+        double mv[kMBand], kv[kMBand], vv[kMBand];
+#pragma unroll
+        for (int o = 0; o < kMBand; o++) {
+            mv[o] = S.M[(size_t)i * kMBand + o];
+            kv[o] = S.K[(size_t)i * kMBand + o];
+            vv[o] = S.vec[min(max(i - kFemKL + o, 0), nd - 1)];
+        }
         double s = 0.0;
-        const int lo = i - kb < 0 ? 0 : i - kb, hi = i + kb > nd - 1 ? nd - 1 : i + kb;
-        for (int j = lo; j <= hi; j++) s += mband(S.M, i, j) * S.vec[j];
+#pragma unroll
+        for (int o = 0; o < kMBand; o++) {
+            const int j = i - kFemKL + o;
+            if (j < 0 || j >= nd) continue;
+            s += mv[o] * vv[o];
+            S.K[(size_t)i * kMBand + o] = kv[o] + a0 * mv[o];
+        }
         S.F[i] = S.R[i] - S.F[i] + s;
-        for (int j = lo; j <= hi; j++) band(S.K, i, j) = band(S.K, i, j) + a0 * mband(S.M, i, j);
     }
     __syncthreads();
     block_solve_d(B, S);
-    for (int k = tid; k < nd; k += nt) U[k] = U[k] + S.x[k];
-    __syncthreads();
-    update_fem_d(B);
-    __shared__ double res_sh;
-    if (tid == 0) {
-        double r = 0.0;
-        for (int k = 0; k < nd; k++) r += S.x[k] * S.x[k];
-        res_sh = sqrt(r) / (B.s.ref_L * sqrt((double)nd));
+    for (int k = tid; k < nd; k += nt) {
+        const double x = S.x[k];
+        U[k] = U[k] + x;
+        S.vec[k] = x * x;
     }
     __syncthreads();
+    // the squares added up in DOF order by a lane of the last wavefront,
+    // beside the elements' update in the first ones
+    __shared__ double res_sh;
+    update_fem_d(B, [&] {
+        if (tid == nt - 64) res_sh = sqrt(serial_sum(0.0, S.vec, nd)) / (B.s.ref_L * sqrt((double)nd));
+    });
     return res_sh;
 }
 
@@ -782,17 +858,20 @@ __global__ __launch_bounds__(kFemThreads) void k_fem_relax(const FemDevBody* __r
 // system-scope fence) writes the launch's sequence number beside the sums.
 FDI void sums_by_last(const FemDevBody* __restrict__ bodies, const FemSumsOut& so) {
     __shared__ int last;
-    __shared__ double t[3 * kFemThreads];
-    __syncthreads();  // every lane's writes of this body precede the count
-    if (threadIdx.x == 0) {
-        __threadfence();
-        last = atomicAdd(so.done, 1) == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
+    constexpr int kStaged = 256;  // bodies whose terms are read side by side
+    __shared__ double t[3 * kStaged];
     const int nb = gridDim.x;
-    for (int b = threadIdx.x; b < nb && b < kFemThreads; b += blockDim.x) {
+    __syncthreads();  // every lane's writes of this body precede the count
+    if (nb > 1) {  // a single body has no one to wait for
+        if (threadIdx.x == 0) {
+            __threadfence();
+            last = atomicAdd(so.done, 1) == nb - 1;
+        }
+        __syncthreads();
+        if (!last) return;
+        __threadfence();
+    }
+    for (int b = threadIdx.x; b < nb && b < kStaged; b += blockDim.x) {
         const double* o = bodies[b].out;
         t[3 * b] = o[0];
         t[3 * b + 1] = o[1];
@@ -805,7 +884,7 @@ FDI void sums_by_last(const FemDevBody* __restrict__ bodies, const FemSumsOut& s
     if (threadIdx.x == 0) {
         double r = 0.0, num = 0.0, den = 0.0;
         for (int b = 0; b < nb; b++) {
-            const double* o = b < kFemThreads ? t + 3 * b : bodies[b].out;
+            const double* o = b < kStaged ? t + 3 * b : bodies[b].out;
             r += o[0];
             num += o[1];
             den += o[2];
@@ -813,7 +892,7 @@ FDI void sums_by_last(const FemDevBody* __restrict__ bodies, const FemSumsOut& s
         so.sums_h[0] = r;
         so.sums_h[1] = num;
         so.sums_h[2] = den;
-        atomicExch(so.done, 0);
+        if (nb > 1) atomicExch(so.done, 0);
         __threadfence_system();
         *(volatile double*)&so.sums_h[3] = so.seq;
     }
@@ -822,12 +901,18 @@ FDI void sums_by_last(const FemDevBody* __restrict__ bodies, const FemSumsOut& s
 // FemBody::dynamic (FEMBody.cpp:26-68) and subResidual (FEMBody.cpp:244-256)
 // redo: the same solve again after epsilon changed (the dense fallback of
 // computeEpsilon): Rkm1 already holds the previous subiteration's Rk.
-__global__ __launch_bounds__(kFemThreads) void k_fem_dynamic(const FemDevBody* __restrict__ bodies,
-                                                            const int* __restrict__ list, int redo,
-                                                            FemSumsOut so) {
+// NT lanes: kFemThreads form the rows of up to 42 elements in one round, 512
+// those of 85.  11 bodies of 20 to 53 elements: 50 us with 512 lanes, 58 with
+// 256; one of 40: 48 and 47.  Many bodies (the canopy's filaments on the CUs
+// of two XCDs) are bound by issue, not by latency: 104 us and 102, 2 % of the
+// step; hence kFemWideBodies.
+constexpr int kFemWideBodies = 32;
+template <int NT>
+__global__ __launch_bounds__(NT) void k_fem_dynamic(const FemDevBody* __restrict__ bodies,
+                                                    const int* __restrict__ list, int redo, FemSumsOut so) {
     extern __shared__ double lds[];
-    const FemDevBody G = bodies[body_index(list)];
-    const FemDevBody B = mirror_in(G, lds, true);
+    const FemDevBody* body = bodies + body_index(list);
+    FemDevBody B = mirror_in(*body, lds, true);
     copy_vec(B, kFU, kFUn);
     copy_vec(B, kFUd, kFUdn);
     copy_vec(B, kFUdd, kFUddn);
@@ -835,41 +920,42 @@ __global__ __launch_bounds__(kFemThreads) void k_fem_dynamic(const FemDevBody* _
     update_fem_d(B);
     const FemLds S = fem_lds(B, lds);
     load_vector_d(B, S);
+    const RowPattern p = row_pattern(threadIdx.x % 6);
     int it = 0;
     double res;
     do {
-        res = newton_d(B, S);
+        res = newton_d(B, S, p);
         it++;
     } while (res > 1e-10 && it < 20);
+    // what only the rest needs is read (again) here, not held in scalar
+    // registers over the iterations
+    asm volatile("" : "+s"(body));
+    const FemDevBody G = *body;
+    B.s = G.s;
+    B.pm_el = G.pm_el;
+    B.pm_zeta = G.pm_zeta;
+    B.out = G.out;
+    B.mpos = G.mpos;
+    B.mvel = G.mvel;
     finish_newmark_d(B);
     update_ibm_d(B, lds);
     // Rkm1 takes Rk, Rk = U - Ukm1
     if (!redo) copy_vec(B, kFRkm1, kFRk);
     __syncthreads();
     double *Rk = vecp(B, kFRk), *Rkm1 = vecp(B, kFRkm1), *U = vecp(B, kFU), *Ukm1 = vecp(B, kFUkm1);
-    // Rk and Rkm1 also into LDS (F and R are free now) for the sums below
+    // the terms of the three sums into LDS (F, R and vec are free now)
     for (int k = threadIdx.x; k < B.ndof; k += blockDim.x) {
-        const double rk = U[k] - Ukm1[k];
+        const double rk = U[k] - Ukm1[k], rm = Rkm1[k];
         Rk[k] = rk;
-        S.F[k] = rk;
-        S.R[k] = Rkm1[k];
+        S.F[k] = rk * rk;
+        S.R[k] = rm * (rk - rm);
+        S.vec[k] = (rk - rm) * (rk - rm);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        // the three sums in DOF order each, side by side
-        double r = 0.0, num = 0.0, den = 0.0;
-        for (int k = 0; k < B.ndof; k++) {
-            const double rk = S.F[k], rm = S.R[k];
-            r += rk * rk;
-            num += rm * (rk - rm);
-            den += (rk - rm) * (rk - rm);
-        }
-        B.out[0] = r;
-        B.out[1] = num;
-        B.out[2] = den;
-        B.out[3] = (double)it;
-        B.out[4] = res;
-    }
+    // the three sums in DOF order each, a lane each
+    if (threadIdx.x < 3) B.out[threadIdx.x] = serial_sum(0.0, threadIdx.x == 0 ? S.F : (threadIdx.x == 1 ? S.R : S.vec), B.ndof);
+    if (threadIdx.x == 3) B.out[3] = (double)it;
+    if (threadIdx.x == 4) B.out[4] = res;
     mirror_out(G, B);
     if (so.done) sums_by_last(bodies, so);
 }
@@ -909,11 +995,14 @@ void launch_fem_relax(const FemDevBody* b, const int* list, int nb, double omega
     LIFE_HIP(hipGetLastError());
 }
 
-void launch_fem_dynamic(const FemDevBody* b, const int* list, int nb, size_t lds, bool redo, hipStream_t st,
-                        const FemSumsOut& so) {
+void launch_fem_dynamic(const FemDevBody* b, const int* list, int nb, size_t lds, int max_nel, bool redo,
+                        hipStream_t st, const FemSumsOut& so) {
     if (nb == 0) return;
     if (so.done && list) throw std::logic_error("device FEM: sums of a listed launch");
-    k_fem_dynamic<<<nb, kFemThreads, lds, st>>>(b, list, redo ? 1 : 0, so);
+    if (max_nel > kFemThreads / 6 && nb <= kFemWideBodies)
+        k_fem_dynamic<512><<<nb, 512, lds, st>>>(b, list, redo ? 1 : 0, so);
+    else
+        k_fem_dynamic<kFemThreads><<<nb, kFemThreads, lds, st>>>(b, list, redo ? 1 : 0, so);
     LIFE_HIP(hipGetLastError());
 }
 
@@ -1003,6 +1092,7 @@ void fem_dev_create(FemDevCase& fc, const std::vector<const FemBody*>& bodies, c
         d.mats = d.el + (size_t)kFemElStride * d.nel;
         d.map_start = upload_vec(fc, lay.map_start, st);
         d.map_node = upload_vec(fc, lay.map_node, st);
+        d.map_el = upload_vec(fc, lay.map_el, st);
         d.map_z = upload_vec(fc, lay.map_z, st);
         d.pm_el = upload_vec(fc, lay.pm_el, st);
         d.pm_zeta = upload_vec(fc, lay.pm_zeta, st);
@@ -1014,11 +1104,13 @@ void fem_dev_create(FemDevCase& fc, const std::vector<const FemBody*>& bodies, c
         fc.host.push_back(d);
         const size_t need = fem_dev_lds_bytes(d.ndof, d.nm);
         if (need > lds) lds = need;
+        fc.max_nel = std::max(fc.max_nel, d.nel);
     }
     if (lds > kFemMaxLds) throw std::runtime_error("flexible body too large for the device FEM");
     fc.lds = lds;
     // dynamic LDS beyond 64 KiB per workgroup
-    for (const void* k : {(const void*)k_fem_predict, (const void*)k_fem_relax, (const void*)k_fem_dynamic})
+    for (const void* k : {(const void*)k_fem_predict, (const void*)k_fem_relax, (const void*)k_fem_dynamic<512>,
+                          (const void*)k_fem_dynamic<kFemThreads>})
         LIFE_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFemMaxLds));
     fc.d_bodies = upload_vec(fc, fc.host, st);
     fc.done = dalloc<int>(1);

@@ -209,6 +209,7 @@ struct life_server {
     // their residual terms
     bool fem_device = false;
     size_t fem_lds = 0;
+    int fem_nel = 0;  // most elements of a body
     Mirror<FemDevBody> fem_bodies;
     Mirror<int> fem_list, fem_list2;
     Mirror<double> fem_param, fem_out;
@@ -341,6 +342,7 @@ void rebuild(life_server* s) {
     std::vector<FemDevBody> fb;
     bool all_dev = true, any_flex = false;
     s->fem_lds = 0;
+    s->fem_nel = 0;
     for (Slot& sl : s->slots) {
         life_case* c = sl.c;
         if (!c->hasFlex) continue;
@@ -352,6 +354,7 @@ void rebuild(life_server* s) {
         sl.fem_off = (int)fb.size();
         fb.insert(fb.end(), c->fdev.host.begin(), c->fdev.host.end());
         s->fem_lds = std::max(s->fem_lds, c->fdev.lds);
+        s->fem_nel = std::max(s->fem_nel, c->fdev.max_nel);
     }
     s->fem_device = any_flex && all_dev;
     if (s->fem_device) {
@@ -609,7 +612,7 @@ int fem_recompute_device(life_server* s, const std::vector<int>& active) {
 // again with it.
 void fem_solve_device(life_server* s, const std::vector<int>& active, const std::vector<CaseSys>& sysl, int nfb) {
     hipStream_t st = s->stream;
-    launch_fem_dynamic(s->fem_bodies.d, s->fem_list.d, nfb, s->fem_lds, false, st);
+    launch_fem_dynamic(s->fem_bodies.d, s->fem_list.d, nfb, s->fem_lds, s->fem_nel, false, st);
     // the device has room beside the FEM's few workgroups: the next step's
     // bulk stream-collide starts now
     if (s->early == 2) launch_bulk_early(s);
@@ -630,7 +633,7 @@ void fem_solve_device(life_server* s, const std::vector<int>& active, const std:
         for (int q : redo)
             for (int b = 0; b < s->slots[q].c->fdev.nb; b++) s->fem_list2.h[n++] = s->slots[q].fem_off + b;
         s->fem_list2.upload(n, st);
-        launch_fem_dynamic(s->fem_bodies.d, s->fem_list2.d, n, s->fem_lds, true, st);
+        launch_fem_dynamic(s->fem_bodies.d, s->fem_list2.d, n, s->fem_lds, s->fem_nel, true, st);
         launch_fem_outs(s->fem_bodies.d, s->fem_list.d, nfb, s->fem_out.h, st);
         LIFE_HIP(hipGetLastError());
         LIFE_HIP(hipStreamSynchronize(st));
