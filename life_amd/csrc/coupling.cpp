@@ -198,7 +198,15 @@ bool finish_epsilon(life_case* c) {
     return !dense.empty();
 }
 
-// Download the marker forces and epsilon; returns once they are on the
+// The markers' positions and velocities on the device, from the host's
+// page-locked copies.
+void upload_markers(life_case* c) {
+    const size_t b2 = 16 * (size_t)c->nm;
+    copy_pinned(c->g, {{c->g->md.pos, c->pos.data(), b2}, {c->g->md.vel, c->vel.data(), b2}});
+}
+
+// Download the marker forces and epsilon (and the banded systems' out-of-band
+// flags, where they wait to be looked at); returns once they are on the
 // host.  With spread set, the spread is queued behind the copies and runs
 // on the device while the host goes on (the FEM does not change what it
 // reads: supports, forces, epsilon); the return value says whether that
@@ -206,9 +214,10 @@ bool finish_epsilon(life_case* c) {
 // rewrites epsilon).
 bool download_forces(life_case* c, bool spread) {
     life_grid* g = c->g;
-    LIFE_HIP(hipMemcpyAsync(c->force.data(), g->md.force, sizeof(double) * 2 * c->nm, hipMemcpyDeviceToHost,
-                            g->stream));
-    LIFE_HIP(hipMemcpyAsync(c->eps.data(), g->md.eps, sizeof(double) * c->nm, hipMemcpyDeviceToHost, g->stream));
+    const size_t n = (size_t)c->nm;
+    copy_pinned(g, {{c->force.data(), g->md.force, 16 * n},
+                    {c->eps.data(), g->md.eps, 8 * n},
+                    {g->eps_outside_h, g->eps_outside, c->eps_check_pending ? sizeof(int) * g->eps_nsys : 0}});
     LIFE_HIP(hipEventRecord(c->ev_forces, g->stream));
     if (spread) ibm_spread(g);
     LIFE_HIP(hipEventSynchronize(c->ev_forces));
@@ -307,8 +316,7 @@ void life::case_solve_eps_dense(life_case* c, int first, int n) {
         lu_solve_sparse(n, 0, c->A.data(), c->rhs.data(), c->sol.data(), c->luw);
     }
     std::memcpy(&c->eps[first], c->sol.data(), sizeof(double) * n);
-    LIFE_HIP(hipMemcpyAsync(c->g->md.eps + first, &c->eps[first], sizeof(double) * n, hipMemcpyHostToDevice,
-                            c->g->stream));
+    copy_pinned(c->g, {{c->g->md.eps + first, &c->eps[first], sizeof(double) * n}});
 }
 
 void life::case_restart_objects(life_case* c) {
@@ -336,11 +344,9 @@ void recompute_object_vals(life_case* c) {
     // the host rewrites pos/vel: the previous step's upload must be done
     LIFE_HIP(hipEventSynchronize(c->ev_upload));
     case_recompute_host(c);
-    life_grid* g = c->g;
-    LIFE_HIP(hipMemcpyAsync(g->md.pos, c->pos.data(), sizeof(double) * 2 * c->nm, hipMemcpyHostToDevice, g->stream));
-    LIFE_HIP(hipMemcpyAsync(g->md.vel, c->vel.data(), sizeof(double) * 2 * c->nm, hipMemcpyHostToDevice, g->stream));
-    ibm_find_support(g, 1);
-    compute_epsilon(c, false);
+    upload_markers(c);
+    ibm_find_support(c->g, 1);
+    compute_epsilon(c, false, false);  // the flags reach the host with the forces
 }
 
 // ObjectsClass::objectKernel, Objects.cpp:26-60.
@@ -481,10 +487,7 @@ void object_kernel(life_case* c, EarlyBulk& eb, int mode) {
         // the last FEM solve moved the markers (FEMBody.cpp:63-64); the
         // spread above used the supports found before it, as the reference
         // does, and the device copy now takes the final positions for output
-        LIFE_HIP(hipMemcpyAsync(c->g->md.pos, c->pos.data(), sizeof(double) * 2 * c->nm, hipMemcpyHostToDevice,
-                                c->g->stream));
-        LIFE_HIP(hipMemcpyAsync(c->g->md.vel, c->vel.data(), sizeof(double) * 2 * c->nm, hipMemcpyHostToDevice,
-                                c->g->stream));
+        upload_markers(c);
         LIFE_HIP(hipEventRecord(c->ev_upload, c->g->stream));
         c->forces_on_host = true;
     }

@@ -762,6 +762,18 @@ void ibm_spread(life_grid* g) {
     LIFE_HIP(hipGetLastError());
 }
 
+void copy_pinned(life_grid* g, std::initializer_list<PinnedCopy> arrays) {
+    WordCopies w{};
+    for (const PinnedCopy& a : arrays) {
+        if (!a.bytes) continue;
+        w.src[w.n] = static_cast<const unsigned*>(a.src);
+        w.dst[w.n] = static_cast<unsigned*>(a.dst);
+        w.words[w.n++] = (int)(a.bytes / 4);
+    }
+    launch_copy_words(w, g->stream);
+    LIFE_HIP(hipGetLastError());
+}
+
 void ibm_interp_spread(life_grid* g) {
     if (g->md.n <= 0) return;
     if (!g->spread_current || g->dense_clear_next || !spread_scans(g->md)) {
