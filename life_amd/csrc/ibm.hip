@@ -1337,14 +1337,13 @@ constexpr int kScanGroup = 7;    // neighbours at a time, of kSupp lanes each
 constexpr int kScanNear = kSupp * kMaxPerSite;
 
 template <typename T, bool INTERP>
-__global__ __launch_bounds__(64 * kScanWaves) void k_spread_scan(const T* __restrict__ f, MarkerDev m, GridScalars g,
-                                                                 SpreadScratch sc, double* __restrict__ fibm) {
+__device__ __forceinline__ void spread_scan_wg(const T* __restrict__ f, const MarkerDev& m, const GridScalars& g,
+                                               const SpreadScratch& sc, double* __restrict__ fibm) {
     __shared__ unsigned short near_s[kScanWaves][kScanWaves][kScanNear];  // marker, quarter
     __shared__ int near_n[kScanWaves][kScanWaves];
     __shared__ double tx_s[kScanWaves][64], ty_s[kScanWaves][64];
     __shared__ int has_s[kScanWaves][64];
     __shared__ double terms_s[kScanWaves][INTERP ? 3 * 64 : 1];
-    coupling_priority();
     const int wv = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
     const int k = (int)blockIdx.x * kScanWaves + wv;
     const int4* box = reinterpret_cast<const int4*>(m.supp_box);
@@ -1497,7 +1496,23 @@ __global__ __launch_bounds__(64 * kScanWaves) void k_spread_scan(const T* __rest
     }
 }
 
-// Batched spread, grid.y = case (the reset: one thread per case).
+template <typename T, bool INTERP>
+__global__ __launch_bounds__(64 * kScanWaves) void k_spread_scan(const T* __restrict__ f, MarkerDev m, GridScalars g,
+                                                                 SpreadScratch sc, double* __restrict__ fibm) {
+    coupling_priority();
+    spread_scan_wg<T, INTERP>(f, m, g, sc, fibm);
+}
+
+// Batched, grid.y = case.  Twelve cases of up to 129 markers: clear and scan
+// 11 us, the five passes 22 us and three more launches.
+__global__ __launch_bounds__(64 * kScanWaves) void k_spread_scan_batch(const CaseDev* __restrict__ cases,
+                                                                       const int* __restrict__ list) {
+    const CaseDev& c = cases[list[blockIdx.y]];
+    if ((int)blockIdx.x * kScanWaves >= c.m.n) return;  // the whole workgroup
+    spread_scan_wg<double, false>(nullptr, c.m, c.g, c.sc, c.fibm);
+}
+
+// Batched spread by passes, grid.y = case (the reset: one thread per case).
 __global__ void k_spread_clear_batch(const CaseDev* __restrict__ cases, const int* __restrict__ list) {
     const CaseDev& c = cases[list[blockIdx.y]];
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < c.sc.cap; k += gridDim.x * blockDim.x)
@@ -1706,6 +1721,11 @@ void launch_spread_batch(const CaseDev* cases, const int* list, int n, int max_m
     const int np = max_markers * kSupp;
     const unsigned nc = (unsigned)((np + 255) / 256);
     if (np > 0) k_spread_clear_batch<<<dim3(nc, (unsigned)n), 256, 0, s>>>(cases, list);
+    if (np > 0 && max_markers <= kScanMaxMarkers) {
+        k_spread_scan_batch<<<dim3((unsigned)((max_markers + kScanWaves - 1) / kScanWaves), (unsigned)n),
+                              64 * kScanWaves, 0, s>>>(cases, list);
+        return;
+    }
     k_spread_reset_batch<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(cases, list, n);
     if (np <= 0) return;
     k_spread_count_batch<<<dim3(nc, (unsigned)n), 256, 0, s>>>(cases, list);
