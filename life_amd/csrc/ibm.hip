@@ -191,6 +191,16 @@ __global__ void k_epsilon_matrix(MarkerDev m, GridScalars g, int first, int n, d
     A[t] = support_sum(m, mi, xj, yj) * m.ds[mj];
 }
 
+// Entry (mi, mj) from the positions of the two markers and the column's
+// spacing.  Markers three spacings apart in x or y have no site in common:
+// their entry is zero.
+__device__ __forceinline__ double eps_entry(const MarkerDev& m, double Dx, int mi, double xi, double yi, double xj,
+                                            double yj, double dsj) {
+    const double lim = 3.01 * Dx;
+    if (fabs(xi - xj) >= lim || fabs(yi - yj) >= lim) return 0.0;  // (a position of NaN shows in the entry)
+    return support_sum(m, mi, xj / Dx, yj / Dx) * dsj;
+}
+
 // The matrix row by row, non-zeros only: a marker couples to the few others
 // within three spacings (a support of marker i lies within 1.5 of x_i and
 // reaches 1.5), so of n^2 entries about ten a row are computed and brought to
@@ -202,7 +212,7 @@ __global__ __launch_bounds__(256) void k_epsilon_rows(MarkerDev m, GridScalars g
                                                       double* __restrict__ val) {
     const int r = blockIdx.x * 4 + (int)threadIdx.x / 64, lane = threadIdx.x % 64;
     if (r >= n) return;
-    const double Dx = g.Dx, lim = 3.01 * Dx;
+    const double Dx = g.Dx;
     const int mi = first + r;
     const double xi = m.pos[2 * mi], yi = m.pos[2 * mi + 1];
     int have = 0;
@@ -210,7 +220,7 @@ __global__ __launch_bounds__(256) void k_epsilon_rows(MarkerDev m, GridScalars g
         const int c = c0 + lane, mj = first + (c < n ? c : 0);
         const double xj = m.pos[2 * mj], yj = m.pos[2 * mj + 1];
         double a = 0.0;
-        if (c < n && fabs(xi - xj) < lim && fabs(yi - yj) < lim) a = support_sum(m, mi, xj / Dx, yj / Dx) * m.ds[mj];
+        if (c < n) a = eps_entry(m, Dx, mi, xi, yi, xj, yj, m.ds[mj]);
         const unsigned long long mask = __ballot(a != 0.0);
         const int at = have + __popcll(mask & ((1ull << lane) - 1));
         if (a != 0.0 && at < kEpsRowCap) {
@@ -230,23 +240,22 @@ __global__ __launch_bounds__(256) void k_epsilon_rows(MarkerDev m, GridScalars g
 // coupling pair outside the band is flagged and solved on the host with the
 // dense path instead.
 
-// One thread per band entry; grid.y = system.
+// One thread per band entry, diagonal by diagonal: of the 3KB + 1 a row is
+// stored with, the few near the main one are formed, the other diagonals'
+// wavefronts only write zeros (row by row: 5.2 us for a filament of 91 markers,
+// 35 for the canopy's 64 on two XCDs, 4.3 and 26 now).  grid.y = system.
 __device__ inline void eps_band_entry(const MarkerDev& m, const GridScalars& g, int first, int n, int KB,
                                       double* __restrict__ band, long long t) {
     const int W = 3 * KB + 1;
     if (t >= (long long)n * W) return;
-    const int r = (int)(t / W), q = (int)(t - (long long)r * W);
+    const int q = (int)(t / n), r = (int)(t - (long long)q * n);
     const int c = r - KB + q;
     double a = 0.0;
     if (q <= 2 * KB && c >= 0 && c < n) {
         const int mi = first + r, mj = first + c;
-        const double Dx = g.Dx;
-        // every read issued before the arithmetic: the support slots past
-        // the count hold zeros and are read but not used
-        const double xj = m.pos[2 * mj] / Dx, yj = m.pos[2 * mj + 1] / Dx, dsj = m.ds[mj];
-        a = support_sum(m, mi, xj, yj) * dsj;
+        a = eps_entry(m, g.Dx, mi, m.pos[2 * mi], m.pos[2 * mi + 1], m.pos[2 * mj], m.pos[2 * mj + 1], m.ds[mj]);
     }
-    band[t] = a;
+    band[(size_t)r * W + q] = a;
 }
 
 // Pairs outside the band that could couple (support of i within 1.5 of
@@ -1081,21 +1090,20 @@ __device__ __forceinline__ void recompute_body(const MarkerDev& m, const GridSca
     }
     __syncthreads();
     // band entries (as eps_band_entry, reading the staged positions and ds)
-    const double Dx = g.Dx;
+    // a wavefront per diagonal (12 bodies of 65 markers beside the bulk kernel:
+    // 69 us row by row, 58 now)
     int bw = 0;
-    for (int t = tid; t < n * W; t += nt) {
-        const int r = t / W, q = t - r * W;
-        const int c = r - KB + q;
-        double a = 0.0;
-        if (q <= 2 * KB && c >= 0 && c < n) {
-            const int mi = first + r;
-            const double xj = P[2 * c] / Dx, yj = P[2 * c + 1] / Dx;
-            a = support_sum(m, mi, xj, yj) * dsl[c];
+    for (int q = tid / 64; q < W; q += nt / 64) {
+        for (int r = tid % 64; r < n; r += 64) {
+            const int c = r - KB + q;
+            double a = 0.0;
+            if (q <= 2 * KB && c >= 0 && c < n)
+                a = eps_entry(m, g.Dx, first + r, P[2 * r], P[2 * r + 1], P[2 * c], P[2 * c + 1], dsl[c]);
+            Bl[r * W + q] = a;
+            if (a != 0.0) bw = max(bw, q < KB ? KB - q : q - KB);
         }
-        Bl[t] = a;
-        if (a != 0.0) bw = max(bw, q < KB ? KB - q : q - KB);
     }
-    atomicMax(bw_sh, bw);
+    if (bw) atomicMax(bw_sh, bw);
     // pairs outside the band that could couple (as eps_far_pair)
     const double lim = 3.01 * g.Dx;
     for (int t = tid; t < n * n; t += nt) {
