@@ -92,6 +92,7 @@ struct life_case {
     std::vector<life::Body*> flex_bodies;  // flexible bodies in body order
     int nm = 0;
     life::pinned_vector pos, vel, force, eps, ds;
+    bool tile_forces = false;  // this call's answer of forces_suit_tiles
     // recorded after the last upload of pos/vel in a step; waited on before
     // the host next writes them
     hipEvent_t ev_upload = nullptr;

@@ -201,4 +201,17 @@ LIFE_DI void load_site(const T* f, long long S, long long id, double fs[kNV]) {
     for (int v = 0; v < kNV; v++) fs[v] = Pops<T>::get(f, S, v, id);
 }
 
+// Terms of the interpolation at one support site (IBMNode.cpp:26-58): rho and
+// rho u (with force_xy F) weighted by the support's delta.
+template <typename T>
+LIFE_DI void interpolate_terms(const T* f, long long S, long long id, double Fx, double Fy, double d, double& a,
+                               double& bx, double& by) {
+    double fs[kNV], rho, ux, uy;
+    load_site(f, S, id, fs);
+    moments64(fs, Fx, Fy, rho, ux, uy);
+    a = rho * d * 1.0 * 1.0;
+    bx = rho * ux * d * 1.0 * 1.0;
+    by = rho * uy * d * 1.0 * 1.0;
+}
+
 }  // namespace life

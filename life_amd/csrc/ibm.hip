@@ -1154,17 +1154,6 @@ constexpr int kInterpMarkers = 28;
 constexpr int kInterpThreads = kInterpMarkers * kSupp;  // 252
 
 template <typename T>
-__device__ __forceinline__ void interpolate_terms(const T* __restrict__ f, const GridScalars& g, long long id, double d,
-                                                  double& a, double& bx, double& by) {
-    double fs[kNV], rho, ux, uy;
-    load_site(f, g.S, id, fs);
-    moments64(fs, g.fcur ? g.fcur[id] : g.Fx, g.fcur ? g.fcur[g.S + id] : g.Fy, rho, ux, uy);
-    a = rho * d * 1.0 * 1.0;
-    bx = rho * ux * d * 1.0 * 1.0;
-    by = rho * uy * d * 1.0 * 1.0;
-}
-
-template <typename T>
 __device__ inline void interpolate_slots(const T* __restrict__ f, const MarkerDev& m, const GridScalars& g,
                                          int k0, double* __restrict__ sh, int t) {
     const int km = t / kSupp, s = t - km * kSupp;
@@ -1173,7 +1162,9 @@ __device__ inline void interpolate_slots(const T* __restrict__ f, const MarkerDe
     double* bx = sh + kInterpThreads;
     double* by = sh + 2 * kInterpThreads;
     if (t < kInterpThreads && k < m.n && s < m.supp_cnt[k]) {
-        interpolate_terms(f, g, m.supp_site[k * kSupp + s], m.supp_delta[k * kSupp + s], a[t], bx[t], by[t]);
+        const long long id = m.supp_site[k * kSupp + s];
+        interpolate_terms(f, g.S, id, g.fcur ? g.fcur[id] : g.Fx, g.fcur ? g.fcur[g.S + id] : g.Fy,
+                          m.supp_delta[k * kSupp + s], a[t], bx[t], by[t]);
     }
     __syncthreads();
     if (t < kInterpThreads && s == 0 && k < m.n) {
@@ -1440,7 +1431,9 @@ __device__ __forceinline__ void spread_scan_wg(const T* __restrict__ f, const Ma
         if constexpr (INTERP) {
             double *ta = terms_s[wv], *tbx = ta + 64, *tby = ta + 128;
             const double vx = m.vel[2 * j], vy = m.vel[2 * j + 1];
-            if (act) interpolate_terms(f, g, site, d, ta[lane], tbx[lane], tby[lane]);
+            if (act)
+                interpolate_terms(f, g.S, site, g.fcur ? g.fcur[site] : g.Fx, g.fcur ? g.fcur[g.S + site] : g.Fy, d,
+                                  ta[lane], tbx[lane], tby[lane]);
             lane_exchange_fence();
             // every lane of the marker adds the terms up in support order
             double iR = 0.0, mx = 0.0, my = 0.0;

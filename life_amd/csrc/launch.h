@@ -49,6 +49,9 @@ struct TileShape {
     int CI, CJ;  // largest tile, without its rim
     int steps;   // steps per launch
 };
+// Markers of a lattice whose tiles form the force: every tile compares them all
+// in one round or two.
+constexpr int kTileMarkers = 256;
 struct TileArgs {
     int steps;
     int per_i, per_j;            // periodic in i / j
@@ -62,6 +65,11 @@ struct TileArgs {
     int one;
     const double* fibm;
     const int *site_uid, *uniq, *uniq_n;  // its support sites (SpreadScratch)
+    // markers > 0: the force is not read but formed in the tiles from these
+    // (MarkerDev) and the populations before the step
+    int markers;
+    const int *supp_box, *supp_site;
+    const double *supp_delta, *eps, *ds, *vel;
     // set by the launcher
     int ni, nj;          // tiles; the first ri (rj) of them have qi + 1 (qj + 1) sites, the others qi (qj)
     int qi, ri, qj, rj;

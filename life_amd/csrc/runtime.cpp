@@ -584,6 +584,16 @@ void tile_launch(life_grid* g, int t, const TileShape& shape, bool one, hipStrea
         a.site_uid = g->sc.site_uid;
         a.uniq = g->sc.uniq;
         a.uniq_n = g->sc.uniq_n;
+        if (g->forces_due) {
+            a.markers = g->md.n;
+            a.supp_box = g->md.supp_box;
+            a.supp_site = g->md.supp_site;
+            a.supp_delta = g->md.supp_delta;
+            a.eps = g->md.eps;
+            a.ds = g->md.ds;
+            a.vel = g->md.vel;
+            g->forces_due = false;
+        }
     }
     a.per_i = g->p.wall_left == LIFE_FLUID;
     a.per_j = g->p.wall_bottom == LIFE_FLUID;
@@ -629,7 +639,17 @@ int lbm_multi_step(life_grid* g, int t, int left) {
     return k;
 }
 
+bool ibm_forces_in_tiles(const life_grid* g) {
+    return g->md.n > 0 && g->md.n <= kTileMarkers && g->spread_current && !g->dense_clear_next && !g->explicit_state &&
+           !g->bulk_pending && !g->stream_pool && tile_shape_one(g).CI > 0;
+}
+
 void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end) {
+    // forces left to this step's tiles, and no tiles after all
+    if (g->forces_due && !ibm_forces_in_tiles(g)) {
+        g->forces_due = false;
+        ibm_interp_spread(g);
+    }
     g->g = step_scalars(*g, t);
     g->t_step = t;
     const double ramp = ramp_coefficient(g->p, g->cs.Dt, t);

@@ -80,6 +80,9 @@ struct life_grid {
     // no site outside the present supports holds a force_ibm: set by a spread
     // (or the clear before it), reset where supports are found again
     bool spread_current = false;
+    // the marker forces of the present populations are left to the next step's
+    // tiles (only between the steps of one call)
+    bool forces_due = false;
     // boundaries
     std::vector<life::BCSite> bc_host;
     life::BCSite* bc = nullptr;
@@ -225,6 +228,11 @@ void copy_pinned(life_grid* g, std::initializer_list<PinnedCopy> arrays);
 // ibm_interpolate then ibm_spread, in one launch where the supports are those
 // of the last spread and the markers few.
 void ibm_interp_spread(life_grid* g);
+// Whether the next step's tiles can form the marker forces themselves
+// (supports of the last spread, few markers, a lattice of the one-step tiles);
+// the caller sees to it that no support lies in a convective outlet's column.
+// Setting forces_due then takes the place of ibm_interp_spread.
+bool ibm_forces_in_tiles(const life_grid* g);
 void ibm_find_support(life_grid* g, int flexible_only);
 void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host);
 // The same matrix by its non-zeros, kEpsRowCap a row, in page-locked memory
