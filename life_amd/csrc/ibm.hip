@@ -258,29 +258,17 @@ __device__ inline void eps_band_entry(const MarkerDev& m, const GridScalars& g, 
     band[(size_t)r * W + q] = a;
 }
 
-// Pairs outside the band that could couple (support of i within 1.5 of
-// x_i, delta of j within 1.5 of the support: |x_i - x_j| < 3 spacings).
-// One thread per pair r < c - KB (the test is symmetric); grid.y = system.
-__device__ inline void eps_far_pair(const MarkerDev& m, const GridScalars& g, int first, int n, int KB,
-                                    int* __restrict__ outside, long long t) {
-    if (t >= (long long)n * n) return;
-    const int r = (int)(t / n), c = (int)(t - (long long)r * n);
-    if (c <= r + KB) return;
-    const double lim = 3.01 * g.Dx;
-    const int mi = first + r, mj = first + c;
-    if (fabs(m.pos[2 * mi] - m.pos[2 * mj]) < lim && fabs(m.pos[2 * mi + 1] - m.pos[2 * mj + 1]) < lim)
-        *outside = 1;
-}
-
-// The out-of-band check of one system (the pairs of eps_far_pair) by one
-// workgroup, which writes the system's flag (1: a pair outside the band
-// couples, 0: none).  Positions are staged in LDS (P: 2n doubles, or null to
+// The out-of-band check of one system: pairs r < c - KB that could couple
+// (support of i within 1.5 of x_i, delta of j within 1.5 of the support: |x_i -
+// x_j| < 3 spacings; the test is symmetric).  One workgroup, which writes the
+// system's flag (1: a pair outside the band couples, 0: none), also to out if
+// that is given (page-locked host memory).  Positions are staged in LDS (P: 2n doubles, or null to
 // read them from device memory).  Eight lanes share a row r and take every
 // eighth column beyond the band, four columns at a time; rows are dealt out
 // in steps of blockDim / 8, so every lane sees about the same number of
 // pairs.
 __device__ inline void eps_far_rows(const MarkerDev& m, const GridScalars& g, int first, int n, int KB,
-                                    int* __restrict__ outside, double* __restrict__ P) {
+                                    int* __restrict__ outside, int* __restrict__ out, double* __restrict__ P) {
     __shared__ int far_sh;
     const double* X = m.pos + 2 * first;
     if (threadIdx.x == 0) far_sh = 0;
@@ -309,7 +297,10 @@ __device__ inline void eps_far_rows(const MarkerDev& m, const GridScalars& g, in
     }
     if (far) atomicOr(&far_sh, 1);
     __syncthreads();
-    if (threadIdx.x == 0) *outside = far_sh;
+    if (threadIdx.x == 0) {
+        *outside = far_sh;
+        if (out) *out = far_sh;
+    }
 }
 
 // Launches whose systems have up to this many markers stage the positions
@@ -332,22 +323,23 @@ __global__ void k_eps_band_prep(MarkerDev m, GridScalars g, const int* __restric
         eps_band_entry(m, g, sys_first[sys], sys_n[sys], KB, band + band_off[sys],
                        (long long)bx * blockDim.x + threadIdx.x);
     else
-        eps_far_rows(m, g, sys_first[sys], sys_n[sys], KB, outside + sys, stage_far ? P : nullptr);
+        eps_far_rows(m, g, sys_first[sys], sys_n[sys], KB, outside + sys, nullptr, stage_far ? P : nullptr);
 }
 
-// Batched assembly: grid.y = entry of the system table.
-__global__ void k_eps_band_entries_batch(const CaseDev* __restrict__ cases, const CaseSys* __restrict__ sys, int KB) {
+// Batched: grid.y = entry of the system table, whose flag goes to out as well.
+// With k_support_ds_batch and the solve 31 us for 12 served filaments, 62 for
+// one workgroup per body that did everything (and the flags' gathering).
+__global__ void k_eps_band_prep_batch(const CaseDev* __restrict__ cases, const CaseSys* __restrict__ sys, int KB, int be,
+                                      int stage_far, int* __restrict__ out) {
+    extern __shared__ double P[];
     const CaseSys q = sys[blockIdx.y];
     const CaseDev& c = cases[q.c];
-    eps_band_entry(c.m, c.g, c.eps.first[q.k], c.eps.n[q.k], KB, c.eps.band + c.eps.off[q.k],
-                   (long long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-__global__ void k_eps_far_check_batch(const CaseDev* __restrict__ cases, const CaseSys* __restrict__ sys, int KB) {
-    const CaseSys q = sys[blockIdx.y];
-    const CaseDev& c = cases[q.c];
-    eps_far_pair(c.m, c.g, c.eps.first[q.k], c.eps.n[q.k], KB, c.eps.outside + q.k,
-                 (long long)blockIdx.x * blockDim.x + threadIdx.x);
+    const int bx = (int)blockIdx.x, first = c.eps.first[q.k], n = c.eps.n[q.k];
+    if (bx < be)
+        eps_band_entry(c.m, c.g, first, n, KB, c.eps.band + c.eps.off[q.k], (long long)bx * blockDim.x + threadIdx.x);
+    else
+        eps_far_rows(c.m, c.g, first, n, KB, c.eps.outside + q.k, out ? out + blockIdx.y : nullptr,
+                     stage_far ? P : nullptr);
 }
 
 // Canonical elimination (partial pivoting, first maximum) of one banded
@@ -1038,110 +1030,7 @@ __global__ __launch_bounds__(256) void k_eps_band_cr_batch(const CaseDev* __rest
     eps_cr_or_pivot(c.eps.band + c.eps.off[q.k], c.eps.first[q.k], n, c.eps.y, c.m.eps, sm, &bw_sh, maxbw);
 }
 
-// ---------------------------------------------------------------- fused recompute
-// The device half of recomputeObjectVals (Objects.cpp:217-227 and the
-// computeEpsilon of flexible bodies, Objects.cpp:235-321) for one flexible
-// body per workgroup, without global round trips between the stages:
-// supports of its markers (to global memory) and spacing, from positions
-// staged in LDS (as k_support_ds), the band of its epsilon
-// system built in LDS (as eps_band_entry), the out-of-band check (as
-// eps_far_pair) and, if the system is banded, the solve by wavefront 0
-// (as k_eps_band_solve).  Same operations in the same order as those
-// kernels.  LDS: n * (3KB + 5) doubles; bodies of up to kFusedMaxMarkers
-// markers.  Used by the serving engine.  A large workgroup needs that many
-// of a CU's wave slots free at once, so beside a concurrent bulk
-// stream-collide (the single-case step schedule, and the serving engine's
-// early bulk kernel) it waits for CUs to drain; the serving engine launches
-// it with kFusedThreads lanes, and the single-case step uses the separate
-// small-block kernels.
-constexpr int kFusedMaxMarkers = 256;
-
-template <int KB>
-__device__ __forceinline__ void recompute_body(const MarkerDev& m, const GridScalars& g, int first, int n,
-                                               int* __restrict__ outside, double* __restrict__ sm,
-                                               int* __restrict__ flag, int* __restrict__ bw_sh, int cr_bw) {
-    constexpr int W = 3 * KB + 1;
-    double* P = sm;                // 2n positions
-    double* dsl = sm + 2 * n;      // n spacings
-    double* Bl = dsl + n;          // n * W band
-    double* yl = Bl + n * W;       // n right-hand side
-    const int tid = threadIdx.x, nt = blockDim.x;
-    if (tid == 0) {
-        *flag = 0;
-        *bw_sh = 0;
-    }
-    const int half = tid / kHalf, nhalf = nt / kHalf, l = tid % kHalf;
-    for (int k = half; k < n; k += nhalf) {
-        // the position and the body kind are read side by side
-        const double x = m.pos[2 * (first + k)], y = m.pos[2 * (first + k) + 1];
-        if (m.body_flex[m.body[first + k]] == 0) find_support_half(m, g, first + k, x, y, l);
-        if (l == 0) {
-            P[2 * k] = x;
-            P[2 * k + 1] = y;
-        }
-    }
-    __syncthreads();
-    for (int k = half; k < n; k += nhalf) {
-        const double ds = spacing_half(P, n, k, P[2 * k], P[2 * k + 1], g.Dx, l);
-        if (l == 0) {
-            m.ds[first + k] = ds;
-            dsl[k] = ds;
-        }
-    }
-    __syncthreads();
-    // band entries (as eps_band_entry, reading the staged positions and ds)
-    // a wavefront per diagonal (12 bodies of 65 markers beside the bulk kernel:
-    // 69 us row by row, 58 now)
-    int bw = 0;
-    for (int q = tid / 64; q < W; q += nt / 64) {
-        for (int r = tid % 64; r < n; r += 64) {
-            const int c = r - KB + q;
-            double a = 0.0;
-            if (q <= 2 * KB && c >= 0 && c < n)
-                a = eps_entry(m, g.Dx, first + r, P[2 * r], P[2 * r + 1], P[2 * c], P[2 * c + 1], dsl[c]);
-            Bl[r * W + q] = a;
-            if (a != 0.0) bw = max(bw, q < KB ? KB - q : q - KB);
-        }
-    }
-    if (bw) atomicMax(bw_sh, bw);
-    // pairs outside the band that could couple (as eps_far_pair)
-    const double lim = 3.01 * g.Dx;
-    for (int t = tid; t < n * n; t += nt) {
-        const int r = t / n, c = t - r * n;
-        if (c <= r + KB) continue;
-        if (fabs(P[2 * r] - P[2 * c]) < lim && fabs(P[2 * r + 1] - P[2 * c + 1]) < lim) *flag = 1;
-    }
-    __syncthreads();
-    const int far = *flag;
-    if (tid == 0) *outside = far;
-    if (far) return;
-    if (*bw_sh <= cr_bw) {
-        // the reduction by the whole workgroup, its blocks after the band
-        double* blk = yl + n;
-        const int nb = (n + kCrMaxBw - 1) / kCrMaxBw;
-        eps_cr_dispatch(*bw_sh, Bl, n, m.eps + first, blk,
-                        blk + (size_t)nb * (3 * kCrMaxBw * kCrMaxBw + kCrMaxBw));
-        return;
-    }
-    eps_band_solve_bw<KB, true>(*bw_sh, first, n, Bl, yl, m.eps);
-}
-
-// Lanes per body workgroup (at least one wavefront for the solve).  Beside
-// the early bulk kernel, 256, 512 and 1024 measured within 3% of each other
-// on MI355X and 128 8% slower (environment LIFE_SERVE_FUSED_THREADS = 64 |
-// 128 | 256 | 512 for sweeps, 0 for the separate batched kernels).
-constexpr int kFusedThreads = 512;
-
-template <int KB>
-__global__ __launch_bounds__(512) void k_recompute_body_batch(const CaseDev* __restrict__ cases,
-                                                              const CaseSys* __restrict__ sys, int cr_bw) {
-    extern __shared__ double sm[];
-    __shared__ int flag, bw;
-    const CaseSys q = sys[blockIdx.x];
-    const CaseDev& c = cases[q.c];
-    recompute_body<KB>(c.m, c.g, c.eps.first[q.k], c.eps.n[q.k], c.eps.outside + q.k, sm, &flag, &bw, cr_bw);
-}
-
+// ---------------------------------------------------------------- interpolation
 // ObjectsClass::ibmKernelInterp body (IBMNode.cpp:26-58): rho and rho*u at
 // the supports (GridClass::macroscopic values: force_xy only) interpolated
 // with the support deltas, then F = 2 (Dt/Dx rho_I U - (rho u)_I).  One
@@ -1564,18 +1453,6 @@ __global__ void k_markers_out_batch(const CaseDev* __restrict__ cases, const int
     q[2] = c.m.eps[k];
 }
 
-__global__ void k_eps_outside_clear_batch(const CaseDev* __restrict__ cases, const CaseSys* __restrict__ sys,
-                                          int nsys) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < nsys) cases[sys[q].c].eps.outside[sys[q].k] = 0;
-}
-
-__global__ void k_eps_outside_gather_batch(const CaseDev* __restrict__ cases, const CaseSys* __restrict__ sys,
-                                           int nsys, int* __restrict__ out) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < nsys) out[q] = cases[sys[q].c].eps.outside[sys[q].k];
-}
-
 static int eps_lds_rows(int KB, int max_n) {
     const int W = 3 * KB + 1;
     const int lds_rows = (int)((60 * 1024) / (sizeof(double) * (W + 1)));
@@ -1690,11 +1567,10 @@ void launch_eps_band_batch(const CaseDev* cases, const CaseSys* sys, int nsys, i
                            bool cr, hipStream_t s) {
     constexpr int KB = 8, W = 3 * KB + 1;
     if (nsys <= 0 || max_n <= 0) return;
-    const unsigned nb = (unsigned)((nsys + 255) / 256);
-    k_eps_outside_clear_batch<<<nb, 256, 0, s>>>(cases, sys, nsys);
-    const long long ne = (long long)max_n * W, np = (long long)max_n * max_n;
-    k_eps_band_entries_batch<<<dim3((unsigned)((ne + 255) / 256), (unsigned)nsys), 256, 0, s>>>(cases, sys, KB);
-    k_eps_far_check_batch<<<dim3((unsigned)((np + 255) / 256), (unsigned)nsys), 256, 0, s>>>(cases, sys, KB);
+    const int be = (int)(((long long)max_n * W + 255) / 256);
+    const bool stage_far = max_n <= kFarLdsMarkers;
+    k_eps_band_prep_batch<<<dim3((unsigned)(be + 1), (unsigned)nsys), 256, stage_far ? 16 * (size_t)max_n : 0, s>>>(
+        cases, sys, KB, be, stage_far ? 1 : 0, outside_out);
     if (cr) {
         static const bool once = (allow_lds((const void*)k_eps_band_cr_batch, eps_cr_lds(kCrMaxRows)), true);
         (void)once;
@@ -1705,7 +1581,6 @@ void launch_eps_band_batch(const CaseDev* cases, const CaseSys* sys, int nsys, i
         k_eps_band_solve_batch<KB><<<(unsigned)nsys, kBandThreads, sizeof(double) * (size_t)rows * (W + 1), s>>>(
             cases, sys, rows, cr ? kCrMaxRows : 0);
     }
-    k_eps_outside_gather_batch<<<nb, 256, 0, s>>>(cases, sys, nsys, outside_out);
 }
 
 template <typename T>
@@ -1744,33 +1619,6 @@ void launch_markers_out_batch(const CaseDev* cases, const int* list, int n, int 
                               hipStream_t s) {
     if (n <= 0 || max_markers <= 0) return;
     k_markers_out_batch<<<dim3((unsigned)((max_markers + 127) / 128), (unsigned)n), 128, 0, s>>>(cases, list, stage);
-}
-
-// Fused recompute (one workgroup per flexible body); false when a body has
-// more markers than the LDS layout takes (the caller uses the separate
-// kernels then).
-static size_t fused_recompute_lds(int max_n, bool cr) {
-    return sizeof(double) * ((size_t)max_n * (3 * 8 + 5) + (cr ? cr_lds_doubles(kCrMaxBw, max_n) : 0));
-}
-
-bool launch_recompute_fused_batch(const CaseDev* cases, const CaseSys* sys, int nsys, int max_n, int* outside_out,
-                                  bool cr, hipStream_t s) {
-    if (max_n > kFusedMaxMarkers) return false;
-    if (nsys <= 0) return true;
-    static const int nt = [] {
-        const char* e = std::getenv("LIFE_SERVE_FUSED_THREADS");
-        const int v = e ? std::atoi(e) : kFusedThreads;
-        return v == 0 || v == 64 || v == 128 || v == 256 ? v : kFusedThreads;
-    }();
-    if (nt == 0) return false;  // the separate batched kernels
-    static const bool once =
-        (allow_lds((const void*)k_recompute_body_batch<8>, fused_recompute_lds(kFusedMaxMarkers, true)), true);
-    (void)once;
-    // cr_bw -1: the pivoted elimination for every system (the plain method)
-    k_recompute_body_batch<8><<<(unsigned)nsys, (unsigned)nt, fused_recompute_lds(max_n, cr), s>>>(
-        cases, sys, cr ? cr_max_bw() : -1);
-    k_eps_outside_gather_batch<<<(unsigned)((nsys + 255) / 256), 256, 0, s>>>(cases, sys, nsys, outside_out);
-    return true;
 }
 
 }  // namespace life

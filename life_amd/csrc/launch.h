@@ -252,13 +252,6 @@ void launch_support_ds_batch(const CaseDev* cases, const int* list, int n, int m
 // cr as for launch_eps_band
 void launch_eps_band_batch(const CaseDev* cases, const CaseSys* sys, int nsys, int max_n, int* outside_out,
                            bool cr, hipStream_t s);
-// Supports and spacing of the listed systems' markers plus their banded
-// epsilon systems, one workgroup per system (the work of
-// launch_find_support_batch(flexible), launch_compute_ds_batch and
-// launch_eps_band_batch in one launch).  Returns false, launching nothing,
-// if a system has more markers than the fused kernel takes.
-bool launch_recompute_fused_batch(const CaseDev* cases, const CaseSys* sys, int nsys, int max_n, int* outside_out,
-                                  bool cr, hipStream_t s);
 template <typename T>
 void launch_interpolate_batch(const CaseDev* cases, const int* list, int n, int max_markers, hipStream_t s);
 void launch_spread_batch(const CaseDev* cases, const int* list, int n, int max_markers, hipStream_t s);

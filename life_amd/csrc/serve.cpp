@@ -694,12 +694,10 @@ void coupling_phase(life_server* s) {
             }
             const int na = (int)active.size();
             int max_n = 0;
-            bool any_uni = false;
             for (int q : active) {
                 life_case* c = s->slots[q].c;
                 life_grid* g = c->g;
                 if (c->p.uni_epsilon) {
-                    any_uni = true;
                     dense.push_back({q, 0});
                     dense_n.push_back(c->nm);
                     continue;
@@ -715,21 +713,14 @@ void coupling_phase(life_server* s) {
                 std::copy(sysl.begin(), sysl.end(), s->sys.h);
                 s->sys.upload(sysl.size(), st);
             }
-            // one workgroup per flexible body for supports, spacing and the
-            // banded epsilon system when every case can take that path
             // FP32-shifted cases solve their banded systems by cyclic
             // reduction, as life_case does
             const bool cr = s->cfg.precision == LIFE_FP32_SHIFTED;
-            // the out-of-band flags are gathered straight into the
-            // page-locked host array, read after the next synchronisation
-            const bool fused = !any_uni && !sysl.empty() &&
-                               launch_recompute_fused_batch(s->cases.d, s->sys.d, (int)sysl.size(), max_n,
-                                                            s->outside.h, cr, st);
-            if (!fused) {
-                launch_support_ds_batch(s->cases.d, s->dyn.d, na, s->max_markers, 1, st);
-                if (!sysl.empty())
-                    launch_eps_band_batch(s->cases.d, s->sys.d, (int)sysl.size(), max_n, s->outside.h, cr, st);
-            }
+            // the out-of-band flags go straight into the page-locked host
+            // array, read after the next synchronisation
+            launch_support_ds_batch(s->cases.d, s->dyn.d, na, s->max_markers, 1, st);
+            if (!sysl.empty())
+                launch_eps_band_batch(s->cases.d, s->sys.d, (int)sysl.size(), max_n, s->outside.h, cr, st);
         }
         // ibmKernelInterp: every case with bodies on the first pass, then
         // the cases still subiterating
