@@ -2,6 +2,7 @@
 // single-case driver (coupling.cpp) and the serving engine (serve.cpp).
 #pragma once
 
+#include <functional>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -149,7 +150,8 @@ void case_push_fem(life_case* c);
 // another subiteration is due (Objects.cpp:59)
 inline bool case_subiterate(const life_case* c) { return c->subIt < kMaxSubIt && c->subRes > c->p.subTol; }
 // computeEpsilon for markers [first, first+n) by the dense path
-void case_solve_eps_dense(life_case* c, int first, int n);
+// beside: what can be queued before the host's solve (it does not read epsilon).
+void case_solve_eps_dense(life_case* c, int first, int n, const std::function<void()>& beside = nullptr);
 // After the marker arrays were restored from a restart file
 // (ObjectsClass::readRestart, Objects.cpp:1186-1198): upload them, find the
 // supports and spacing of every marker and recompute epsilon as at t > 0.

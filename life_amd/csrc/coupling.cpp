@@ -171,10 +171,17 @@ void finalise_markers(life_case* c) {
 // Later calls (flexible bodies only): banded systems assembled and solved
 // on the device, with the dense host path for any system that is not banded.
 // copy_flags: queue the copy of the banded systems' out-of-band flags to the
-// host (the device FEM's last workgroup brings them over otherwise).
-void compute_epsilon(life_case* c, bool initial, bool copy_flags = true) {
+// host (the device FEM's last workgroup brings them over otherwise).  then:
+// the interpolation, which does not read epsilon: queued before the host
+// solves where it does (cylinder with plate: 4.5 us and its launch beside a
+// solve of 75 us, not behind it).
+void compute_epsilon(life_case* c, bool initial, bool copy_flags = true, const std::function<void()>& then = nullptr) {
     auto solve = [&](int first, int n) { case_solve_eps_dense(c, first, n); };
     if (c->p.uni_epsilon) {
+        if (!c->timing->on) {
+            case_solve_eps_dense(c, 0, c->nm, then);
+            return;
+        }
         solve(0, c->nm);
     } else if (initial) {
         for (auto& b : c->bodies)
@@ -186,6 +193,7 @@ void compute_epsilon(life_case* c, bool initial, bool copy_flags = true) {
         ibm_epsilon_band_launch(c->g, copy_flags);
         c->eps_check_pending = true;
     }
+    if (then) then();
 }
 
 // Dense solves of the systems that the banded path left (after a
@@ -302,13 +310,16 @@ void life::case_fem(life_case* c) {
 
 // computeEpsilon's solve of one system on the host: its non-zeros from the
 // device, or the whole matrix where a row has too many of them.
-void life::case_solve_eps_dense(life_case* c, int first, int n) {
-    if (n <= 0) return;
+void life::case_solve_eps_dense(life_case* c, int first, int n, const std::function<void()>& beside) {
+    if (n <= 0) {
+        if (beside) beside();
+        return;
+    }
     c->rhs.assign(n, 1.0);
     c->sol.assign(n, 0.0);
     const int *count, *col;
     const double* val;
-    if (ibm_epsilon_rows(c->g, first, n, count, col, val)) {
+    if (ibm_epsilon_rows(c->g, first, n, count, col, val, c->ev_forces, beside)) {
         lu_solve_rows(n, kEpsRowCap, count, col, val, c->rhs.data(), c->sol.data(), c->luw);
     } else {
         c->A.resize((size_t)n * n);
@@ -346,7 +357,11 @@ void recompute_object_vals(life_case* c) {
     case_recompute_host(c);
     upload_markers(c);
     ibm_find_support(c->g, 1);
-    compute_epsilon(c, false, false);  // the flags reach the host with the forces
+    // the flags reach the host with the forces
+    compute_epsilon(c, false, false, [&] {
+        c->timing->lap(c->g, 1);
+        ibm_interpolate(c->g, true);
+    });
 }
 
 // ObjectsClass::objectKernel, Objects.cpp:26-60.
@@ -393,9 +408,10 @@ void object_kernel_dev(life_case* c, EarlyBulk& eb, int mode) {
         LIFE_HIP(hipGetLastError());
         ibm_find_support(g, 1);
         // the out-of-band flags reach the host with the FEM's sums
-        compute_epsilon(c, false, false);
-        T.lap(g, 1);
-        ibm_interpolate(g, true);
+        compute_epsilon(c, false, false, [&] {
+            T.lap(g, 1);
+            ibm_interpolate(g, true);
+        });
         if (mode == 2) launch_pending(c, eb);
         T.lap(g, 2);
         // femKernel; again with epsilon from the dense path if a system was
@@ -490,9 +506,12 @@ void object_kernel(life_case* c, EarlyBulk& eb, int mode, bool more_steps) {
     }
     bool spread_final = false, more = false;
     do {
-        if (c->hasFlex) recompute_object_vals(c);
-        T.lap(c->g, 1);
-        ibm_interpolate(c->g, true);
+        if (c->hasFlex) {
+            recompute_object_vals(c);  // and the interpolation
+        } else {
+            T.lap(c->g, 1);
+            ibm_interpolate(c->g, true);
+        }
         // mode 2: the next step's stream-collide starts once the first
         // pass of the coupling kernels is queued, beside the host FEM
         if (mode == 2) launch_pending(c, eb);

@@ -906,7 +906,8 @@ void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host) {
     LIFE_HIP(hipStreamSynchronize(g->stream));
 }
 
-bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const int*& col, const double*& val) {
+bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const int*& col, const double*& val,
+                      hipEvent_t ev, const std::function<void()>& beside) {
     // values, then counts, then columns, in the page-locked block
     const size_t nv = (size_t)n * kEpsRowCap;
     char* p = stage(g, nv * sizeof(double) + (size_t)n * sizeof(int) + nv * sizeof(int));
@@ -915,7 +916,13 @@ bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const i
     int* j = c + n;
     launch_epsilon_rows(g->md, g->g, first, n, c, j, v, g->stream);
     LIFE_HIP(hipGetLastError());
-    LIFE_HIP(hipStreamSynchronize(g->stream));
+    if (beside) {
+        LIFE_HIP(hipEventRecord(ev, g->stream));
+        beside();
+        LIFE_HIP(hipEventSynchronize(ev));
+    } else {
+        LIFE_HIP(hipStreamSynchronize(g->stream));
+    }
     count = c;
     col = j;
     val = v;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <functional>
 #include <initializer_list>
 #include <string>
 #include <vector>
@@ -238,7 +239,10 @@ void ibm_epsilon_matrix(life_grid* g, int first, int n, double* A_host);
 // The same matrix by its non-zeros, kEpsRowCap a row, in page-locked memory
 // that stays valid until the grid's next marker transfer; false where a row
 // has more.  Waits for the stream.
-bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const int*& col, const double*& val);
+// beside: work to queue behind the rows while the host waits for them (on ev)
+// and solves.
+bool ibm_epsilon_rows(life_grid* g, int first, int n, const int*& count, const int*& col, const double*& val,
+                      hipEvent_t ev = nullptr, const std::function<void()>& beside = nullptr);
 // Declare the banded epsilon systems [first[k], first[k]+n[k]) once.
 void ibm_epsilon_band_setup(life_grid* g, const std::vector<int>& first, const std::vector<int>& n, int KB);
 // Assemble and solve them on the device (epsilon lands in md.eps) and, with
