@@ -70,13 +70,6 @@ LIFE_DI void moments64(const double fs[kNV], double Fx, double Fy, double& rho, 
 LIFE_DI double site_force_x(const GridScalars& g, double rho) { return (rho * g.fDrho * g.fgx + g.fdx) * g.fsc / g.fDm; }
 LIFE_DI double site_force_y(const GridScalars& g, double rho) { return (rho * g.fDrho * g.fgy + g.fdy) * g.fsc / g.fDm; }
 
-LIFE_DI double density64(const double fs[kNV]) {
-    double r = 0.0;
-#pragma unroll
-    for (int v = 0; v < kNV; v++) r += fs[v];
-    return r;
-}
-
 // BGK collision + Guo forcing (Grid.cpp:236-244).  FORCE false: the site's
 // force is zero, whose terms (a zero each) are left out.
 template <bool FORCE = true>

@@ -23,7 +23,6 @@ constexpr int kMaxPerSite = 64; // markers that may share one support site
 // D2Q9 tables (Grid.cpp:1247-1250).
 constexpr int kCX[kNV] = {0, 1, -1, 0, 0, 1, -1, 1, -1};
 constexpr int kCY[kNV] = {0, 0, 0, 1, -1, 1, -1, -1, 1};
-constexpr int kOpp[kNV] = {0, 2, 1, 4, 3, 6, 5, 8, 7};
 
 enum Prec : int { kFP64 = 0, kFP32 = 1 };
 
