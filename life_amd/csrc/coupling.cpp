@@ -197,11 +197,13 @@ void compute_epsilon(life_case* c, bool initial, bool copy_flags = true, const s
 }
 
 // Dense solves of the systems that the banded path left (after a
-// synchronisation of the grid stream).
-bool finish_epsilon(life_case* c) {
+// synchronisation of the grid stream).  before: run ahead of them if there are
+// any.
+bool finish_epsilon(life_case* c, const std::function<void()>& before = nullptr) {
     if (!c->eps_check_pending) return false;
     c->eps_check_pending = false;
     const std::vector<int> dense = ibm_epsilon_band_dense(c->g);
+    if (before && !dense.empty()) before();
     for (int k : dense) case_solve_eps_dense(c, c->g->eps_first_h[k], c->g->eps_n_h[k]);
     return !dense.empty();
 }
@@ -442,8 +444,14 @@ void object_kernel_dev(life_case* c, EarlyBulk& eb, int mode) {
             // the host polls the sequence word the launch writes last (an
             // event wait wakes the host tens of microseconds later)
             fem_wait_sums(so, c->ev_forces, sums_spin_us());
-            // a redo changes epsilon: the spread is queued again behind it
-            if (!finish_epsilon(c)) break;
+            // a redo changes epsilon: the spread is queued again behind it.
+            // The FEM has moved the markers: a relaxation by nothing takes
+            // them back to the positions whose supports the system is formed
+            // from (those of the predictor or of the last relaxation)
+            if (!finish_epsilon(c, [&] {
+                    launch_fem_relax(fd.d_bodies, nullptr, fd.nb, 0.0, nullptr, fd.lds, g->stream);
+                }))
+                break;
             redo = true;
         }
         T.subits++;

@@ -193,7 +193,8 @@ __global__ void k_epsilon_matrix(MarkerDev m, GridScalars g, int first, int n, d
 
 // Entry (mi, mj) from the positions of the two markers and the column's
 // spacing.  Markers three spacings apart in x or y have no site in common:
-// their entry is zero.
+// their entry is zero.  The supports are those of the positions (every caller
+// forms the system before the markers move on).
 __device__ __forceinline__ double eps_entry(const MarkerDev& m, double Dx, int mi, double xi, double yi, double xj,
                                             double yj, double dsj) {
     const double lim = 3.01 * Dx;

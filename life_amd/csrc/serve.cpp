@@ -620,19 +620,24 @@ void fem_solve_device(life_server* s, const std::vector<int>& active, const std:
     launch_fem_outs(s->fem_bodies.d, s->fem_list.d, nfb, s->fem_out.h, st);
     LIFE_HIP(hipGetLastError());
     LIFE_HIP(hipStreamSynchronize(st));
-    std::vector<int> redo;  // slots whose epsilon changed
+    std::vector<int> redo;  // slots whose epsilon changes
     for (size_t k = 0; k < sysl.size(); k++)
-        if (s->outside.h[k]) {
-            life_case* c = s->slots[sysl[k].c].c;
-            case_solve_eps_dense(c, c->g->eps_first_h[sysl[k].k], c->g->eps_n_h[sysl[k].k]);
-            LIFE_HIP(hipStreamSynchronize(c->g->stream));
-            if (redo.empty() || redo.back() != sysl[k].c) redo.push_back(sysl[k].c);
-        }
+        if (s->outside.h[k] && (redo.empty() || redo.back() != sysl[k].c)) redo.push_back(sysl[k].c);
     if (!redo.empty()) {
         int n = 0;
         for (int q : redo)
             for (int b = 0; b < s->slots[q].c->fdev.nb; b++) s->fem_list2.h[n++] = s->slots[q].fem_off + b;
         s->fem_list2.upload(n, st);
+        // the FEM has moved the markers: a relaxation by nothing takes them
+        // back to the positions whose supports the systems are formed from
+        launch_fem_relax(s->fem_bodies.d, s->fem_list2.d, n, 0.0, nullptr, s->fem_lds, st);
+        LIFE_HIP(hipStreamSynchronize(st));
+        for (size_t k = 0; k < sysl.size(); k++)
+            if (s->outside.h[k]) {
+                life_case* c = s->slots[sysl[k].c].c;
+                case_solve_eps_dense(c, c->g->eps_first_h[sysl[k].k], c->g->eps_n_h[sysl[k].k]);
+                LIFE_HIP(hipStreamSynchronize(c->g->stream));
+            }
         launch_fem_dynamic(s->fem_bodies.d, s->fem_list2.d, n, s->fem_lds, s->fem_nel, true, st);
         launch_fem_outs(s->fem_bodies.d, s->fem_list.d, nfb, s->fem_out.h, st);
         LIFE_HIP(hipGetLastError());
