@@ -737,6 +737,14 @@ void coupling_phase(life_server* s) {
         first = false;
         if (active.empty()) break;
         if (devfem) {
+            // one system over all markers of a case (UNI_EPSILON): solved by
+            // the host before the FEM reads it
+            if (!dense.empty()) LIFE_HIP(hipStreamSynchronize(st));
+            for (size_t k = 0; k < dense.size(); k++) {
+                life_case* c = s->slots[dense[k].first].c;
+                case_solve_eps_dense(c, dense[k].second, dense_n[k]);
+                LIFE_HIP(hipStreamSynchronize(c->g->stream));
+            }
             fem_solve_device(s, active, sysl, nfb);
             std::vector<int> next;
             for (int q : active)
