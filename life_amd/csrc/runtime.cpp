@@ -556,6 +556,9 @@ TileShape tile_shape_one(const life_grid* g) {
     const TileShape plain{0, 0, 0};
     if (!g->tile_ok || std::getenv("LIFE_PUSH32") || std::getenv("LIFE_PUSH64")) return plain;
     if (g->convective && g->p.Ny > kTileMaxOutlet) return plain;
+    // A force outside the list of the last spread (an upload, new markers): the
+    // plain kernels leave it out at support sites, the tiles would take it in.
+    if (g->md.n > 0 && g->dense_clear_next) return plain;
     if (const char* e = std::getenv("LIFE_TILE"))
         if (std::atoi(e) == 0) return plain;
     const long long N = (long long)g->p.Nx * g->p.Ny;
