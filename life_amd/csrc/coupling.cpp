@@ -340,6 +340,7 @@ void life::case_restart_objects(life_case* c) {
     LIFE_HIP(hipMemcpyAsync(g->md.pos, c->pos.data(), b2, hipMemcpyHostToDevice, g->stream));
     LIFE_HIP(hipMemcpyAsync(g->md.vel, c->vel.data(), b2, hipMemcpyHostToDevice, g->stream));
     LIFE_HIP(hipMemcpyAsync(g->md.force, c->force.data(), b2, hipMemcpyHostToDevice, g->stream));
+    g->markers_by_caller = false;
     ibm_find_support(g, 0);
     compute_epsilon(c, false);
     LIFE_HIP(hipStreamSynchronize(g->stream));
@@ -477,9 +478,10 @@ void object_kernel_dev(life_case* c, EarlyBulk& eb, int mode) {
 // circles gain 3-6 us of 16-24 a step, 114 piled up within 8 sites 1.5 of 27,
 // 254 within 13 sites lose 12 of 29.  A tile with its rim (at most 16 x 32
 // sites) and the supports that reach it lie in two by two buckets of 20 x 36.
+// Both are read off the host's copy of the positions, which has to be current.
 bool forces_suit_tiles(const life_case* c) {
     constexpr int kBi = 20, kBj = 36, kMost = 128;
-    if (c->hasFlex || c->nm > kTileMarkers) return false;
+    if (c->hasFlex || c->nm > kTileMarkers || c->g->markers_by_caller) return false;
     const int ni = c->p.Nx / kBi + 2, nj = c->p.Ny / kBj + 2;
     std::vector<int> count((size_t)ni * nj, 0);
     for (int k = 0; k < c->nm; k++) {
@@ -695,6 +697,7 @@ int life_case_create(const life_params* p, const char* geometry, int precision, 
             if (life_ibm_set_markers(c->g, c->nm, c->pos.data(), c->vel.data(), c->mbody.data(),
                                      (int)c->bodies.size(), flex.data()))
                 throw std::runtime_error(life_last_error());
+            c->g->markers_by_caller = false;
             // ObjectsClass::initialiseObjects, Objects.cpp:941-961
             ibm_find_support(c->g, 0);
             compute_epsilon(c, true);

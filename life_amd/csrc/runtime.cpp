@@ -1599,6 +1599,7 @@ int life_ibm_set_markers(life_grid* g, int n, const double* pos, const double* v
         LIFE_HIP(hipStreamSynchronize(s));
         g->dense_clear_next = true;
         g->spread_current = false;
+        g->markers_by_caller = true;
     });
 }
 
@@ -1606,6 +1607,7 @@ int life_ibm_update_markers(life_grid* g, const double* pos, const double* vel) 
     return guarded([&] {
         LIFE_HIP(hipSetDevice(g->device));
         const size_t n = (size_t)g->md.n;
+        if (pos) g->markers_by_caller = true;
         move_markers(g, {{const_cast<double*>(pos), g->md.pos, 16 * n}, {const_cast<double*>(vel), g->md.vel, 16 * n}},
                      false);
     });

@@ -81,6 +81,9 @@ struct life_grid {
     // no site outside the present supports holds a force_ibm: set by a spread
     // (or the clear before it), reset where supports are found again
     bool spread_current = false;
+    // the caller has set markers or their positions through this handle: a
+    // case's host copy of them may lag behind
+    bool markers_by_caller = false;
     // the marker forces of the present populations are left to the next step's
     // tiles (only between the steps of one call)
     bool forces_due = false;
