@@ -1624,6 +1624,7 @@ int life_ibm_find_support(life_grid* g, int flexible_only) {
 int life_ibm_epsilon_matrix(life_grid* g, int first, int n, double* A) {
     return guarded([&] {
         if (first < 0 || n < 0 || first + n > g->md.n) throw std::runtime_error("epsilon system out of range");
+        if (!A && n > 0) throw std::runtime_error("life_ibm_epsilon_matrix needs the matrix");
         LIFE_HIP(hipSetDevice(g->device));
         ibm_epsilon_matrix(g, first, n, A);
     });
@@ -1631,6 +1632,7 @@ int life_ibm_epsilon_matrix(life_grid* g, int first, int n, double* A) {
 
 int life_ibm_set_epsilon(life_grid* g, const double* eps) {
     return guarded([&] {
+        if (!eps && g->md.n > 0) throw std::runtime_error("life_ibm_set_epsilon needs epsilon");
         LIFE_HIP(hipSetDevice(g->device));
         move_markers(g, {{const_cast<double*>(eps), g->md.eps, sizeof(double) * g->md.n}}, false);
     });
