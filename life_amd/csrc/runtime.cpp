@@ -858,7 +858,10 @@ void move_markers(life_grid* g, std::initializer_list<MarkerCopy> copies, bool t
     size_t bytes = 0;
     for (const MarkerCopy& c : copies)
         if (c.host) bytes += (c.bytes + 15) / 16 * 16;
-    if (bytes == 0) return;
+    if (bytes == 0) {
+        if (to_host) LIFE_HIP(hipStreamSynchronize(g->stream));
+        return;
+    }
     char* const base = stage(g, bytes);
     size_t at = 0;
     for (const MarkerCopy& c : copies) {
@@ -1468,6 +1471,7 @@ int life_grid_download(life_grid* g, double* f_aos, double* rho, double* u, doub
         lbm_join(g);
         StateChunks ch(g, f_aos, rho, u, force_ibm);
         const size_t n = ch.count(), depth = ch.depth();
+        if (n == 0) LIFE_HIP(hipStreamSynchronize(g->stream));  // no array asked for
         // a buffer is filled by the device while the host empties the others
         for (size_t k = 0; k < n + depth; k++) {
             if (k >= depth) {
