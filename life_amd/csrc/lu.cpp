@@ -144,11 +144,12 @@ int lu_solve_sparse(int n, int bc, const double* A, const double* b, double* x, 
 int lu_solve_rows(int n, int cap, const int* count, const int* col, const double* val, const double* b, double* x,
                   LuWork& w) {
     const int words = (n + 63) / 64;
-    if (w.rows_m != n) {
+    const bool fits = w.rows_m == n;
+    w.rows_m = 0;  // until B is zero again (memory may run out on the way)
+    if (!fits) {
         w.B.assign((size_t)n * n, 0.0);
         w.bits.assign((size_t)n * words, 0);
         w.y.resize(n);
-        w.rows_m = n;
     }
     for (int r = 0; r < n; r++) {
         double* const ri = &w.B[(size_t)r * n];
@@ -170,6 +171,7 @@ int lu_solve_rows(int n, int cap, const int* count, const int* col, const double
             p[q] = 0;
         }
     }
+    w.rows_m = n;
     return info;
 }
 
