@@ -9,10 +9,9 @@
 #include <climits>
 #include <cstdlib>
 
-#include <stdexcept>
-
 #include "d2q9_f64.h"
 #include "launch.h"
+#include "lds_limit.h"
 
 namespace life {
 
@@ -986,14 +985,6 @@ static size_t eps_cr_lds(int max_n) {
     return sizeof(double) * cr_lds_doubles(kCrMaxBw, n);
 }
 
-// Dynamic LDS beyond 64 KiB per workgroup (gfx950 has 160 KiB) for a kernel,
-// allowed once per process.
-static void allow_lds(const void* kernel, size_t bytes) {
-    if (bytes > 64 * 1024 &&
-        hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
-        throw std::runtime_error("hipFuncSetAttribute: dynamic LDS of the epsilon solve");
-}
-
 // One system per workgroup: the reduction, or for a band wider than
 // kCrMaxBw the pivoted elimination on the band in device memory (ywork: its
 // right-hand side) by wavefront 0.
@@ -1475,8 +1466,8 @@ void launch_eps_band(const MarkerDev& m, const GridScalars& g, const int* sys_fi
                                                                           outside, be, stage_far ? 1 : 0);
     if (cr) {
         const size_t lds = eps_cr_lds(max_n);
-        static const bool once = (allow_lds((const void*)k_eps_band_cr, eps_cr_lds(kCrMaxRows)), true);
-        (void)once;
+        static LdsLimit limit;
+        limit.allow((const void*)k_eps_band_cr, lds, eps_cr_lds(kCrMaxRows));
         k_eps_band_cr<<<nsys, 256, lds, s>>>(sys_first, sys_n, outside, band, band_off, ywork, m.eps, cr_max_bw());
         if (max_n <= kCrMaxRows) return;
     }
@@ -1573,9 +1564,10 @@ void launch_eps_band_batch(const CaseDev* cases, const CaseSys* sys, int nsys, i
     k_eps_band_prep_batch<<<dim3((unsigned)(be + 1), (unsigned)nsys), 256, stage_far ? 16 * (size_t)max_n : 0, s>>>(
         cases, sys, KB, be, stage_far ? 1 : 0, outside_out);
     if (cr) {
-        static const bool once = (allow_lds((const void*)k_eps_band_cr_batch, eps_cr_lds(kCrMaxRows)), true);
-        (void)once;
-        k_eps_band_cr_batch<<<(unsigned)nsys, 256, eps_cr_lds(max_n), s>>>(cases, sys, cr_max_bw());
+        static LdsLimit limit;
+        const size_t lds = eps_cr_lds(max_n);
+        limit.allow((const void*)k_eps_band_cr_batch, lds, eps_cr_lds(kCrMaxRows));
+        k_eps_band_cr_batch<<<(unsigned)nsys, 256, lds, s>>>(cases, sys, cr_max_bw());
     }
     if (!cr || max_n > kCrMaxRows) {
         const int rows = eps_lds_rows(KB, max_n);

@@ -23,6 +23,7 @@
 #include "bc_site.h"
 #include "dev_util.h"
 #include "launch.h"
+#include "lds_limit.h"
 
 namespace life {
 
@@ -410,9 +411,8 @@ template <typename T, bool CM, bool FORCE, bool ONE, bool MARK>
 void launch_tile_t(const T* src, T* dst, const GridScalars& g, const TileArgs& a, unsigned threads, size_t lds,
                    hipStream_t s) {
     // tiles of four steps with their rim exceed the default limit in FP64
-    static const bool once = (hipFuncSetAttribute((const void*)k_tile_step<T, CM, FORCE, ONE, MARK>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) == hipSuccess);
-    (void)once;
+    static LdsLimit limit;
+    limit.allow((const void*)k_tile_step<T, CM, FORCE, ONE, MARK>, lds, 128 * 1024);
     k_tile_step<T, CM, FORCE, ONE, MARK><<<(unsigned)(a.ni * a.nj), threads, lds, s>>>(src, dst, g, a);
 }
 
