@@ -163,7 +163,10 @@ int life_case_destroy(life_case *c);
 int life_case_step(life_case *c, int nsteps);
 /* As life_case_step, also returning the elapsed device time of the steps
  * (ms, HIP events on the case stream) and of the fused stream-collide kernel
- * launches alone (ms, summed). */
+ * launches alone (ms, summed).  Where one launch does whole steps (lattices
+ * that are stepped in tiles: stream-collide, boundaries and outlet, marker
+ * forces of rigid bodies, several steps without bodies), that launch is the
+ * one timed. */
 int life_case_step_timed(life_case *c, int nsteps, double *ms_total, double *ms_kernel);
 int life_case_time(const life_case *c, int *t);
 /* Cadence of the blow-up test (the NaN velocity scan of GridClass::writeInfo,

@@ -611,6 +611,17 @@ void case_step(life_case* c, hipEvent_t ev_begin, hipEvent_t ev_end, bool more, 
     T.t[5] += 1;
 }
 
+// Steps of a case without bodies, several in one launch, up to the next step
+// that the blow-up scan reads; 0: none launched, a case_step is due.
+int case_multi_step(life_case* c, int left, hipEvent_t ev_begin, hipEvent_t ev_end) {
+    if (c->hasIBM || c->timing->on) return 0;
+    const int every = c->g->check_every;
+    const int to_check = every > 0 ? every - c->t % every : left;
+    const int k = lbm_multi_step(c->g, c->t + 1, std::min(left, to_check), ev_begin, ev_end);
+    c->t += k;
+    return k;
+}
+
 // The blow-up test of the reference's writeInfo (Grid.cpp:562-581) at the
 // grid's cadence, after step c->t.
 void case_blowup_cadence(life_case* c) {
@@ -749,15 +760,7 @@ int life_case_step(life_case* c, int nsteps) {
         const ForcesDone done{c->g};
         c->tile_forces = c->hasIBM && nsteps > 1 && forces_suit_tiles(c);
         for (int s = 0; s < nsteps;) {
-            // without bodies, several steps go in one launch, up to the next
-            // step that the blow-up scan reads
-            int k = 0;
-            if (!c->hasIBM && !c->timing->on) {
-                const int every = c->g->check_every;
-                const int to_check = every > 0 ? every - c->t % every : nsteps;
-                k = lbm_multi_step(c->g, c->t + 1, std::min(nsteps - s, to_check));
-                c->t += k;
-            }
+            int k = case_multi_step(c, nsteps - s, nullptr, nullptr);
             if (k == 0) {
                 k = 1;
                 case_step(c, nullptr, nullptr, s + 1 < nsteps, nullptr, nullptr);
@@ -782,7 +785,7 @@ int life_case_step_timed(life_case* c, int nsteps, double* ms_total, double* ms_
         life_grid* g = c->g;
         LIFE_HIP(hipSetDevice(g->device));
         LIFE_HIP(hipStreamSynchronize(g->stream));
-        // one event pair per step around the stream-collide launch, read
+        // an event pair around each stream-collide launch, one to a step, read
         // after the last step so the host never waits inside the loop.
         // They order nothing, so they are recorded without the system-scope
         // fence (cache writeback and invalidate) that a default event adds
@@ -795,14 +798,22 @@ int life_case_step_timed(life_case* c, int nsteps, double* ms_total, double* ms_
         LIFE_HIP(hipEventRecord(g->ev_a, g->stream));
         const ForcesDone done{g};
         c->tile_forces = c->hasIBM && nsteps > 1 && forces_suit_tiles(c);
-        // a step's stream-collide events are recorded where it is launched:
-        // in the step itself, or during the previous step when launched early
-        for (int s = 0; s < nsteps; s++) {
-            const bool early = g->bulk_pending;
-            hipEvent_t nb = s + 1 < nsteps ? c->kev[2 * (s + 1)] : nullptr;
-            hipEvent_t ne = s + 1 < nsteps ? c->kev[2 * (s + 1) + 1] : nullptr;
-            case_step(c, early ? nullptr : c->kev[2 * s], early ? nullptr : c->kev[2 * s + 1], s + 1 < nsteps, nb,
-                      ne);
+        // the steps of life_case_step; a step's stream-collide events are
+        // recorded where it is launched: in the step itself, or during the
+        // previous step when launched early
+        std::vector<int> launches;  // first steps of the stream-collide launches
+        for (int s = 0; s < nsteps;) {
+            launches.push_back(s);
+            int k = case_multi_step(c, nsteps - s, c->kev[2 * s], c->kev[2 * s + 1]);
+            if (k == 0) {
+                k = 1;
+                const bool early = g->bulk_pending;
+                hipEvent_t nb = s + 1 < nsteps ? c->kev[2 * (s + 1)] : nullptr;
+                hipEvent_t ne = s + 1 < nsteps ? c->kev[2 * (s + 1) + 1] : nullptr;
+                case_step(c, early ? nullptr : c->kev[2 * s], early ? nullptr : c->kev[2 * s + 1], s + 1 < nsteps, nb,
+                          ne);
+            }
+            s += k;
             case_blowup_cadence(c);
         }
         lbm_join(g);
@@ -812,7 +823,7 @@ int life_case_step_timed(life_case* c, int nsteps, double* ms_total, double* ms_
         float ms = 0.0f;
         LIFE_HIP(hipEventElapsedTime(&ms, g->ev_a, g->ev_b));
         double kms = 0.0;
-        for (int s = 0; s < nsteps; s++) {
+        for (int s : launches) {
             float k = 0.0f;
             LIFE_HIP(hipEventElapsedTime(&k, c->kev[2 * s], c->kev[2 * s + 1]));
             kms += k;

@@ -522,14 +522,16 @@ void tile_launch(life_grid* g, int t, const TileShape& shape, bool one, hipStrea
 
 }  // namespace
 
-int lbm_multi_step(life_grid* g, int t, int left) {
+int lbm_multi_step(life_grid* g, int t, int left, hipEvent_t ev_begin, hipEvent_t ev_end) {
     if (!g->tile_multi || g->explicit_state || g->md.n > 0 || g->bulk_pending || g->stream_pool) return 0;
     TileShape shape = tile_shape(g);
     if (shape.CI <= 0) return 0;
     if (shape.steps > left) shape.steps = left;
     lbm_join(g);
     g->g = step_scalars(*g, t);
+    if (ev_begin) LIFE_HIP(hipEventRecord(ev_begin, g->stream));
     tile_launch(g, t, shape, false, g->stream);
+    if (ev_end) LIFE_HIP(hipEventRecord(ev_end, g->stream));
     LIFE_HIP(hipGetLastError());
     const int k = shape.steps;
     g->g = step_scalars(*g, t + k - 1);

@@ -160,11 +160,13 @@ struct life_grid {
 
 namespace life {
 // Enqueue one lbmKernel on the grid stream; if ev_begin/ev_end are given,
-// they are recorded around the fused stream-collide launch.
+// they are recorded around the fused stream-collide launch (the tiled step's
+// where that does the whole step).
 void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end);
 // Steps t .. t + k - 1 of a lattice without bodies in one launch, 1 <= k <=
-// left; returns k, or 0 (nothing launched) where lbm_step is to be used.
-int lbm_multi_step(life_grid* g, int t, int left);
+// left; returns k, or 0 (nothing launched) where lbm_step is to be used.  The
+// events, if given, are recorded around the launch.
+int lbm_multi_step(life_grid* g, int t, int left, hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr);
 // The same step in two parts.  lbm_bulk_early launches the bulk
 // stream-collide of the next step on the second stream as soon as the
 // populations of the current step are final (it reads only f and the
