@@ -12,6 +12,15 @@
 
 namespace life {
 
+// delU of GridClass::convectiveSpeed (Grid.cpp:488-494) at outlet row j: the
+// velocities of the last three columns, and their mean behind them.
+__device__ __forceinline__ void outlet_delta(const double* __restrict__ ucol, int Ny, int j, double& dux, double& duy) {
+    const double uOut = ucol[6 * (long long)Ny];
+    const double* u = ucol + j;
+    dux = (-uOut / 2.0) * (3.0 * u[0] - 4.0 * u[2LL * Ny] + u[4LL * Ny]);
+    duy = (-uOut / 2.0) * (3.0 * u[Ny] - 4.0 * u[3LL * Ny] + u[5LL * Ny]);
+}
+
 // GridClass::applyBCs + regularisedBC / convectiveBC (Grid.cpp:302-474) on
 // the populations just streamed into dst, nine lanes per boundary site
 // (bc_site.h).  rho_n/u_n start as the site's end-of-previous-step moments
@@ -38,11 +47,8 @@ __device__ __forceinline__ void bc_wave(const T* __restrict__ src, T* __restrict
     const int Ny = g.Ny, j = b.j;
     if (b.type == 5) {  // convective: f[2,6,8] = f_n + 3 w (delU . c)
         if (v == 2 || v == 6 || v == 8) {
-            // delU of GridClass::convectiveSpeed (Grid.cpp:488-494)
-            const double uOut = a.ucol[6 * (long long)Ny];
-            const double* u = a.ucol + j;
-            const double dux = (-uOut / 2.0) * (3.0 * u[0] - 4.0 * u[2LL * Ny] + u[4LL * Ny]);
-            const double duy = (-uOut / 2.0) * (3.0 * u[Ny] - 4.0 * u[3LL * Ny] + u[5LL * Ny]);
+            double dux, duy;
+            outlet_delta(a.ucol, Ny, j, dux, duy);
             Pops<T>::put(dst, S, v, id, bc_convective(v, Pops<T>::get(src, S, v, id), dux, duy));
         }
         return;
@@ -88,6 +94,170 @@ __device__ __forceinline__ void bc_wave(const T* __restrict__ src, T* __restrict
     Pops<T>::put(dst, S, v, id, bc_value<CM>(l, g, q, r1, u1, r2, u2, uwx, uwy, rin, pun, share + slot * kNV));
 }
 
+// The same with one lane per site, for lattices and batches of so many sites
+// that the launch is bound by the instructions issued and not by one chain:
+// nine lanes form each sum nine times over (one_lane_each has the line between
+// the two).  The values are the same.
+constexpr __device__ int opposite(int v) { return v == 0 ? 0 : ((v - 1) ^ 1) + 1; }
+
+__device__ __forceinline__ double density(const double f[kNV]) {
+    double r = 0.0;
+#pragma unroll
+    for (int v = 0; v < kNV; v++) r += f[v];
+    return r;
+}
+
+// GridClass::regularisedBC (Grid.cpp:387-465, Latt et al. 2008) on one
+// site's nine post-stream populations fs, with rho_n/u_n as set by applyBCs.
+// rhoNb1/rhoNb2 are the current densities at site + n and site + 2n, used
+// by the corner extrapolation (Utils.h:150-162).
+template <bool CM>
+__device__ void regularised64(const GridScalars& g, int type, int nx, int ny, int nd, double fs[kNV], double& rn,
+                              double& uxn, double& uyn, double rhoNb1, double rhoNb2) {
+    const bool velocity_like = (type == 1 || type == 2 || type == 3);  // wall, velocity, free-slip
+    const bool corner = (nx != 0 && ny != 0);
+    if (corner) {
+        if (velocity_like) rn = 2.0 * rhoNb1 - rhoNb2;
+    } else {
+        const int nn = nd == 0 ? nx : ny;
+        double fplus = 0.0, fzero = 0.0;
+#pragma unroll
+        for (int v = 0; v < kNV; v++) {
+            const int cn = nd == 0 ? kCX[v] : kCY[v];
+            if (cn == -nn) fplus += fs[v];
+            else if (cn == 0) fzero += fs[v];
+        }
+        if (velocity_like) rn = (2.0 * fplus + fzero) / (1.0 - nn * (nd == 0 ? uxn : uyn));
+        else if (type == 4) {
+            const double un = nn * (1.0 - (2.0 * fplus + fzero) / rn);
+            if (nd == 0) uxn = un;
+            else uyn = un;
+        }
+    }
+    const double rho = rn, ux = uxn, uy = uyn;
+    double Sxx = 0.0, Syy = 0.0, Sxy = 0.0;
+#pragma unroll
+    for (int v = 0; v < kNV; v++) {
+        const double feq = feq64<CM>(rho, ux, uy, v);
+        bool unknown;
+        if (corner) unknown = (kCX[v] == nx || kCY[v] == ny);
+        else unknown = ((nd == 0 ? kCX[v] : kCY[v]) == (nd == 0 ? nx : ny));
+        if (unknown) {
+            if (corner && nx * kCX[v] + ny * kCY[v] == 0) fs[v] = feq;
+            else fs[v] = feq + (fs[opposite(v)] - feq64<CM>(rho, ux, uy, opposite(v)));
+        }
+        const double fneq = fs[v] - feq;
+        Sxx += kCX[v] * kCX[v] * fneq;
+        Syy += kCY[v] * kCY[v] * fneq;
+        Sxy += kCX[v] * kCY[v] * fneq;
+    }
+#pragma unroll
+    for (int v = 0; v < kNV; v++)
+        fs[v] = feq64<CM>(rho, ux, uy, v) +
+                (w64(v) / (2.0 * g.cs4)) * (((kCX[v] * kCX[v] - g.cs2) * Sxx) + ((kCY[v] * kCY[v] - g.cs2) * Syy) +
+                                            (2.0 * kCX[v] * kCY[v] * Sxy));
+}
+
+template <typename T, bool CM>
+__device__ inline void bc_site(const T* __restrict__ src, T* __restrict__ dst, const GridScalars& g, const BCArgs& a,
+                               const double* __restrict__ fibm, const double* __restrict__ rho0,
+                               const double* __restrict__ u0, int explicit_state, int k) {
+    if (k >= a.nbc) return;
+    const BCSite b = a.sites[k];
+    const long long S = g.S, id = b.id;
+    const int Ny = g.Ny, j = b.j;
+    if (b.type == 5) {  // convective: f[2,6,8] = f_n + 3 w (delU . c)
+        double dux, duy;
+        outlet_delta(a.ucol, Ny, j, dux, duy);
+        const int vs[3] = {2, 6, 8};
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const int v = vs[q];
+            Pops<T>::put(dst, S, v, id, Pops<T>::get(src, S, v, id) + 3.0 * w64(v) * (dux * kCX[v] + duy * kCY[v]));
+        }
+        return;
+    }
+    if (b.type == 0) return;
+    // the populations regularisedBC rebuilds from the others (the ones that
+    // entered from outside the domain) are never read, so only the known
+    // ones are loaded: six of nine on an edge
+    const bool corner = b.nx != 0 && b.ny != 0;
+    // Every load the site needs is issued before the arithmetic (one round
+    // trip to memory, not up to three): its known populations, the two
+    // inward neighbours' populations (the zero gradient of free-slip and
+    // pressure sites, the density extrapolation of corners) and, at a
+    // pressure corner, its previous populations.
+    const bool nbr = b.type == 3 || b.type == 4 || corner;
+    const bool prev = b.type == 4 && corner && !explicit_state;
+    const long long id1 = (long long)(b.i + b.nx) * Ny + (j + b.ny);
+    const long long id2 = (long long)(b.i + 2 * b.nx) * Ny + (j + 2 * b.ny);
+    double fs[kNV], f1[kNV], f2[kNV], fp[kNV];
+#pragma unroll
+    for (int v = 0; v < kNV; v++) {
+        const bool unknown = corner ? (kCX[v] == b.nx || kCY[v] == b.ny)
+                                    : ((b.nd == 0 ? kCX[v] : kCY[v]) == (b.nd == 0 ? b.nx : b.ny));
+        fs[v] = unknown ? 0.0 : Pops<T>::get(dst, S, v, id);
+    }
+    if (nbr) {
+        load_site(dst, S, id1, f1);
+        load_site(dst, S, id2, f2);
+    }
+    if (prev) load_site(src, S, id, fp);
+    // rho_n/u_n of the previous step outlive applyBCs + regularisedBC only
+    // at a pressure corner: everywhere else all three are overwritten below
+    // (wall/velocity set u, free-slip and pressure take u from the normal
+    // condition and the zero gradient, rho comes from the post-stream
+    // populations, the corner extrapolation or rho_in).  The previous
+    // populations, nine scattered loads per site, are read only there.
+    double rn = 0.0, uxn = 0.0, uyn = 0.0;
+    if (b.type == 4 && corner) {
+        if (explicit_state) {
+            rn = rho0[id];
+            uxn = u0[2 * id];
+            uyn = u0[2 * id + 1];
+        } else {
+            moments64(fp, (g.fprev ? g.fprev[id] : g.Fxm) + fibm[id], (g.fprev ? g.fprev[S + id] : g.Fym) + fibm[S + id],
+                      rn, uxn, uyn);
+        }
+    }
+    double rho1 = 0.0, rho2 = 0.0;
+    switch (b.type) {
+        case 1:  // wall
+            uxn = 0.0;
+            uyn = 0.0;
+            break;
+        case 2:  // velocity
+            uxn = a.u_in[2 * j] * a.ramp;
+            uyn = a.u_in[2 * j + 1] * a.ramp;
+            break;
+        case 3:    // free slip
+        case 4: {  // pressure
+            if (b.type == 3) {
+                if (b.nd == 0) uxn = 0.0;
+                else uyn = 0.0;
+            } else {
+                rn = a.rho_in[j];
+            }
+            // Utils::zeroGradient order 2 on the current velocity (Utils.h:200-210)
+            double r1, r2, u1x, u1y, u2x, u2y;
+            moments64(f1, g.fcur ? g.fcur[id1] : g.Fx, g.fcur ? g.fcur[S + id1] : g.Fy, r1, u1x, u1y);
+            moments64(f2, g.fcur ? g.fcur[id2] : g.Fx, g.fcur ? g.fcur[S + id2] : g.Fy, r2, u2x, u2y);
+            if (b.nd != 0) uxn = (4.0 / 3.0) * u1x - (1.0 / 3.0) * u2x;
+            if (b.nd != 1) uyn = (4.0 / 3.0) * u1y - (1.0 / 3.0) * u2y;
+            break;
+        }
+        default:
+            break;
+    }
+    if (corner) {
+        rho1 = density(f1);
+        rho2 = density(f2);
+    }
+    regularised64<CM>(g, b.type, b.nx, b.ny, b.nd, fs, rn, uxn, uyn, rho1, rho2);
+#pragma unroll
+    for (int v = 0; v < kNV; v++) Pops<T>::put(dst, S, v, id, fs[v]);
+}
+
 template <typename T, bool CM>
 __global__ __launch_bounds__(kBCBlock) void k_bc(const T* __restrict__ src, T* __restrict__ dst, GridScalars g,
                                                  BCArgs a, const double* __restrict__ fibm,
@@ -106,10 +276,46 @@ __global__ __launch_bounds__(kBCBlock) void k_bc_batch(const CaseDev* __restrict
                    c.explicit_state, blockIdx.x, share);
 }
 
+template <typename T, bool CM>
+__global__ __launch_bounds__(256) void k_bc_sites(const T* __restrict__ src, T* __restrict__ dst, GridScalars g,
+                                                  BCArgs a, const double* __restrict__ fibm,
+                                                  const double* __restrict__ rho0, const double* __restrict__ u0,
+                                                  int explicit_state) {
+    bc_site<T, CM>(src, dst, g, a, fibm, rho0, u0, explicit_state, blockIdx.x * 256 + threadIdx.x);
+}
+
+template <typename T, bool CM>
+__global__ __launch_bounds__(256) void k_bc_sites_batch(const CaseDev* __restrict__ cases,
+                                                        const int* __restrict__ list) {
+    const CaseDev& c = cases[list[blockIdx.y]];
+    bc_site<T, CM>(static_cast<const T*>(c.src), static_cast<T*>(c.dst), c.g, c.bc, c.fibm, c.rho0, c.u0,
+                   c.explicit_state, blockIdx.x * 256 + threadIdx.x);
+}
+
+// Whether a launch of this many sites takes one lane each.  A wall and a
+// free-slip side of n/2 sites each, nine lanes a site | one:
+//   n        FP64              FP32
+//   12 000    8.2 |  10.2 us    6.5 | 11.0
+//   20 000    8.7 |   9.6       8.8 | 12.3
+//   28 000   11.3 |  10.5      10.8 | 12.7
+//   36 000   14.0 |  11.7      11.9 | 12.1
+//   44 000   16.2 |  12.3      13.3 | 12.2
+//   200 000    61 |    51        44 |   27
+template <typename T>
+bool one_lane_each(long long sites) {
+    return sites > (sizeof(T) == 8 ? 24000 : 36000);
+}
+
 template <typename T>
 void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, const double* fibm, const double* rho0,
                const double* u0, bool explicit_state, hipStream_t s) {
     if (a.nbc <= 0) return;
+    if (one_lane_each<T>(a.nbc)) {
+        const unsigned nl = (unsigned)((a.nbc + 255) / 256);
+        if (g.cm) k_bc_sites<T, true><<<nl, 256, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
+        else k_bc_sites<T, false><<<nl, 256, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
+        return;
+    }
     const unsigned nb = (unsigned)((a.nbc + kBCPerWave - 1) / kBCPerWave);
     if (g.cm) k_bc<T, true><<<nb, kBCBlock, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
     else k_bc<T, false><<<nb, kBCBlock, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
@@ -235,6 +441,12 @@ void launch_convective_speed(const T* src, const GridScalars& g, const double* f
 template <typename T>
 void launch_bc_batch(bool cm, const CaseDev* cases, const int* list, int n, int max_nbc, hipStream_t s) {
     if (n <= 0 || max_nbc <= 0) return;
+    if (one_lane_each<T>((long long)n * max_nbc)) {
+        const dim3 lanes((unsigned)((max_nbc + 255) / 256), (unsigned)n);
+        if (cm) k_bc_sites_batch<T, true><<<lanes, 256, 0, s>>>(cases, list);
+        else k_bc_sites_batch<T, false><<<lanes, 256, 0, s>>>(cases, list);
+        return;
+    }
     const dim3 grid((unsigned)((max_nbc + kBCPerWave - 1) / kBCPerWave), (unsigned)n);
     if (cm) k_bc_batch<T, true><<<grid, kBCBlock, 0, s>>>(cases, list);
     else k_bc_batch<T, false><<<grid, kBCBlock, 0, s>>>(cases, list);
