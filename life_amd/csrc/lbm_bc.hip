@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256) void k_bc_sites_batch(const CaseDev* __restric
 }
 
 // Whether a launch of this many sites takes one lane each.  A wall and a
-// free-slip side of n/2 sites each, nine lanes a site | one:
+// free-slip side of n/2 sites each, 16 apart, nine lanes a site | one:
 //   n        FP64              FP32
 //   12 000    8.2 |  10.2 us    6.5 | 11.0
 //   20 000    8.7 |   9.6       8.8 | 12.3
@@ -301,16 +301,19 @@ __global__ __launch_bounds__(256) void k_bc_sites_batch(const CaseDev* __restric
 //   36 000   14.0 |  11.7      11.9 | 12.1
 //   44 000   16.2 |  12.3      13.3 | 12.2
 //   200 000    61 |    51        44 |   27
+// few: the lattice has fewer than 20 sites across, so that the lanes of both
+// sides share cache lines.  Whole steps of a channel of 4 rows: 12 000 sites FP64
+// 13.1 | 11.8 us, 28 000 FP32 13.9 | 13.6, 34 000 FP32 15.1 | 13.9.
 template <typename T>
-bool one_lane_each(long long sites) {
-    return sites > (sizeof(T) == 8 ? 24000 : 36000);
+bool one_lane_each(long long sites, bool few) {
+    return sites > (sizeof(T) == 8 ? (few ? 11000 : 24000) : (few ? 28000 : 36000));
 }
 
 template <typename T>
 void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, const double* fibm, const double* rho0,
                const double* u0, bool explicit_state, hipStream_t s) {
     if (a.nbc <= 0) return;
-    if (one_lane_each<T>(a.nbc)) {
+    if (one_lane_each<T>(a.nbc, g.Nx < 20 || g.Ny < 20)) {
         const unsigned nl = (unsigned)((a.nbc + 255) / 256);
         if (g.cm) k_bc_sites<T, true><<<nl, 256, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
         else k_bc_sites<T, false><<<nl, 256, 0, s>>>(src, dst, g, a, fibm, rho0, u0, explicit_state ? 1 : 0);
@@ -441,7 +444,7 @@ void launch_convective_speed(const T* src, const GridScalars& g, const double* f
 template <typename T>
 void launch_bc_batch(bool cm, const CaseDev* cases, const int* list, int n, int max_nbc, hipStream_t s) {
     if (n <= 0 || max_nbc <= 0) return;
-    if (one_lane_each<T>((long long)n * max_nbc)) {
+    if (one_lane_each<T>((long long)n * max_nbc, false)) {
         const dim3 lanes((unsigned)((max_nbc + 255) / 256), (unsigned)n);
         if (cm) k_bc_sites_batch<T, true><<<lanes, 256, 0, s>>>(cases, list);
         else k_bc_sites_batch<T, false><<<lanes, 256, 0, s>>>(cases, list);

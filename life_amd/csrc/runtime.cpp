@@ -7,6 +7,7 @@
 #include "state_chunks.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -398,6 +399,54 @@ void lbm_bulk_early(life_grid* g, hipEvent_t ev_begin, hipEvent_t ev_end) {
 
 namespace {
 
+// Few sites across a long lattice put a boundary in every tile and rows
+// shorter than a wavefront in the lanes: past these sizes the plain kernels are
+// the better choice, whatever tiles_pay estimates.
+bool thin(const life_grid* g, long long narrow, long long slim) {
+    const long long N = (long long)g->p.Nx * g->p.Ny;
+    const int across = std::min(g->p.Nx, g->p.Ny);
+    return (across < 8 && N > 40000) || (across < 20 && N > narrow) || (across < 56 && N > slim);
+}
+
+// Whether tiles of this shape are expected to step a lattice without bodies
+// faster than the plain kernels.  Past 150 000 sites both are estimated from
+// what bounds them, in us and us per million:
+//   tiles: the chain of a step, the lanes of tile and rim in whole wavefronts
+//          (more with a body force), the boundary sites of tile and rim
+//   plain: the launches, the sites, the boundary sites
+// The rates are least-squares fits to 1 800 pairs of runs (20 sites by 140 000 to
+// 1 800 by 2 800; walls on four, two and no sides); they name the faster side of
+// all but a few within 10 % of each other.  Plain | tiled, us a step, BGK and then
+// central moments:
+//   cavity 900 x 1 334     FP64 42.9 | 22.6, 43.3 | 28.7   FP32 22.1 | 17.4, 22.9 | 21.1
+//   cavity 450 x 6 223     FP64 84.7 | 49.8, 86.2 | 67.9   FP32 42.9 | 37.3, 44.0 | 45.4
+//   cavity 112 x 25 001    FP64 86.8 | 67.1, 87.1 | 83.1   FP32 48.7 | 55.8, 49.0 | 63.1
+//   cavity 8 x 62 501      FP64 22.2 | 29.5, 23.7 | 32.4   FP32 16.6 | 27.8, 17.1 | 29.5
+//   channel, body force, 1 300 x 2 154                     FP32 42.7 | 41.1, 44.6 | 53.0
+//   periodic 900 x 1 334   FP64 38.4 | 21.7, 39.7 | 30.4   FP32 17.9 | 15.7, 18.8 | 23.0
+bool tiles_pay(const life_grid* g, const TileShape& shape) {
+    const life_params& p = g->p;
+    const int Nx = p.Nx, Ny = p.Ny, n = shape.steps, across = std::min(Nx, Ny);
+    const bool fp64 = g->prec == LIFE_FP64, cm = p.central_moments != 0;
+    const bool force = p.gravityX != 0.0 || p.gravityY != 0.0 || p.dpdx != 0.0 || p.dpdy != 0.0;
+    const double N = 1e-6 * (double)Nx * Ny;
+    if (thin(g, 150000, LLONG_MAX)) return false;
+    if ((across < (fp64 ? 41 : 120) && N > 0.4) || (across < 100 && N > 1.5)) return false;
+    if (N <= 0.15) return true;
+    const int ni = (Nx + shape.CI - 1) / shape.CI, nj = (Ny + shape.CJ - 1) / shape.CJ;
+    const int EI = (Nx + ni - 1) / ni + 2 * n, EJ = (Ny + nj - 1) / nj + 2 * n;
+    const double lanes = 1e-6 * ni * nj * ((EI * EJ + 63) / 64 * 64);
+    // the sites of the two sides across i (and j), each in the tiles that reach it
+    const bool wi = p.wall_left != LIFE_FLUID, wj = p.wall_bottom != LIFE_FLUID;
+    const double si = wi ? 2e-6 * std::min(ni, 1 + n / (Nx / ni)) * nj * EJ : 0.0;
+    const double sj = wj ? 2e-6 * std::min(nj, 1 + n / (Ny / nj)) * ni * EI : 0.0;
+    const double lane_us = (fp64 ? (cm ? 14.8 : 8.0) : (cm ? 10.4 : 5.7)) + (force ? (fp64 ? 3.0 : 2.0) : 0.0);
+    const double site_us = (fp64 ? 26.3 : 12.1) + (force ? 1.0 : 0.0);
+    const double tiled = 2.8 + lane_us * lanes + 163.0 * (si + sj);
+    const double plain = 3.2 + (wi || wj ? 4.3 : 0.0) + site_us * N + 172.0 * 2e-6 * ((wi ? Ny : 0) + (wj ? Nx : 0));
+    return tiled <= 0.97 * plain;
+}
+
 // The tiled step's tile and steps per launch for a lattice without bodies,
 // or CI = 0 where the plain kernels (a bulk launch and a boundary launch per
 // step) are the better choice.  Measured per step on cavities, plain | tiled:
@@ -406,15 +455,14 @@ namespace {
 //   512 x 512    11.5 | 7.8, 9.0 | 6.5
 //   1501 x 377   FP64 CM 22.9 | 16.2, FP32 CM 14.5 | 12.3
 //   2048 x 2048  FP64 BGK 113 | 69, FP64 CM 109 | 94, FP32 BGK 57 | 50, FP32 CM 55 | 61
-// Small lattices are bound by the launch and by the chain of one step on a
-// tile, so they take square tiles of four steps, of the smallest size that
-// gives every tile a CU of its own (two for the smallest tile, whose
+// (plain: then with one lane a boundary site).  Small lattices are bound by the
+// launch and by the chain of one step on a tile, so they take square tiles of
+// four steps, of the smallest size that gives every tile a CU of its own (two for the smallest tile, whose
 // workgroups share a CU at little cost).  Larger ones are bound by the
 // arithmetic of tile and rim and by memory: tiles of 512 sites with their rim
 // (three workgroups to a CU), three steps where a step is cheap (BGK) and two
-// where the rim costs more (central moments).  FP32 central moments above
-// 3 M sites stay on the plain kernels, which move 72 B a site at close to the
-// copy rate.  LIFE_TILE = 0 (plain) or "steps,CI,CJ" overrides, for sweeps.
+// where the rim costs more (central moments), where tiles_pay.  LIFE_TILE = 0
+// (plain) or "steps,CI,CJ" overrides, for sweeps.
 TileShape tile_shape(const life_grid* g) {
     const TileShape plain{0, 0, 0};
     const int Nx = g->p.Nx, Ny = g->p.Ny;
@@ -432,9 +480,8 @@ TileShape tile_shape(const life_grid* g) {
         const long long tiles = (long long)((Nx + c - 1) / c) * ((Ny + c - 1) / c);
         if (tiles <= (c == 8 ? 400 : 256)) return TileShape{c, c, 4};
     }
-    const bool cm = g->p.central_moments != 0;
-    if (cm && g->prec == LIFE_FP32_SHIFTED && (long long)Nx * Ny > 3000000LL) return plain;
-    return cm ? TileShape{12, 28, 2} : TileShape{10, 26, 3};
+    const TileShape large = g->p.central_moments != 0 ? TileShape{12, 28, 2} : TileShape{10, 26, 3};
+    return tiles_pay(g, large) ? large : plain;
 }
 
 // As tile_shape, for a launch of one step of any lattice, bodies and
@@ -446,7 +493,9 @@ TileShape tile_shape(const life_grid* g) {
 // 256 without bodies FP64 8.5 | 6.8, of 512 x 512 11.5 | 12.6.  Tiles of
 // 14 x 14 sites with their rim while they are few, of 16 x 32 (three
 // workgroups to a CU, longer rows) above; past the sizes below the rim's
-// second reading costs more than the launches.  LIFE_TILE = 0 selects the
+// second reading costs more than the launches, and on a long lattice of few
+// sites across the boundaries do: convective outlet, 32 across, FP32 300 000
+// sites 23.8 | 20.3, 500 000 25.9 | 29.2.  LIFE_TILE = 0 selects the
 // plain kernels here too, LIFE_TILE1 = "CI,CJ" a tile, for sweeps.
 TileShape tile_shape_one(const life_grid* g) {
     const TileShape plain{0, 0, 0};
@@ -468,6 +517,7 @@ TileShape tile_shape_one(const life_grid* g) {
     const bool f32 = g->prec == LIFE_FP32_SHIFTED;
     const long long most = g->convective ? 1100000 : (g->md.n > 0 ? (f32 ? 300000 : 1100000) : 150000);
     if (N > most) return plain;
+    if (thin(g, 100000, 300000)) return plain;
     return N <= 150000 ? TileShape{12, 12, 1} : TileShape{14, 30, 1};
 }
 
