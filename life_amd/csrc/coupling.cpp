@@ -709,6 +709,7 @@ int life_case_create(const life_params* p, const char* geometry, int precision, 
                                      (int)c->bodies.size(), flex.data()))
                 throw std::runtime_error(life_last_error());
             c->g->markers_by_caller = false;
+            c->g->md.along_bodies = 1;
             // ObjectsClass::initialiseObjects, Objects.cpp:941-961
             ibm_find_support(c->g, 0);
             compute_epsilon(c, true);

@@ -1206,10 +1206,14 @@ __global__ void k_spread_reduce(MarkerDev m, SpreadScratch sc, double* __restric
 // and lists in device memory, took 26 us for 530 markers against 6 us here; with
 // the interpolation 17 us for 126 markers against 6 us.
 // Up to kScanMaxMarkers markers: the comparisons grow with the square of their
-// number, the five passes do not.  Spread with the clear at 1000, 2000, 4000
-// and 8000 markers: 10, 12, 15 and 24 us here, 19, 21, 25 and 33 us by the
-// passes.
+// number, the five passes do not.  The markers of a case lie one after the other
+// along its bodies, so the four of a workgroup are close together and most rounds
+// of 64 meet none of them; a caller's may lie anywhere, and then every round is
+// opened: hence two limits.  Spread alone at 2000, 4000, 6000 and 8192 markers,
+// here | passes: filaments 6.0 | 21.0, 8.5 | 23.3, 11.7 | 26.2, 17.6 | 29.7 us,
+// scattered 8.6 | 20.3, 18.5 | 23.9, 31.6 | 27.9, 51.4 | 32.8.
 constexpr int kScanMaxMarkers = 8192;
+constexpr int kScanMaxScattered = 5000;
 constexpr int kScanWaves = 4;    // markers per workgroup
 constexpr int kScanGroup = 7;    // neighbours at a time, of kSupp lanes each
 // More overlapping markers than this put more than kMaxPerSite pairs on one
@@ -1512,7 +1516,7 @@ template void launch_interpolate<double>(const double*, const MarkerDev&, const 
 template void launch_interpolate<float>(const float*, const MarkerDev&, const GridScalars&, bool, double*,
                                         const SpreadScratch&, hipStream_t);
 
-bool spread_scans(const MarkerDev& m) { return m.n <= kScanMaxMarkers; }
+bool spread_scans(const MarkerDev& m) { return m.n <= (m.along_bodies ? kScanMaxMarkers : kScanMaxScattered); }
 
 static unsigned scan_blocks(const MarkerDev& m) { return (unsigned)((m.n + kScanWaves - 1) / kScanWaves); }
 

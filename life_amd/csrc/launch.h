@@ -113,6 +113,7 @@ void launch_fill_i32(int* p, int v, long long n, hipStream_t s);
 // IBM (ibm.hip)
 struct MarkerDev {
     int n;
+    int along_bodies;  // 1: markers one after the other along their bodies (a case's own)
     double* pos;       // n*2 (physical)
     double* vel;       // n*2 (physical)
     double* force;     // n*2 (lattice)
