@@ -758,8 +758,9 @@ int life_case_destroy(life_case* c) {
 int life_case_step(life_case* c, int nsteps) {
     return guarded([&] {
         LIFE_HIP(hipSetDevice(c->g->device));
+        const ShapesHeld shapes(c->g);
         const ForcesDone done{c->g};
-        c->tile_forces = c->hasIBM && nsteps > 1 && forces_suit_tiles(c);
+        c->tile_forces = c->hasIBM && nsteps > 1 && c->g->shape_one.CI > 0 && forces_suit_tiles(c);
         for (int s = 0; s < nsteps;) {
             int k = case_multi_step(c, nsteps - s, nullptr, nullptr);
             if (k == 0) {
@@ -797,8 +798,9 @@ int life_case_step_timed(life_case* c, int nsteps, double* ms_total, double* ms_
             c->kev.push_back(e);
         }
         LIFE_HIP(hipEventRecord(g->ev_a, g->stream));
+        const ShapesHeld shapes(g);
         const ForcesDone done{g};
-        c->tile_forces = c->hasIBM && nsteps > 1 && forces_suit_tiles(c);
+        c->tile_forces = c->hasIBM && nsteps > 1 && g->shape_one.CI > 0 && forces_suit_tiles(c);
         // the steps of life_case_step; a step's stream-collide events are
         // recorded where it is launched: in the step itself, or during the
         // previous step when launched early

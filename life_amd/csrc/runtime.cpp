@@ -405,7 +405,7 @@ namespace {
 bool thin(const life_grid* g, long long narrow, long long slim) {
     const long long N = (long long)g->p.Nx * g->p.Ny;
     const int across = std::min(g->p.Nx, g->p.Ny);
-    return (across < 8 && N > 40000) || (across < 20 && N > narrow) || (across < 56 && N > slim);
+    return (across < 8 && N > 40000 && g->nbc > 0) || (across < 20 && N > narrow) || (across < 56 && N > slim);
 }
 
 // Whether tiles of this shape are expected to step a lattice without bodies
@@ -464,6 +464,7 @@ bool tiles_pay(const life_grid* g, const TileShape& shape) {
 // where the rim costs more (central moments), where tiles_pay.  LIFE_TILE = 0
 // (plain) or "steps,CI,CJ" overrides, for sweeps.
 TileShape tile_shape(const life_grid* g) {
+    if (g->shapes_held) return g->shape_multi;
     const TileShape plain{0, 0, 0};
     const int Nx = g->p.Nx, Ny = g->p.Ny;
     // the knobs of the plain kernels select them
@@ -499,11 +500,12 @@ TileShape tile_shape(const life_grid* g) {
 // plain kernels here too, LIFE_TILE1 = "CI,CJ" a tile, for sweeps.
 TileShape tile_shape_one(const life_grid* g) {
     const TileShape plain{0, 0, 0};
-    if (!g->tile_ok || std::getenv("LIFE_PUSH32") || std::getenv("LIFE_PUSH64")) return plain;
-    if (g->convective && g->p.Ny > kTileMaxOutlet) return plain;
     // A force outside the list of the last spread (an upload, new markers): the
     // plain kernels leave it out at support sites, the tiles would take it in.
     if (g->md.n > 0 && g->dense_clear_next) return plain;
+    if (g->shapes_held) return g->shape_one;
+    if (!g->tile_ok || std::getenv("LIFE_PUSH32") || std::getenv("LIFE_PUSH64")) return plain;
+    if (g->convective && g->p.Ny > kTileMaxOutlet) return plain;
     if (const char* e = std::getenv("LIFE_TILE"))
         if (std::atoi(e) == 0) return plain;
     const long long N = (long long)g->p.Nx * g->p.Ny;
@@ -571,6 +573,17 @@ void tile_launch(life_grid* g, int t, const TileShape& shape, bool one, hipStrea
 }
 
 }  // namespace
+
+ShapesHeld::ShapesHeld(life_grid* grid) : g(grid) {
+    const bool dense = g->dense_clear_next;
+    g->dense_clear_next = false;  // asked for at each step (tile_shape_one)
+    g->shape_multi = tile_shape(g);
+    g->shape_one = tile_shape_one(g);
+    g->dense_clear_next = dense;
+    g->shapes_held = true;
+}
+
+ShapesHeld::~ShapesHeld() { g->shapes_held = false; }
 
 int lbm_multi_step(life_grid* g, int t, int left, hipEvent_t ev_begin, hipEvent_t ev_end) {
     if (!g->tile_multi || g->explicit_state || g->md.n > 0 || g->bulk_pending || g->stream_pool) return 0;

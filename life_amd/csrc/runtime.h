@@ -100,6 +100,10 @@ struct life_grid {
     // the sides allow the tiled step (lbm_tile.hip), and several steps per
     // launch of it without bodies
     bool tile_ok = false, tile_multi = false;
+    // the tiles of this lattice (tile_shape, tile_shape_one), for the length of a
+    // call of many steps (ShapesHeld)
+    bool shapes_held = false;
+    life::TileShape shape_multi{0, 0, 0}, shape_one{0, 0, 0};
     // markers
     life::MarkerDev md{};
     int nbodies = 0;
@@ -163,6 +167,16 @@ namespace life {
 // they are recorded around the fused stream-collide launch (the tiled step's
 // where that does the whole step).
 void lbm_step(life_grid* g, int t, hipEvent_t ev_begin, hipEvent_t ev_end);
+// The choice of tiles, which reads the environment, made once for a call: a
+// plain step of a small lattice without walls is a launch of 5 us, which the
+// host's reading of six variables a step held up by 0.3.
+struct ShapesHeld {
+    life_grid* g;
+    explicit ShapesHeld(life_grid* g);
+    ~ShapesHeld();
+    ShapesHeld(const ShapesHeld&) = delete;
+    ShapesHeld& operator=(const ShapesHeld&) = delete;
+};
 // Steps t .. t + k - 1 of a lattice without bodies in one launch, 1 <= k <=
 // left; returns k, or 0 (nothing launched) where lbm_step is to be used.  The
 // events, if given, are recorded around the launch.
