@@ -356,7 +356,15 @@ void rebuild(life_server* s) {
         s->fem_lds = std::max(s->fem_lds, c->fdev.lds);
         s->fem_nel = std::max(s->fem_nel, c->fdev.max_nel);
     }
-    s->fem_device = any_flex && all_dev;
+    // the beams of cases that go on with the other FEM than before go along
+    const bool device = any_flex && all_dev;
+    if (device != s->fem_device)
+        for (Slot& sl : s->slots) {
+            if (!sl.c->hasFlex || sl.c->t == 0) continue;
+            if (device) case_push_fem(sl.c);
+            else case_sync_host(sl.c);
+        }
+    s->fem_device = device;
     if (s->fem_device) {
         s->fem_bodies.reserve(fb.size());
         std::copy(fb.begin(), fb.end(), s->fem_bodies.h);
