@@ -10,7 +10,9 @@
 // SITE selects between the two roundings in use: false, the bulk
 // stream-collide's, which rounds some products before they are added; true,
 // the support sites', fused throughout.  Both are the same expressions; `mad`
-// marks where they differ.  FORCE false: the site's force is zero, whose
+// marks where they differ.  Which products those are has no numerical reason: it
+// is how the two kernels were contracted when their results became the ones to
+// keep, bit for bit.  FORCE false: the site's force is zero, whose
 // terms (a zero each) are left out.
 #pragma once
 

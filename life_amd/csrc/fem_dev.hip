@@ -266,13 +266,11 @@ FDI void update_ibm_d(const FemDevBody& B, double* elu) {
 
 // LDS of the dynamic solve (doubles): K band (ndof x kFemBandW), M band
 // (ndof x kMBand), the force vector F, the load vector R, the Newmark
-// vector, the increment delU, the elimination's row extents, and the
-// body's marker forces and epsilon (3 per marker).  update_ibm's element
-// terms reuse the K band.
+// vector, the increment delU, and the body's marker forces and epsilon (3 per
+// marker).  update_ibm's element terms reuse the K band.
 constexpr int kMBand = 2 * kFemKL + 1;
 struct FemLds {
     double *K, *M, *F, *R, *vec, *x, *mk;
-    int* last;
 };
 FDI FemLds fem_lds(const FemDevBody& B, double* lds) {
     FemLds L;
@@ -283,8 +281,7 @@ FDI FemLds fem_lds(const FemDevBody& B, double* lds) {
     L.R = L.F + n;
     L.vec = L.R + n;
     L.x = L.vec + n;
-    L.last = reinterpret_cast<int*>(L.x + n);
-    L.mk = L.x + 2 * n;
+    L.mk = L.x + n;
     return L;
 }
 FDI double& mband(double* M, int r, int c) { return M[(size_t)r * kMBand + (c - r + kFemKL)]; }
@@ -758,7 +755,7 @@ FDI void copy_vec(const FemDevBody& B, int to, int from) {
 // from device memory: its state vectors U .. Rkm1, nodes, elements and
 // element matrices.  The kernels run on the mirror (one round trip to
 // device memory in, one out) and write the markers and out[] directly.
-__host__ __device__ inline size_t scratch_doubles(int ndof, int nm) { return (size_t)ndof * (kFemBandW + kMBand + 5) + 3 * (size_t)nm; }
+__host__ __device__ inline size_t scratch_doubles(int ndof, int nm) { return (size_t)ndof * (kFemBandW + kMBand + 4) + 3 * (size_t)nm; }
 
 FDI FemDevBody mirror_in(const FemDevBody& G, double* lds, bool mats) {
     FemDevBody B = G;

@@ -35,10 +35,12 @@ template <typename T>
 void launch_bc(const T* src, T* dst, const GridScalars& g, const BCArgs& a, const double* fibm, const double* rho0,
                const double* u0, bool explicit_state, hipStream_t s);
 // Tiled step (lbm_tile.hip): stream-collide and boundaries of a.steps steps
-// in one launch.  The lattice has no immersed bodies, no convective outlet
-// and no pressure corner, has in each direction boundary conditions on both
-// sides or on neither, and is periodic in i if it is in j; tiles are at
-// least 3 sites wide (CI, CJ >= 5).
+// in one launch.  The lattice has in each direction boundary conditions on both
+// sides or on neither, and is periodic in i if it is in j; tiles are at least 3
+// sites wide (CI, CJ >= 5).  Several steps: no immersed bodies, no convective
+// outlet, no pressure corner.  One step (a.one) takes all of them: the force at
+// the support sites of the last spread (or formed here, a.markers), the outlet's
+// mean, the corners' previous velocity.
 constexpr int kTileMaxSteps = 8;
 constexpr int kTileMaxOutlet = 2048;  // rows of a lattice whose convective outlet a tile takes
 // Threads of the outlet-mean kernel, whose tree of sums the FP32-shifted

@@ -1,5 +1,6 @@
 // Tiled lattice step: stream-collide and boundaries of several time steps in
-// one launch, for a lattice without immersed bodies.
+// one launch, for a lattice without immersed bodies, convective outlet or
+// pressure corner, or of one step of any lattice.
 //
 // The plain step is a bulk push kernel and a boundary kernel that wait for
 // each other: two launches of 4-5 us on a small lattice, and one trip of the
