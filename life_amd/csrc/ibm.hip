@@ -358,8 +358,8 @@ __global__ void k_eps_band_prep_batch(const CaseDev* __restrict__ cases, const C
 //  - otherwise the first row of maximum magnitude is found, and the two lanes'
 //    registers change places;
 //  - every lane divides (l = a(i, k) / a(k, k)) and the window's lanes take
-//    l times row k from their own row: columns k+1..k+KB, and up to k+2KB
-//    within KB steps of a swap, past which those columns of row k are zero.
+//    l times row k from their own row: columns k+1..k+KB, and those up to
+//    k+d+KB that a row come up by d has brought in.
 // Rows of U stay in place; half the lanes at a time store theirs and take the
 // rows 64 further on.  The skipped dense operations all involve an exact
 // zero, so the values equal the dense elimination's.
@@ -368,10 +368,14 @@ __global__ void k_eps_band_prep_batch(const CaseDev* __restrict__ cases, const C
 // (readlane, compare, a division of ten operations, product, difference), about
 // 330 cycles a step at KB = 3; the back substitution, with the diagonal's
 // reciprocals formed beforehand, 175.  Columns in lanes and rows in registers,
-// shifted every step, took 950 for both; with swaps at every step 1500 (1030
-// before), which the matrices of markers one spacing apart do not have.
-// 91 markers, KB = 3: 39 us before, 25 us with the staging by four
-// wavefronts.
+// shifted every step, took 950 for both.  A moved row costs its exchange and the
+// columns that it brings in.  Markers one spacing apart, or up to half a per cent
+// less, move none; 2 % less, nearly every second row.  97 rows, before | now: none
+// moved, KB = 3, 45.8 | 28.9 us; 14 % 46.2 | 34.0; 58 % 48.5 | 46.4; KB = 4, 71 %
+// 55.3 | 54.9; 76 % 78.3 | 76.4.  (With the exchange by readlane, all
+// KB further columns for KB steps and divisions in the back substitution 28.1,
+// 42.0, 61.0, 78.2, 131.)  91 markers, KB = 3: 39 us before, 25 us with the staging
+// by four wavefronts.
 
 // Lane `lane`'s value as a wavefront-uniform (SGPR) value.
 __device__ inline double uniform64(double v, int lane) {
@@ -391,7 +395,7 @@ template <int KB, int KBS>
 struct BandRows {
     static constexpr int C = 2 * KB + 1, W = 3 * KBS + 1;
     double w[C], wr;       // this lane's row and its right-hand side
-    bool swapped = false;  // a pivot was not on the diagonal
+    int moved = 0;         // most rows a pivot has come up by
 
     // Row r of the band (zero past n): register j takes column
     // (r - KB) + (j - (r - KB)) mod C.
@@ -423,39 +427,46 @@ struct BandRows {
         y[r] = wr;
     }
 
+    // The rows of lanes a and b change places, each value by one exchange over
+    // the LDS crossbar (all of them in flight together).
     __device__ __forceinline__ void swap_lanes(int L, int a, int b) {
-        auto sw = [&](double& v) {
-            const double va = uniform64(v, a), vb = uniform64(v, b);
-            v = L == a ? vb : (L == b ? va : v);
-        };
+        const int from = L == a ? b : (L == b ? a : L);
 #pragma unroll
-        for (int j = 0; j < C; j++) sw(w[j]);
-        sw(wr);
+        for (int j = 0; j < C; j++) w[j] = __shfl(w[j], from);
+        wr = __shfl(wr, from);
     }
 
     // Step k, column k in register J; window: the lanes of rows k+1..k+KB;
-    // wide: steps left in which row k may reach past column k+KB.
+    // reach: a pivot row, widened by swaps, has no entry past this column or
+    // column k+KB.
     template <int J>
-    __device__ __forceinline__ void step(int k, unsigned long long window, int& wide, int L) {
+    __device__ __forceinline__ void step(int k, unsigned long long window, int& reach, int L) {
         const int a = k & 63;
         const double p0 = uniform64(w[J], a);
         double piv = p0;
-        // also where the whole column is zero (rows past n are zero)
-        if (__builtin_expect((__ballot(fabs(w[J]) >= fabs(p0)) & window) != 0, 0)) {
+        const unsigned long long reached = __ballot(fabs(w[J]) >= fabs(p0)) & window;
+        if (__builtin_expect(reached != 0, 0)) {
+            const unsigned long long above = __ballot(fabs(w[J]) > fabs(p0)) & window;
+            // the first largest, among the rows above the diagonal's magnitude,
+            // in row order (bit d of m: row k + d)
+            unsigned long long m = (above >> a) | (above << ((64 - a) & 63));
             double best = fabs(p0);
             int b = a;
-            for (int r = 1; r <= KB; r++) {
-                const double v = fabs(uniform64(w[J], (k + r) & 63));
-                if (v > best) {
-                    best = v;
-                    b = (k + r) & 63;
+            for (; m; m &= m - 1) {
+                const int lane = (a + __builtin_ctzll(m)) & 63;
+                const double v = uniform64(w[J], lane);
+                if (fabs(v) > best) {
+                    best = fabs(v);
+                    piv = v;
+                    b = lane;
                 }
             }
             if (b != a) {
                 swap_lanes(L, a, b);
-                piv = uniform64(w[J], a);
-                wide = KB + 1;
-                swapped = true;
+                // row k + d has entries up to column k + d + KB
+                const int up = (b - a) & 63;
+                reach = max(reach, k + up + KB);
+                moved = max(moved, up);
             }
             if (piv == 0.0) piv = 1.0;  // zero column: all multipliers 0
         }
@@ -470,38 +481,38 @@ struct BandRows {
             for (int d = 1; d <= KB; d++) w[(J + d) % C] = w[(J + d) % C] - l * p[d];
             wr = wr - l * pr;
         }
-        if (__builtin_expect(wide > 0, 0)) {
-            wide--;
+        if (__builtin_expect(reach > k + KB, 0)) {
 #pragma unroll
-            for (int d = KB + 1; d <= 2 * KB; d++) {
-                const double q = uniform64(w[(J + d) % C], a);
-                if (lane_in(window)) w[(J + d) % C] = w[(J + d) % C] - l * q;
-            }
+            for (int d = KB + 1; d <= 2 * KB; d++)
+                if (d <= reach - k) {
+                    const double q = uniform64(w[(J + d) % C], a);
+                    if (lane_in(window)) w[(J + d) % C] = w[(J + d) % C] - l * q;
+                }
         }
     }
 
     // Steps k .. k+C-1 (FULL) or those of them below kend.
     template <bool FULL, int J = 0>
-    __device__ __forceinline__ void steps(int k, int kend, unsigned long long& window, int& wide, int L) {
+    __device__ __forceinline__ void steps(int k, int kend, unsigned long long& window, int& reach, int L) {
         if constexpr (J < C) {
             if (FULL || k < kend) {
-                step<J>(k, window, wide, L);
+                step<J>(k, window, reach, L);
                 window = (window << 1) | (window >> 63);
-                steps<FULL, J + 1>(k + 1, kend, window, wide, L);
+                steps<FULL, J + 1>(k + 1, kend, window, reach, L);
             }
         }
     }
 };
 
-// One wavefront; true if a row swap was made.
+// One wavefront; returns the most rows a pivot has come up by, which widen U.
 template <int KB, int KBS>
-__device__ __forceinline__ bool band_eliminate(int n, double* __restrict__ B, double* __restrict__ y) {
+__device__ __forceinline__ int band_eliminate(int n, double* __restrict__ B, double* __restrict__ y) {
     constexpr int C = 2 * KB + 1;
     const int L = threadIdx.x;
     BandRows<KB, KBS> s;
     s.load(L, n, B);
     unsigned long long window = ((1ull << KB) - 1) << 1;
-    int wide = 0, saved = 0;
+    int reach = 0, saved = 0;
     for (int k = 0; k < n; k += C) {
         // the half wavefront whose rows are done: a block of C steps and its
         // window stay within the 64 rows from `saved`
@@ -513,12 +524,12 @@ __device__ __forceinline__ bool band_eliminate(int n, double* __restrict__ B, do
             }
             saved += 32;
         }
-        if (k + C <= n) s.template steps<true>(k, n, window, wide, L);
-        else s.template steps<false>(k, n, window, wide, L);
+        if (k + C <= n) s.template steps<true>(k, n, window, reach, L);
+        else s.template steps<false>(k, n, window, reach, L);
     }
     for (int end = saved + 64; saved < end; saved += 32)
         if (L / 32 == (saved / 32) % 2) s.store(saved + L % 32, n, B, y);
-    return s.swapped;
+    return s.moved;
 }
 
 // Between the solve's phases: writes of some lanes, reads by others of the
@@ -545,7 +556,7 @@ __device__ __forceinline__ double div_by(double a, double b, double y) {
 }
 
 // Back substitution by one wavefront (every lane the same), in increasing
-// column order: rows of U of half-bandwidth T = KB, no swap having widened
+// column order: rows of U of half-bandwidth T, KB where no swap has widened
 // them.  Terms past n are 0 * 0, which leaves a sum unchanged.  The
 // reciprocals and the results go into the two sub-diagonal entries that the
 // elimination left unused.  False, with nothing of use written, if a diagonal
@@ -635,10 +646,13 @@ __device__ __forceinline__ void eps_band_solve_impl(int first, int n, double* __
                                                     double* __restrict__ eps) {
     static_assert(KB <= KBS && KB >= 2, "window wider than the stored band, or no sub-diagonal pair");
     if (threadIdx.x >= 64) return;
-    const bool swapped = band_eliminate<KB, KBS>(n, B, y);
+    const int moved = band_eliminate<KB, KBS>(n, B, y);
     band_fence<LDS_>();
-    if (!swapped && band_back_fast<KB, KBS, LDS_>(first, n, B, y, eps)) return;
-    band_back_rows<2 * KB, KBS>(first, n, B, y, eps);
+    bool done;
+    if (moved == 0) done = band_back_fast<KB, KBS, LDS_>(first, n, B, y, eps);
+    else if (moved <= 2) done = band_back_fast<KB + 2, KBS, LDS_>(first, n, B, y, eps);
+    else done = band_back_fast<2 * KB, KBS, LDS_>(first, n, B, y, eps);
+    if (!done) band_back_rows<2 * KB, KBS>(first, n, B, y, eps);
 }
 
 // Largest |column - row| over the non-zero entries of rows [r0, r1) of a
