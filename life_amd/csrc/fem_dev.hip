@@ -567,7 +567,11 @@ constexpr int kBackNodes = 21;   // nodes per wavefront, three lanes each
 // took both neighbours' whole products, the inverse by one lane and three
 // barriers a level, 19 000 now.
 FDI void block_solve_d(const FemDevBody& B, const FemLds& S) {
-    const int tid = threadIdx.x, nt = blockDim.x, lane = tid % 64, wave = tid / 64, waves = nt / 64;
+    int tid = threadIdx.x;
+    // keeps the addresses formed from it here: moved out of the Newton iterations
+    // they take registers over all of them (262 with them, 233 without)
+    asm("" : "+v"(tid));
+    const int nt = blockDim.x, lane = tid % 64, wave = tid / 64, waves = nt / 64;
     const int N = B.nnode, nbc = B.nbc;
     double* blk = S.M;
     {
@@ -902,10 +906,11 @@ FDI void sums_by_last(const FemDevBody* __restrict__ bodies, const FemSumsOut& s
 // those of 85.  11 bodies of 20 to 53 elements: 50 us with 512 lanes, 58 with
 // 256; one of 40: 48 and 47.  Many bodies (the canopy's filaments on the CUs
 // of two XCDs) are bound by issue, not by latency: 104 us and 102, 2 % of the
-// step; hence kFemWideBodies.
+// step; hence kFemWideBodies.  Two wavefronts a SIMD (256 registers): two bodies
+// share a CU (50 elements: 74 KB), and a body its CU with the bulk kernel.
 constexpr int kFemWideBodies = 32;
 template <int NT>
-__global__ __launch_bounds__(NT) void k_fem_dynamic(const FemDevBody* __restrict__ bodies,
+__global__ __launch_bounds__(NT, 2) void k_fem_dynamic(const FemDevBody* __restrict__ bodies,
                                                     const int* __restrict__ list, int redo, FemSumsOut so) {
     extern __shared__ double lds[];
     const FemDevBody* body = bodies + body_index(list);
