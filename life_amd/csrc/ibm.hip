@@ -1223,11 +1223,16 @@ __global__ void k_spread_reduce(MarkerDev m, SpreadScratch sc, double* __restric
 // number, the five passes do not.  The markers of a case lie one after the other
 // along its bodies, so the four of a workgroup are close together and most rounds
 // of 64 meet none of them; a caller's may lie anywhere, and then every round is
-// opened: hence two limits.  Spread alone at 2000, 4000, 6000 and 8192 markers,
-// here | passes: filaments 6.0 | 21.0, 8.5 | 23.3, 11.7 | 26.2, 17.6 | 29.7 us,
-// scattered 8.6 | 20.3, 18.5 | 23.9, 31.6 | 27.9, 51.4 | 32.8.
-constexpr int kScanMaxMarkers = 8192;
-constexpr int kScanMaxScattered = 5000;
+// opened: hence limits of their own.  Spread alone at 2000, 4000, 6000 and 8192
+// markers, here | passes: filaments 6.0 | 21.0, 8.5 | 23.3, 11.7 | 26.2, 17.6 |
+// 29.7 us, scattered 8.6 | 20.3, 18.5 | 23.9, 31.6 | 27.9, 51.4 | 32.8.  Where
+// the coupling keeps to a quarter of the device (few_cus), the comparisons take
+// longer and the passes, atomics most of them, hardly: a step of 4096 x 1040 with
+// filaments, 2904, 4961, 5929 and 7986 markers 123 | 132, 138 | 139, 146 | 143,
+// 174 | 155 us; scattered, spread alone at 1000, 2000 and 3000 markers 7.8 | 15.4,
+// 17.2 | 17.9, 31 | 20.
+constexpr int kScanMaxMarkers = 8192, kScanMaxMarkersFew = 5000;
+constexpr int kScanMaxScattered = 5000, kScanMaxScatteredFew = 2000;
 constexpr int kScanWaves = 4;    // markers per workgroup
 constexpr int kScanGroup = 7;    // neighbours at a time, of kSupp lanes each
 // More overlapping markers than this put more than kMaxPerSite pairs on one
@@ -1530,7 +1535,10 @@ template void launch_interpolate<double>(const double*, const MarkerDev&, const 
 template void launch_interpolate<float>(const float*, const MarkerDev&, const GridScalars&, bool, double*,
                                         const SpreadScratch&, hipStream_t);
 
-bool spread_scans(const MarkerDev& m) { return m.n <= (m.along_bodies ? kScanMaxMarkers : kScanMaxScattered); }
+bool spread_scans(const MarkerDev& m) {
+    if (m.few_cus) return m.n <= (m.along_bodies ? kScanMaxMarkersFew : kScanMaxScatteredFew);
+    return m.n <= (m.along_bodies ? kScanMaxMarkers : kScanMaxScattered);
+}
 
 static unsigned scan_blocks(const MarkerDev& m) { return (unsigned)((m.n + kScanWaves - 1) / kScanWaves); }
 

@@ -116,6 +116,7 @@ void launch_fill_i32(int* p, int v, long long n, hipStream_t s);
 struct MarkerDev {
     int n;
     int along_bodies;  // 1: markers one after the other along their bodies (a case's own)
+    int few_cus;       // 1: their kernels run on a quarter of the device, beside the bulk kernel
     double* pos;       // n*2 (physical)
     double* vel;       // n*2 (physical)
     double* force;     // n*2 (lattice)

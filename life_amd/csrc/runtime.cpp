@@ -1123,6 +1123,7 @@ void grid_split_coupling(life_grid* g, int xcds, int fallback_cus) {
     if (!g->stream_pool) g->stream_pool = g->stream;
     g->stream = cs;
     g->stream2 = bs;
+    g->md.few_cus = 1;
 }
 
 }  // namespace life
@@ -1510,6 +1511,7 @@ int life_ibm_set_markers(life_grid* g, int n, const double* pos, const double* v
         g->nbodies = nbodies;
         MarkerDev& m = g->md;
         m.n = n;
+        m.few_cus = g->stream_pool != nullptr;  // grid_split_coupling
         m.pos = dalloc<double>(2 * (size_t)n);
         m.vel = dalloc<double>(2 * (size_t)n);
         m.force = dalloc<double>(2 * (size_t)n);
