@@ -1227,10 +1227,10 @@ __global__ void k_spread_reduce(MarkerDev m, SpreadScratch sc, double* __restric
 // markers, here | passes: filaments 6.0 | 21.0, 8.5 | 23.3, 11.7 | 26.2, 17.6 |
 // 29.7 us, scattered 8.6 | 20.3, 18.5 | 23.9, 31.6 | 27.9, 51.4 | 32.8.  Where
 // the coupling keeps to a quarter of the device (few_cus), the comparisons take
-// longer and the passes, atomics most of them, hardly: a step of 4096 x 1040 with
-// filaments, 2904, 4961, 5929 and 7986 markers 123 | 132, 138 | 139, 146 | 143,
-// 174 | 155 us; scattered, spread alone at 1000, 2000 and 3000 markers 7.8 | 15.4,
-// 17.2 | 17.9, 31 | 20.
+// longer and the passes, atomics most of them, hardly: in a step of 4096 x 1040,
+// 2420, 4840 and 7744 markers of filaments 14 | 26, 28 | 30, 52 | 36 us of kernels;
+// scattered, spread alone, 1000, 2000 and 3000 markers 7.8 | 15.4, 17.2 | 17.9,
+// 31 | 20.
 constexpr int kScanMaxMarkers = 8192, kScanMaxMarkersFew = 5000;
 constexpr int kScanMaxScattered = 5000, kScanMaxScatteredFew = 2000;
 constexpr int kScanWaves = 4;    // markers per workgroup
