@@ -566,11 +566,12 @@ constexpr int kBackNodes = 21;   // nodes per wavefront, three lanes each
 // one after the other.  41 nodes: 25 000 cycles with nine lanes per node that
 // took both neighbours' whole products, the inverse by one lane and three
 // barriers a level, 19 000 now.
+template <bool SHARED>
 FDI void block_solve_d(const FemDevBody& B, const FemLds& S) {
     int tid = threadIdx.x;
     // keeps the addresses formed from it here: moved out of the Newton iterations
     // they take registers over all of them (262 with them, 233 without)
-    asm("" : "+v"(tid));
+    if constexpr (SHARED) asm("" : "+v"(tid));
     const int nt = blockDim.x, lane = tid % 64, wave = tid / 64, waves = nt / 64;
     const int N = B.nnode, nbc = B.nbc;
     double* blk = S.M;
@@ -701,6 +702,7 @@ FDI void block_solve_d(const FemDevBody& B, const FemLds& S) {
 
 // FemBody::newton_dynamic (FEMBody.cpp:71-87, 112-126) and the residual
 // test of dynamic(): returns resNR (every lane).
+template <bool SHARED>
 FDI double newton_d(const FemDevBody& B, const FemLds& S, const RowPattern& p) {
     const int tid = threadIdx.x, nt = blockDim.x;
     build_global_d(B, S, p);
@@ -733,7 +735,7 @@ FDI double newton_d(const FemDevBody& B, const FemLds& S, const RowPattern& p) {
         S.F[i] = S.R[i] - S.F[i] + s;
     }
     __syncthreads();
-    block_solve_d(B, S);
+    block_solve_d<SHARED>(B, S);
     for (int k = tid; k < nd; k += nt) {
         const double x = S.x[k];
         U[k] = U[k] + x;
@@ -906,11 +908,18 @@ FDI void sums_by_last(const FemDevBody* __restrict__ bodies, const FemSumsOut& s
 // those of 85.  11 bodies of 20 to 53 elements: 50 us with 512 lanes, 58 with
 // 256; one of 40: 48 and 47.  Many bodies (the canopy's filaments on the CUs
 // of two XCDs) are bound by issue, not by latency: 104 us and 102, 2 % of the
-// step; hence kFemWideBodies.  Two wavefronts a SIMD (256 registers): two bodies
-// share a CU (50 elements: 74 KB), and a body its CU with the bulk kernel.
+// step; hence kFemWideBodies.
+// SHARED: two wavefronts a SIMD (256 registers), so that two bodies share a CU (50
+// elements: 74 KB) and a body its CU with the bulk kernel.  Without, the solve's
+// addresses stay in registers over the Newton iterations, and a body has a CU for
+// itself.  Which one: a case has 64 CUs for its bodies (33, 64, 80 and 128 of 50
+// elements, without | shared: 62 | 65, 65 | 68, 120 | 75, 124 | 79 us; 80 of 20: 84 |
+// 54); listed bodies are those of many cases and run beside the bulk kernel (36, 48,
+// 64 and 96 served cases, a step 0.48 | 0.46, 0.53 | 0.52, 0.60 | 0.59, 0.80 | 0.75 ms).
 constexpr int kFemWideBodies = 32;
-template <int NT>
-__global__ __launch_bounds__(NT, 2) void k_fem_dynamic(const FemDevBody* __restrict__ bodies,
+constexpr int kFemOwnCus = 64;
+template <int NT, bool SHARED>
+__global__ __launch_bounds__(NT, SHARED ? 2 : 1) void k_fem_dynamic(const FemDevBody* __restrict__ bodies,
                                                     const int* __restrict__ list, int redo, FemSumsOut so) {
     extern __shared__ double lds[];
     const FemDevBody* body = bodies + body_index(list);
@@ -926,7 +935,7 @@ __global__ __launch_bounds__(NT, 2) void k_fem_dynamic(const FemDevBody* __restr
     int it = 0;
     double res;
     do {
-        res = newton_d(B, S, p);
+        res = newton_d<SHARED>(B, S, p);
         it++;
     } while (res > 1e-10 && it < 20);
     // what only the rest needs is read (again) here, not held in scalar
@@ -1002,9 +1011,11 @@ void launch_fem_dynamic(const FemDevBody* b, const int* list, int nb, size_t lds
     if (nb == 0) return;
     if (so.done && list) throw std::logic_error("device FEM: sums of a listed launch");
     if (max_nel > kFemThreads / 6 && nb <= kFemWideBodies)
-        k_fem_dynamic<512><<<nb, 512, lds, st>>>(b, list, redo ? 1 : 0, so);
+        k_fem_dynamic<512, false><<<nb, 512, lds, st>>>(b, list, redo ? 1 : 0, so);
+    else if (nb <= (list ? kFemWideBodies : kFemOwnCus))
+        k_fem_dynamic<kFemThreads, false><<<nb, kFemThreads, lds, st>>>(b, list, redo ? 1 : 0, so);
     else
-        k_fem_dynamic<kFemThreads><<<nb, kFemThreads, lds, st>>>(b, list, redo ? 1 : 0, so);
+        k_fem_dynamic<kFemThreads, true><<<nb, kFemThreads, lds, st>>>(b, list, redo ? 1 : 0, so);
     LIFE_HIP(hipGetLastError());
 }
 
@@ -1111,8 +1122,8 @@ void fem_dev_create(FemDevCase& fc, const std::vector<const FemBody*>& bodies, c
     if (lds > kFemMaxLds) throw std::runtime_error("flexible body too large for the device FEM");
     fc.lds = lds;
     // dynamic LDS beyond 64 KiB per workgroup
-    for (const void* k : {(const void*)k_fem_predict, (const void*)k_fem_relax, (const void*)k_fem_dynamic<512>,
-                          (const void*)k_fem_dynamic<kFemThreads>})
+    for (const void* k : {(const void*)k_fem_predict, (const void*)k_fem_relax, (const void*)k_fem_dynamic<512, false>,
+                          (const void*)k_fem_dynamic<kFemThreads, false>, (const void*)k_fem_dynamic<kFemThreads, true>})
         LIFE_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFemMaxLds));
     fc.d_bodies = upload_vec(fc, fc.host, st);
     fc.done = dalloc<int>(1);
